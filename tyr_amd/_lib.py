@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -18,18 +19,44 @@ SYMBOLS = (
     "tyr_hip_decode_rope_append", "tyr_hip_rope_fwd", "tyr_hip_layernorm_residual", "tyr_hip_copy", "tyr_hip_mfma_sustain", "tyr_hip_mse_loss_grad_workspace_bytes", "tyr_hip_mse_loss_grad", "tyr_hip_sgd_step",
 )
 
+BINDING_PATH = os.path.join(_HERE, "lib", "_tyr_torch.so")
+
 _lib = None
+
+
+def _require(path: str) -> None:
+    if not os.path.exists(path):
+        raise RuntimeError(
+            f"{path} is missing: build it with `make -C tyr_amd/csrc` "
+            "(or `python -c 'import __graft_entry__ as g; g.build()'`). "
+            "tyr_amd has no CPU or PyTorch fallback.")
+
+
+class _Unbuilt:
+    """Stands for the binding where it is not built yet (the package can be imported then, nothing can be called)."""
+
+    def __getattr__(self, name):
+        _require(BINDING_PATH)
+        _require(LIB_PATH)
+        raise RuntimeError("the libraries were built after tyr_amd was imported: import it again in a new process")
+
+
+def load_binding(error: type):
+    """The native host layer (csrc/torch_binding.cpp), bound to the C ABI of LIB_PATH; it raises ``error``."""
+    if not (os.path.exists(BINDING_PATH) and os.path.exists(LIB_PATH)):
+        return _Unbuilt()
+    spec = importlib.util.spec_from_file_location("_tyr_torch", BINDING_PATH)
+    binding = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(binding)
+    binding.load(LIB_PATH, error)
+    return binding
 
 
 def load() -> ctypes.CDLL:
     global _lib
     if _lib is not None:
         return _lib
-    if not os.path.exists(LIB_PATH):
-        raise RuntimeError(
-            f"{LIB_PATH} is missing: build it with `make -C tyr_amd/csrc` "
-            "(or `python -c 'import __graft_entry__ as g; g.build()'`). "
-            "tyr_amd has no CPU or PyTorch fallback.")
+    _require(LIB_PATH)
     L = ctypes.CDLL(LIB_PATH)
     u64, vp, ci, f32, sz = ctypes.c_uint64, ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_size_t
     L.tyr_hip_strerror.argtypes = [ci]
