@@ -319,6 +319,17 @@ int tyr_hip_gemm_bf16_batched(const void* a, const void* b, void* c, uint64_t ba
                               uint64_t stride_a, uint64_t stride_b, uint64_t stride_c,
                               int trans_b, void* stream);
 
+/* The same products with device scratch.  A product with few output tiles and a long K leaves most of the device idle
+ * unless K is split over workgroups; the f32 partial sums then pass through `workspace` (16-byte aligned device memory of
+ * tyr_hip_gemm_workspace_bytes bytes; a smaller one, or NULL, only means that K is not split).  elem_bytes: 2 = bf16,
+ * 1 = e4m3; 0 bytes = this shape is never split.  Results are reproducible launch to launch either way; splitting sums
+ * K in another order, so the two forms may differ in the last bit of the output. */
+size_t tyr_hip_gemm_workspace_bytes(uint64_t batch, uint64_t M, uint64_t N, uint64_t K, int elem_bytes, int trans_b);
+int tyr_hip_gemm_bf16_batched_ws(const void* a, const void* b, void* c, uint64_t batch,
+                                 uint64_t M, uint64_t N, uint64_t K,
+                                 uint64_t stride_a, uint64_t stride_b, uint64_t stride_c,
+                                 int trans_b, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Test switch (no counterpart in the reference).  The bf16 and fp8 GEMMs have a fast kernel and a
  * general (register-staged) kernel that otherwise serves only shapes whose 256-row panels or whose
  * [K, N] B exceed 32-bit byte offsets.  on != 0 sends every shape through the general kernels,
@@ -365,6 +376,11 @@ int tyr_hip_gemm_fp8_ex(const void* aq, const void* bq, void* c,
                         uint64_t M, uint64_t N, uint64_t K,
                         float scale, const float* row_scale, const float* col_scale, int out_dtype,
                         int trans_b, void* stream);
+/* tyr_hip_gemm_fp8_ex with scratch for split-K partials, as tyr_hip_gemm_bf16_batched_ws. */
+int tyr_hip_gemm_fp8_ws(const void* aq, const void* bq, void* c,
+                        uint64_t M, uint64_t N, uint64_t K,
+                        float scale, const float* row_scale, const float* col_scale, int out_dtype,
+                        int trans_b, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------
  * The element-wise half of the attention train step, fused.

@@ -1,0 +1,86 @@
+"""The small and medium GEMM tiles and their dispatch: sizes around every tile edge, ragged K (a last piece of 16 bytes
+up to 128), one to many pieces per k-group, K split over workgroups, and outputs that must stay inside C."""
+import pytest
+import torch
+
+from oracle import libtorch_path as lt
+from tests.util import rel_fro
+
+pytestmark = pytest.mark.gpu
+TOL_FRO = 1e-2
+
+# (M, N, K): the first extents pick tiles of 16..192 rows and 16..256 columns, one less and one more row than a tile each
+SHAPES = [(1, 16, 16), (1, 272, 2048), (15, 4096, 144), (17, 1040, 4096), (33, 272, 528), (31, 4112, 1040), (64, 48, 80), (65, 1296, 3088),
+          (95, 4096, 2064), (97, 2064, 272), (127, 1024, 4112), (129, 528, 1296), (200, 16, 8192), (3, 512, 8192), (333, 1408, 6608),
+          (255, 6144, 400), (385, 2560, 2048), (1000, 2576, 1024), (1290, 4080, 256), (2050, 1040, 1552)]
+
+
+def worst_line(got, want):
+    """Largest relative error of a row or column (a wrong tile edge would drown in the norm of the whole)."""
+    err, worst = got.float() - want, 0.0
+    for dim in (0, 1):
+        n = want.norm(dim=dim)
+        worst = max(worst, float((err.norm(dim=dim) / n.clamp_min(float(n.mean()))).max()))
+    return worst
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_tiles_match_the_f32_product(M, N, K, trans_b):
+    import tyr_amd
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = (torch.randn(M, K, generator=g, device="cuda") * K ** -0.25).bfloat16()
+    b = (torch.randn(K, N, generator=g, device="cuda") * K ** -0.25).bfloat16()
+    bb = b.t().contiguous() if trans_b else b
+    want = a.float() @ b.float()
+    c = tyr_amd.gemm_bf16(a, bb, trans_b=trans_b)
+    assert rel_fro(c, want) <= 3e-3
+    assert torch.equal(tyr_amd.gemm_bf16(a, bb, trans_b=trans_b), c)
+    assert worst_line(c, want) <= TOL_FRO
+    aq, sa = tyr_amd.quantize_e4m3(a)
+    bq, sb = tyr_amd.quantize_e4m3(b)
+    bqb = bq.t().contiguous() if trans_b else bq
+    want8 = (aq.float() @ bq.float()) * (sa * sb)
+    rs = torch.rand(M, generator=g, device="cuda") + 0.5
+    cs = torch.rand(N, generator=g, device="cuda") + 0.5
+    f = tyr_amd.gemm_fp8_scaled(aq, bqb, rs, cs, scale=sa * sb, trans_b=trans_b)
+    assert rel_fro(f, want8 * rs[:, None] * cs[None, :]) <= 1e-4
+    c8 = tyr_amd.gemm_fp8(aq, bqb, sa, sb, trans_b=trans_b)
+    assert rel_fro(c8, want8) <= 3e-3
+    assert worst_line(c8, want8) <= TOL_FRO
+
+
+def test_every_k_step_of_a_sum_arrives():
+    # operands of ones: each output counts the k it saw (the last products of a tile included)
+    import tyr_amd
+    for M, N in ((16, 64), (40, 1024), (130, 4096), (333, 4096), (640, 2048), (1500, 4096)):
+        for K in (128, 144, 1024, 4096):
+            for trans_b in (False, True):
+                a = torch.ones(M, K, device="cuda").to(torch.float8_e4m3fn)
+                b = torch.ones((N, K) if trans_b else (K, N), device="cuda").to(torch.float8_e4m3fn)
+                c = tyr_amd.gemm_fp8_scaled(a, b, trans_b=trans_b)
+                assert bool((c == K).all()), (M, N, K, trans_b)
+                c = tyr_amd.gemm_bf16(a.bfloat16(), b.bfloat16(), trans_b=trans_b)
+                assert bool((c == K).all()), (M, N, K, trans_b)
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("M,N,K", [(5, 24, 4096), (33, 1032, 264), (100, 8, 6000), (130, 4088, 512)])
+def test_tiles_write_only_c(M, N, K, trans_b):
+    from tyr_amd import _lib
+    lib = _lib.load()
+    a, b = lt.make_inputs(M + N + K, (M, K), (K, N), std=K ** -0.25)
+    ad, bd = a.cuda(), (b.t().contiguous() if trans_b else b).cuda()
+    guard = 4096
+    buf = torch.full((guard + M * N + guard,), -7.0, dtype=torch.bfloat16, device="cuda")
+    need = lib.tyr_hip_gemm_workspace_bytes(1, M, N, K, 2, int(trans_b))
+    ws = torch.full((need // 4 + 64,), 5.0, device="cuda")
+    for w, nbytes in ((ws.data_ptr(), need), (None, 0)):
+        buf.fill_(-7.0)
+        rc = lib.tyr_hip_gemm_bf16_batched_ws(ad.data_ptr(), bd.data_ptr(), buf.data_ptr() + 2 * guard, 1, M, N, K, 0, 0, 0, int(trans_b),
+                                              w, nbytes, 0)
+        assert rc == 0
+        torch.cuda.synchronize()
+        assert bool((buf[:guard] == -7.0).all()) and bool((buf[guard + M * N:] == -7.0).all())
+        assert bool((ws[need // 4:] == 5.0).all())
+        assert rel_fro(buf[guard:guard + M * N].view(M, N).cpu(), a.float() @ b.float()) <= TOL_FRO

@@ -15,7 +15,7 @@ SYMBOLS = (
     "tyr_hip_flash_attn_fwd", "tyr_hip_flash_attn_fwd_gqa", "tyr_hip_flash_attn_bwd_workspace_bytes", "tyr_hip_flash_attn_bwd",
     "tyr_hip_flash_attn_bwd_gqa", "tyr_hip_flash_attn_fwd_mask", "tyr_hip_flash_attn_bwd_mask",
     "tyr_hip_gqa_decode_workspace_bytes", "tyr_hip_gqa_decode_auto_splits",
-    "tyr_hip_gqa_decode", "tyr_hip_gqa_decode_varlen", "tyr_hip_gqa_decode_static", "tyr_hip_gemm_bf16", "tyr_hip_gemm_bf16_batched", "tyr_hip_gemm_force_general", "tyr_hip_flash_attn_fwd_persistent", "tyr_hip_gemm_fp8", "tyr_hip_gemm_fp8_ex",
+    "tyr_hip_gqa_decode", "tyr_hip_gqa_decode_varlen", "tyr_hip_gqa_decode_static", "tyr_hip_gemm_bf16", "tyr_hip_gemm_bf16_batched", "tyr_hip_gemm_bf16_batched_ws", "tyr_hip_gemm_workspace_bytes", "tyr_hip_gemm_force_general", "tyr_hip_flash_attn_fwd_persistent", "tyr_hip_gemm_fp8", "tyr_hip_gemm_fp8_ex", "tyr_hip_gemm_fp8_ws",
     "tyr_hip_decode_rope_append", "tyr_hip_rope_fwd", "tyr_hip_layernorm_residual", "tyr_hip_copy", "tyr_hip_mfma_sustain", "tyr_hip_mse_loss_grad_workspace_bytes", "tyr_hip_mse_loss_grad", "tyr_hip_sgd_step",
 )
 
@@ -96,6 +96,10 @@ def load() -> ctypes.CDLL:
     L.tyr_hip_gemm_bf16.restype = ci
     L.tyr_hip_gemm_bf16_batched.argtypes = [vp, vp, vp, u64, u64, u64, u64, u64, u64, u64, ci, vp]
     L.tyr_hip_gemm_bf16_batched.restype = ci
+    L.tyr_hip_gemm_workspace_bytes.argtypes = [u64] * 4 + [ci, ci]
+    L.tyr_hip_gemm_workspace_bytes.restype = sz
+    L.tyr_hip_gemm_bf16_batched_ws.argtypes = [vp, vp, vp, u64, u64, u64, u64, u64, u64, u64, ci, vp, sz, vp]
+    L.tyr_hip_gemm_bf16_batched_ws.restype = ci
     L.tyr_hip_gemm_force_general.argtypes = [ci]
     L.tyr_hip_gemm_force_general.restype = ci
     L.tyr_hip_flash_attn_fwd_persistent.argtypes = [ci]
@@ -104,6 +108,8 @@ def load() -> ctypes.CDLL:
     L.tyr_hip_gemm_fp8.restype = ci
     L.tyr_hip_gemm_fp8_ex.argtypes = [vp, vp, vp, u64, u64, u64, f32, vp, vp, ci, ci, vp]
     L.tyr_hip_gemm_fp8_ex.restype = ci
+    L.tyr_hip_gemm_fp8_ws.argtypes = [vp, vp, vp, u64, u64, u64, f32, vp, vp, ci, ci, vp, sz, vp]
+    L.tyr_hip_gemm_fp8_ws.restype = ci
     L.tyr_hip_decode_rope_append.argtypes = [vp] * 8 + [u64] * 6 + [vp]
     L.tyr_hip_decode_rope_append.restype = ci
     L.tyr_hip_rope_fwd.argtypes = [vp, vp, vp, vp, u64, u64, u64, u64, ci, vp]

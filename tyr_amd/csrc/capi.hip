@@ -387,12 +387,24 @@ int tyr_hip_gemm_bf16(const void* a, const void* b, void* c, uint64_t M, uint64_
 int tyr_hip_gemm_bf16_batched(const void* a, const void* b, void* c, uint64_t batch, uint64_t M, uint64_t N,
                               uint64_t K, uint64_t stride_a, uint64_t stride_b, uint64_t stride_c, int trans_b,
                               void* stream) {
+    return tyr_hip_gemm_bf16_batched_ws(a, b, c, batch, M, N, K, stride_a, stride_b, stride_c, trans_b, nullptr, 0, stream);
+}
+
+size_t tyr_hip_gemm_workspace_bytes(uint64_t batch, uint64_t M, uint64_t N, uint64_t K, int elem_bytes, int trans_b) {
+    if (batch == 0 || M == 0 || N == 0 || K == 0 || batch > 65535 || !fits_int(M) || !fits_int(N) || !fits_int(K)) return 0;
+    if (elem_bytes != 1 && elem_bytes != 2) return 0;
+    return tyr::gemm_workspace_bytes((int)M, (int)N, (int)K, elem_bytes, trans_b != 0, (int)batch);
+}
+
+int tyr_hip_gemm_bf16_batched_ws(const void* a, const void* b, void* c, uint64_t batch, uint64_t M, uint64_t N,
+                                 uint64_t K, uint64_t stride_a, uint64_t stride_b, uint64_t stride_c, int trans_b,
+                                 void* workspace, size_t workspace_bytes, void* stream) {
     if (!a || !b || !c) return TYR_HIP_ERR_NULL_POINTER;
     if (batch == 0 || M == 0 || N == 0 || K == 0) return TYR_HIP_ERR_BAD_SHAPE;
     if (!fits_int(M) || !fits_int(N) || !fits_int(K) || batch > 65535) return TYR_HIP_ERR_BAD_SHAPE;
     if (((M + 255) / 256) * ((N + 255) / 256) > (uint64_t)INT_MAX) return TYR_HIP_ERR_BAD_SHAPE;
     if (K % 8 != 0 || N % 8 != 0) return TYR_HIP_ERR_UNSUPPORTED;
-    if (!aligned16(a) || !aligned16(b) || !aligned16(c)) return TYR_HIP_ERR_MISALIGNED;
+    if (!aligned16(a) || !aligned16(b) || !aligned16(c) || !aligned16(workspace)) return TYR_HIP_ERR_MISALIGNED;
     if (batch > 1) {
         // every batch entry keeps 16-byte alignment; outputs of different entries must not overlap
         if (stride_a % 8 != 0 || stride_b % 8 != 0 || stride_c % 8 != 0) return TYR_HIP_ERR_MISALIGNED;
@@ -401,8 +413,8 @@ int tyr_hip_gemm_bf16_batched(const void* a, const void* b, void* c, uint64_t ba
             return TYR_HIP_ERR_BAD_SHAPE;
     }
     const int rc = tyr::launch_gemm_bf16(a, b, c, (int)M, (int)N, (int)K, trans_b != 0, (int)batch,
-                                         (int64_t)stride_a, (int64_t)stride_b, (int64_t)stride_c,
-                                         static_cast<hipStream_t>(stream));
+                                         (int64_t)stride_a, (int64_t)stride_b, (int64_t)stride_c, workspace,
+                                         workspace_bytes, static_cast<hipStream_t>(stream));
     return rc == 0 ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }
 
@@ -418,6 +430,12 @@ int tyr_hip_gemm_fp8(const void* aq, const void* bq, void* c, uint64_t M, uint64
 int tyr_hip_gemm_fp8_ex(const void* aq, const void* bq, void* c, uint64_t M, uint64_t N, uint64_t K,
                         float scale, const float* row_scale, const float* col_scale, int out_dtype,
                         int trans_b, void* stream) {
+    return tyr_hip_gemm_fp8_ws(aq, bq, c, M, N, K, scale, row_scale, col_scale, out_dtype, trans_b, nullptr, 0, stream);
+}
+
+int tyr_hip_gemm_fp8_ws(const void* aq, const void* bq, void* c, uint64_t M, uint64_t N, uint64_t K,
+                        float scale, const float* row_scale, const float* col_scale, int out_dtype,
+                        int trans_b, void* workspace, size_t workspace_bytes, void* stream) {
     if (!aq || !bq || !c) return TYR_HIP_ERR_NULL_POINTER;
     if (M == 0 || N == 0 || K == 0) return TYR_HIP_ERR_BAD_SHAPE;
     if (!fits_int(M) || !fits_int(N) || !fits_int(K)) return TYR_HIP_ERR_BAD_SHAPE;
@@ -425,11 +443,11 @@ int tyr_hip_gemm_fp8_ex(const void* aq, const void* bq, void* c, uint64_t M, uin
     if (K % 16 != 0 || N % 16 != 0) return TYR_HIP_ERR_UNSUPPORTED;
     if (out_dtype != TYR_HIP_OUT_BF16 && out_dtype != TYR_HIP_OUT_F32 && out_dtype != TYR_HIP_OUT_E4M3)
         return TYR_HIP_ERR_UNSUPPORTED;
-    if (!aligned16(aq) || !aligned16(bq) || !aligned16(c)) return TYR_HIP_ERR_MISALIGNED;
+    if (!aligned16(aq) || !aligned16(bq) || !aligned16(c) || !aligned16(workspace)) return TYR_HIP_ERR_MISALIGNED;
     if ((row_scale && (reinterpret_cast<uintptr_t>(row_scale) & 3u)) || (col_scale && !aligned16(col_scale)))
         return TYR_HIP_ERR_MISALIGNED;
     const int rc = tyr::launch_gemm_fp8(aq, bq, c, (int)M, (int)N, (int)K, scale, trans_b != 0, row_scale, col_scale,
-                                        out_dtype, static_cast<hipStream_t>(stream));
+                                        out_dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
     return rc == 0 ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }
 

@@ -17,6 +17,7 @@
 //   * The MFMA is issued with the B fragment as its row operand, so every lane ends up with
 //     4 consecutive n for one m and stores 8-byte pieces of a C row.
 #include "common.hpp"
+#include "gemm_tile.hpp"
 #include "launch.hpp"
 
 namespace tyr {
@@ -390,8 +391,15 @@ __global__ __launch_bounds__(gemm2::THREADS, 1) void gemm_bf16_fast_kernel(
                            M - (m0 + wm * 128), N - (n0 + wn * 64));
 }
 
+size_t gemm_workspace_bytes(int M, int N, int K, int elem_bytes, int trans_b, int batch) {
+    if (gemm_general_only() || !gt::offsets_fit(N, K, elem_bytes, trans_b != 0)) return 0;
+    const gt::Plan p = gt::plan(M, N, K, elem_bytes, trans_b != 0, batch, true);
+    return p.splits > 1 ? (size_t)p.splits * batch * M * N * sizeof(float) : 0;
+}
+
 int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K, int trans_b,
-                     int batch, int64_t stride_a, int64_t stride_b, int64_t stride_c, hipStream_t stream) {
+                     int batch, int64_t stride_a, int64_t stride_b, int64_t stride_c, void* workspace, size_t workspace_bytes,
+                     hipStream_t stream) {
     using namespace gemm;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const bool edge = (M % BM) || (N % BN) || (K % BK);
@@ -399,15 +407,22 @@ int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K,
     auto A = static_cast<const uint16_t*>(a);
     auto Bp = static_cast<const uint16_t*>(b);
     auto Cp = static_cast<uint16_t*>(c);
-    // 32-bit buffer offsets: one 256-row panel of A (and of B^T), or all of B, must stay below 4 GiB
-    // The fast kernel needs rows of whole 16-byte chunks; ragged M, N and K are handled by the zero
+    // The tile and 256x256 fast kernels need rows of whole 16-byte chunks; ragged M, N and K are handled by the zero
     // fill of the buffer loads (rows past the end, chunks past K) and by the guarded epilogue (columns
-    // past N only ever contribute to outputs that are not stored).
-    // gemm_general_only() sends every shape to the general kernels, which otherwise only shapes beyond
-    // the 32-bit offsets reach: a switch for tests and for comparing the two paths.
-    const bool general_only = gemm_general_only();
-    const bool fast_ok = !general_only && (K % 8 == 0) && (size_t)256 * K * 2 < ((size_t)1 << 31) &&
-                         (trans_b || (size_t)K * N * 2 < ((size_t)1 << 32));
+    // past N only ever contribute to outputs that are not stored).  Beyond their 32-bit offsets the general kernels serve.
+    // gemm_general_only() sends every shape there: a switch for tests and for comparing the paths.
+    const bool fast_ok = !gemm_general_only() && (K % 8 == 0) && gt::offsets_fit(N, K, 2, trans_b != 0);
+    if (fast_ok) {
+        gt::Plan p = gt::plan(M, N, K, 2, trans_b != 0, batch, workspace != nullptr);
+        if (workspace_bytes < (size_t)(p.splits > 1 ? p.splits : 0) * batch * M * N * sizeof(float))
+            p = gt::plan(M, N, K, 2, trans_b != 0, batch, false);
+        if (p.tile != gt::T256x256) {
+            const GemmEpilogue ep{1.0f, nullptr, nullptr, 0};
+            auto part = static_cast<float*>(workspace);
+            return trans_b ? gt::launch_plan<2, true>(p, a, b, c, M, N, K, part, batch, stride_a, stride_b, stride_c, ep, stream)
+                           : gt::launch_plan<2, false>(p, a, b, c, M, N, K, part, batch, stride_a, stride_b, stride_c, ep, stream);
+        }
+    }
     if (fast_ok) {
 #define TYR_GEMM_FAST(TB, KT)                                                                     \
         do {                                                                                      \

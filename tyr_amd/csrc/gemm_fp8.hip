@@ -14,6 +14,7 @@
 // (further down; every shape whose offsets fit 32 bits takes it) moves slices straight into LDS and runs
 // the same tile with eight waves.
 #include "common.hpp"
+#include "gemm_tile.hpp"
 #include "launch.hpp"
 
 namespace tyr {
@@ -410,7 +411,8 @@ __global__ __launch_bounds__(gemm8f::THREADS, 1) void gemm_fp8_fast_kernel(
 }
 
 int launch_gemm_fp8(const void* aq, const void* bq, void* c, int M, int N, int K, float scale,
-                    int trans_b, const float* row_scale, const float* col_scale, int out_kind, hipStream_t stream) {
+                    int trans_b, const float* row_scale, const float* col_scale, int out_kind, void* workspace,
+                    size_t workspace_bytes, hipStream_t stream) {
     const GemmEpilogue ep{scale, row_scale, col_scale, out_kind};
     using namespace gemm8;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
@@ -419,14 +421,18 @@ int launch_gemm_fp8(const void* aq, const void* bq, void* c, int M, int N, int K
     auto A = static_cast<const uint8_t*>(aq);
     auto Bp = static_cast<const uint8_t*>(bq);
     auto Cp = static_cast<uint16_t*>(c);
-    // 32-bit buffer offsets: a 256-row panel of A (and of B^T), or all of B, must stay below 4 GiB
-    // The fast kernel needs whole K slices; ragged M and N are handled by the zero fill of the
-    // buffer loads and by the guarded epilogue.
-    // gemm_general_only() sends every shape to the general kernels, which otherwise only
-    // shapes beyond the 32-bit offsets reach: a switch for tests and for comparing the two paths.
-    const bool general_only = gemm_general_only();
-    const bool fast_ok = !general_only && (K % 16 == 0) && (size_t)256 * K < ((size_t)1 << 31) &&
-                         (trans_b || (size_t)K * N < ((size_t)1 << 32));
+    // As in launch_gemm_bf16: tiles or 256x256 tiles within the 32-bit offsets, the general kernels beyond them.
+    const bool fast_ok = !gemm_general_only() && (K % 16 == 0) && gt::offsets_fit(N, K, 1, trans_b != 0);
+    if (fast_ok) {
+        gt::Plan p = gt::plan(M, N, K, 1, trans_b != 0, 1, workspace != nullptr);
+        if (workspace_bytes < (size_t)(p.splits > 1 ? p.splits : 0) * M * N * sizeof(float))
+            p = gt::plan(M, N, K, 1, trans_b != 0, 1, false);
+        if (p.tile != gt::T256x256) {
+            auto part = static_cast<float*>(workspace);
+            return trans_b ? gt::launch_plan<1, true>(p, aq, bq, c, M, N, K, part, 1, 0, 0, 0, ep, stream)
+                           : gt::launch_plan<1, false>(p, aq, bq, c, M, N, K, part, 1, 0, 0, 0, ep, stream);
+        }
+    }
     if (fast_ok) {
 #define TYR_GEMM8_FAST(TB, KT)                                                                      \
         do {                                                                                      \

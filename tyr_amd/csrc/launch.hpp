@@ -8,16 +8,20 @@
 namespace tyr {
 
 // `batch` independent products; strides in elements between consecutive batch entries (stride_b = 0
-// uses one B for every entry).
+// uses one B for every entry).  workspace (may be null): device scratch for split-K partials, gemm_workspace_bytes bytes.
 int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K, int trans_b,
-                     int batch, int64_t stride_a, int64_t stride_b, int64_t stride_c, hipStream_t stream);
+                     int batch, int64_t stride_a, int64_t stride_b, int64_t stride_c, void* workspace, size_t workspace_bytes,
+                     hipStream_t stream);
+// Scratch that lets a product with few output tiles and a long K split K over workgroups; 0 = it would not.
+size_t gemm_workspace_bytes(int M, int N, int K, int elem_bytes, int trans_b, int batch);
 // Process-wide switch that sends every GEMM shape through the general (register-staged) kernels.
 // Its initial value is taken once from the environment variable TYR_HIP_GEMM_GENERAL.
 bool gemm_general_only();
 int set_gemm_general_only(int on);   // returns the previous value
 // row_scale [M] / col_scale [N] (device f32, may be null); out_kind 0 = bf16, 1 = f32, 2 = e4m3
 int launch_gemm_fp8(const void* aq, const void* bq, void* c, int M, int N, int K, float scale,
-                    int trans_b, const float* row_scale, const float* col_scale, int out_kind, hipStream_t stream);
+                    int trans_b, const float* row_scale, const float* col_scale, int out_kind, void* workspace,
+                    size_t workspace_bytes, hipStream_t stream);
 // Process-wide choice between persistent forward workgroups (two per CU walking the job ids) and one workgroup per job
 // id.  Its initial value is taken once from the environment variable TYR_HIP_FA_PERSISTENT ("1" = persistent).
 bool flash_attn_fwd_persistent();

@@ -31,7 +31,7 @@ namespace {
     X(tyr_hip_strerror) X(tyr_hip_flash_attn_fwd_gqa) X(tyr_hip_flash_attn_fwd_mask) X(tyr_hip_flash_attn_bwd_workspace_bytes) \
     X(tyr_hip_flash_attn_bwd_gqa) X(tyr_hip_flash_attn_bwd_mask) X(tyr_hip_gqa_decode_workspace_bytes)                        \
     X(tyr_hip_gqa_decode_varlen) X(tyr_hip_decode_rope_append) X(tyr_hip_rope_fwd) X(tyr_hip_layernorm_residual)             \
-    X(tyr_hip_copy) X(tyr_hip_gemm_bf16) X(tyr_hip_gemm_bf16_batched) X(tyr_hip_gemm_fp8_ex)                                  \
+    X(tyr_hip_copy) X(tyr_hip_gemm_workspace_bytes) X(tyr_hip_gemm_bf16_batched_ws) X(tyr_hip_gemm_fp8_ws)                    \
     X(tyr_hip_mse_loss_grad_workspace_bytes) X(tyr_hip_mse_loss_grad) X(tyr_hip_sgd_step)
 struct Api {
 #define X(f) decltype(&::f) f = nullptr;
@@ -321,6 +321,17 @@ Extents extents(const at::Tensor& a, const at::Tensor& b, bool trans_b) {
     return {M, N, K};
 }
 
+// scratch for split-K partials, where the library splits this product
+struct Partials {
+    size_t bytes;
+    at::Tensor block;
+    Partials(int64_t batch, const Extents& e, int elem_bytes, bool trans_b, const at::Tensor& like)
+        : bytes(api.tyr_hip_gemm_workspace_bytes(batch, e.M, e.N, e.K, elem_bytes, trans_b)) {
+        if (bytes) block = scratch(bytes, like);
+    }
+    void* ptr() const { return bytes ? block.data_ptr() : nullptr; }
+};
+
 // (a, b, trans_b)
 PyObject* gemm_bf16(PyObject* const* a) {
     const at::Tensor &x = checked(a[0], "a", at::kBFloat16, 2), &y = checked(a[1], "b", at::kBFloat16, 2);
@@ -331,7 +342,9 @@ PyObject* gemm_bf16(PyObject* const* a) {
     {
         NoGil nogil;
         c = empty({e.M, e.N}, at::kBFloat16, x);
-        rc = api.tyr_hip_gemm_bf16(x.data_ptr(), y.data_ptr(), c.data_ptr(), e.M, e.N, e.K, trans_b, stream());
+        const Partials ws(1, e, 2, trans_b, x);
+        rc = api.tyr_hip_gemm_bf16_batched_ws(x.data_ptr(), y.data_ptr(), c.data_ptr(), 1, e.M, e.N, e.K, 0, 0, 0, trans_b, ws.ptr(),
+                                              ws.bytes, stream());
     }
     check_status(rc, "gemmBf16");
     return wrap(std::move(c));
@@ -355,8 +368,9 @@ PyObject* matmul_bf16(PyObject* const* a) {
     {
         NoGil nogil;
         c = empty(sizes, at::kBFloat16, x);
-        rc = api.tyr_hip_gemm_bf16_batched(x.data_ptr(), y.data_ptr(), c.data_ptr(), batch, e.M, e.N, e.K, e.M * e.K,
-                                           y.dim() == 2 ? 0 : e.K * e.N, e.M * e.N, trans_b, stream());
+        const Partials ws(batch, e, 2, trans_b, x);
+        rc = api.tyr_hip_gemm_bf16_batched_ws(x.data_ptr(), y.data_ptr(), c.data_ptr(), batch, e.M, e.N, e.K, e.M * e.K,
+                                              y.dim() == 2 ? 0 : e.K * e.N, e.M * e.N, trans_b, ws.ptr(), ws.bytes, stream());
     }
     check_status(rc, "matmul");
     return wrap(std::move(c));
@@ -385,7 +399,9 @@ PyObject* fp8(PyObject* pa, PyObject* pb, float scale, PyObject* row, PyObject* 
     {
         NoGil nogil;
         c = empty({e.M, e.N}, out, x);
-        rc = api.tyr_hip_gemm_fp8_ex(x.data_ptr(), y.data_ptr(), c.data_ptr(), e.M, e.N, e.K, scale, rs, cs, kind, trans_b, stream());
+        const Partials ws(1, e, 1, trans_b, x);
+        rc = api.tyr_hip_gemm_fp8_ws(x.data_ptr(), y.data_ptr(), c.data_ptr(), e.M, e.N, e.K, scale, rs, cs, kind, trans_b, ws.ptr(),
+                                     ws.bytes, stream());
     }
     check_status(rc, what);
     return wrap(std::move(c));
