@@ -286,4 +286,60 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t pid, uint32_t n) {
     return (pid % 8u) * (n / 8u) + pid / 8u;
 }
 
+// ---- order of the query tiles of an attention launch ---------------------------------------------------------
+// A launch has one job per (query head, tile rank); rank 0 is the longest causal tile.  Consecutive workgroup ids go to the
+// 8 XCDs in turn, and of the ids an XCD gets, id i and id i + 32 share a CU (two workgroups fit).
+//   paired (causal, many jobs): a job is the tiles ntq-1-rank and rank one after the other, so all jobs are equal; group
+//     by group, so that the jobs that share a K / V run together.
+//   single (few jobs): one tile per job, longest first -- and the first 32 of an XCD in ascending order, so that the
+//     second workgroup of a CU is the longer the shorter its first one is.
+// With grouped queries the unit dealt to an XCD is a (batch, kv head) group, whose G heads share one K / V.
+struct AttnOrder {
+    int BH, Hq, G, ntr, single;                      // ntr = ranks per head
+    __device__ __forceinline__ void decode(int id, int& bh, int& rank, int& kvbh) const {
+        const int ngroups = BH / G, hkv = Hq / G;
+        if ((ngroups & 7) == 0) {
+            const int xcd = id & 7, heads = BH >> 3;
+            int slot = id >> 3, head;
+            if (single) {
+                if (slot < 32 && heads * ntr > 32) slot = 31 - slot;
+                rank = slot / heads;
+                const int r = slot % heads;
+                kvbh = (r / G) * 8 + xcd;
+                head = r % G;
+            } else {
+                const int per_group = G * ntr, within = slot % per_group;
+                kvbh = (slot / per_group) * 8 + xcd;
+                rank = within / G;
+                head = within % G;
+            }
+            bh = (kvbh / hkv) * Hq + (kvbh % hkv) * G + head;
+        } else {
+            if (single) {
+                if (id < 256 && BH * ntr > 256) id = 255 - id;
+                rank = id / BH;
+                bh = id % BH;
+            } else {
+                bh = id / ntr;
+                rank = id % ntr;
+            }
+            kvbh = (bh / Hq) * hkv + (bh % Hq) / G;
+        }
+    }
+};
+// Paired or single tiles for a causal launch, by the time the busiest of 256 CUs needs: tile t of a head walks 2 (t + 1)
+// 64-key steps and costs about 2.6 steps more for its start and end (1 more as the second tile of a pair).
+inline bool attn_single_tiles(int64_t bh, int ntq) {
+    const int64_t pairs = bh * ((ntq + 1) / 2), singles = bh * ntq;
+    const double pair_work = 2.0 * (ntq + 1) + 3.6, longest = 2.0 * ntq + 2.6, total = (double)bh * ntq * (ntq + 1 + 2.6);
+    const double paired = (double)((pairs + 255) / 256) * pair_work;
+    // up to 256 jobs run alone; beyond, the longest-first order leaves about half a mean job of imbalance
+    double single = longest;
+    if (singles > 256) {
+        single = total / 256 + 0.5 * (ntq + 1 + 2.6);
+        if (single < longest) single = longest;
+    }
+    return single < 0.95 * paired;
+}
+
 }  // namespace tyr

@@ -126,7 +126,7 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
     uint16_t* __restrict__ dQ, float2* __restrict__ stats, int BH, int N, int ntq, float scale,
     float scale_log2, int Hq, int G, int window, const int* __restrict__ kv_lens,
-    const uint8_t* __restrict__ key_mask, int pair) {
+    const uint8_t* __restrict__ key_mask, int pair, int single) {
     using namespace fab;
     using C = CfgQ<D>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -135,27 +135,9 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
     const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int r = lane & 31, g = lane >> 5;
 
-    // With `pair` (causal) a workgroup handles query tile ntq-1-tr and then tile tr (equal work
-    // for every workgroup, half as many of them).
-    const int ntr = pair ? (ntq + 1) / 2 : ntq;
+    // With `pair` (causal) a workgroup handles query tile ntq-1-tr and then tile tr.
     int bh, tr, kvbh;
-    {
-        const int id = blockIdx.x;
-        const int ngroups = BH / G;              // B * Hkv: the unit dealt to an XCD shares one K / V
-        if ((ngroups & 7) == 0) {
-            const int xcd = id & 7, slot = id >> 3;
-            const int per_group = G * ntr;
-            kvbh = (slot / per_group) * 8 + xcd;
-            const int within = slot % per_group;
-            tr = within / G;
-            const int hkv = Hq / G;
-            bh = (kvbh / hkv) * Hq + (kvbh % hkv) * G + within % G;
-        } else {
-            bh = id / ntr;
-            tr = id % ntr;
-            kvbh = (bh / Hq) * (Hq / G) + (bh % Hq) / G;
-        }
-    }
+    AttnOrder{BH, Hq, G, pair ? (ntq + 1) / 2 : ntq, single}.decode(blockIdx.x, bh, tr, kvbh);
     const int npass = (pair && ntq - 1 - tr != tr) ? 2 : 1;
     for (int pass = 0; pass < npass; ++pass) {
     const int qt = CAUSAL ? (pass == 0 ? ntq - 1 - tr : tr) : tr;
@@ -765,7 +747,9 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     const int ntq = (N + 127) / 128;
     const int npad = ntq * 128;
     const bool ext = window > 0 || kv_lens != nullptr || key_mask != nullptr;
-    const int pair = (causal && window <= 0 && ntq > 1) ? 1 : 0;   // lengths and key masks keep tile 0 starting at key 0
+    // lengths and key masks keep tile 0 starting at key 0; a window makes the tiles equal
+    const int single = (causal && window <= 0 && ntq > 1 && attn_single_tiles(BH, ntq)) ? 1 : 0;
+    const int pair = (causal && window <= 0 && ntq > 1 && !single) ? 1 : 0;
     dim3 grid_q((unsigned)(BH * (pair ? (ntq + 1) / 2 : ntq))), grid_k((unsigned)(BHkv * ntq)), block(THREADS);
     const float scale_log2 = scale * LOG2E;
     auto Qp = static_cast<const uint16_t*>(q);
@@ -785,7 +769,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
         if (a1 != hipSuccess || a2 != hipSuccess) return -1;                                          \
         hipLaunchKernelGGL((flash_attn_bwd_dq_kernel<DD, CC, EE>), grid_q, block, CfgQ<DD>::LDS, stream, \
                            Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st, BH, N, ntq,      \
-                           scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair);                \
+                           scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single);                \
         hipLaunchKernelGGL((flash_attn_bwd_dkv_kernel<DD, CC, EE>), grid_k, block, CfgK<DD>::LDS, stream, \
                            Qp, Kp, Vp, dOp, st, static_cast<uint16_t*>(dk),                           \
                            static_cast<uint16_t*>(dv), BHkv, N, ntq, npad, scale, scale_log2, Hq, G,  \

@@ -75,7 +75,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     uint16_t* __restrict__ O, float* __restrict__ LSE, int BH, int N, int ntq, float scale_log2,
     int Hq, int G, int window, const int* __restrict__ kv_lens, const uint8_t* __restrict__ key_mask, int pair,
-    int total_ids) {
+    int single, int total_ids) {
     using namespace fa;
     using C = Cfg<D>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -84,35 +84,14 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     const int lane = t & 63, w = t >> 6;
     const int r = lane & 31, g = lane >> 5;
 
-    // workgroup -> (head, query tile).  Heads are dealt to the 8 XCDs so that all query tiles of a
-    // head run on one XCD (shared K/V in its L2); within a head the longest (last) causal tiles
-    // are issued first.
-    // With grouped queries (G > 1) the unit dealt to an XCD is a (batch, kv head) group: its G
-    // query heads times ntq tiles share one K/V; the G heads of a tile are adjacent.
-    // With `pair` (causal) a workgroup handles query tile ntq-1-tr and then tile tr: every
-    // workgroup does the same amount of work and there are half as many of them to start.
+    // workgroup -> (head, query tile): AttnOrder.
     // A launch has either one workgroup per job id, or (persistent launch) two workgroups per CU, of which workgroup p
     // walks the job ids p, p + gridDim.x, ... (the host makes gridDim.x a multiple of 8 then, so with the XCD mapping
-    // above all of them belong to its XCD).  The hand-over from a job's last tile to the next job's first one is the
+    // of AttnOrder all of them belong to its XCD).  The hand-over from a job's last tile to the next job's first one is the
     // hand-over between the two tiles of a pair: the next tile's K(0), K(1) and Q are requested under the end of the
     // current one.
-    const int ntr = pair ? (ntq + 1) / 2 : ntq;  // tile ranks per head
-    auto decode = [&](int id, int& bh_, int& tr_, int& kvbh_) {
-        const int ngroups = BH / G;              // B * Hkv
-        if ((ngroups & 7) == 0) {
-            const int xcd = id & 7, slot = id >> 3;
-            const int per_group = G * ntr;
-            kvbh_ = (slot / per_group) * 8 + xcd;
-            const int within = slot % per_group;
-            tr_ = within / G;
-            const int hkv = Hq / G;
-            bh_ = (kvbh_ / hkv) * Hq + (kvbh_ % hkv) * G + within % G;
-        } else {
-            bh_ = id / ntr;
-            tr_ = id % ntr;
-            kvbh_ = (bh_ / Hq) * (Hq / G) + (bh_ % Hq) / G;
-        }
-    };
+    const AttnOrder order{BH, Hq, G, pair ? (ntq + 1) / 2 : ntq, single};
+    auto decode = [&](int id, int& bh_, int& tr_, int& kvbh_) { order.decode(id, bh_, tr_, kvbh_); };
     bf16x8 qf[C::KSTEPS];                        // Q^T fragments: lane holds row qw0+r, columns 16i + 8g + [0,8)
     bool preloaded = false;                      // this tile's K(0), K(1) and Q were requested by the previous one
     for (int id = blockIdx.x; id < total_ids; id += gridDim.x) {
@@ -452,7 +431,9 @@ int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, 
     const int G = Hq / Hkv;
     const int ntq = (N + BM - 1) / BM;
     const bool ext = window > 0 || kv_lens != nullptr || key_mask != nullptr;
-    const int pair = (causal && window <= 0 && ntq > 1) ? 1 : 0;   // lengths and key masks keep tile 0 starting at key 0
+    // lengths and key masks keep tile 0 starting at key 0; a window makes the tiles equal
+    const int single = (causal && window <= 0 && ntq > 1 && attn_single_tiles(BH, ntq)) ? 1 : 0;
+    const int pair = (causal && window <= 0 && ntq > 1 && !single) ? 1 : 0;
     const int total_ids = BH * (pair ? (ntq + 1) / 2 : ntq);
     // One workgroup per job id, or persistent workgroups: two per CU (what registers and 64 KB of LDS at D = 128 allow),
     // rounded down to a multiple of 8 so that a workgroup's job ids stay on one XCD, and never fewer than 8.
@@ -484,7 +465,7 @@ int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, 
             hipFuncAttributeMaxDynamicSharedMemorySize, Cfg<DD>::LDS);                           \
         if (attr != hipSuccess) return -1;                                                       \
         hipLaunchKernelGGL((flash_attn_fwd_kernel<DD, CC, EE>), grid, block, Cfg<DD>::LDS, stream, \
-                           Qp, Kp, Vp, Op, lse, BH, N, ntq, scale_log2, Hq, G, window, kv_lens, key_mask, pair, total_ids); \
+                           Qp, Kp, Vp, Op, lse, BH, N, ntq, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single, total_ids); \
     } while (0)
 #define TYR_FA_PICK(DD)                                                                          \
     do {                                                                                         \
