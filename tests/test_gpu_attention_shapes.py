@@ -1,0 +1,61 @@
+"""The forms an attention launch can take (paired query tiles, single ones, 64-row tiles whose keys two waves share) and the
+backward's dK / dV cut into parts: head counts and lengths on both sides of where the choice changes, with every mask."""
+import math
+
+import pytest
+import torch
+
+from tests.util import rel_fro
+
+pytestmark = pytest.mark.gpu
+
+# (B, Hq, Hkv, N, D): few heads with short and long rows, part of a tile in the last one, more heads than CUs
+SHAPES = [(1, 1, 1, 65, 128), (1, 4, 4, 191, 64), (2, 4, 1, 257, 128), (1, 8, 2, 1000, 128), (1, 16, 16, 1025, 64), (3, 8, 4, 577, 128),
+          (4, 16, 16, 700, 128), (2, 32, 8, 449, 64), (8, 32, 8, 300, 128), (1, 4, 1, 3001, 128)]
+
+
+def reference(q, k, v, g, visible):
+    """f32 attention and its gradients; visible [B, 1, N, N]."""
+    B, Hq, N, D = q.shape
+    rep = Hq // k.shape[1]
+    q, k, v = (t.float().requires_grad_() for t in (q, k, v))
+    kk, vv = k.repeat_interleave(rep, 1), v.repeat_interleave(rep, 1)
+    s = (torch.matmul(q, kk.transpose(-1, -2).contiguous()) / math.sqrt(D)).masked_fill(~visible, float("-inf"))
+    lse = torch.logsumexp(s, -1)
+    p = torch.exp(s - lse.masked_fill(lse == float("-inf"), 0.0)[..., None])
+    o = torch.matmul(p, vv)
+    return (o.detach(), lse.detach(), *torch.autograd.grad(o, (q, k, v), g.float()))
+
+
+@pytest.mark.parametrize("mask", ["causal", "full", "window", "lens", "keys"])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", SHAPES)
+def test_every_launch_form_matches_the_f32_reference(B, Hq, Hkv, N, D, mask):
+    import tyr_amd
+    if mask == "keys" and N > 2000:
+        pytest.skip("the reference would not fit the time of a small test")
+    gen = torch.Generator(device="cuda").manual_seed(B + Hq + N)
+    q, k, v, g = (torch.randn(B, h, N, D, device="cuda", generator=gen).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    i = torch.arange(N, device="cuda")
+    visible = (i[None, :] <= i[:, None] if mask != "full" else torch.ones(N, N, dtype=torch.bool, device="cuda"))[None, None].expand(B, 1, N, N)
+    opt = dict(causal=mask != "full")
+    if mask == "window":
+        opt["window"] = N // 3 + 1
+        visible = visible & (i[:, None] - i[None, :] < opt["window"])
+    if mask == "lens":
+        opt["kv_lens"] = torch.tensor([N - b * (N // (2 * B)) for b in range(B)], dtype=torch.int32, device="cuda")
+        visible = visible & (i[None, None, None, :] < opt["kv_lens"][:, None, None, None])
+    if mask == "keys":
+        opt["key_mask"] = torch.rand(B, N, device="cuda", generator=gen) > 0.3
+        opt["key_mask"][:, 0] = True
+        visible = visible & opt["key_mask"][:, None, None, :]
+    o, lse = tyr_amd.flash_attn_fwd(q, k, v, **opt)
+    grads = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)
+    want_o, want_lse, *want = reference(q, k, v, g, visible)
+    assert float((o.float() - want_o).abs().max()) <= 2e-2 and float((lse - want_lse).abs().max()) <= 2e-2
+    for got, ref in zip(grads, want):
+        assert rel_fro(got, ref) <= 1e-2
+        # a row lost at the edge of a tile or part would drown in the norm of the whole
+        err, n = (got.float() - ref).norm(dim=-1), ref.norm(dim=-1)
+        assert float((err / n.clamp_min(float(n[n > 0].mean()))).max()) <= 4e-2
+    again = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)
+    assert all(torch.equal(a, b) for a, b in zip(grads, again))

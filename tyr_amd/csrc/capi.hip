@@ -206,6 +206,14 @@ size_t tyr_hip_flash_attn_bwd_workspace_bytes(uint64_t B, uint64_t H, uint64_t N
     return tyr::flash_attn_bwd_workspace_bytes((int)B, (int)H, (int)N);
 }
 
+size_t tyr_hip_flash_attn_bwd_full_workspace_bytes(uint64_t B, uint64_t Hq, uint64_t Hkv, uint64_t N, uint64_t D, int causal,
+                                                   uint64_t window) {
+    if (B == 0 || Hq == 0 || Hkv == 0 || N == 0 || Hq % Hkv != 0 || (D != 64 && D != 128)) return 0;
+    if (!fits_int(N) || !fits_int(B * Hq) || B * Hq > (uint64_t)INT_MAX / ((N + 127) / 128)) return 0;
+    return tyr::flash_attn_bwd_full_workspace_bytes((int)B, (int)Hq, (int)Hkv, (int)N, (int)D, causal != 0,
+                                                    (int)(window > (uint64_t)INT_MAX ? INT_MAX : window));
+}
+
 int tyr_hip_flash_attn_bwd(const void* q, const void* k, const void* v, const void* o,
                            const void* d_o, const float* lse, void* dq, void* dk, void* dv,
                            uint64_t B, uint64_t H, uint64_t N, uint64_t D, int causal, float scale,
@@ -239,7 +247,7 @@ static int attn_bwd_checked(const void* q, const void* k, const void* v, const v
     const int rc = tyr::launch_flash_attn_bwd(q, k, v, o, d_o, lse, dq, dk, dv, (int)B, (int)Hq, (int)Hkv, (int)N,
                                               (int)D, causal != 0,
                                               (int)(window > (uint64_t)INT_MAX ? INT_MAX : window), kv_lens, key_mask,
-                                              scale, workspace, static_cast<hipStream_t>(stream));
+                                              scale, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
     return rc == 0 ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }
 

@@ -327,19 +327,9 @@ struct AttnOrder {
         }
     }
 };
-// Paired or single tiles for a causal launch, by the time the busiest of 256 CUs needs: tile t of a head walks 2 (t + 1)
-// 64-key steps and costs about 2.6 steps more for its start and end (1 more as the second tile of a pair).
-inline bool attn_single_tiles(int64_t bh, int ntq) {
-    const int64_t pairs = bh * ((ntq + 1) / 2), singles = bh * ntq;
-    const double pair_work = 2.0 * (ntq + 1) + 3.6, longest = 2.0 * ntq + 2.6, total = (double)bh * ntq * (ntq + 1 + 2.6);
-    const double paired = (double)((pairs + 255) / 256) * pair_work;
-    // up to 256 jobs run alone; beyond, the longest-first order leaves about half a mean job of imbalance
-    double single = longest;
-    if (singles > 256) {
-        single = total / 256 + 0.5 * (ntq + 1 + 2.6);
-        if (single < longest) single = longest;
-    }
-    return single < 0.95 * paired;
-}
+// What one job of a launch is: `rows` query rows (128, or 64 with the keys of every tile shared by two waves), and for
+// causal launches paired tiles or single ones.
+struct AttnShape { int rows, pair, single; };
+AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window);
 
 }  // namespace tyr

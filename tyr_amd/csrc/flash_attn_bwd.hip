@@ -36,7 +36,11 @@
 // conflict-free both for row fragments (16-byte reads, lane = row) and for transposed fragments
 // (ds_read_b64_tr_b16 over 4 rows x 64 bytes per lane-group pair).
 #include <limits.h>
+
+#include <algorithm>
+#include <functional>
 #include <type_traits>
+#include <vector>
 
 #include "common.hpp"
 #include "launch.hpp"
@@ -119,21 +123,25 @@ __device__ __forceinline__ void store_transposed_bf16(const f32x16 (&acc)[D / 32
 // ------------------------------------------------------------------------------------------
 // dQ (and the (lse2, delta) pairs)
 // EXT adds the per-sequence key length and the sliding window (same rule as the forward kernel);
-// G = query heads per kv head.
-template <int D, bool CAUSAL, bool EXT>
+// G = query heads per kv head.  SPLIT: 64 query rows per workgroup, the two 32-key sub-tiles of a tile on two waves whose
+// dQ are added through LDS at the end (same use as in the forward kernel: launches with few tiles).
+template <int D, bool CAUSAL, bool EXT, bool SPLIT>
 __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
-    uint16_t* __restrict__ dQ, float2* __restrict__ stats, int BH, int N, int ntq, float scale,
+    uint16_t* __restrict__ dQ, float2* __restrict__ stats, int BH, int N, int ntq, int npad, float scale,
     float scale_log2, int Hq, int G, int window, const int* __restrict__ kv_lens,
     const uint8_t* __restrict__ key_mask, int pair, int single) {
     using namespace fab;
     using C = CfgQ<D>;
+    constexpr int TBM = SPLIT ? 64 : C::BM;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
     const int t = threadIdx.x;
     const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int r = lane & 31, g = lane >> 5;
+    const int wr = SPLIT ? w & 1 : w;            // which 32 rows of the tile
+    const int T0 = SPLIT ? w >> 1 : 0;           // SPLIT: the one sub-tile of this wave
 
     // With `pair` (causal) a workgroup handles query tile ntq-1-tr and then tile tr.
     int bh, tr, kvbh;
@@ -141,14 +149,14 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
     const int npass = (pair && ntq - 1 - tr != tr) ? 2 : 1;
     for (int pass = 0; pass < npass; ++pass) {
     const int qt = CAUSAL ? (pass == 0 ? ntq - 1 - tr : tr) : tr;
-    const int q0 = qt * C::BM;
-    const int qw0 = q0 + w * 32;
+    const int q0 = qt * TBM;
+    const int qw0 = q0 + wr * 32;
     const size_t head_off = (size_t)bh * N * D;
     const uint16_t* Kh = Kp + (size_t)kvbh * N * D;
     const uint16_t* Vh = Vp + (size_t)kvbh * N * D;
     const int Nk = (EXT && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / Hq])) : N;
     const uint8_t* km = (EXT && key_mask != nullptr) ? key_mask + (size_t)(bh / Hq) * N : nullptr;
-    const int kv_end = CAUSAL ? min(Nk, q0 + C::BM) : Nk;
+    const int kv_end = CAUSAL ? min(Nk, q0 + TBM) : Nk;
     const int nkv_abs = max(1, (kv_end + C::BN - 1) / C::BN);   // a sequence without keys still walks one (fully masked) tile
     const int jbase = (EXT && window > 0) ? min(max(0, q0 - window + 1) / C::BN, nkv_abs - 1) : 0;
     const int nkv = nkv_abs - jbase;             // tiles are numbered from jbase below
@@ -173,8 +181,7 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
         delta = part + xor32(part);
         lse2 = LSE[(size_t)bh * N + qrow] * LOG2E;
         if (EXT && lse2 == -INFINITY) lse2 = INFINITY;      // a row that saw no key: every probability is 0
-        if (g == 0) {
-            const size_t npad = (size_t)ntq * C::BM;
+        if (g == 0 && T0 == 0) {
             stats[(size_t)bh * npad + qpos] = qpos < N ? make_float2(lse2, delta) : make_float2(INFINITY, 0.0f);
         }
     }
@@ -235,7 +242,7 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
         const int j0 = (jbase + j) * C::BN;
         if (j + 1 < nkv) issue_kv((j + 1) & 1, j0 + C::BN);
         if (j < nkv_w) {
-            const unsigned char* Kt = lds + (j & 1) * C::TILE;
+            const unsigned char* Kt = lds + (j & 1) * C::TILE + (SPLIT ? T0 * 32 * C::ROW : 0);
             const unsigned char* Vt = Kt + C::V_BASE;
             // The two 32-row sub-tiles of the tile are taken one after the other (scores, probabilities, dQ
             // products): only one sub-tile's scores are live, which leaves the registers the fragment read-ahead
@@ -283,8 +290,8 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
                 if (need_mask) {
                     const int lim = CAUSAL ? min(qpos, Nk - 1) : Nk - 1;
                     const int low = (EXT && window > 0) ? qpos - window + 1 : INT_MIN;
-                    const int base = j0 + 4 * g;
-                    const uint64_t hidden = tile_hidden >> (4 * g + 32 * T);      // shifted to this lane's rows
+                    const int base = j0 + 32 * T0 + 4 * g;
+                    const uint64_t hidden = tile_hidden >> (4 * g + 32 * (T0 + T));      // shifted to this lane's rows
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
                         const int kv = base + 32 * T + 8 * (e >> 2) + (e & 3);
@@ -311,27 +318,59 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
                 for (int n = 0; n < 2 * C::DT; ++n) {
                     const int c = 2 * T + n / C::DT, dt = n % C::DT;
                     if (n + 1 < 2 * C::DT) read_transposed(T, n + 1, (n + 1) & 1);
-                    else if (T == 0) read_rows(1, 0, 0);         // first fragments of the second sub-tile's scores
+                    else if (T == 0 && !SPLIT) read_rows(1, 0, 0);   // first fragments of the second sub-tile's scores
                     __builtin_amdgcn_sched_barrier(0);
                     const bf16x8 kt = __builtin_shufflevector(lo[n & 1], hi[n & 1], 0, 1, 2, 3, 4, 5, 6, 7);
                     dq[dt] = mfma_32x32x16_bf16(kt, dsf[c], dq[dt]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             };
-            read_rows(0, 0, 0);
-            scores(0);
-            probabilities(0);
-            accumulate(0);
-            scores(1);
-            probabilities(1);
-            accumulate(1);
+            if constexpr (SPLIT) {
+                // one sub-tile per wave: register arrays are indexed as sub-tile 0, addresses and masks are of sub-tile T0
+                read_rows(0, 0, 0);
+                scores(0);
+                probabilities(0);
+                accumulate(0);
+            } else {
+                read_rows(0, 0, 0);
+                scores(0);
+                probabilities(0);
+                accumulate(0);
+                scores(1);
+                probabilities(1);
+                accumulate(1);
+            }
         }
         wait_vmcnt0();
         __syncthreads();
     }
 
-    store_transposed_bf16<D>(dq, scale, lds + w * (32 * (D * 2 + 16)), dQ + head_off + (size_t)qw0 * D,
-                             N - qw0, lane);
+    if constexpr (SPLIT) {
+        f32x4* other = reinterpret_cast<f32x4*>(lds) + wr * (C::DT * 4 * 64) + lane;
+        if (w >= 2) {
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4)
+                    other[(dt * 4 + q4) * 64] = f32x4{dq[dt][4 * q4], dq[dt][4 * q4 + 1], dq[dt][4 * q4 + 2], dq[dt][4 * q4 + 3]};
+        }
+        __syncthreads();
+        if (w < 2) {
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    const f32x4 o = other[(dt * 4 + q4) * 64];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) dq[dt][4 * q4 + x] += o[x];
+                }
+            store_transposed_bf16<D>(dq, scale, lds + C::LDS / 2 + w * (32 * (D * 2 + 16)), dQ + head_off + (size_t)qw0 * D,
+                                     N - qw0, lane);
+        }
+    } else {
+        store_transposed_bf16<D>(dq, scale, lds + w * (32 * (D * 2 + 16)), dQ + head_off + (size_t)qw0 * D,
+                                 N - qw0, lane);
+    }
     __syncthreads();                             // the scratch is read; the stages may be refilled
     }
 }
@@ -341,12 +380,47 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
 // BHkv = batch * kv heads; the G query heads of a kv head are walked one after the other and
 // accumulate into the same dK / dV (the gradient of repeat_interleave).  EXT as above; with it
 // every step carries the mask instructions.
-template <int D, bool CAUSAL, bool EXT>
+// Where (key tile, kv head) pairs are too few or too unequal for the device (causal: the first key tile meets every query
+// tile, the last one two; all times G), the steps of a key tile -- its 64-row query tiles, head after head -- are cut
+// into equal parts of at most `chunk` for as many workgroups, which leave f32 partial sums that flash_attn_bwd_sum_kernel adds.
+namespace fab {
+struct Parts {
+    int G, nq, causal, window, chunk;                // chunk = 0: one part per key tile
+    // 64-row query tiles that see key tile kt: [first(kt), last(kt))
+    __host__ __device__ int first(int kt) const { return causal ? 2 * kt : 0; }
+    __host__ __device__ int last(int kt) const {
+        if (window <= 0) return nq;                  // the last query that sees a key of the tile is 128 kt + 127 + window - 1
+        const int64_t e = ((int64_t)128 * kt + 126 + window) / 64 + 1;
+        return e < nq ? (int)e : nq;
+    }
+    __host__ __device__ int steps(int kt) const { return G * (last(kt) - first(kt)); }
+    __host__ __device__ int parts(int kt) const { return chunk == 0 ? 1 : (steps(kt) + chunk - 1) / chunk; }
+    __host__ __device__ int part_steps(int kt) const { const int n = parts(kt); return (steps(kt) + n - 1) / n; }
+    // item = position in the list of all parts of a kv head (chunk > 0: there are at most 64 key tiles)
+    __device__ void find(int item, int ntk, int& kt, int& part) const {
+        const int lane = threadIdx.x & 63;
+        int upto = lane < ntk ? parts(lane) : 0;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int below = __shfl_up(upto, o, 64);
+            if (lane >= o) upto += below;
+        }
+        kt = __builtin_amdgcn_readfirstlane(__builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < ntk && upto <= item)));
+        part = __builtin_amdgcn_readfirstlane(item - (kt > 0 ? __shfl(upto, kt > 0 ? kt - 1 : 0, 64) : 0));
+    }
+};
+}  // namespace fab
+
+// CUT: the launch has parts.  (Whole key tiles keep their own instantiation: with the bookkeeping of the parts in the same
+// code the pipeline below, which has no register to spare, is 4-8 % slower.)
+template <int D, bool CAUSAL, bool EXT, bool CUT>
 __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     const uint16_t* __restrict__ dO, const float2* __restrict__ stats, uint16_t* __restrict__ dK,
     uint16_t* __restrict__ dV, int BHkv, int N, int ntk, int npad, float scale, float scale_log2,
-    int Hq, int G, int window, const int* __restrict__ kv_lens, const uint8_t* __restrict__ key_mask) {
+    int Hq, int window, const int* __restrict__ kv_lens, const uint8_t* __restrict__ key_mask, fab::Parts plan, int items,
+    float* __restrict__ partial) {
+    const int G = plan.G;
     using namespace fab;
     using C = CfgK<D>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -355,18 +429,22 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int r = lane & 31, g = lane >> 5;
 
-    int bh, kt;                           // bh indexes (batch, kv head)
+    int bh, item;                         // bh indexes (batch, kv head)
     {
         const int id = blockIdx.x;
+        // causal: key tile 0 meets every query tile, so heavy first; parts of all kv heads of an XCD in that order, or
+        // head after head where whole key tiles are many (their Q / dO then share the L2)
         if ((BHkv & 7) == 0) {
-            const int xcd = id & 7, slot = id >> 3;
-            bh = (slot / ntk) * 8 + xcd;
-            kt = slot % ntk;              // causal: key tile 0 meets every query tile, so heavy first
+            const int xcd = id & 7, slot = id >> 3, heads = BHkv >> 3;
+            bh = (CUT ? slot % heads : slot / items) * 8 + xcd;
+            item = CUT ? slot / heads : slot % items;
         } else {
-            bh = id / ntk;
-            kt = id % ntk;
+            bh = CUT ? id % BHkv : id / items;
+            item = CUT ? id / BHkv : id % items;
         }
     }
+    int kt = item, part = 0;
+    if constexpr (CUT) plan.find(item, ntk, kt, part);
     const int n0 = kt * C::BNK;
     const int nw0 = n0 + w * 32;
     const int kvpos = nw0 + r;
@@ -406,13 +484,11 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     }
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
     const uint32_t wave_dst = __builtin_amdgcn_readfirstlane(lds_base + (uint32_t)w * C::PT * 1024u);
-    const int nq = (N + C::BQ - 1) / C::BQ;
-    // Tiles past the end are requested at an offset beyond the buffer (they read as zero), so that
+    // Tiles past the end of a segment are requested at an offset beyond the buffer (they read as zero), so that
     // every iteration issues the same number of loads and the wait count below stays constant.
-    const int jq0 = CAUSAL ? n0 / C::BQ : 0;
-    // with a window the last query that sees a key of this block is n0 + 127 + window - 1
-    const int jq_end = (EXT && window > 0) ? min(nq, (n0 + C::BNK + window - 2) / C::BQ + 1) : nq;
-    int hq = 0;                                      // query head of the group being walked
+    const int jq_first = CAUSAL ? n0 / C::BQ : 0, jq_last = plan.last(kt);      // query tiles that see the block's keys
+    // a segment = the tiles [jq0, jq_end) of query head hq of the group
+    int hq = 0, jq0 = jq_first, jq_end = jq_last;
     auto issue_tile = [&](int stage, int jq) {
         const uint32_t dst = wave_dst + (uint32_t)stage * C::STAGE;
         const bool live = jq < jq_end;
@@ -444,13 +520,6 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     for (int i = 0; i < C::DT; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) { dk[i][e] = 0.0f; dv[i][e] = 0.0f; }
-
-    const int ntile = jq_end - jq0;
-    const int nsub = 2 * ntile;                       // 32-row sub-tiles, numbered from the block's first tile
-    // First sub-tile with a visible (query, key) pair for this wave.  Causal: the block's first
-    // tile starts at query n0 and the wave's keys at n0 + 32w, so sub-tile w is the wave's diagonal
-    // one (the only partially masked one); earlier sub-tiles are skipped.
-    const int u0 = CAUSAL ? w : 0;
 
     // LDS addresses.  Inside the pipeline the stage and the sub-tile of every access are
     // compile-time constants, so an address is a per-lane base register plus an immediate; the
@@ -667,7 +736,24 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
 
 #pragma unroll
     for (int i = 0; i < C::KSTEPS; ++i) { pin_registers(kf[i]); pin_registers(vf[i]); }
-    for (hq = 0; hq < G; ++hq) {
+    // this part's steps of the block; a block whose keys all lie beyond the sequence's length has none (its rows are 0)
+    const int per_head = jq_last - jq_first, per_part = CUT ? plan.part_steps(kt) : 0;
+    const int step_end = EXT && n0 >= Nk ? 0 : CUT ? min(G * per_head, (part + 1) * per_part) : G;
+    for (int step_at = CUT ? part * per_part : 0; step_at < step_end;) {
+    if constexpr (CUT) {
+        hq = step_at / per_head;
+        jq0 = jq_first + step_at % per_head;
+        jq_end = min(jq_last, jq0 + step_end - step_at);
+        step_at += jq_end - jq0;
+    } else {
+        hq = step_at++;
+    }
+    const int ntile = jq_end - jq0;
+    const int nsub = 2 * ntile;                       // 32-row sub-tiles, numbered from the segment's first tile
+    // First sub-tile with a visible (query, key) pair for this wave.  Causal: the block's first
+    // tile starts at query n0 and the wave's keys at n0 + 32w, so sub-tile w of the head is the wave's diagonal
+    // one (the only partially masked one); earlier sub-tiles are skipped.
+    const int u0 = !CAUSAL ? 0 : CUT ? max(0, w - 2 * (jq0 - jq_first)) : w;
     issue_tile(0, jq0);
     issue_tile(1, jq0 + 1);
     issue_tile(2, jq0 + 2);
@@ -723,13 +809,58 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     }
 pipeline_done:
 #undef TYR_STEP
-    wait_vmcnt0();                                   // drain before the next head reuses the stages
+    wait_vmcnt0();                                   // drain before the next segment reuses the stages
     __syncthreads();
     }
 
+    if (CUT && plan.parts(kt) > 1) {
+        // [2 (dV, dK)][wave][register group of four][lane] f32x4: coalesced as the accumulators lie
+        f32x4* out = reinterpret_cast<f32x4*>(partial) + ((size_t)bh * items + item) * (2 * 4 * C::DT * 4 * 64) + w * (C::DT * 4 * 64) + lane;
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+                out[(dt * 4 + q4) * 64] = f32x4{dv[dt][4 * q4], dv[dt][4 * q4 + 1], dv[dt][4 * q4 + 2], dv[dt][4 * q4 + 3]};
+                out[(4 * C::DT * 4 + dt * 4 + q4) * 64] = f32x4{dk[dt][4 * q4], dk[dt][4 * q4 + 1], dk[dt][4 * q4 + 2], dk[dt][4 * q4 + 3]};
+            }
+        return;
+    }
     unsigned char* scratch = lds + w * (32 * (D * 2 + 16));
     store_transposed_bf16<D>(dv, 1.0f, scratch, dV + head_off + (size_t)nw0 * D, N - nw0, lane);
     store_transposed_bf16<D>(dk, scale, scratch, dK + head_off + (size_t)nw0 * D, N - nw0, lane);
+}
+
+// dK and dV of the key tiles that were cut into parts: the parts' f32 sums added in order, 8 elements of a row per thread.
+template <int D>
+__global__ __launch_bounds__(256) void flash_attn_bwd_sum_kernel(const float* __restrict__ partial, uint16_t* __restrict__ dK,
+                                                                uint16_t* __restrict__ dV, int N, int ntk, int items, float scale,
+                                                                fab::Parts plan) {
+    constexpr int CH = D / 8, DT = D / 32, TILE16 = 2 * 4 * DT * 4 * 64;      // 16-byte pieces of one part
+    const int id = blockIdx.x * 256 + threadIdx.x;
+    constexpr int PER_TILE = 2 * 128 * CH;
+    const int tile = (blockIdx.x * 256) / PER_TILE;                          // a workgroup stays inside one tile
+    const int bh = tile / ntk, kt = tile % ntk;
+    const int parts = plan.parts(kt);
+    if (parts == 1) return;
+    int first = 0;
+    for (int k = 0; k < kt; ++k) first += plan.parts(k);
+    const int within = id % PER_TILE, which = within / (128 * CH), row = (within / CH) % 128, c = within % CH;
+    // d = 8c .. 8c + 7 of key row `row`: register group dt = c / 4, q4 = c % 4 of wave row / 32, lanes row % 32 (+ 32)
+    const f32x4* in = reinterpret_cast<const f32x4*>(partial) + ((size_t)bh * items + first) * TILE16 +
+                      (which * 4 * DT * 4 + (row >> 5) * (DT * 4) + c) * 64 + (row & 31);
+    f32x4 lo = in[0], hi = in[32];
+    for (int p = 1; p < parts; ++p) {
+        lo += in[(size_t)p * TILE16];
+        hi += in[(size_t)p * TILE16 + 32];
+    }
+    if (kt * 128 + row >= N) return;
+    const float mul = which ? scale : 1.0f;
+    u32x4 v;
+    v[0] = pack_bf16(lo[0] * mul, lo[1] * mul);
+    v[1] = pack_bf16(lo[2] * mul, lo[3] * mul);
+    v[2] = pack_bf16(hi[0] * mul, hi[1] * mul);
+    v[3] = pack_bf16(hi[2] * mul, hi[3] * mul);
+    st_global_16((which ? dK : dV) + ((size_t)bh * N + kt * 128 + row) * D + c * 8, v);
 }
 
 size_t flash_attn_bwd_workspace_bytes(int B, int H, int N) {
@@ -737,20 +868,111 @@ size_t flash_attn_bwd_workspace_bytes(int B, int H, int N) {
     return (size_t)B * H * npad * sizeof(float2);
 }
 
+namespace {
+// How the dK / dV work is cut.  A workgroup has a CU to itself; a step (64 queries x 128 keys) takes 1.55 us at D = 128, 0.9
+// at 64, a segment (one head's range) 1.5 us to start and end, the sum of the parts 4 us and the traffic of its partials
+// (written and read at 4 TB/s).  Tried: whole key tiles, and the finest cut with at most 256, 512 or 768 workgroups.
+fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window) {
+    const int ntk = (N + 127) / 128, nq = (N + 63) / 64;
+    const fab::Parts whole{G, nq, causal, window, 0};
+    fab::Parts best = whole;
+    if (ntk > 64) return best;
+    const double step = D == 128 ? 1.55 : 0.9;
+    int64_t total = 0;
+    int most = 1;
+    for (int kt = 0; kt < ntk; ++kt) {
+        total += whole.steps(kt);
+        most = std::max(most, whole.steps(kt));
+    }
+    double least = 1e300;
+    std::vector<int> sizes;
+    for (int round = 0; round <= 3; ++round) {
+        fab::Parts p = whole;
+        auto count = [&](int chunk) {
+            p.chunk = chunk;
+            int64_t n = 0;
+            for (int kt = 0; kt < ntk; ++kt) n += p.parts(kt);
+            return n * BHkv;
+        };
+        if (round) {
+            int lo = std::max<int64_t>(2, total * BHkv / (256 * round)), hi = most;     // least chunk with few enough parts
+            if (lo >= hi || count(hi) > 256 * round) continue;
+            while (lo < hi) {
+                const int mid = (lo + hi) / 2;
+                if (count(mid) <= 256 * round) hi = mid; else lo = mid + 1;
+            }
+            p.chunk = lo;
+        }
+        int64_t cut = 0;
+        sizes.clear();
+        for (int kt = 0; kt < ntk; ++kt) {
+            const int n = p.parts(kt);
+            if (n > 1) cut += n;
+            for (int i = 0; i < n; ++i) sizes.push_back(p.chunk ? p.part_steps(kt) : p.steps(kt));
+        }
+        if (round && cut == 0) continue;
+        std::sort(sizes.begin(), sizes.end(), std::greater<int>());
+        // every size BHkv times, longest first over 256 CUs
+        const int64_t n = (int64_t)sizes.size() * BHkv;
+        double steps = sizes[0];
+        if (n > 256 && n <= 512) {
+            for (int64_t j = 0; j < n - 256; ++j) steps = std::max(steps, (double)sizes[(255 - j) / BHkv] + sizes[(256 + j) / BHkv]);
+        } else if (n > 512) {
+            steps = std::max(steps, (double)total * BHkv / 256 + 0.5 * total / sizes.size());
+        }
+        const double heads = std::max(1.0, std::min((double)G, (double)sizes[0] / std::max(1, p.last(0) - p.first(0))));
+        double us = step * steps + 1.5 * (heads + std::max(0.0, (double)n / 256 - 1));
+        if (round) us += 4.0 + cut * BHkv * (128.0 * D * 8 * 2) / 4.0e6;
+        if (us < least) { least = us; best = p; }
+    }
+    return best;
+}
+// some microseconds of host time: each thread keeps its last plans
+fab::Parts dkv_plan(int BHkv, int G, int N, int D, bool causal, int window) {
+    struct Entry { int BHkv, G, N, D, causal, window; fab::Parts plan; };
+    static thread_local Entry kept[16];
+    const uint32_t h = ((uint32_t)BHkv * 0x9e3779b1u ^ (uint32_t)N * 0x85ebca6bu ^ (uint32_t)(G * 131 + D) * 0xc2b2ae35u ^ (uint32_t)(window * 2 + causal) * 0x27d4eb2fu) * 0x9e3779b1u;
+    Entry& e = kept[h >> 28];
+    if (e.BHkv != BHkv || e.G != G || e.N != N || e.D != D || e.causal != causal || e.window != window)
+        e = {BHkv, G, N, D, causal, window, make_dkv_plan(BHkv, G, N, D, causal, window)};
+    return e.plan;
+}
+int dkv_items(const fab::Parts& p, int N) {
+    const int ntk = (N + 127) / 128;
+    if (p.chunk == 0) return ntk;
+    int n = 0;
+    for (int kt = 0; kt < ntk; ++kt) n += p.parts(kt);
+    return n;
+}
+size_t dkv_partial_bytes(const fab::Parts& p, int BHkv, int N, int D) {
+    return p.chunk ? (size_t)BHkv * dkv_items(p, N) * 128 * D * 8 : 0;
+}
+}  // namespace
+
+size_t flash_attn_bwd_full_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int causal, int window) {
+    const fab::Parts p = dkv_plan(B * Hkv, Hq / Hkv, N, D, causal != 0, window);
+    return flash_attn_bwd_workspace_bytes(B, Hq, N) + dkv_partial_bytes(p, B * Hkv, N, D);
+}
+
 int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                           const float* lse, void* dq, void* dk, void* dv, int B, int Hq, int Hkv, int N, int D,
                           int causal, int window, const int* kv_lens, const uint8_t* key_mask, float scale,
-                          void* workspace,
+                          void* workspace, size_t workspace_bytes,
                           hipStream_t stream) {
     using namespace fab;
     const int BH = B * Hq, BHkv = B * Hkv, G = Hq / Hkv;
-    const int ntq = (N + 127) / 128;
-    const int npad = ntq * 128;
+    const int ntk = (N + 127) / 128, npad = ntk * 128;
     const bool ext = window > 0 || kv_lens != nullptr || key_mask != nullptr;
-    // lengths and key masks keep tile 0 starting at key 0; a window makes the tiles equal
-    const int single = (causal && window <= 0 && ntq > 1 && attn_single_tiles(BH, ntq)) ? 1 : 0;
-    const int pair = (causal && window <= 0 && ntq > 1 && !single) ? 1 : 0;
-    dim3 grid_q((unsigned)(BH * (pair ? (ntq + 1) / 2 : ntq))), grid_k((unsigned)(BHkv * ntq)), block(THREADS);
+    const AttnShape shape = attn_shape(BH, N, D, causal != 0, window);
+    const int ntq = (N + shape.rows - 1) / shape.rows;
+    const int pair = shape.pair, single = shape.single;
+    dim3 grid_q((unsigned)(BH * (pair ? (ntq + 1) / 2 : ntq))), block(THREADS);
+    const size_t stat_bytes = flash_attn_bwd_workspace_bytes(B, Hq, N);
+    Parts plan = dkv_plan(BHkv, G, N, D, causal != 0, window);
+    if (workspace_bytes < stat_bytes + dkv_partial_bytes(plan, BHkv, N, D)) plan.chunk = 0;
+    const int items = dkv_items(plan, N);
+    dim3 grid_k((unsigned)(BHkv * items));
+    float* partial = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + stat_bytes);
     const float scale_log2 = scale * LOG2E;
     auto Qp = static_cast<const uint16_t*>(q);
     auto Kp = static_cast<const uint16_t*>(k);
@@ -758,22 +980,37 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     auto Op = static_cast<const uint16_t*>(o);
     auto dOp = static_cast<const uint16_t*>(d_o);
     auto st = static_cast<float2*>(workspace);
-#define TYR_FAB_LAUNCH(DD, CC, EE)                                                                    \
+#define TYR_FAB_DQ(DD, CC, EE, SS)                                                                    \
     do {                                                                                              \
         static const hipError_t a1 = hipFuncSetAttribute(                                             \
-            reinterpret_cast<const void*>(&flash_attn_bwd_dq_kernel<DD, CC, EE>),                     \
+            reinterpret_cast<const void*>(&flash_attn_bwd_dq_kernel<DD, CC, EE, SS>),                 \
             hipFuncAttributeMaxDynamicSharedMemorySize, CfgQ<DD>::LDS);                               \
+        if (a1 != hipSuccess) return -1;                                                              \
+        hipLaunchKernelGGL((flash_attn_bwd_dq_kernel<DD, CC, EE, SS>), grid_q, block, CfgQ<DD>::LDS, stream, \
+                           Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st, BH, N, ntq, npad, \
+                           scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single);        \
+    } while (0)
+#define TYR_FAB_DKV(DD, CC, EE, UU)                                                                   \
+    do {                                                                                              \
         static const hipError_t a2 = hipFuncSetAttribute(                                             \
-            reinterpret_cast<const void*>(&flash_attn_bwd_dkv_kernel<DD, CC, EE>),                    \
+            reinterpret_cast<const void*>(&flash_attn_bwd_dkv_kernel<DD, CC, EE, UU>),                \
             hipFuncAttributeMaxDynamicSharedMemorySize, CfgK<DD>::LDS);                               \
-        if (a1 != hipSuccess || a2 != hipSuccess) return -1;                                          \
-        hipLaunchKernelGGL((flash_attn_bwd_dq_kernel<DD, CC, EE>), grid_q, block, CfgQ<DD>::LDS, stream, \
-                           Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st, BH, N, ntq,      \
-                           scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single);                \
-        hipLaunchKernelGGL((flash_attn_bwd_dkv_kernel<DD, CC, EE>), grid_k, block, CfgK<DD>::LDS, stream, \
+        if (a2 != hipSuccess) return -1;                                                              \
+        hipLaunchKernelGGL((flash_attn_bwd_dkv_kernel<DD, CC, EE, UU>), grid_k, block, CfgK<DD>::LDS, stream, \
                            Qp, Kp, Vp, dOp, st, static_cast<uint16_t*>(dk),                           \
-                           static_cast<uint16_t*>(dv), BHkv, N, ntq, npad, scale, scale_log2, Hq, G,  \
-                           window, kv_lens, key_mask);                                                \
+                           static_cast<uint16_t*>(dv), BHkv, N, ntk, npad, scale, scale_log2, Hq,     \
+                           window, kv_lens, key_mask, plan, items, partial);                          \
+    } while (0)
+#define TYR_FAB_LAUNCH(DD, CC, EE)                                                                    \
+    do {                                                                                              \
+        if (shape.rows == 64) TYR_FAB_DQ(DD, CC, EE, true); else TYR_FAB_DQ(DD, CC, EE, false);       \
+        if (plan.chunk) {                                                                             \
+            TYR_FAB_DKV(DD, CC, EE, true);                                                            \
+            hipLaunchKernelGGL(flash_attn_bwd_sum_kernel<DD>, dim3((unsigned)(BHkv * ntk * (DD / 8))), dim3(256), 0, stream, \
+                               partial, static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), N, ntk, items, scale, plan); \
+        } else {                                                                                      \
+            TYR_FAB_DKV(DD, CC, EE, false);                                                           \
+        }                                                                                             \
     } while (0)
 #define TYR_FAB_PICK(DD)                                                                              \
     do {                                                                                              \
@@ -783,6 +1020,8 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     if (D == 128) TYR_FAB_PICK(128); else TYR_FAB_PICK(64);
 #undef TYR_FAB_PICK
 #undef TYR_FAB_LAUNCH
+#undef TYR_FAB_DKV
+#undef TYR_FAB_DQ
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -32,6 +32,7 @@
 // pointing at 4 consecutive d of 4 kv rows hand every lane "its" d for those 4 rows.
 #include <limits.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "common.hpp"
@@ -70,7 +71,10 @@ template <int D> __device__ __forceinline__ int v_swz(int row, int c) { return c
 
 // EXT adds the per-sequence key length (padding mask over the tail) and the sliding window; the
 // plain instantiation carries none of their instructions.  G = query heads per kv head.
-template <int D, bool CAUSAL, bool EXT>
+// SPLIT (launches with few tiles): a workgroup takes 64 query rows; waves w and w + 2 own the same 32 rows, one the first
+// and one the second 32 keys of every tile, and merge their (m, l, O) through LDS at the end.  Half the work per tile
+// step and twice the workgroups; the step's requests and barrier cost what they did, so it pays only on an idle device.
+template <int D, bool CAUSAL, bool EXT, bool SPLIT>
 __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     uint16_t* __restrict__ O, float* __restrict__ LSE, int BH, int N, int ntq, float scale_log2,
@@ -78,11 +82,15 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     int single, int total_ids) {
     using namespace fa;
     using C = Cfg<D>;
+    constexpr int TBM = SPLIT ? 64 : BM;         // query rows of a workgroup
+    constexpr int NT = SPLIT ? 1 : 2;            // 32-key sub-tiles of a key tile that a wave computes
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
     const int t = threadIdx.x;
     const int lane = t & 63, w = t >> 6;
     const int r = lane & 31, g = lane >> 5;
+    const int wr = SPLIT ? w & 1 : w;            // which 32 rows of the tile
+    const int T0 = SPLIT ? w >> 1 : 0;           // first sub-tile
 
     // workgroup -> (head, query tile): AttnOrder.
     // A launch has either one workgroup per job id, or (persistent launch) two workgroups per CU, of which workgroup p
@@ -109,8 +117,8 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
         n_qt = CAUSAL ? ntq - 1 - n_tr : n_tr;
         has_next = true;
     }
-    const int q0 = qt * BM;
-    const int qw0 = q0 + w * 32;                 // first query row of this wave
+    const int q0 = qt * TBM;
+    const int qw0 = q0 + wr * 32;                // first query row of this wave
     const size_t head_off = (size_t)bh * N * D;
     const size_t kv_head_off = (size_t)kvbh * N * D;
     const uint16_t* Qh = Q + head_off;
@@ -122,7 +130,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     const int Nk = (EXT && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / Hq])) : N;
     // per-sequence key mask (nonzero = visible), any pattern
     const uint8_t* km = (EXT && key_mask != nullptr) ? key_mask + (size_t)(bh / Hq) * N : nullptr;
-    const int kv_end = CAUSAL ? min(Nk, q0 + BM) : Nk;
+    const int kv_end = CAUSAL ? min(Nk, q0 + TBM) : Nk;
     const int nkv_abs = max(1, (kv_end + BN - 1) / BN);   // a sequence without keys still walks one (fully masked) tile
     const int jbase = (EXT && window > 0) ? min(max(0, q0 - window + 1) / BN, nkv_abs - 1) : 0;   // first tile any row sees
     const int nkv = nkv_abs - jbase;             // tiles are numbered from jbase below
@@ -178,13 +186,14 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
         for (int e = 0; e < 16; ++e) oacc[i][e] = 0.0f;
     // running row maximum, in log2 units (score * scale * log2 e).  With a window a row's first
     // tiles can be wholly masked; a finite start keeps (-inf) - m2 from becoming NaN there.
-    float m2 = EXT ? -1.0e30f : -INFINITY;
+    // (SPLIT: so can the keys of one wave.)
+    float m2 = EXT || SPLIT ? -1.0e30f : -INFINITY;
     float lsum = 0.0f;         // this lane's share of the running row sum
 
     // K fragment (sub-tile T, k-step i): row 32T + r, chunk 2i + g.
     int k_roff[C::KSTEPS];
 #pragma unroll
-    for (int i = 0; i < C::KSTEPS; ++i) k_roff[i] = r * C::ROW + k_swz<D>(r, 2 * i + g) * 16;
+    for (int i = 0; i < C::KSTEPS; ++i) k_roff[i] = (32 * T0 + r) * C::ROW + k_swz<D>(r, 2 * i + g) * 16;
     // V^T fragment (d tile dt; rows 32T + 16s + 8h + 4g + [0,4)): as a source lane of the transposing
     // read this lane points at row 4g + (lane%16)/4 of that group, 8 bytes at d = 32dt + 16(b&1) + 4(lane%4).
     int v_roff[C::DT];
@@ -194,7 +203,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
 #pragma unroll
         for (int dt = 0; dt < C::DT; ++dt) {
             const int dcol = 32 * dt + 16 * (b16 & 1) + 4 * (i16 & 3);
-            v_roff[dt] = C::V_BASE + row * C::ROW + v_swz<D>(row, dcol >> 3) * 16 + (dcol & 7) * 2;
+            v_roff[dt] = C::V_BASE + (32 * T0 + row) * C::ROW + v_swz<D>(row, dcol >> 3) * 16 + (dcol & 7) * 2;
         }
     }
     const int qpos = qw0 + r;
@@ -206,18 +215,18 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     const int nkv_w = CAUSAL ? min(nkv, (qw0 + 31) / BN + 1 - jbase) : nkv;
 
     constexpr int NG = C::KSTEPS / 2;            // S^T is built in NG groups of (2 k-steps x 2 sub-tiles)
-    auto read_k_group = [&](const unsigned char* Kt, int grp, bf16x8 (&dst)[4]) {
+    auto read_k_group = [&](const unsigned char* Kt, int grp, bf16x8 (&dst)[2 * NT]) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            dst[u] = *reinterpret_cast<const bf16x8*>(Kt + k_roff[2 * grp + (u >> 1)] + (u & 1) * 32 * C::ROW);
+        for (int u = 0; u < 2 * NT; ++u)
+            dst[u] = *reinterpret_cast<const bf16x8*>(Kt + k_roff[2 * grp + u / NT] + (u % NT) * 32 * C::ROW);
     };
-    auto mfma_k_group = [&](f32x16 (&sacc)[2], int grp, const bf16x8 (&kf)[4]) {
+    auto mfma_k_group = [&](f32x16 (&sacc)[NT], int grp, const bf16x8 (&kf)[2 * NT]) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) sacc[u & 1] = mfma_32x32x16_bf16(kf[u], qf[2 * grp + (u >> 1)], sacc[u & 1]);
+        for (int u = 0; u < 2 * NT; ++u) sacc[u % NT] = mfma_32x32x16_bf16(kf[u], qf[2 * grp + u / NT], sacc[u % NT]);
     };
-    auto zero_s = [&](f32x16 (&sacc)[2]) {
+    auto zero_s = [&](f32x16 (&sacc)[NT]) {
 #pragma unroll
-        for (int T = 0; T < 2; ++T)
+        for (int T = 0; T < NT; ++T)
 #pragma unroll
             for (int e = 0; e < 16; ++e) sacc[T][e] = 0.0f;
     };
@@ -235,10 +244,10 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     wait_vmcnt0();
     __syncthreads();
 
-    f32x16 sA[2], sB[2];
+    f32x16 sA[NT], sB[NT];
     zero_s(sA);
     {
-        bf16x8 kf[2][4];
+        bf16x8 kf[2][2 * NT];
         read_k_group(lds, 0, kf[0]);
 #pragma unroll
         for (int grp = 0; grp < NG; ++grp) {
@@ -255,7 +264,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     // One kv tile: softmax and P V of tile j (scores in `cur`), overlapped with the score MFMAs of
     // tile j+1 (into `nxt`).  K runs one tile ahead of V in LDS: at entry K(j+1) and V(j) are
     // resident; K(j+2) and V(j+1) are requested here and awaited at the end.
-    auto tile_step = [&](f32x16 (&cur)[2], f32x16 (&nxt)[2], int j) {
+    auto tile_step = [&](f32x16 (&cur)[NT], f32x16 (&nxt)[NT], int j) {
         const int j0 = (jbase + j) * BN;
         // The two requests are issued apart (K here, V after the row-max reduction) so the waves of
         // a CU do not all queue on the texture path at once.
@@ -281,10 +290,10 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
             if (need_mask) {
                 const int lim = CAUSAL ? min(qpos, Nk - 1) : Nk - 1;   // largest visible kv row
                 const int low = (EXT && window > 0) ? qpos - window + 1 : INT_MIN;   // smallest visible kv row
-                const int base = j0 + 4 * g;
-                const uint64_t hidden = tile_hidden >> (4 * g);      // shifted to this lane's rows
+                const int base = j0 + 32 * T0 + 4 * g;
+                const uint64_t hidden = tile_hidden >> (32 * T0 + 4 * g);      // shifted to this lane's rows
 #pragma unroll
-                for (int T = 0; T < 2; ++T)
+                for (int T = 0; T < NT; ++T)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
                         const int kv = base + 32 * T + 8 * (e >> 2) + (e & 3);
@@ -295,10 +304,11 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
             }
 
             // ---- next tile's scores, first group, under the row-max reduction of this tile
-            bf16x8 kf[2][4];
+            // (SPLIT has the registers to hold all fragments of the next tile's scores at once)
+            bf16x8 kf[SPLIT ? NG : 2][2 * NT];
             zero_s(nxt);
-            read_k_group(Kt, 0, kf[0]);
-            read_k_group(Kt, 1, kf[1]);
+#pragma unroll
+            for (int grp = 0; grp < (SPLIT ? NG : 2); ++grp) read_k_group(Kt, grp, kf[grp]);
 
             // online softmax on this lane's query column.  The reference maximum m2 is only
             // advanced (and O, l rescaled) when some row of the wave outgrew it by more than
@@ -306,7 +316,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
             // sums and bf16 P hold without loss.
             float mx = cur[0][0];
 #pragma unroll
-            for (int T = 0; T < 2; ++T)
+            for (int T = 0; T < NT; ++T)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) mx = fmaxf(mx, cur[T][e]);
             mfma_k_group(nxt, 0, kf[0]);
@@ -326,7 +336,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
 
             // ---- exponentials of this tile under the remaining score MFMAs of the next
             float psum = 0.0f;
-            bf16x8 pf[2][2];
+            bf16x8 pf[NT][2];
             bf16x8 vf[2][C::DT];
             auto read_v_group = [&](int c, bf16x8 (&dst)[C::DT]) {
 #pragma unroll
@@ -338,13 +348,16 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
                 }
             };
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {                 // c = 2T + s : 8 scores each
+            for (int c = 0; c < 2 * NT; ++c) {            // c = 2T + s : 8 scores each
                 const int T = c >> 1, sh = c & 1;
-                if (c + 1 < NG) {
+                if constexpr (SPLIT) {
+#pragma unroll
+                    for (int grp = 1 + c * (NG / 2); grp < min(NG, 1 + (c + 1) * (NG / 2)); ++grp) mfma_k_group(nxt, grp, kf[grp]);
+                } else if (c + 1 < NG) {
                     if (c + 2 < NG) read_k_group(Kt, c + 2, kf[c & 1]);
                     mfma_k_group(nxt, c + 1, kf[(c + 1) & 1]);
                 }
-                if (c == 3) read_v_group(0, vf[0]);       // first V^T fragments arrive under the last exponentials
+                if (c == 2 * NT - 1) read_v_group(0, vf[0]);       // first V^T fragments arrive under the last exponentials
                 u32x4 pk;
 #pragma unroll
                 for (int jj = 0; jj < 4; ++jj) {
@@ -360,8 +373,8 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
             // ---- O^T += V^T P^T; fragment reads run one group ahead.  Group c = (T, s).
             {
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    if (c + 1 < 4) read_v_group(c + 1, vf[(c + 1) & 1]);
+                for (int c = 0; c < 2 * NT; ++c) {
+                    if (c + 1 < 2 * NT) read_v_group(c + 1, vf[(c + 1) & 1]);
 #pragma unroll
                     for (int dt = 0; dt < C::DT; ++dt)
                         oacc[dt] = mfma_32x32x16_bf16(vf[c & 1][dt], pf[c >> 1][c & 1], oacc[dt]);
@@ -383,14 +396,42 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     // the second tile of a pair) so that global stores are 16 bytes per lane along rows.  Rows are
     // unpadded; 16-byte chunks are XOR-swizzled by row.
     if (overlap_next) {
-        const int qrow = min(n_qt * BM + w * 32 + r, N - 1);
+        const int qrow = min(n_qt * TBM + wr * 32 + r, N - 1);
         const uint16_t* qp = Q + (size_t)n_bh * N * D + (size_t)qrow * D + g * 8;
 #pragma unroll
         for (int i = 0; i < C::KSTEPS; ++i) qf[i] = __builtin_bit_cast(bf16x8, ld_global_16(qp + i * 16));
     }
-    const float ltot = sum_xor32(lsum);
+    float ltot = sum_xor32(lsum);
+    if constexpr (SPLIT) {
+        // waves 2, 3 hand their (m, l, O) to waves 0, 1 through the K stages (dead now: a SPLIT launch has no next tile)
+        f32x4* mine = reinterpret_cast<f32x4*>(lds) + wr * (C::DT * 4 * 64) + lane;
+        float2* stat = reinterpret_cast<float2*>(lds + C::LDS - 1024) + wr * 64 + lane;     // behind the O scratch below
+        if (w >= 2) {
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4)
+                    mine[(dt * 4 + q4) * 64] = f32x4{oacc[dt][4 * q4], oacc[dt][4 * q4 + 1], oacc[dt][4 * q4 + 2], oacc[dt][4 * q4 + 3]};
+            *stat = make_float2(m2, ltot);
+        }
+        __syncthreads();
+        if (w < 2) {
+            const float2 other = *stat;
+            const float m = fmaxf(m2, other.x), wa = fast_exp2(m2 - m), wb = fast_exp2(other.x - m);
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    const f32x4 o = mine[(dt * 4 + q4) * 64];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) oacc[dt][4 * q4 + x] = oacc[dt][4 * q4 + x] * wa + o[x] * wb;
+                }
+            ltot = ltot * wa + other.y * wb;
+            m2 = m;
+        }
+    }
     const float inv = (!EXT || ltot > 0.0f) ? 1.0f / ltot : 0.0f;    // EXT: a row that saw no key gives 0
-    {
+    if (!SPLIT || w < 2) {
         constexpr int SROW = D * 2;
         constexpr int CH = D / 8;                   // 16-byte chunks per row
         auto s_swz = [](int row) { return (D == 128 ? row : (row >> 1)) & (CH - 1); };
@@ -415,11 +456,70 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
             if (qw0 + row < N) st_global_16(O + head_off + (size_t)(qw0 + row) * D + (lane % CH) * 8, v);
         }
     }
-    if (qpos < N && LSE != nullptr && g == 0) LSE[(size_t)bh * N + qpos] = logf(ltot) + m2 * LN2;
+    if ((!SPLIT || w < 2) && qpos < N && LSE != nullptr && g == 0) LSE[(size_t)bh * N + qpos] = logf(ltot) + m2 * LN2;
     __syncthreads();                             // the scratch is read; the stages may be refilled
     preloaded = overlap_next;
     }
     }
+}
+
+// The jobs of a launch and the time of its busiest CU.  Times are microseconds on an MI355X, measured on 150 shapes (4 to
+// 256 heads, 64 to 4096 rows): a key-tile step of a 128-row workgroup takes 1.0 us at D = 128 (0.64 at D = 64) with the device
+// busy, of a 64-row one 0.61 (0.38); a launch costs 5.6-6.1 us besides, a second workgroup of a CU and the second tile of
+// a pair 1-2.  The choice is 1.3 % slower on those shapes than the best of the three forms.
+namespace {
+struct AttnJobs {
+    int ntq, steps0;             // tiles per head; steps of the longest
+    bool causal, paired;
+    int rows, N;
+    // steps of the job of rank r (rank 0 = longest)
+    double work(int r) const {
+        auto tile = [&](int rank) { return causal ? std::min(steps0, ((ntq - rank) * rows + 63) / 64) : steps0; };
+        if (!paired) return tile(r);
+        const int other = ntq - 1 - r;
+        return other == r ? tile(r) : tile(r) + tile(other) + 2.0;
+    }
+    int ranks() const { return paired ? (ntq + 1) / 2 : ntq; }
+};
+double busiest_cu_us(const AttnJobs& jobs, int64_t bh, double step, double alone, double fixed, double extra) {
+    const int64_t n = bh * jobs.ranks();
+    if (n <= 256) return fixed + step * alone * jobs.work(0);
+    if (n <= 512) {
+        // job 256 + j is the second of the CU that has job 255 - j (AttnOrder)
+        double worst = alone * jobs.work(0);
+        for (int64_t j = 0; j < n - 256;) {
+            const int64_t a = 255 - j, b = 256 + j;
+            worst = std::max(worst, jobs.work((int)(a / bh)) + jobs.work((int)(b / bh)));
+            j += std::min(a % bh + 1, bh - b % bh);
+        }
+        return fixed + step * worst + extra;
+    }
+    double total = 0;
+    for (int r = 0; r < jobs.ranks(); ++r) total += jobs.work(r);
+    // more: pairs are equal and fill whole rounds; single tiles, longest first, leave about half a mean job of imbalance
+    // (and 5 % for the L2, see attn_shape)
+    if (jobs.paired) return fixed + step * jobs.work(0) * (double)((n + 255) / 256) + extra * ((double)n / 256 - 1);
+    return fixed + step * (total * bh / 256 * 1.05 + 0.5 * total / jobs.ranks()) + extra * ((double)n / 256 - 1);
+}
+}  // namespace
+
+AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window) {
+    const bool ordered = causal && window <= 0;      // a window makes the tiles equal
+    AttnShape best{128, 0, 0};
+    double least = 1e300;
+    for (int form = 0; form < 3; ++form) {           // 0 = pairs, 1 = single tiles, 2 = 64-row tiles
+        const int rows = form == 2 ? 64 : 128, ntq = (N + rows - 1) / rows;
+        if (form == 0 && (!ordered || ntq == 1)) continue;
+        // many single tiles, longest first, walk all heads at once: their K / V do not fit an L2 (the backward of 256 heads
+        // of 4096 rows was 14 % slower that way than with pairs, head after head)
+        if (form != 0 && ordered && ntq > 1 && bh * ntq > 2048) continue;
+        const int all = (N + 63) / 64, seen = window > 0 ? std::min<int64_t>(all, ((int64_t)window + rows) / 64 + 1) : all;
+        const AttnJobs jobs{ntq, seen, ordered, form == 0, rows, N};
+        const double us = D == 128 ? (form == 2 ? busiest_cu_us(jobs, bh, 0.61, 0.97, 6.1, 1.0) : busiest_cu_us(jobs, bh, 1.0, 0.95, 5.6, 1.3))
+                                   : (form == 2 ? busiest_cu_us(jobs, bh, 0.38, 1.3, 5.0, 0.8) : busiest_cu_us(jobs, bh, 0.64, 1.1, 4.7, 1.0));
+        if (us < least) { least = us; best = {rows, form == 0, form != 0 && ordered}; }
+    }
+    return best;
 }
 
 int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B,
@@ -429,16 +529,16 @@ int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, 
     using namespace fa;
     const int BH = B * Hq;
     const int G = Hq / Hkv;
-    const int ntq = (N + BM - 1) / BM;
     const bool ext = window > 0 || kv_lens != nullptr || key_mask != nullptr;
-    // lengths and key masks keep tile 0 starting at key 0; a window makes the tiles equal
-    const int single = (causal && window <= 0 && ntq > 1 && attn_single_tiles(BH, ntq)) ? 1 : 0;
-    const int pair = (causal && window <= 0 && ntq > 1 && !single) ? 1 : 0;
+    // a window makes the tiles equal; lengths and key masks keep tile 0 starting at key 0
+    const AttnShape shape = attn_shape(BH, N, D, causal != 0, window);
+    const int ntq = (N + shape.rows - 1) / shape.rows;
+    const int pair = shape.pair, single = shape.single;
     const int total_ids = BH * (pair ? (ntq + 1) / 2 : ntq);
     // One workgroup per job id, or persistent workgroups: two per CU (what registers and 64 KB of LDS at D = 128 allow),
     // rounded down to a multiple of 8 so that a workgroup's job ids stay on one XCD, and never fewer than 8.
     unsigned nwg = (unsigned)total_ids;
-    if (flash_attn_fwd_persistent()) {
+    if (flash_attn_fwd_persistent() && shape.rows == BM) {
         static std::atomic<int> resident_of[kMaxDevices];       // per device, 0 = not asked yet
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) dev = 0;
@@ -458,22 +558,25 @@ int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, 
     auto Kp = static_cast<const uint16_t*>(k);
     auto Vp = static_cast<const uint16_t*>(v);
     auto Op = static_cast<uint16_t*>(o);
-#define TYR_FA_LAUNCH(DD, CC, EE)                                                                \
+#define TYR_FA_LAUNCH(DD, CC, EE, SS)                                                            \
     do {                                                                                         \
         static const hipError_t attr = hipFuncSetAttribute(                                      \
-            reinterpret_cast<const void*>(&flash_attn_fwd_kernel<DD, CC, EE>),                   \
+            reinterpret_cast<const void*>(&flash_attn_fwd_kernel<DD, CC, EE, SS>),               \
             hipFuncAttributeMaxDynamicSharedMemorySize, Cfg<DD>::LDS);                           \
         if (attr != hipSuccess) return -1;                                                       \
-        hipLaunchKernelGGL((flash_attn_fwd_kernel<DD, CC, EE>), grid, block, Cfg<DD>::LDS, stream, \
+        hipLaunchKernelGGL((flash_attn_fwd_kernel<DD, CC, EE, SS>), grid, block, Cfg<DD>::LDS, stream, \
                            Qp, Kp, Vp, Op, lse, BH, N, ntq, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single, total_ids); \
     } while (0)
+#define TYR_FA_SHAPE(DD, CC, EE)                                                                 \
+    do { if (shape.rows == BM) TYR_FA_LAUNCH(DD, CC, EE, false); else TYR_FA_LAUNCH(DD, CC, EE, true); } while (0)
 #define TYR_FA_PICK(DD)                                                                          \
     do {                                                                                         \
-        if (ext) { if (causal) TYR_FA_LAUNCH(DD, true, true); else TYR_FA_LAUNCH(DD, false, true); }   \
-        else     { if (causal) TYR_FA_LAUNCH(DD, true, false); else TYR_FA_LAUNCH(DD, false, false); } \
+        if (ext) { if (causal) TYR_FA_SHAPE(DD, true, true); else TYR_FA_SHAPE(DD, false, true); }   \
+        else     { if (causal) TYR_FA_SHAPE(DD, true, false); else TYR_FA_SHAPE(DD, false, false); } \
     } while (0)
     if (D == 128) TYR_FA_PICK(128); else TYR_FA_PICK(64);
 #undef TYR_FA_PICK
+#undef TYR_FA_SHAPE
 #undef TYR_FA_LAUNCH
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
