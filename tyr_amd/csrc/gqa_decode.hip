@@ -9,8 +9,7 @@
 // partial results are merged with the online-softmax algebra
 //   m = max m_s ; l = sum l_s 2^(m_s-m) ; O = sum O_s 2^(m_s-m) / l ; LSE = ln l + m ln 2.
 //
-// First pass.  grid = splits * B*Hkv workgroups (the splits of a group adjacent), 8 waves per workgroup; the waves take the 32-row steps of
-// the split in turn, each with the 16x16x32 bf16 MFMA:
+// First pass.  grid = splits * B*Hkv workgroups of 4 or 8 waves; the waves take the 32-row steps of the split in turn, each with the 16x16x32 bf16 MFMA:
 //   S^T (16 kv x 16 q)  = K rows (row operand: lane l holds row l%16, 8 d at 32i + 8(l/16))
 //                         x Q^T (column operand, zero beyond the G = Hq/Hkv real heads)
 //   O^T_j (16 d x 16 q) += V^T (row operand) x P^T (column operand),  j = 0..7
@@ -55,9 +54,12 @@ __global__ __launch_bounds__(64 * WAVES) void gqa_decode_split_kernel(
     const int t = threadIdx.x;
     const int lane = t & 63, w = t >> 6;
     const int x = lane & 15, g = lane >> 4;
-    // one-dimensional grid, the splits of a (batch, kv head) group adjacent: any number of groups fits
-    const int split = (int)(blockIdx.x % (unsigned)S);
-    const int bg = (int)(blockIdx.x / (unsigned)S);   // b * Hkv + kv head
+    // One-dimensional grid, so any number of (batch, kv head) groups fits.  The first splits of all groups come first: the
+    // last ones, empty in a batch of unequal lengths, then neither fall on the same XCDs nor hold up others (272 groups of
+    // 1000-2000 rows, 4 splits, next to each other 47.7 us, so 42.1).
+    const unsigned groups = gridDim.x / (unsigned)S;
+    const int split = (int)(blockIdx.x / groups);
+    const int bg = (int)(blockIdx.x % groups);        // b * Hkv + kv head
     const int b = bg / Hkv, kvh = bg % Hkv;
 
     const uint16_t* Kb = Kp + (size_t)bg * kv_stride * D;
@@ -218,43 +220,68 @@ __global__ __launch_bounds__(64 * WAVES) void gqa_decode_split_kernel(
     }
 }
 
-// Second pass: one workgroup of D threads per (batch, query head).
+// Second pass: one workgroup per (batch, query head).  It is all latency, so the partials of the splits are read side by
+// side (D/4 threads of 4 elements per split, CG splits at once, up to four of each in flight) and merged through LDS.
 template <int D>
-__global__ __launch_bounds__(D) void gqa_decode_combine_kernel(
+__global__ __launch_bounds__(256) void gqa_decode_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_m, const float* __restrict__ part_l,
     uint16_t* __restrict__ O, float* __restrict__ LSE, int S) {
     using namespace dec;
-    const int bh = blockIdx.x, d = threadIdx.x;
+    constexpr int TPS = D / 4, CG = 256 / TPS;       // threads per split; splits side by side
+    __shared__ f32x4 so[CG][TPS];
+    __shared__ float sm[CG], sl[CG];
+    const int bh = blockIdx.x, t = threadIdx.x, c = t % TPS, sg = t / TPS;
     const float* pm = part_m + (size_t)bh * S;
     const float* pl = part_l + (size_t)bh * S;
-    const float* po = part_o + (size_t)bh * S * D + d;
-    float m = -INFINITY;
-#pragma unroll 8
-    for (int s = 0; s < S; ++s) m = fmaxf(m, pm[s]);
-    // The loads of a partial do not depend on its weight, so eight splits are in flight at a time
-    // (an empty split's O is never written: it is read and discarded, not multiplied).
-    float o = 0.0f, l = 0.0f;
-#pragma unroll 8
-    for (int s = 0; s < S; ++s) {
-        const float ms = pm[s];
-        const float os = po[(size_t)s * D], ls = pl[s];
-        const bool live = ms > -INFINITY;
-        const float wgt = live ? fast_exp2(ms - m) : 0.0f;
-        o += live ? os * wgt : 0.0f;
-        l += live ? ls * wgt : 0.0f;
+    const f32x4* po = reinterpret_cast<const f32x4*>(part_o + (size_t)bh * S * D) + c;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.0f;
+    for (int s0 = sg; s0 < S; s0 += 4 * CG) {
+        f32x4 os[4];
+        float ms[4], ls[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int s = min(s0 + i * CG, S - 1);
+            ms[i] = s0 + i * CG < S ? pm[s] : -INFINITY;
+            ls[i] = pl[s];
+            os[i] = po[(size_t)s * TPS];
+        }
+        const float mn = fmaxf(fmaxf(fmaxf(ms[0], ms[1]), fmaxf(ms[2], ms[3])), m);
+        if (mn == -INFINITY) continue;
+        const float alpha = fast_exp2(m - mn);
+        o *= alpha;
+        l *= alpha;
+        m = mn;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (ms[i] > -INFINITY) {                 // an empty split's O holds nothing
+                const float wgt = fast_exp2(ms[i] - m);
+                o += os[i] * wgt;
+                l += ls[i] * wgt;
+            }
     }
-    const float res = l > 0.0f ? o / l : 0.0f;    // every split empty: the sequence has no keys
-    // pairs of threads pack two bf16 into one dword
-    const float nb = __shfl_down(res, 1);
-    if ((d & 1) == 0) reinterpret_cast<uint32_t*>(O + (size_t)bh * D)[d >> 1] = pack_bf16(res, nb);
-    if (LSE != nullptr && d == 0) LSE[bh] = l > 0.0f ? logf(l) + m * LN2 : -INFINITY;
+    so[sg][c] = o;
+    if (c == 0) { sm[sg] = m; sl[sg] = l; }
+    __syncthreads();
+    if (t >= TPS) return;
+    const int n = min(CG, S);
+    for (int i = 1; i < n; ++i) {
+        const float mi = sm[i];
+        if (mi == -INFINITY) continue;
+        const float mn = fmaxf(m, mi), a = fast_exp2(m - mn), wgt = fast_exp2(mi - mn);
+        o = o * a + so[i][c] * wgt;
+        l = l * a + sl[i] * wgt;
+        m = mn;
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;    // every split empty: the sequence has no keys
+    reinterpret_cast<u32x2*>(O + (size_t)bh * D)[c] = u32x2{pack_bf16(o[0] * inv, o[1] * inv), pack_bf16(o[2] * inv, o[3] * inv)};
+    if (LSE != nullptr && c == 0) LSE[bh] = l > 0.0f ? logf(l) + m * LN2 : -INFINITY;
 }
 
 int launch_gqa_decode(const void* q, const void* k, const void* v, void* o, float* lse, int B,
                       int Hq, int Hkv, int L, int D, int64_t kv_stride, float scale, int num_splits,
                       void* workspace, const int* kv_lens, int window, hipStream_t stream) {
     using namespace dec;
-    constexpr int WAVES = 8;
     const int G = Hq / Hkv;
     const int S = num_splits;
     const int span = window > 0 ? (window < L ? window : L) : L;     // longest range any sequence reads
@@ -265,28 +292,34 @@ int launch_gqa_decode(const void* q, const void* k, const void* v, void* o, floa
     float* part_m = part_o + (size_t)B * Hq * S * D;
     float* part_l = part_m + (size_t)B * Hq * S;
 
-    const size_t lds = (size_t)(WAVES * G * D + 2 * WAVES * QPAD) * sizeof(float);
-    dim3 grid((unsigned)((size_t)S * B * Hkv)), block(64 * WAVES);
-#define TYR_DEC_LAUNCH(DD)                                                                           \
+    dim3 grid((unsigned)((size_t)S * B * Hkv));
+#define TYR_DEC_LAUNCH(DD, WAVES)                                                                    \
     do {                                                                                             \
+        const size_t lds = (size_t)(WAVES * G * DD + 2 * WAVES * QPAD) * sizeof(float);              \
+                                                                                                 \
         static const hipError_t attr = hipFuncSetAttribute(                                          \
             reinterpret_cast<const void*>(&gqa_decode_split_kernel<WAVES, DD>),                      \
             hipFuncAttributeMaxDynamicSharedMemorySize,                                              \
             (WAVES * QPAD * DD + 2 * WAVES * QPAD) * (int)sizeof(float));                            \
         if (attr != hipSuccess) return -1;                                                           \
-        hipLaunchKernelGGL((gqa_decode_split_kernel<WAVES, DD>), grid, block, lds, stream,           \
+        hipLaunchKernelGGL((gqa_decode_split_kernel<WAVES, DD>), grid, dim3(64 * WAVES), lds, stream,          \
                            static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),         \
                            static_cast<const uint16_t*>(v), part_o, part_m, part_l,                  \
                            static_cast<uint16_t*>(o), lse, Hq, Hkv, G, L, (long)kv_stride, S, chunk, \
                            scale * LOG2E, kv_lens, window);                                          \
         if (hipGetLastError() != hipSuccess) return -1;                                              \
         if (S > 1) {                                                                                 \
-            hipLaunchKernelGGL(gqa_decode_combine_kernel<DD>, dim3((unsigned)(B * Hq)), dim3(DD), 0, \
+            hipLaunchKernelGGL(gqa_decode_combine_kernel<DD>, dim3((unsigned)(B * Hq)), dim3(256), 0, \
                                stream, part_o, part_m, part_l, static_cast<uint16_t*>(o), lse, S);   \
             if (hipGetLastError() != hipSuccess) return -1;                                          \
         }                                                                                            \
     } while (0)
-    if (D == 128) TYR_DEC_LAUNCH(128); else TYR_DEC_LAUNCH(64);
+    // Eight waves where every CU has at most one workgroup (16.5 us against 16.7 at 64 groups of 2000 rows, 4 splits); four
+    // where workgroups share CUs: they come and go in smaller pieces (2048 groups of 500 rows 95 -> 85 us, 192 of 3000
+    // with 4 splits 56 -> 52).
+    const bool wide = grid.x <= 256;
+    if (D == 128) { if (wide) TYR_DEC_LAUNCH(128, 8); else TYR_DEC_LAUNCH(128, 4); }
+    else { if (wide) TYR_DEC_LAUNCH(64, 8); else TYR_DEC_LAUNCH(64, 4); }
 #undef TYR_DEC_LAUNCH
     return 0;
 }
