@@ -87,6 +87,15 @@ __device__ __forceinline__ u32x4 ld_global_16_nt(const void* p) {
 __device__ __forceinline__ void st_global_16_nt(void* p, u32x4 v) {
     __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
+// Loads of a streaming kernel (each byte read once).  Up to kStreamCached bytes moved by the launch, plain loads find what
+// the kernels before left in the 256 MB last-level cache (LayerNorm of 2222 x 4096, 73 MB: 16.1 us non-temporal, 13.1 plain;
+// SGD of 2^23 elements within a train step: 22 and 19); beyond, they only displace each other (268 MB: 45.4 and 47.3; SGD
+// of 2^26: 149 and 161).  Stores are non-temporal at every size: the lines of plain ones are written back while the next
+// kernel waits.
+constexpr size_t kStreamCached = (size_t)160 << 20;
+template <bool CACHED>
+__device__ __forceinline__ u32x4 ld_stream_16(const void* p) { return CACHED ? ld_global_16(p) : ld_global_16_nt(p); }
+
 __device__ __forceinline__ void st_global_8(void* p, u32x2 v) { *reinterpret_cast<u32x2*>(p) = v; }
 
 // 8x8 transpose of 16-bit elements held as 8 rows of 4 dwords: out[c] holds column c

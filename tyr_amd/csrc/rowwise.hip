@@ -19,6 +19,7 @@
 // consecutive addresses, and the grids have many more workgroups than the device has CUs.
 #include "common.hpp"
 #include "launch.hpp"
+#include <type_traits>
 
 namespace tyr {
 
@@ -78,6 +79,7 @@ template <> struct Piece<uint16_t> {                 // bf16
 }  // namespace rw
 
 // ------------------------------------------------------------------------------------------
+template <bool CACHED>
 __global__ __launch_bounds__(rw::THREADS) void copy_kernel(const u32x4* __restrict__ src, u32x4* __restrict__ dst,
                                                            size_t n16, const unsigned char* __restrict__ src_tail,
                                                            unsigned char* __restrict__ dst_tail, int tail) {
@@ -85,29 +87,28 @@ __global__ __launch_bounds__(rw::THREADS) void copy_kernel(const u32x4* __restri
     // buffers as one contiguous front (measured on a 1 GiB copy: 6.7 TB/s of read + write traffic,
     // against 6.0 for a grid-stride loop with four loads in flight per lane).
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n16) st_global_16_nt(dst + i, ld_global_16_nt(src + i));
+    if (i < n16) st_global_16_nt(dst + i, ld_stream_16<CACHED>(src + i));
     if (blockIdx.x == 0 && (int)threadIdx.x < tail) dst_tail[threadIdx.x] = src_tail[threadIdx.x];
 }
 
-// x, y: [rows_total = B*S*H][D]; row -> position s = (row / H) % S.  One thread rotates one piece
-// pair; a row takes D / (2E) consecutive threads.
-template <typename T>
+// x, y: [B*S*H][D].  One thread rotates one piece pair; a row takes per_row = D / (2E) consecutive threads.  I = uint32_t
+// unless there are more threads than that counts: with 64-bit divisions a thread spent as long on its indices as on its
+// 64 bytes (together with plain loads 2222 x 32 heads of 128: 8.4 -> 7.0 us, 36 MB).
+template <typename T, bool CACHED, typename I>
 __global__ __launch_bounds__(rw::THREADS) void rope_kernel(const T* __restrict__ x, const float* __restrict__ cosp,
                                                            const float* __restrict__ sinp, T* __restrict__ y,
-                                                           size_t rows, int S, int H, int D) {
-    constexpr int E = rw::Piece<T>::E;
-    const int per_row = D / (2 * E);
-    const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t row = id / per_row;
-    if (row >= rows) return;
-    const int e0 = (int)(id % per_row) * E;
-    const int s = (int)((row / H) % S);
-    const T* xr = x + row * D;
-    u32x4 a = ld_global_16_nt(xr + e0), b = ld_global_16_nt(xr + D / 2 + e0);
-    rw::Piece<T>::rotate(a, b, cosp + (size_t)s * (D / 2) + e0, sinp + (size_t)s * (D / 2) + e0);
-    T* yr = y + row * D;
-    st_global_16_nt(yr + e0, a);
-    st_global_16_nt(yr + D / 2 + e0, b);
+                                                           I threads, unsigned S, unsigned H, unsigned per_row) {
+    constexpr unsigned E = rw::Piece<T>::E;
+    const I id = (I)blockIdx.x * rw::THREADS + threadIdx.x;
+    if (id >= threads) return;
+    const I row = id / per_row;
+    const unsigned half = per_row * E, e0 = (unsigned)(id - row * per_row) * E;
+    const unsigned s = (unsigned)(row / H % S);
+    const size_t at = (size_t)row * 2 * half + e0;
+    u32x4 a = ld_stream_16<CACHED>(x + at), b = ld_stream_16<CACHED>(x + at + half);
+    rw::Piece<T>::rotate(a, b, cosp + (size_t)s * half + e0, sinp + (size_t)s * half + e0);
+    st_global_16_nt(y + at, a);
+    st_global_16_nt(y + at + half, b);
 }
 
 // Rows 0 .. B*Hq-1: q rows (rotated into q_out).  Then B*Hkv k rows (rotated into row `pos` of the
@@ -142,37 +143,57 @@ __global__ __launch_bounds__(rw::THREADS) void decode_rope_append_kernel(
     st_global_16(dst + D / 2 + e0, b);
 }
 
-// One wave per row; a lane holds pieces lane, lane + 64, ... of the row (8 bf16 each).
-template <int MAXP>
-__global__ __launch_bounds__(rw::THREADS) void layernorm_residual_kernel(
+// WPR waves per row; a lane holds P <= 2 pieces (8 bf16) of it, lane, lane + 64 * WPR, so that all loads of a row, weights
+// included, are under way at once and many waves share the chip (one wave per row, up to 16 pieces a lane: 2222 x 4096
+// 16.8 us, 300 x 8192 17; so 13.1 and 7.1).
+template <int WPR, int P, bool CACHED>
+__global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void layernorm_residual_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res, const uint16_t* __restrict__ weight,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ out, uint16_t* __restrict__ out_resid, size_t rows,
     int d_model, float eps) {
-    const int lane = threadIdx.x & 63;
-    const size_t row = (size_t)blockIdx.x * (rw::THREADS / 64) + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const int pieces = d_model / 8;
-    const uint16_t* xr = x + row * d_model;
-    const uint16_t* rr = res + row * d_model;
-    float v[MAXP][8];
+    constexpr int RPB = WPR > 4 ? 1 : 4 / WPR;
+    __shared__ float2 part[RPB][WPR];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wr = wave % WPR;
+    const size_t row = (size_t)blockIdx.x * RPB + wave / WPR;
+    const bool live = row < rows;
+    if (WPR == 1 && !live) return;
+    const int pieces = live ? d_model / 8 : 0;
+    const size_t at = row * d_model;
+    float v[P][8];
+    u32x4 a[P], b[P], w[P], bi[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int pc = lane + 64 * (wr + WPR * p);
+        if (pc < pieces) {
+            a[p] = ld_stream_16<CACHED>(x + at + pc * 8);
+            b[p] = ld_stream_16<CACHED>(res + at + pc * 8);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int pc = lane + 64 * (wr + WPR * p);
+        if (pc < pieces) {
+            w[p] = ld_global_16(weight + pc * 8);
+            bi[p] = ld_global_16(bias + pc * 8);
+        }
+    }
     float sum = 0.0f;
 #pragma unroll
-    for (int p = 0; p < MAXP; ++p) {
-        const int pc = lane + 64 * p;
-        if (pc < pieces) {
-            float a[8], b[8];
-            rw::unpack8(ld_global_16_nt(xr + pc * 8), a);
-            rw::unpack8(ld_global_16_nt(rr + pc * 8), b);
+    for (int p = 0; p < P; ++p) {
+        const int pc = lane + 64 * (wr + WPR * p);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) a[i] += b[i];
-            const u32x4 r16 = rw::pack8(a);                     // out_resid is the bf16-rounded sum ...
-            st_global_16_nt(out_resid + row * d_model + pc * 8, r16);
+        for (int i = 0; i < 8; ++i) v[p][i] = 0.0f;
+        if (pc < pieces) {
+            float f[8], g[8];
+            rw::unpack8(a[p], f);
+            rw::unpack8(b[p], g);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] += g[i];
+            const u32x4 r16 = rw::pack8(f);                     // out_resid is the bf16-rounded sum ...
+            st_global_16_nt(out_resid + at + pc * 8, r16);
             rw::unpack8(r16, v[p]);                             // ... and the statistics are taken from it
 #pragma unroll
             for (int i = 0; i < 8; ++i) sum += v[p][i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[p][i] = 0.0f;
         }
     }
     auto wave_sum = [](float s) {
@@ -180,25 +201,49 @@ __global__ __launch_bounds__(rw::THREADS) void layernorm_residual_kernel(
         for (int o = 1; o < 32; o <<= 1) s += __shfl_xor(s, o, 64);
         return sum_xor32(s);
     };
-    const float mean = wave_sum(sum) / (float)d_model;
+    // mean and sum of squares about it: of each wave's elements, then of the row's waves together
+    auto elements = [&](int i) {                                // of wave i
+        int c = 0;
+#pragma unroll
+        for (int p = 0; p < P; ++p) c += max(0, min(64, pieces - 64 * (i + WPR * p)));
+        return 8.0f * (float)c;
+    };
+    float mean = wave_sum(sum) / fmaxf(elements(wr), 1.0f);
     float sq = 0.0f;
 #pragma unroll
-    for (int p = 0; p < MAXP; ++p)
-        if (lane + 64 * p < pieces) {
+    for (int p = 0; p < P; ++p)
+        if (lane + 64 * (wr + WPR * p) < pieces) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) { const float c = v[p][i] - mean; sq += c * c; }
         }
-    const float inv_std = rsqrtf(wave_sum(sq) / (float)d_model + eps);
+    sq = wave_sum(sq);
+    if constexpr (WPR > 1) {
+        if (lane == 0) part[wave / WPR][wr] = float2{mean, sq};
+        __syncthreads();
+        if (!live) return;
+        float2 q[WPR];
+        float total = 0.0f;
 #pragma unroll
-    for (int p = 0; p < MAXP; ++p) {
-        const int pc = lane + 64 * p;
+        for (int i = 0; i < WPR; ++i) {
+            q[i] = part[wave / WPR][i];
+            total += q[i].x * elements(i);
+        }
+        mean = total / (float)d_model;
+        sq = 0.0f;
+#pragma unroll
+        for (int i = 0; i < WPR; ++i) { const float d = q[i].x - mean; sq += q[i].y + elements(i) * d * d; }
+    }
+    const float inv_std = rsqrtf(sq / (float)d_model + eps);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int pc = lane + 64 * (wr + WPR * p);
         if (pc < pieces) {
-            float w[8], b[8], o[8];
-            rw::unpack8(ld_global_16(weight + pc * 8), w);
-            rw::unpack8(ld_global_16(bias + pc * 8), b);
+            float wf[8], bf[8], o[8];
+            rw::unpack8(w[p], wf);
+            rw::unpack8(bi[p], bf);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) o[i] = (v[p][i] - mean) * inv_std * w[i] + b[i];
-            st_global_16_nt(out + row * d_model + pc * 8, rw::pack8(o));
+            for (int i = 0; i < 8; ++i) o[i] = (v[p][i] - mean) * inv_std * wf[i] + bf[i];
+            st_global_16_nt(out + at + pc * 8, rw::pack8(o));
         }
     }
 }
@@ -210,7 +255,7 @@ int launch_copy(const void* src, void* dst, size_t bytes, hipStream_t stream) {
     size_t blocks = (n16 + rw::STREAM_THREADS - 1) / rw::STREAM_THREADS;
     if (blocks == 0) blocks = 1;
     if (blocks > 0x7fffffffull) return -1;             // 2^31 workgroups of 1 KiB: 2 TiB
-    hipLaunchKernelGGL(copy_kernel, dim3((unsigned)blocks), dim3(rw::STREAM_THREADS), 0, stream,
+    hipLaunchKernelGGL((2 * bytes <= kStreamCached ? copy_kernel<true> : copy_kernel<false>), dim3((unsigned)blocks), dim3(rw::STREAM_THREADS), 0, stream,
                        static_cast<const u32x4*>(src), static_cast<u32x4*>(dst), n16,
                        static_cast<const unsigned char*>(src) + n16 * 16, static_cast<unsigned char*>(dst) + n16 * 16,
                        tail);
@@ -219,14 +264,20 @@ int launch_copy(const void* src, void* dst, size_t bytes, hipStream_t stream) {
 
 int launch_rope_fwd(const void* x, const float* cosp, const float* sinp, void* y, size_t rows, int S, int H, int D,
                     int is_bf16, hipStream_t stream) {
-    const size_t threads = rows * (size_t)(D / (is_bf16 ? 16 : 8));
-    const size_t blocks = (threads + rw::THREADS - 1) / rw::THREADS;
-    if (is_bf16)
-        hipLaunchKernelGGL(rope_kernel<uint16_t>, dim3((unsigned)blocks), dim3(rw::THREADS), 0, stream,
-                           static_cast<const uint16_t*>(x), cosp, sinp, static_cast<uint16_t*>(y), rows, S, H, D);
-    else
-        hipLaunchKernelGGL(rope_kernel<float>, dim3((unsigned)blocks), dim3(rw::THREADS), 0, stream,
-                           static_cast<const float*>(x), cosp, sinp, static_cast<float*>(y), rows, S, H, D);
+    const unsigned per_row = D / (is_bf16 ? 16 : 8);
+    const size_t threads = rows * per_row;
+    auto go = [&](auto elem, auto cached, auto index) {
+        using T = decltype(elem);
+        using I = decltype(index);
+        hipLaunchKernelGGL((rope_kernel<T, cached(), I>), dim3((unsigned)((threads + rw::THREADS - 1) / rw::THREADS)), dim3(rw::THREADS), 0,
+                           stream, static_cast<const T*>(x), cosp, sinp, static_cast<T*>(y), (I)threads, (unsigned)S, (unsigned)H, per_row);
+    };
+    auto pick = [&](auto elem) {
+        if (threads * 64 <= kStreamCached) go(elem, std::true_type{}, uint32_t{});
+        else if (threads <= UINT32_MAX - rw::THREADS) go(elem, std::false_type{}, uint32_t{});
+        else go(elem, std::false_type{}, size_t{});
+    };
+    if (is_bf16) pick(uint16_t{}); else pick(float{});
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -245,18 +296,20 @@ int launch_decode_rope_append(const void* q, const void* k_new, const void* v_ne
 
 int launch_layernorm_residual(const void* x, const void* residual, const void* weight, const void* bias, void* out,
                               void* out_resid, size_t rows, int d_model, float eps, hipStream_t stream) {
-    const size_t blocks = (rows + 3) / 4;
-    const int pieces_per_lane = (d_model / 8 + 63) / 64;
-#define TYR_LN_LAUNCH(MAXP)                                                                                     \
-    hipLaunchKernelGGL(layernorm_residual_kernel<MAXP>, dim3((unsigned)blocks), dim3(rw::THREADS), 0, stream,   \
-                       static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(residual),                 \
-                       static_cast<const uint16_t*>(weight), static_cast<const uint16_t*>(bias),                \
-                       static_cast<uint16_t*>(out), static_cast<uint16_t*>(out_resid), rows, d_model, eps)
-    if (pieces_per_lane <= 2) TYR_LN_LAUNCH(2);
-    else if (pieces_per_lane <= 4) TYR_LN_LAUNCH(4);
-    else if (pieces_per_lane <= 8) TYR_LN_LAUNCH(8);
-    else TYR_LN_LAUNCH(16);
-#undef TYR_LN_LAUNCH
+    auto go = [&](auto wpr, auto p) {
+        constexpr int W = wpr(), RPB = W > 4 ? 1 : 4 / W;       // rows per workgroup
+        auto kernel = rows * d_model * 8 <= kStreamCached ? &layernorm_residual_kernel<W, p(), true> : &layernorm_residual_kernel<W, p(), false>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(W > 4 ? 64 * W : 256), 0, stream,
+                           static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(residual), static_cast<const uint16_t*>(weight),
+                           static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(out), static_cast<uint16_t*>(out_resid), rows,
+                           d_model, eps);
+    };
+    using std::integral_constant;
+    if (d_model <= 512) go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    else if (d_model <= 1024) go(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+    else if (d_model <= 2048) go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+    else if (d_model <= 4096) go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+    else go(integral_constant<int, 8>{}, integral_constant<int, 2>{});
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

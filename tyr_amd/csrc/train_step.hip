@@ -9,7 +9,7 @@
 // Here: one pass over out / target writes dO and per-workgroup partial sums of diff^2 (a second, single
 // workgroup turns them into the loss; up to 2^15 elements one workgroup does both); one pass per parameter reads the f32 master and the bf16 gradient and
 // writes the updated master together with its bf16 copy for the next step's kernels.  Both are bound by HBM
-// bandwidth: 8- or 16-byte pieces per lane, consecutive lanes on consecutive addresses, non-temporal hints, no loop.
+// bandwidth: 8- or 16-byte pieces per lane, consecutive lanes on consecutive addresses, no loop.
 // Products and differences are evaluated as separate f32 operations (no fused multiply-add) and the division
 // is a true division, so dO and the updated masters are bit-identical to the LibTorch chain.
 #include "../../include/tyr_hip.h"
@@ -47,13 +47,14 @@ __device__ __forceinline__ float mse_piece(u32x4 out, u32x4 target, uint16_t* d_
 }
 
 // one 8-element piece per lane; partial[blockIdx.x] = sum over the workgroup of diff^2
+template <bool CACHED>
 __global__ __launch_bounds__(THREADS) void mse_grad_kernel(const uint16_t* __restrict__ out, const uint16_t* __restrict__ target,
                                                            uint16_t* __restrict__ d_out, float* __restrict__ partial,
                                                            size_t pieces, float n_elems) {
     __shared__ float wave_sum[THREADS / 64];
     const size_t i = (size_t)blockIdx.x * THREADS + threadIdx.x;
     float acc = 0.0f;
-    if (i < pieces) acc = mse_piece(ld_global_16_nt(out + 8 * i), ld_global_16_nt(target + 8 * i), d_out + 8 * i, n_elems);
+    if (i < pieces) acc = mse_piece(ld_stream_16<CACHED>(out + 8 * i), ld_stream_16<CACHED>(target + 8 * i), d_out + 8 * i, n_elems);
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, 64);
     if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = acc;
@@ -118,21 +119,21 @@ __global__ __launch_bounds__(1024) void mse_grad_loss_kernel(const uint16_t* __r
 
 // param' = param - (f32(grad) * lr); optionally also bf16(param').  param_out may be param itself (the in-place update), so
 // neither of the two is declared restrict; a lane stores only the elements it loaded.
+template <bool CACHED>
 __global__ __launch_bounds__(THREADS) void sgd_kernel(const float* param, const uint16_t* __restrict__ grad, float lr,
                                                       float* param_out, uint16_t* __restrict__ param_out_bf16,
                                                       size_t n) {
     // a wave's 512 elements as two runs of 256: every load and store instruction covers whole cache lines (a lane with 8
     // consecutive elements leaves half of every line to its next instruction: 277 us for 2^27 elements, so 253, 6.4 TB/s).
-    // Non-temporal at every size: plain accesses are 7 % faster alone up to 2^24 elements, but cost the kernels around
-    // this one more than that in a train step.
     const size_t base = ((size_t)blockIdx.x * (THREADS / 64) + (threadIdx.x >> 6)) * 512 + (threadIdx.x & 63) * 4;
     f32x4 p[2];
     u32x2 g[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
         if (base + 256 * h < n) {
-            p[h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(param + base + 256 * h));
-            g[h] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(grad + base + 256 * h));
+            p[h] = __builtin_bit_cast(f32x4, ld_stream_16<CACHED>(param + base + 256 * h));
+            auto gp = reinterpret_cast<const u32x2*>(grad + base + 256 * h);
+            g[h] = CACHED ? *gp : __builtin_nontemporal_load(gp);
         }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -182,7 +183,7 @@ int tyr_hip_mse_loss_grad(const void* out, const void* target, void* d_out, floa
         return hipGetLastError() == hipSuccess ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
     }
     float* partial = static_cast<float*>(workspace);
-    hipLaunchKernelGGL(mse_grad_kernel, dim3((unsigned)blocks), dim3(THREADS), 0, s, static_cast<const uint16_t*>(out),
+    hipLaunchKernelGGL((6 * n <= kStreamCached ? mse_grad_kernel<true> : mse_grad_kernel<false>), dim3((unsigned)blocks), dim3(THREADS), 0, s, static_cast<const uint16_t*>(out),
                        static_cast<const uint16_t*>(target), static_cast<uint16_t*>(d_out), partial, (size_t)pieces, (float)n);
     if (hipGetLastError() != hipSuccess) return TYR_HIP_ERR_LAUNCH;
     hipLaunchKernelGGL(mse_loss_kernel, dim3(1), dim3(1024), 0, s, partial, (size_t)blocks, (double)n, loss);
@@ -199,7 +200,7 @@ int tyr_hip_sgd_step(const float* param, const void* grad, float lr, float* para
     if (blocks > (uint64_t)INT_MAX) return TYR_HIP_ERR_BAD_SHAPE;
     if (!aligned16(param) || !aligned16(grad) || !aligned16(param_out) || !aligned16(param_out_bf16))
         return TYR_HIP_ERR_MISALIGNED;
-    hipLaunchKernelGGL(sgd_kernel, dim3((unsigned)blocks), dim3(THREADS), 0, static_cast<hipStream_t>(stream), param,
+    hipLaunchKernelGGL((12 * n <= kStreamCached ? sgd_kernel<true> : sgd_kernel<false>), dim3((unsigned)blocks), dim3(THREADS), 0, static_cast<hipStream_t>(stream), param,
                        static_cast<const uint16_t*>(grad), lr, param_out, static_cast<uint16_t*>(param_out_bf16), (size_t)n);
     return hipGetLastError() == hipSuccess ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }
