@@ -59,3 +59,45 @@ def test_every_launch_form_matches_the_f32_reference(B, Hq, Hkv, N, D, mask):
         assert float((err / n.clamp_min(float(n[n > 0].mean()))).max()) <= 4e-2
     again = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)
     assert all(torch.equal(a, b) for a, b in zip(grads, again))
+
+
+def padded_masks(N):
+    """Key masks by what is hidden: nothing, either end across tile edges, both, all but one key, a hole of whole tiles, all."""
+    i = torch.arange(N)
+    return torch.stack([i >= 0, i >= 64, i >= min(63, N - 1), i >= min(65, N - 1), i >= N // 2, i < N - N // 3, (i >= N // 4) & (i < N - N // 4),
+                        i == N - 1, i == 0, (i < 40) | (i >= N - 40), i < 0])
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,N,D", [(1, 1, 3, 64), (2, 1, 65, 128), (4, 2, 130, 64), (4, 1, 700, 128), (16, 4, 700, 64), (2, 2, 1350, 128)])
+def test_tiles_hidden_by_the_key_mask_are_skipped(Hq, Hkv, N, D, causal):
+    import tyr_amd
+    gen = torch.Generator(device="cuda").manual_seed(N + D)
+    mask = padded_masks(N).cuda().contiguous()
+    B = mask.shape[0]
+    q, k, v, g = (torch.randn(B, h, N, D, device="cuda", generator=gen).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    i = torch.arange(N, device="cuda")
+    visible = mask[:, None, None, :].expand(B, 1, N, N)
+    if causal:
+        visible = visible & (i[None, :] <= i[:, None])
+    opt = dict(causal=causal, key_mask=mask)
+    o, lse = tyr_amd.flash_attn_fwd(q, k, v, **opt)
+    grads = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)
+
+    rq, rk, rv = (t.float().requires_grad_() for t in (q, k, v))
+    kk, vv = rk.repeat_interleave(Hq // Hkv, 1), rv.repeat_interleave(Hq // Hkv, 1)
+    s = (torch.matmul(rq, kk.transpose(-1, -2).contiguous()) / math.sqrt(D)).masked_fill(~visible, -1e30)
+    m = s.detach().amax(-1, keepdim=True)
+    p = torch.exp(s - m) * visible
+    total = p.sum(-1, keepdim=True)
+    want_o = torch.matmul(p / total.clamp_min(1e-30), vv)
+    seen = visible.any(-1).expand(B, Hq, N)
+    want_lse = (m + torch.log(total)).squeeze(-1).detach()
+    want = torch.autograd.grad(want_o, (rq, rk, rv), g.float())
+    assert torch.equal(torch.isneginf(lse), ~seen) and not bool(o[~seen].any())
+    assert float((o.float() - want_o).abs().max()) <= 2e-2
+    assert float((lse - want_lse)[seen].abs().max()) <= 2e-2
+    used = visible.any(-2).expand(B, Hkv, N)             # keys that some query sees
+    for got, ref, alive in zip(grads, want, (seen, used, used)):
+        assert rel_fro(got, ref) <= 1e-2
+        assert not bool(got[~alive].any())

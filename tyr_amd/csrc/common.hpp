@@ -295,6 +295,43 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t pid, uint32_t n) {
     return (pid % 8u) * (n / 8u) + pid / 8u;
 }
 
+// What an attention launch masks besides the causal rule: nothing, lengths and / or a window, or a key mask.
+enum class AttnMask { None, Limits, Keys };
+
+// ---- key mask: the 64-key tiles among keys [0, end) that hold a visible one lie in [first, last) ------------------
+// Read from both ends, 8 tiles an end and round (one byte a lane and tile, all 16 loads in flight), until a visible key is
+// met: one memory latency where nothing is hidden at the ends, and a padded batch's empty tiles cost 1/8 of one each
+// instead of a step of the attention loop (1 us).  end >= 1; nothing visible: first == last.
+struct TileSpan { int first, last; };
+__device__ __forceinline__ TileSpan visible_tiles(const uint8_t* mask, int end, int lane) {
+    constexpr int AT_ONCE = 8;
+    TileSpan s{0, (end + 63) / 64};
+    bool front = false, back = false;
+    while (s.first < s.last && !(front && back)) {
+        uint8_t f[AT_ONCE], b[AT_ONCE];
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+            f[u] = mask[min((s.first + u) * 64 + lane, end - 1)];
+            b[u] = mask[max(0, min((s.last - 1 - u) * 64 + lane, end - 1))];
+        }
+        uint32_t in_front = 0, in_back = 0;
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+            in_front |= (uint32_t)(__builtin_amdgcn_ballot_w64(f[u] != 0) != 0) << u;
+            in_back |= (uint32_t)(__builtin_amdgcn_ballot_w64(b[u] != 0) != 0) << u;
+        }
+        if (!front) {
+            front = in_front != 0;
+            s.first = front ? s.first + __builtin_ctz(in_front) : min(s.first + AT_ONCE, s.last);
+        }
+        if (!back) {
+            back = in_back != 0;
+            s.last = back ? s.last - __builtin_ctz(in_back) : max(s.last - AT_ONCE, s.first);
+        }
+    }
+    return {__builtin_amdgcn_readfirstlane(s.first), __builtin_amdgcn_readfirstlane(max(s.first, s.last))};
+}
+
 // ---- order of the query tiles of an attention launch ---------------------------------------------------------
 // A launch has one job per (query head, tile rank); rank 0 is the longest causal tile.  Consecutive workgroup ids go to the
 // 8 XCDs in turn, and of the ids an XCD gets, id i and id i + 32 share a CU (two workgroups fit).

@@ -122,10 +122,10 @@ __device__ __forceinline__ void store_transposed_bf16(const f32x16 (&acc)[D / 32
 
 // ------------------------------------------------------------------------------------------
 // dQ (and the (lse2, delta) pairs)
-// EXT adds the per-sequence key length and the sliding window (same rule as the forward kernel);
+// MASK as in the forward kernel;
 // G = query heads per kv head.  SPLIT: 64 query rows per workgroup, the two 32-key sub-tiles of a tile on two waves whose
 // dQ are added through LDS at the end (same use as in the forward kernel: launches with few tiles).
-template <int D, bool CAUSAL, bool EXT, bool SPLIT>
+template <int D, bool CAUSAL, AttnMask MASK, bool SPLIT>
 __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
@@ -134,6 +134,7 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
     const uint8_t* __restrict__ key_mask, int pair, int single) {
     using namespace fab;
     using C = CfgQ<D>;
+    constexpr bool LIMITS = MASK == AttnMask::Limits, KEYS = MASK == AttnMask::Keys;
     constexpr int TBM = SPLIT ? 64 : C::BM;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
@@ -154,12 +155,12 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
     const size_t head_off = (size_t)bh * N * D;
     const uint16_t* Kh = Kp + (size_t)kvbh * N * D;
     const uint16_t* Vh = Vp + (size_t)kvbh * N * D;
-    const int Nk = (EXT && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / Hq])) : N;
-    const uint8_t* km = (EXT && key_mask != nullptr) ? key_mask + (size_t)(bh / Hq) * N : nullptr;
+    const int Nk = (LIMITS && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / Hq])) : N;
+    const uint8_t* km = KEYS ? key_mask + (size_t)(bh / Hq) * N : nullptr;
     const int kv_end = CAUSAL ? min(Nk, q0 + TBM) : Nk;
     const int nkv_abs = max(1, (kv_end + C::BN - 1) / C::BN);   // a sequence without keys still walks one (fully masked) tile
-    const int jbase = (EXT && window > 0) ? min(max(0, q0 - window + 1) / C::BN, nkv_abs - 1) : 0;
-    const int nkv = nkv_abs - jbase;             // tiles are numbered from jbase below
+    int jbase = (LIMITS && window > 0) ? min(max(0, q0 - window + 1) / C::BN, nkv_abs - 1) : 0;
+    int nkv = nkv_abs - jbase;                   // tiles are numbered from jbase below
     const int qpos = qw0 + r;
 
     // ---- this wave's Q^T and dO^T fragments (lane = query row, columns 16i + 8g + [0,8)),
@@ -180,7 +181,7 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
         }
         delta = part + xor32(part);
         lse2 = LSE[(size_t)bh * N + qrow] * LOG2E;
-        if (EXT && lse2 == -INFINITY) lse2 = INFINITY;      // a row that saw no key: every probability is 0
+        if (MASK != AttnMask::None && lse2 == -INFINITY) lse2 = INFINITY;      // a row that saw no key: every probability is 0
         if (g == 0 && T0 == 0) {
             stats[(size_t)bh * npad + qpos] = qpos < N ? make_float2(lse2, delta) : make_float2(INFINITY, 0.0f);
         }
@@ -230,9 +231,21 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
 #pragma unroll
         for (int e = 0; e < 16; ++e) dq[i][e] = 0.0f;
 
+    issue_kv(0, jbase * C::BN);
+    uint64_t next_hidden = 0;                    // KEYS: bit r set = kv row r of the next step's tile is hidden
+    if constexpr (KEYS) {                        // tiles before the first and after the last visible key are not walked
+        const TileSpan span = visible_tiles(km, kv_end, lane);
+        const int end = max(1, span.last);
+        jbase = min(span.first, end - 1);
+        nkv = end - jbase;
+        if (jbase > 0) {
+            wait_vmcnt0();
+            issue_kv(0, jbase * C::BN);
+        }
+        next_hidden = __builtin_amdgcn_ballot_w64(km[min(jbase * C::BN + lane, N - 1)] == 0);
+    }
     const int nkv_w = CAUSAL ? min(nkv, (qw0 + 31) / C::BN + 1 - jbase) : nkv;
 
-    issue_kv(0, jbase * C::BN);
 #pragma unroll
     for (int i = 0; i < C::KSTEPS; ++i) { pin_registers(qf[i]); pin_registers(dof[i]); }
     wait_vmcnt0();
@@ -240,6 +253,11 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
 
     for (int j = 0; j < nkv; ++j) {
         const int j0 = (jbase + j) * C::BN;
+        // the tile's 64 key-mask bytes as one word (bit r set: kv row j0 + r is hidden): one byte per lane and a ballot,
+        // read one step ahead; a tile without hidden rows skips the masking
+        const uint64_t tile_hidden = next_hidden;
+        uint32_t mask_byte = 1;
+        if (KEYS && j + 1 < nkv) mask_byte = km[min(j0 + C::BN + lane, N - 1)];
         if (j + 1 < nkv) issue_kv((j + 1) & 1, j0 + C::BN);
         if (j < nkv_w) {
             const unsigned char* Kt = lds + (j & 1) * C::TILE + (SPLIT ? T0 * 32 * C::ROW : 0);
@@ -249,12 +267,8 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
             // needs; the other wave of the SIMD has matrix work while this one does its exponentials.
             f32x16 s[2], dp[2];
             bf16x8 dsf[4];
-            // the tile's 64 key-mask bytes as one word (bit r set: kv row j0 + r is hidden): one byte per
-            // lane and a ballot; a tile without hidden rows skips the masking
-            uint64_t tile_hidden = 0;
-            if (EXT && km != nullptr) tile_hidden = __builtin_amdgcn_ballot_w64(km[min(j0 + lane, N - 1)] == 0);
             const bool need_mask = (CAUSAL && (j0 + C::BN - 1 > qw0)) || (j0 + C::BN > Nk) ||
-                                   (EXT && window > 0 && j0 < qw0 + 32 - window) || (EXT && tile_hidden != 0);
+                                   (LIMITS && window > 0 && j0 < qw0 + 32 - window) || (KEYS && tile_hidden != 0);
             // Fragments are read one k-step ahead of the products that take them, also across the phases of a tile (the
             // first fragments of a phase are requested under the last products of the phase before it), and the
             // scheduling barriers keep that order: left to itself the compiler, at its register limit, puts every read
@@ -289,13 +303,13 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
             auto probabilities = [&](int T) {
                 if (need_mask) {
                     const int lim = CAUSAL ? min(qpos, Nk - 1) : Nk - 1;
-                    const int low = (EXT && window > 0) ? qpos - window + 1 : INT_MIN;
+                    const int low = (LIMITS && window > 0) ? qpos - window + 1 : INT_MIN;
                     const int base = j0 + 32 * T0 + 4 * g;
                     const uint64_t hidden = tile_hidden >> (4 * g + 32 * (T0 + T));      // shifted to this lane's rows
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
                         const int kv = base + 32 * T + 8 * (e >> 2) + (e & 3);
-                        const bool off = kv > lim || (EXT && kv < low) || ((hidden >> (8 * (e >> 2) + (e & 3))) & 1u);
+                        const bool off = kv > lim || (LIMITS && kv < low) || ((hidden >> (8 * (e >> 2) + (e & 3))) & 1u);
                         s[T][e] = off ? -INFINITY : s[T][e];
                     }
                 }
@@ -342,6 +356,7 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
             }
         }
         wait_vmcnt0();
+        if constexpr (KEYS) next_hidden = __builtin_amdgcn_ballot_w64(mask_byte == 0);
         __syncthreads();
     }
 
@@ -378,8 +393,10 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
 // ------------------------------------------------------------------------------------------
 // dK, dV
 // BHkv = batch * kv heads; the G query heads of a kv head are walked one after the other and
-// accumulate into the same dK / dV (the gradient of repeat_interleave).  EXT as above; with it
-// every step carries the mask instructions.
+// accumulate into the same dK / dV (the gradient of repeat_interleave).  A lane owns one
+// key, so lengths and key masks (Keys) need no instructions in the steps: what a hidden key's lane summed is set to zero at
+// the end, and a block of 128 hidden keys walks no query (padded batch of 8, 2000 rows, whole backward: 933 -> 428 us with a
+// key mask, 747 -> 558 with lengths).  Limits is a window, with or without lengths: its steps carry mask instructions.
 // Where (key tile, kv head) pairs are too few or too unequal for the device (causal: the first key tile meets every query
 // tile, the last one two; all times G), the steps of a key tile -- its 64-row query tiles, head after head -- are cut
 // into equal parts of at most `chunk` for as many workgroups, which leave f32 partial sums that flash_attn_bwd_sum_kernel adds.
@@ -413,13 +430,14 @@ struct Parts {
 
 // CUT: the launch has parts.  (Whole key tiles keep their own instantiation: with the bookkeeping of the parts in the same
 // code the pipeline below, which has no register to spare, is 4-8 % slower.)
-template <int D, bool CAUSAL, bool EXT, bool CUT>
+template <int D, bool CAUSAL, AttnMask MASK, bool CUT>
 __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     const uint16_t* __restrict__ dO, const float2* __restrict__ stats, uint16_t* __restrict__ dK,
     uint16_t* __restrict__ dV, int BHkv, int N, int ntk, int npad, float scale, float scale_log2,
     int Hq, int window, const int* __restrict__ kv_lens, const uint8_t* __restrict__ key_mask, fab::Parts plan, int items,
     float* __restrict__ partial) {
+    constexpr bool WINDOW = MASK == AttnMask::Limits, PER_KEY = MASK != AttnMask::None;
     const int G = plan.G;
     using namespace fab;
     using C = CfgK<D>;
@@ -451,9 +469,13 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     const size_t head_off = (size_t)bh * N * D;                       // of K, V, dK, dV
     const int hkv = Hq / G;
     const size_t qh0 = (size_t)(bh / hkv) * Hq + (size_t)(bh % hkv) * G;   // first query head of the group
-    const int Nk = (EXT && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / hkv])) : N;
-    // this lane's key is hidden from every query by the key mask
-    const bool key_off = EXT && key_mask != nullptr && key_mask[(size_t)(bh / hkv) * N + min(kvpos, N - 1)] == 0;
+    const int Nk = (PER_KEY && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / hkv])) : N;
+    // no key of the block is seen by any query (beyond the length, or all 128 hidden by the key mask)
+    bool block_hidden = PER_KEY && n0 >= Nk;
+    if (PER_KEY && key_mask != nullptr && !block_hidden) {
+        const TileSpan span = visible_tiles(key_mask + (size_t)(bh / hkv) * N + n0, min(C::BNK, Nk - n0), lane);
+        block_hidden = span.first >= span.last;
+    }
 
     // ---- this wave's K and V rows as column operands (lane = key row, columns 16i + 8g + [0,8))
     bf16x8 kf[C::KSTEPS], vf[C::KSTEPS];
@@ -605,8 +627,7 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
 #pragma unroll
                 for (int x = 0; x < 4; ++x) {
                     const int qrow = qs0 + 8 * (2 * sh + h) + 4 * g + x;
-                    const bool hidden = (CAUSAL && kvpos > qrow) ||
-                                        (EXT && ((window > 0 && qrow - kvpos >= window) || kvpos >= Nk || key_off));
+                    const bool hidden = (CAUSAL && kvpos > qrow) || (WINDOW && qrow - kvpos >= window);
                     if (hidden) p[x] = 0.0f;
                 }
             }
@@ -636,12 +657,10 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
         }
     };
 
-    // With EXT a step applies the mask only where some pair of the 64 query rows it touches (the second
-    // half of u, the first half of u+1) is hidden from this wave's keys: a key at or beyond the sequence's
-    // length or switched off by the key mask, the causal diagonal, the far edge of the window.
-    const bool wave_key_hidden = EXT && __builtin_amdgcn_ballot_w64(kvpos >= Nk || key_off) != 0;
+    // With WINDOW a step applies the mask only where some pair of the 64 query rows it touches (the second
+    // half of u, the first half of u+1) is hidden from this wave's keys: the causal diagonal, the far edge of the window.
     auto rows_are_masked = [&](int qs0) {
-        return wave_key_hidden || (CAUSAL && qs0 < nw0 + 32) || (window > 0 && qs0 + 63 - nw0 >= window);
+        return (CAUSAL && qs0 < nw0 + 32) || (window > 0 && qs0 + 63 - nw0 >= window);
     };
     bf16x8 rq[C::KSTEPS], rd[C::KSTEPS];              // row fragments of the next sub-tile, read one step ahead
     bf16x8 pf0, dsf0;                                 // P, dS of the first half of the current sub-tile
@@ -712,7 +731,7 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     };
     // What a step expects of the step before it, for the wave's first sub-tile: its scores, P and dS
     // of its first half, the pairs of its second half, and the row fragments of the sub-tile after
-    // it.  Without EXT the only partially masked sub-tile of a causal wave is this one (its
+    // it.  Without WINDOW the only partially masked sub-tile of a causal wave is this one (its
     // diagonal): hidden scores become -inf here, which the steps turn into P = 0 and dS = 0 like any
     // other score, so they carry no mask instructions.
     auto first_scores = [&](auto masked, auto stg, auto sub, int qs0, f32x16& sc, f32x16& dpc) {
@@ -724,7 +743,7 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
         read_pairs(stg, sub, Half0{}, st0);
         read_pairs(stg, sub, Half1{}, st1);
         scores(rq, rd, sc, dpc);
-        if (CAUSAL && !EXT) {
+        if (CAUSAL && !WINDOW) {
 #pragma unroll
             for (int e = 0; e < 16; ++e)
                 if (kvpos > qs0 + 8 * (e >> 2) + 4 * g + (e & 3)) sc[e] = -INFINITY;
@@ -736,9 +755,9 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
 
 #pragma unroll
     for (int i = 0; i < C::KSTEPS; ++i) { pin_registers(kf[i]); pin_registers(vf[i]); }
-    // this part's steps of the block; a block whose keys all lie beyond the sequence's length has none (its rows are 0)
+    // this part's steps of the block; a block that no query sees has none (its rows are 0)
     const int per_head = jq_last - jq_first, per_part = CUT ? plan.part_steps(kt) : 0;
-    const int step_end = EXT && n0 >= Nk ? 0 : CUT ? min(G * per_head, (part + 1) * per_part) : G;
+    const int step_end = block_hidden ? 0 : CUT ? min(G * per_head, (part + 1) * per_part) : G;
     for (int step_at = CUT ? part * per_part : 0; step_at < step_end;) {
     if constexpr (CUT) {
         hq = step_at / per_head;
@@ -770,7 +789,7 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
         }
     };
     using std::integral_constant;
-    using MaskedT = integral_constant<bool, EXT>;
+    using MaskedT = integral_constant<bool, WINDOW>;
     const int qbase = jq0 * C::BQ;
     // Scores ping-pong between two register sets by the parity of u (no copies).
     f32x16 sA, dpA, sB, dpB;
@@ -813,6 +832,14 @@ pipeline_done:
     __syncthreads();
     }
 
+    if constexpr (PER_KEY) {
+        if (kvpos >= Nk || (key_mask != nullptr && key_mask[(size_t)(bh / hkv) * N + min(kvpos, N - 1)] == 0)) {
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) dv[dt][e] = dk[dt][e] = 0.0f;
+        }
+    }
     if (CUT && plan.parts(kt) > 1) {
         // [2 (dV, dK)][wave][register group of four][lane] f32x4: coalesced as the accumulators lie
         f32x4* out = reinterpret_cast<f32x4*>(partial) + ((size_t)bh * items + item) * (2 * 4 * C::DT * 4 * 64) + w * (C::DT * 4 * 64) + lane;
@@ -962,7 +989,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     using namespace fab;
     const int BH = B * Hq, BHkv = B * Hkv, G = Hq / Hkv;
     const int ntk = (N + 127) / 128, npad = ntk * 128;
-    const bool ext = window > 0 || kv_lens != nullptr || key_mask != nullptr;
+    const bool limits = window > 0 || kv_lens != nullptr;     // never together with a key mask
     const AttnShape shape = attn_shape(BH, N, D, causal != 0, window);
     const int ntq = (N + shape.rows - 1) / shape.rows;
     const int pair = shape.pair, single = shape.single;
@@ -1001,25 +1028,35 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
                            static_cast<uint16_t*>(dv), BHkv, N, ntk, npad, scale, scale_log2, Hq,     \
                            window, kv_lens, key_mask, plan, items, partial);                          \
     } while (0)
+#define TYR_FAB_DKV_MASK(DD, CC, EE, UU)      /* lengths alone are a mask of keys here */             \
+    do {                                                                                              \
+        if (EE == AttnMask::Limits && window <= 0) TYR_FAB_DKV(DD, CC, AttnMask::Keys, UU);           \
+        else TYR_FAB_DKV(DD, CC, EE, UU);                                                             \
+    } while (0)
 #define TYR_FAB_LAUNCH(DD, CC, EE)                                                                    \
     do {                                                                                              \
         if (shape.rows == 64) TYR_FAB_DQ(DD, CC, EE, true); else TYR_FAB_DQ(DD, CC, EE, false);       \
         if (plan.chunk) {                                                                             \
-            TYR_FAB_DKV(DD, CC, EE, true);                                                            \
+            TYR_FAB_DKV_MASK(DD, CC, EE, true);                                                            \
             hipLaunchKernelGGL(flash_attn_bwd_sum_kernel<DD>, dim3((unsigned)(BHkv * ntk * (DD / 8))), dim3(256), 0, stream, \
                                partial, static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), N, ntk, items, scale, plan); \
         } else {                                                                                      \
-            TYR_FAB_DKV(DD, CC, EE, false);                                                           \
+            TYR_FAB_DKV_MASK(DD, CC, EE, false);                                                           \
         }                                                                                             \
     } while (0)
-#define TYR_FAB_PICK(DD)                                                                              \
+#define TYR_FAB_PICK(DD, MM)                                                                          \
+    do { if (causal) TYR_FAB_LAUNCH(DD, true, MM); else TYR_FAB_LAUNCH(DD, false, MM); } while (0)
+#define TYR_FAB_MASK(DD)                                                                              \
     do {                                                                                              \
-        if (ext) { if (causal) TYR_FAB_LAUNCH(DD, true, true); else TYR_FAB_LAUNCH(DD, false, true); }    \
-        else     { if (causal) TYR_FAB_LAUNCH(DD, true, false); else TYR_FAB_LAUNCH(DD, false, false); }  \
+        if (key_mask != nullptr) TYR_FAB_PICK(DD, AttnMask::Keys);                                    \
+        else if (limits) TYR_FAB_PICK(DD, AttnMask::Limits);                                          \
+        else TYR_FAB_PICK(DD, AttnMask::None);                                                        \
     } while (0)
-    if (D == 128) TYR_FAB_PICK(128); else TYR_FAB_PICK(64);
+    if (D == 128) TYR_FAB_MASK(128); else TYR_FAB_MASK(64);
+#undef TYR_FAB_MASK
 #undef TYR_FAB_PICK
 #undef TYR_FAB_LAUNCH
+#undef TYR_FAB_DKV_MASK
 #undef TYR_FAB_DKV
 #undef TYR_FAB_DQ
     return hipGetLastError() == hipSuccess ? 0 : -1;

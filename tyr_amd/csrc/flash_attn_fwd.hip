@@ -69,12 +69,13 @@ template <int D> __device__ __forceinline__ int k_swz(int row, int c) { return c
 template <int D> __device__ __forceinline__ int v_swz(int row, int c) { return c ^ (((row & 3) << 2) & (Cfg<D>::KCH - 1)); }
 }  // namespace fa
 
-// EXT adds the per-sequence key length (padding mask over the tail) and the sliding window; the
-// plain instantiation carries none of their instructions.  G = query heads per kv head.
+// MASK: Limits adds the per-sequence key length (padding mask over the tail) and the sliding window, Keys the key mask; an
+// instantiation carries none of the others' instructions (the scalar registers of the one cost the other 3 %).
+// G = query heads per kv head.
 // SPLIT (launches with few tiles): a workgroup takes 64 query rows; waves w and w + 2 own the same 32 rows, one the first
 // and one the second 32 keys of every tile, and merge their (m, l, O) through LDS at the end.  Half the work per tile
 // step and twice the workgroups; the step's requests and barrier cost what they did, so it pays only on an idle device.
-template <int D, bool CAUSAL, bool EXT, bool SPLIT>
+template <int D, bool CAUSAL, AttnMask MASK, bool SPLIT>
 __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     uint16_t* __restrict__ O, float* __restrict__ LSE, int BH, int N, int ntq, float scale_log2,
@@ -82,6 +83,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     int single, int total_ids) {
     using namespace fa;
     using C = Cfg<D>;
+    constexpr bool LIMITS = MASK == AttnMask::Limits, KEYS = MASK == AttnMask::Keys;
     constexpr int TBM = SPLIT ? 64 : BM;         // query rows of a workgroup
     constexpr int NT = SPLIT ? 1 : 2;            // 32-key sub-tiles of a key tile that a wave computes
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -127,13 +129,13 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
 
     // keys at or beyond Nk are masked (Nk = 0: the sequence has no keys, O = 0 and LSE = -inf); with a window,
     // query i sees keys (i - window, i]
-    const int Nk = (EXT && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / Hq])) : N;
+    const int Nk = (LIMITS && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / Hq])) : N;
     // per-sequence key mask (nonzero = visible), any pattern
-    const uint8_t* km = (EXT && key_mask != nullptr) ? key_mask + (size_t)(bh / Hq) * N : nullptr;
+    const uint8_t* km = KEYS ? key_mask + (size_t)(bh / Hq) * N : nullptr;
     const int kv_end = CAUSAL ? min(Nk, q0 + TBM) : Nk;
     const int nkv_abs = max(1, (kv_end + BN - 1) / BN);   // a sequence without keys still walks one (fully masked) tile
-    const int jbase = (EXT && window > 0) ? min(max(0, q0 - window + 1) / BN, nkv_abs - 1) : 0;   // first tile any row sees
-    const int nkv = nkv_abs - jbase;             // tiles are numbered from jbase below
+    int jbase = (LIMITS && window > 0) ? min(max(0, q0 - window + 1) / BN, nkv_abs - 1) : 0;   // first tile any row sees
+    int nkv = nkv_abs - jbase;                   // tiles are numbered from jbase below
 
     auto load_q = [&](int first_row) {
         const int qrow = min(first_row + r, N - 1);
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     // running row maximum, in log2 units (score * scale * log2 e).  With a window a row's first
     // tiles can be wholly masked; a finite start keeps (-inf) - m2 from becoming NaN there.
     // (SPLIT: so can the keys of one wave.)
-    float m2 = EXT || SPLIT ? -1.0e30f : -INFINITY;
+    float m2 = LIMITS || KEYS || SPLIT ? -1.0e30f : -INFINITY;
     float lsum = 0.0f;         // this lane's share of the running row sum
 
     // K fragment (sub-tile T, k-step i): row 32T + r, chunk 2i + g.
@@ -207,13 +209,6 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
         }
     }
     const int qpos = qw0 + r;
-    // The second tile of a pair starts under the end of the first: its K(0), K(1) are requested
-    // in the first tile's last two steps (stage parity needs an even tile count), its Q rows
-    // before the first tile's output is written.
-    const bool overlap_next = has_next && (nkv & 1) == 0 && !(EXT && window > 0);
-    // number of kv tiles that intersect this wave's visible region
-    const int nkv_w = CAUSAL ? min(nkv, (qw0 + 31) / BN + 1 - jbase) : nkv;
-
     constexpr int NG = C::KSTEPS / 2;            // S^T is built in NG groups of (2 k-steps x 2 sub-tiles)
     auto read_k_group = [&](const unsigned char* Kt, int grp, bf16x8 (&dst)[2 * NT]) {
 #pragma unroll
@@ -239,6 +234,29 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     } else {
         issue_v(0, 0);                           // K(0), K(1) and Q were requested by the first tile
     }
+    uint64_t next_hidden = 0;                    // KEYS: bit r set = row r of the next step's tile is hidden
+    if constexpr (KEYS) {
+        // Tiles before the first and after the last visible key are not walked: a batch of 8 padded on the left to 2000 rows
+        // 183 -> 122 us.  The mask is read under the requests above, which are the right ones where nothing is padded.
+        const TileSpan span = visible_tiles(km, kv_end, lane);
+        const int end = max(1, span.last);
+        jbase = min(span.first, end - 1);
+        nkv = end - jbase;
+        if (jbase > 0) {
+            wait_vmcnt0();
+            issue_k(0, jbase * BN);
+            issue_v(0, jbase * BN);
+            if (nkv > 1) issue_k(1, (jbase + 1) * BN);
+        }
+        next_hidden = __builtin_amdgcn_ballot_w64(km[min(jbase * BN + lane, N - 1)] == 0);
+    }
+    // The second tile of a pair starts under the end of the first: its K(0), K(1) are requested
+    // in the first tile's last two steps (stage parity needs an even tile count), its Q rows
+    // before the first tile's output is written.
+    const bool overlap_next = has_next && (nkv & 1) == 0 && !KEYS && !(LIMITS && window > 0);
+    // number of kv tiles that intersect this wave's visible region
+    const int nkv_w = CAUSAL ? min(nkv, (qw0 + 31) / BN + 1 - jbase) : nkv;
+
 #pragma unroll
     for (int i = 0; i < C::KSTEPS; ++i) pin_registers(qf[i]);
     wait_vmcnt0();
@@ -266,6 +284,11 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     // resident; K(j+2) and V(j+1) are requested here and awaited at the end.
     auto tile_step = [&](f32x16 (&cur)[NT], f32x16 (&nxt)[NT], int j) {
         const int j0 = (jbase + j) * BN;
+        // The next tile's key-mask bytes travel under this step and become a word behind its wait (read where they are used,
+        // they made every step wait for the K request in front of them: B1 Hq8 N8192 all visible, 178 -> 156 us with the mask out of the other form).
+        const uint64_t tile_hidden = next_hidden;
+        uint32_t mask_byte = 1;
+        if (KEYS && j + 1 < nkv) mask_byte = km[min(j0 + BN + lane, N - 1)];
         // The two requests are issued apart (K here, V after the row-max reduction) so the waves of
         // a CU do not all queue on the texture path at once.
         // In the last two steps of the first tile of a pair the freed K stages take K(0) and K(1) of
@@ -283,13 +306,11 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
             // The tile's 64 key-mask bytes are the same for every lane: lane l reads the byte of kv row
             // j0 + l and a ballot makes them one 64-bit word (bit r set: row j0 + r is hidden).  A tile
             // without hidden rows skips the masking.  (Rows at or beyond N are hidden by `lim` already.)
-            uint64_t tile_hidden = 0;
-            if (EXT && km != nullptr) tile_hidden = __builtin_amdgcn_ballot_w64(km[min(j0 + lane, N - 1)] == 0);
             const bool need_mask = (CAUSAL && (j0 + BN - 1 > qw0)) || (j0 + BN > Nk) ||
-                                   (EXT && window > 0 && j0 < qw0 + 32 - window) || (EXT && tile_hidden != 0);
+                                   (LIMITS && window > 0 && j0 < qw0 + 32 - window) || (KEYS && tile_hidden != 0);
             if (need_mask) {
                 const int lim = CAUSAL ? min(qpos, Nk - 1) : Nk - 1;   // largest visible kv row
-                const int low = (EXT && window > 0) ? qpos - window + 1 : INT_MIN;   // smallest visible kv row
+                const int low = (LIMITS && window > 0) ? qpos - window + 1 : INT_MIN;   // smallest visible kv row
                 const int base = j0 + 32 * T0 + 4 * g;
                 const uint64_t hidden = tile_hidden >> (32 * T0 + 4 * g);      // shifted to this lane's rows
 #pragma unroll
@@ -297,7 +318,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
                         const int kv = base + 32 * T + 8 * (e >> 2) + (e & 3);
-                        const bool off = kv > lim || (EXT && kv < low) ||
+                        const bool off = kv > lim || (LIMITS && kv < low) ||
                                          ((hidden >> (32 * T + 8 * (e >> 2) + (e & 3))) & 1u);
                         cur[T][e] = off ? -INFINITY : cur[T][e];
                     }
@@ -383,6 +404,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
         }
 
         wait_vmcnt0();
+        if constexpr (KEYS) next_hidden = __builtin_amdgcn_ballot_w64(mask_byte == 0);
         __syncthreads();
     };
 
@@ -430,7 +452,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
             m2 = m;
         }
     }
-    const float inv = (!EXT || ltot > 0.0f) ? 1.0f / ltot : 0.0f;    // EXT: a row that saw no key gives 0
+    const float inv = (MASK == AttnMask::None || ltot > 0.0f) ? 1.0f / ltot : 0.0f;    // masked: a row that saw no key gives 0
     if (!SPLIT || w < 2) {
         constexpr int SROW = D * 2;
         constexpr int CH = D / 8;                   // 16-byte chunks per row
@@ -529,7 +551,7 @@ int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, 
     using namespace fa;
     const int BH = B * Hq;
     const int G = Hq / Hkv;
-    const bool ext = window > 0 || kv_lens != nullptr || key_mask != nullptr;
+    const bool limits = window > 0 || kv_lens != nullptr;     // never together with a key mask
     // a window makes the tiles equal; lengths and key masks keep tile 0 starting at key 0
     const AttnShape shape = attn_shape(BH, N, D, causal != 0, window);
     const int ntq = (N + shape.rows - 1) / shape.rows;
@@ -569,12 +591,16 @@ int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, 
     } while (0)
 #define TYR_FA_SHAPE(DD, CC, EE)                                                                 \
     do { if (shape.rows == BM) TYR_FA_LAUNCH(DD, CC, EE, false); else TYR_FA_LAUNCH(DD, CC, EE, true); } while (0)
-#define TYR_FA_PICK(DD)                                                                          \
+#define TYR_FA_PICK(DD, MM)                                                                      \
+    do { if (causal) TYR_FA_SHAPE(DD, true, MM); else TYR_FA_SHAPE(DD, false, MM); } while (0)
+#define TYR_FA_MASK(DD)                                                                          \
     do {                                                                                         \
-        if (ext) { if (causal) TYR_FA_SHAPE(DD, true, true); else TYR_FA_SHAPE(DD, false, true); }   \
-        else     { if (causal) TYR_FA_SHAPE(DD, true, false); else TYR_FA_SHAPE(DD, false, false); } \
+        if (key_mask != nullptr) TYR_FA_PICK(DD, AttnMask::Keys);                                \
+        else if (limits) TYR_FA_PICK(DD, AttnMask::Limits);                                      \
+        else TYR_FA_PICK(DD, AttnMask::None);                                                    \
     } while (0)
-    if (D == 128) TYR_FA_PICK(128); else TYR_FA_PICK(64);
+    if (D == 128) TYR_FA_MASK(128); else TYR_FA_MASK(64);
+#undef TYR_FA_MASK
 #undef TYR_FA_PICK
 #undef TYR_FA_SHAPE
 #undef TYR_FA_LAUNCH
