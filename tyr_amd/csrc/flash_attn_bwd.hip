@@ -9,7 +9,7 @@
 // Examples/GPU/RunMhaH100.lean:56-64).  exp is evaluated as exp2 with log2(e) folded into the
 // scale and into the saved log-sum-exp.  causal: key j visible to query i iff j <= i.
 //
-// Two kernels, no atomics, every output written once (results are deterministic):
+// Two kernels (one launch where they leave CUs idle), no atomics, every output written once (results are deterministic):
 //
 //  1. flash_attn_bwd_dq_kernel: one workgroup = 128 query rows (4 waves x 32 rows), keys/values
 //     stream through LDS in tiles of 64 rows exactly as in the forward kernel.  Products are
@@ -126,7 +126,7 @@ __device__ __forceinline__ void store_transposed_bf16(const f32x16 (&acc)[D / 32
 // G = query heads per kv head.  SPLIT: 64 query rows per workgroup, the two 32-key sub-tiles of a tile on two waves whose
 // dQ are added through LDS at the end (same use as in the forward kernel: launches with few tiles).
 template <int D, bool CAUSAL, AttnMask MASK, bool SPLIT>
-__global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
+__device__ __forceinline__ void bwd_dq(int block,
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
     uint16_t* __restrict__ dQ, float2* __restrict__ stats, int BH, int N, int ntq, int npad, float scale,
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
 
     // With `pair` (causal) a workgroup handles query tile ntq-1-tr and then tile tr.
     int bh, tr, kvbh;
-    AttnOrder{BH, Hq, G, pair ? (ntq + 1) / 2 : ntq, single}.decode(blockIdx.x, bh, tr, kvbh);
+    AttnOrder{BH, Hq, G, pair ? (ntq + 1) / 2 : ntq, single}.decode(block, bh, tr, kvbh);
     const int npass = (pair && ntq - 1 - tr != tr) ? 2 : 1;
     for (int pass = 0; pass < npass; ++pass) {
     const int qt = CAUSAL ? (pass == 0 ? ntq - 1 - tr : tr) : tr;
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
         delta = part + xor32(part);
         lse2 = LSE[(size_t)bh * N + qrow] * LOG2E;
         if (MASK != AttnMask::None && lse2 == -INFINITY) lse2 = INFINITY;      // a row that saw no key: every probability is 0
-        if (g == 0 && T0 == 0) {
+        if (stats != nullptr && g == 0 && T0 == 0) {
             stats[(size_t)bh * npad + qpos] = qpos < N ? make_float2(lse2, delta) : make_float2(INFINITY, 0.0f);
         }
     }
@@ -390,6 +390,17 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
     }
 }
 
+template <int D, bool CAUSAL, AttnMask MASK, bool SPLIT>
+__global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
+    const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
+    uint16_t* __restrict__ dQ, float2* __restrict__ stats, int BH, int N, int ntq, int npad, float scale,
+    float scale_log2, int Hq, int G, int window, const int* __restrict__ kv_lens,
+    const uint8_t* __restrict__ key_mask, int pair, int single) {
+    bwd_dq<D, CAUSAL, MASK, SPLIT>(blockIdx.x, Q, Kp, Vp, O, dO, LSE, dQ, stats, BH, N, ntq, npad, scale, scale_log2, Hq, G, window,
+                                   kv_lens, key_mask, pair, single);
+}
+
 // ------------------------------------------------------------------------------------------
 // dK, dV
 // BHkv = batch * kv heads; the G query heads of a kv head are walked one after the other and
@@ -430,14 +441,16 @@ struct Parts {
 
 // CUT: the launch has parts.  (Whole key tiles keep their own instantiation: with the bookkeeping of the parts in the same
 // code the pipeline below, which has no register to spare, is 4-8 % slower.)
-template <int D, bool CAUSAL, AttnMask MASK, bool CUT>
-__global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
+// OWN_STATS: nothing ran before this kernel, so the workgroup makes the (lse2, delta) pairs of its query rows itself.
+template <int D, bool CAUSAL, AttnMask MASK, bool CUT, bool OWN_STATS>
+__device__ __forceinline__ void bwd_dkv(int block,
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
-    const uint16_t* __restrict__ dO, const float2* __restrict__ stats, uint16_t* __restrict__ dK,
-    uint16_t* __restrict__ dV, int BHkv, int N, int ntk, int npad, float scale, float scale_log2,
+    const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE, float2* stats,
+    uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int BHkv, int N, int ntk, int npad, float scale, float scale_log2,
     int Hq, int window, const int* __restrict__ kv_lens, const uint8_t* __restrict__ key_mask, fab::Parts plan, int items,
     float* __restrict__ partial) {
     constexpr bool WINDOW = MASK == AttnMask::Limits, PER_KEY = MASK != AttnMask::None;
+    if (WINDOW && OWN_STATS && window <= 0) window = INT_MAX;      // lengths alone have no instantiation of their own there
     const int G = plan.G;
     using namespace fab;
     using C = CfgK<D>;
@@ -449,7 +462,7 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
 
     int bh, item;                         // bh indexes (batch, kv head)
     {
-        const int id = blockIdx.x;
+        const int id = block;
         // causal: key tile 0 meets every query tile, so heavy first; parts of all kv heads of an XCD in that order, or
         // head after head where whole key tiles are many (their Q / dO then share the L2)
         if ((BHkv & 7) == 0) {
@@ -475,6 +488,28 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     if (PER_KEY && key_mask != nullptr && !block_hidden) {
         const TileSpan span = visible_tiles(key_mask + (size_t)(bh / hkv) * N + n0, min(C::BNK, Nk - n0), lane);
         block_hidden = span.first >= span.last;
+    }
+    if constexpr (OWN_STATS) {
+        if (!block_hidden) {
+            const int first = plan.first(kt), per_head = plan.last(kt) - first, all = G * per_head;
+            const int begin = CUT ? part * plan.part_steps(kt) : 0, end = CUT ? min(all, begin + plan.part_steps(kt)) : all;
+#pragma unroll 2
+            for (int s = 2 * begin + w; s < 2 * end; s += 4) {           // 32 rows a wave, as in the dQ kernel
+                const size_t head = qh0 + (s >> 1) / per_head;
+                const int qpos = (first + (s >> 1) % per_head) * C::BQ + (s & 1) * 32 + r, qrow = min(qpos, N - 1);
+                const size_t off = (head * N + qrow) * D + g * 8;
+                float part_sum = 0.0f;
+#pragma unroll
+                for (int i = 0; i < C::KSTEPS; ++i) part_sum += dot8_bf16(ld_global_16(dO + off + i * 16), ld_global_16(O + off + i * 16));
+                const float delta = part_sum + xor32(part_sum);
+                float lse2 = LSE[head * N + qrow] * LOG2E;
+                if (MASK != AttnMask::None && lse2 == -INFINITY) lse2 = INFINITY;
+                if (g == 0) stats[head * npad + qpos] = qpos < N ? make_float2(lse2, delta) : make_float2(INFINITY, 0.0f);
+            }
+            __threadfence_block();       // before the requests below read the pairs back (other workgroups write equal bytes)
+            wait_vmcnt0();
+            __syncthreads();
+        }
     }
 
     // ---- this wave's K and V rows as column operands (lane = key row, columns 16i + 8g + [0,8))
@@ -857,6 +892,36 @@ pipeline_done:
     store_transposed_bf16<D>(dk, scale, scratch, dK + head_off + (size_t)nw0 * D, N - nw0, lane);
 }
 
+template <int D, bool CAUSAL, AttnMask MASK, bool CUT>
+__global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
+    const uint16_t* __restrict__ dO, float2* stats, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int BHkv, int N,
+    int ntk, int npad, float scale, float scale_log2, int Hq, int window, const int* __restrict__ kv_lens,
+    const uint8_t* __restrict__ key_mask, fab::Parts plan, int items, float* __restrict__ partial) {
+    bwd_dkv<D, CAUSAL, MASK, CUT, false>(blockIdx.x, Q, Kp, Vp, nullptr, dO, nullptr, stats, dK, dV, BHkv, N, ntk, npad, scale, scale_log2,
+                                         Hq, window, kv_lens, key_mask, plan, items, partial);
+}
+
+// Both at once for launches that leave CUs idle anyway (rule at one_launch): the first `ndkv` workgroups are dK/dV's, the
+// rest dQ's (64-row form).  The dQ kernel then need not end before dK/dV starts -- a launch, a prologue and a drain, 3.5 us
+// of 11 for one head of 128 rows, 12 of 41 for 8 heads of 700.
+template <int D, bool CAUSAL, AttnMask MASK, bool CUT>
+__global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_both_kernel(
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
+    const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
+    uint16_t* __restrict__ dQ, float2* stats, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int BH, int N, int ntq,
+    int ntk, int npad, float scale, float scale_log2, int Hq, int window, const int* __restrict__ kv_lens,
+    const uint8_t* __restrict__ key_mask, int single, fab::Parts plan, int items, float* __restrict__ partial, int ndkv) {
+    const int at = blockIdx.x;
+    if (at < ndkv) {
+        bwd_dkv<D, CAUSAL, MASK, CUT, true>(at, Q, Kp, Vp, O, dO, LSE, stats, dK, dV, BH / plan.G, N, ntk, npad, scale, scale_log2, Hq,
+                                         window, kv_lens, key_mask, plan, items, partial);
+    } else {
+        bwd_dq<D, CAUSAL, MASK, true>(at - ndkv, Q, Kp, Vp, O, dO, LSE, dQ, nullptr, BH, N, ntq, npad, scale, scale_log2, Hq, plan.G,
+                                      window, kv_lens, key_mask, 0, single);
+    }
+}
+
 // dK and dV of the key tiles that were cut into parts: the parts' f32 sums added in order, 8 elements of a row per thread.
 template <int D>
 __global__ __launch_bounds__(256) void flash_attn_bwd_sum_kernel(const float* __restrict__ partial, uint16_t* __restrict__ dK,
@@ -971,6 +1036,14 @@ int dkv_items(const fab::Parts& p, int N) {
     for (int kt = 0; kt < ntk; ++kt) n += p.parts(kt);
     return n;
 }
+// dQ and dK/dV as one launch: where every workgroup gets a CU to itself, and up to 1024 rows while there are not many more
+// than that.  Measured (MI355X, us, two launches -> one): B1 H1 N128 D64 11.0 -> 7.5, B1 H4 N512 D128 causal 27.2 -> 18.3,
+// B1 Hq8 Hkv2 N700 40.6 -> 28.8; 384 workgroups, N1000 43.7 -> 39.8; beyond, a dK/dV workgroup waits longer for the pairs of
+// all its rows and dQ comes last: 512 workgroups, N2048 69 -> 73.
+bool one_launch(int N, int64_t dq_blocks, int64_t dkv_blocks) {
+    const int64_t n = dq_blocks + dkv_blocks;
+    return n <= 256 || (n <= 640 && N <= 1024);
+}
 size_t dkv_partial_bytes(const fab::Parts& p, int BHkv, int N, int D) {
     return p.chunk ? (size_t)BHkv * dkv_items(p, N) * 128 * D * 8 : 0;
 }
@@ -999,6 +1072,8 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     if (workspace_bytes < stat_bytes + dkv_partial_bytes(plan, BHkv, N, D)) plan.chunk = 0;
     const int items = dkv_items(plan, N);
     dim3 grid_k((unsigned)(BHkv * items));
+    const int64_t dq_blocks = (int64_t)BH * ((N + 63) / 64);
+    const bool both = one_launch(N, dq_blocks, grid_k.x);
     float* partial = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + stat_bytes);
     const float scale_log2 = scale * LOG2E;
     auto Qp = static_cast<const uint16_t*>(q);
@@ -1033,13 +1108,32 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
         if (EE == AttnMask::Limits && window <= 0) TYR_FAB_DKV(DD, CC, AttnMask::Keys, UU);           \
         else TYR_FAB_DKV(DD, CC, EE, UU);                                                             \
     } while (0)
+#define TYR_FAB_SUM(DD)                                                                               \
+    hipLaunchKernelGGL(flash_attn_bwd_sum_kernel<DD>, dim3((unsigned)(BHkv * ntk * (DD / 8))), dim3(256), 0, stream, \
+                       partial, static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), N, ntk, items, scale, plan)
+#define TYR_FAB_BOTH(DD, CC, EE, UU)                                                                  \
+    do {                                                                                              \
+        static const hipError_t a3 = hipFuncSetAttribute(                                             \
+            reinterpret_cast<const void*>(&flash_attn_bwd_both_kernel<DD, CC, EE, UU>),               \
+            hipFuncAttributeMaxDynamicSharedMemorySize, CfgK<DD>::LDS);                               \
+        if (a3 != hipSuccess) return -1;                                                              \
+        hipLaunchKernelGGL((flash_attn_bwd_both_kernel<DD, CC, EE, UU>), dim3(grid_k.x + (unsigned)dq_blocks), block, CfgK<DD>::LDS, \
+                           stream, Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st,          \
+                           static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), BH, N, (N + 63) / 64, ntk, \
+                           npad, scale, scale_log2, Hq, window, kv_lens, key_mask, causal && window <= 0, plan, items, partial, (int)grid_k.x); \
+    } while (0)
 #define TYR_FAB_LAUNCH(DD, CC, EE)                                                                    \
     do {                                                                                              \
+        if (both) {                                                                                   \
+            if (!plan.chunk) { TYR_FAB_BOTH(DD, CC, EE, false); break; }                              \
+            TYR_FAB_BOTH(DD, CC, EE, true);                                                           \
+            TYR_FAB_SUM(DD);                                                                          \
+            break;                                                                                    \
+        }                                                                                             \
         if (shape.rows == 64) TYR_FAB_DQ(DD, CC, EE, true); else TYR_FAB_DQ(DD, CC, EE, false);       \
         if (plan.chunk) {                                                                             \
             TYR_FAB_DKV_MASK(DD, CC, EE, true);                                                            \
-            hipLaunchKernelGGL(flash_attn_bwd_sum_kernel<DD>, dim3((unsigned)(BHkv * ntk * (DD / 8))), dim3(256), 0, stream, \
-                               partial, static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), N, ntk, items, scale, plan); \
+            TYR_FAB_SUM(DD);                                                                          \
         } else {                                                                                      \
             TYR_FAB_DKV_MASK(DD, CC, EE, false);                                                           \
         }                                                                                             \
@@ -1056,6 +1150,8 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
 #undef TYR_FAB_MASK
 #undef TYR_FAB_PICK
 #undef TYR_FAB_LAUNCH
+#undef TYR_FAB_BOTH
+#undef TYR_FAB_SUM
 #undef TYR_FAB_DKV_MASK
 #undef TYR_FAB_DKV
 #undef TYR_FAB_DQ
