@@ -537,8 +537,12 @@ AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window) {
         if (form != 0 && ordered && ntq > 1 && bh * ntq > 2048) continue;
         const int all = (N + 63) / 64, seen = window > 0 ? std::min<int64_t>(all, ((int64_t)window + rows) / 64 + 1) : all;
         const AttnJobs jobs{ntq, seen, ordered, form == 0, rows, N};
-        const double us = D == 128 ? (form == 2 ? busiest_cu_us(jobs, bh, 0.61, 0.97, 6.1, 1.0) : busiest_cu_us(jobs, bh, 1.0, 0.95, 5.6, 1.3))
-                                   : (form == 2 ? busiest_cu_us(jobs, bh, 0.38, 1.3, 5.0, 0.8) : busiest_cu_us(jobs, bh, 0.64, 1.1, 4.7, 1.0));
+        // under a window two tiles of a job are masked, and a 128-row workgroup alone on its CU hides none of that (1.25 us a
+        // step; B1 Hq16 N1800 window 600: 20.3 us, 19.1 with 64 rows)
+        const bool edges = window > 0 && window < N;
+        const double us =
+            D == 128 ? (form == 2 ? busiest_cu_us(jobs, bh, edges ? 0.56 : 0.61, 0.97, 6.1, 1.0) : busiest_cu_us(jobs, bh, 1.0, edges ? 1.25 : 0.95, 5.6, 1.3))
+                     : (form == 2 ? busiest_cu_us(jobs, bh, edges ? 0.36 : 0.38, 1.3, 5.0, 0.8) : busiest_cu_us(jobs, bh, 0.64, edges ? 1.4 : 1.1, 4.7, 1.0));
         if (us < least) { least = us; best = {rows, form == 0, form != 0 && ordered}; }
     }
     return best;
