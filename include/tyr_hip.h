@@ -171,14 +171,18 @@ int tyr_hip_gqa_decode(const void* q, const void* k, const void* v, void* o, flo
  * The partial results of the split pass go to a fixed device array of
  * TYR_HIP_GQA_DECODE_STATIC_SCRATCH_BYTES bytes that the library holds on every GPU it runs on
  * until the process ends; the call makes no hipMalloc / hipFree and uses no allocating library
- * routine.  Arguments and results are those of tyr_hip_gqa_decode (same kernels).
+ * routine.  Arguments and results are those of tyr_hip_gqa_decode with the split count that runs
+ * (same kernels).  num_splits = 0 takes one split where B * Hkv >= 256 or L < 1024, and elsewhere
+ * the count of tyr_hip_gqa_decode_auto_splits, lowered to what the array holds.
  *
- * Limit: tyr_hip_gqa_decode_workspace_bytes(B, Hq, Hkv, L, D, num_splits) must not exceed
- * TYR_HIP_GQA_DECODE_STATIC_SCRATCH_BYTES, else TYR_HIP_ERR_WORKSPACE is returned and nothing is
- * launched (B * Hq * num_splits <= 16131 at D = 128).
- * Every call on one GPU uses the same array: calls that overlap in time on one GPU (different
- * streams, different threads) race on it; calls on one stream are ordered and safe.  Nothing in
- * the array has to start at zero (the split pass writes every partial the combine pass reads).
+ * Limit: for a num_splits > 0, tyr_hip_gqa_decode_workspace_bytes(B, Hq, Hkv, L, D, num_splits) must
+ * not exceed TYR_HIP_GQA_DECODE_STATIC_SCRATCH_BYTES, else TYR_HIP_ERR_WORKSPACE is returned and
+ * nothing is launched (B * Hq * num_splits <= 16131 at D = 128); num_splits = 0 is refused so where
+ * not even one split's partials would fit (B * Hq > 16131).
+ * Every call on one GPU that runs more than one split uses the same array: such calls that overlap in
+ * time on one GPU (different streams, different threads) race on it; calls on one stream are ordered
+ * and safe, and a call that runs one split does not touch the array.  Nothing in the array has to
+ * start at zero (the split pass writes every partial the combine pass reads).
  * The first call on a device looks the array's address up (hipGetSymbolAddress); make that call
  * outside stream capture.
  */

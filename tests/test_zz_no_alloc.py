@@ -67,6 +67,41 @@ def test_static_decode_single_split_and_auto():
         assert np.array_equal(lse_s.cpu().numpy().view(np.uint32), lse_w.cpu().numpy().view(np.uint32))
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,L", [(40, 8, 8, 3000), (32, 8, 8, 1500), (1, 16, 8, 1000), (2, 16, 4, 1023)])
+def test_static_decode_takes_one_split_where_calls_may_overlap(B, Hq, Hkv, L):
+    """num_splits = 0 with 256 groups or more, or fewer than 1024 rows: the partials' array stays untouched, i.e. the bits
+    are those of one split (the logs of sums added in another order differ in some rows)."""
+    from tyr_amd import _lib
+    L_ = _lib.load()
+    D = 128
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q = torch.randn(B, Hq, 1, D, device="cuda", generator=g).bfloat16()
+    k, v = (torch.randn(B, Hkv, L, D, device="cuda", generator=g).bfloat16() for _ in range(2))
+    (o_auto, lse_auto), _ = _call_pair(L_, q, k, v, 0, L)
+    (o_one, lse_one), _ = _call_pair(L_, q, k, v, 1, L)
+    assert torch.equal(o_auto, o_one) and torch.equal(lse_auto, lse_one)
+
+
+def test_static_decode_lowers_the_automatic_count_to_what_the_array_holds():
+    from tyr_amd import _lib
+    L_ = _lib.load()
+    B, Hq, Hkv, L, D = 13, 192, 12, 1024, 128
+    auto = L_.tyr_hip_gqa_decode_auto_splits(B, Hkv, L)
+    fits = (8 << 20) // (B * Hq * (D + 2) * 4)
+    assert L_.tyr_hip_gqa_decode_workspace_bytes(B, Hq, Hkv, L, D, 0) == B * Hq * auto * (D + 2) * 4
+    g = torch.Generator(device="cuda").manual_seed(7)
+    q = torch.randn(B, Hq, 1, D, device="cuda", generator=g).bfloat16()
+    k, v = (torch.randn(B, Hkv, L, D, device="cuda", generator=g).bfloat16() for _ in range(2))
+    (o_auto, lse_auto), _ = _call_pair(L_, q, k, v, 0, L)
+    assert fits < auto
+    (o_most, lse_most), _ = _call_pair(L_, q, k, v, fits, L)
+    assert torch.equal(o_auto, o_most) and torch.equal(lse_auto, lse_most)
+    # one split of more heads than the array holds is refused, before anything is looked at
+    t = torch.zeros(16, dtype=torch.bfloat16, device="cuda")
+    rc = L_.tyr_hip_gqa_decode_static(t.data_ptr(), t.data_ptr(), t.data_ptr(), t.data_ptr(), None, 8, 2048, 256, 2048, D, 2048, 0.1, 0, None)
+    assert rc == -5
+
+
 def test_static_decode_rejects_oversized_request():
     from tyr_amd import _lib
     L_ = _lib.load()

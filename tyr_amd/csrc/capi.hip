@@ -328,8 +328,12 @@ int tyr_hip_gqa_decode_static(const void* q, const void* k, const void* v, void*
     if (num_splits > kMaxSplits) return TYR_HIP_ERR_UNSUPPORTED;
     if (B > (uint64_t)INT_MAX || Hq > (uint64_t)INT_MAX || B * Hq > (uint64_t)INT_MAX || Hkv > Hq || D > 4096)
         return TYR_HIP_ERR_BAD_SHAPE;
-    if (num_splits == 0)                             // as many as the array holds
-        num_splits = std::max<uint64_t>(1, std::min<uint64_t>(auto_splits(B, Hkv, L), kStaticScratchBytes / (B * Hq * (D + 2) * sizeof(float))));
+    if (num_splits == 0) {
+        // A call with one split does not touch the array, so such calls may overlap on the device; from 256 groups on and
+        // below 1024 rows callers can rely on it.  Elsewhere as many splits as the array holds.
+        const uint64_t most = B * Hkv >= 256 || L < 1024 ? 1 : auto_splits(B, Hkv, L);
+        num_splits = std::max<uint64_t>(1, std::min<uint64_t>(most, kStaticScratchBytes / (B * Hq * (D + 2) * sizeof(float))));
+    }
     const size_t need = tyr_hip_gqa_decode_workspace_bytes(B, Hq, Hkv, L, D, num_splits);
     if (need > kStaticScratchBytes) return TYR_HIP_ERR_WORKSPACE;
     void* ptr = nullptr;
