@@ -76,6 +76,19 @@ def test_host_validation_needs_no_gpu():
     assert OK == 0
 
 
+def test_automatic_decode_splits_all_hold_rows():
+    """The count the library reports, sizes the workspace for and launches is one count: chunks are whole 32-row steps, and
+    every one of them holds rows."""
+    L = _lib.load()
+    for B in (1, 2, 3, 5, 8, 13, 20, 33, 40, 64):
+        for Hkv in (1, 2, 4, 8, 15, 32):
+            for rows in (1, 64, 383, 385, 416, 417, 700, 1023, 1500, 2000, 2049, 3001, 8191, 32768, 100001):
+                s = L.tyr_hip_gqa_decode_auto_splits(B, Hkv, rows)
+                chunk = -(-(-(-rows // s)) // 32) * 32
+                assert 1 <= s <= 64 and -(-rows // chunk) == s, (B, Hkv, rows, s, chunk)
+                assert L.tyr_hip_gqa_decode_workspace_bytes(B, Hkv, Hkv, rows, 128, 0) == B * Hkv * s * 130 * 4
+
+
 def test_python_mirror_refuses_cpu_tensors_without_a_gpu():
     import torch
     import tyr_amd

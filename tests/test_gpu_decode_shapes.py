@@ -35,3 +35,19 @@ def test_decode_launch_shapes(B, Hq, Hkv, L, D, splits, lens):
         want_o, want_lse = oracle.gqa_decode(bits(q[b:b + 1]), bits(kb), bits(vb), sc, 1)
         assert float((o[b:b + 1].cpu().float() - from_bits(want_o).float()).abs().max()) <= 8e-3, (b, n[b])
         assert float(np.abs(lse[b:b + 1].cpu().numpy() - np.asarray(want_lse)).max()) <= 1e-3, (b, n[b])
+
+
+@pytest.mark.parametrize("Hq,Hkv,L,D,splits", [(4, 2, 1056, 128, 33), (2, 1, 2048, 128, 64), (4, 1, 2017, 64, 64), (8, 8, 1500, 128, 23),
+                                               (4, 4, 33, 128, 4), (2, 2, 20, 64, 4)])
+@pytest.mark.parametrize("window", [0, 19, 1000])
+def test_more_splits_than_chunks_with_rows(Hq, Hkv, L, D, splits, window):
+    """Counts whose chunks, rounded up to whole steps, are fewer than asked for, down to one; and 33 and 64 that all hold rows."""
+    import tyr_amd as gpu
+    q, = lt.make_inputs(60 + L, (1, Hq, 1, D))
+    k, v = lt.make_inputs(61 + L, (1, Hkv, L, D), (1, Hkv, L, D))
+    sc = 1 / math.sqrt(D)
+    o, lse = gpu.gqa_decode(q.cuda(), k.cuda(), v.cuda(), scale=sc, num_splits=splits, window=window)
+    lo = max(0, L - window) if window else 0
+    want_o, want_lse = oracle.gqa_decode(bits(q), bits(k[:, :, lo:].contiguous()), bits(v[:, :, lo:].contiguous()), sc, 1)
+    assert float((o.cpu().float() - from_bits(want_o).float()).abs().max()) <= 8e-3
+    assert float(np.abs(lse.cpu().numpy() - np.asarray(want_lse)).max()) <= 1e-3

@@ -22,23 +22,27 @@ inline bool fits_int(uint64_t v) { return v <= (uint64_t)INT_MAX; }
 
 constexpr uint64_t kMaxSplits = 64;
 
-// Splits per (batch, kv head), for 256 CUs.  A second pass costs 2.5 us, what a CU reads of 100 rows, and more than one
-// workgroup's 384 rows take.  A CU with one workgroup reads 20-40 GB/s (K and V go from the L2 to registers in 64-byte
-// pieces), so fewer groups than CUs are cut until every CU has a workgroup: B1 Hkv8 L1500 16.6 us with 2 splits (one per
-// 512 rows, the former rule), 8.6 with 23.  More groups than 128 are cut where that fills the last round of workgroups:
-// 320 groups of 3000 rows 110 us whole, 87 with 4 splits.  On 30 shapes (2 to 2048 groups, 64 to 32768 rows) the choice
-// is 1 % slower than the best.
+// Splits per (batch, kv head), for 256 CUs: as many as the launch has chunks with rows (a chunk is a multiple of the 32 rows
+// of a step).  A second pass costs 2.5 us, what a CU reads of 100 rows, and more than one workgroup's 384 rows take.  A CU
+// with one workgroup reads 20-40 GB/s (K and V go from the L2 to registers in 64-byte pieces), so fewer groups than CUs are
+// cut towards a workgroup on every CU, in chunks of 64 rows or more; rounding a chunk up to whole steps leaves some CUs
+// without one (8 groups of 1500 rows: 16 chunks of 96; both passes take 7.6 us, one split 16.5).  More groups than 128 are cut where that
+// fills the last round of workgroups: 320 groups of 3000 rows 110 us whole, 87 with 4 splits.
 uint64_t auto_splits(uint64_t B, uint64_t Hkv, uint64_t L) {
     const uint64_t groups = B * Hkv;
     if (groups == 0 || L <= 384) return 1;
-    if (groups <= 128) return std::min({256 / groups, L / 64, kMaxSplits});
+    auto chunk_rows = [L](uint64_t s) { return ((L + s - 1) / s + 31) / 32 * 32; };
     uint64_t best = 1, least = UINT64_MAX;
-    for (uint64_t s = 1; s <= 8; ++s) {
-        const uint64_t chunk = ((L + s - 1) / s + 31) / 32 * 32, rounds = (groups * s + 255) / 256;
-        const uint64_t rows = std::max(groups * L / 325, rounds * chunk) + 20 * rounds + (s > 1 ? 100 : 0);
-        if (rows < least) { least = rows; best = s; }
+    if (groups <= 128) {
+        best = std::min({256 / groups, L / 64, kMaxSplits});
+    } else {
+        for (uint64_t s = 1; s <= 8; ++s) {
+            const uint64_t rounds = (groups * s + 255) / 256;
+            const uint64_t rows = std::max(groups * L / 325, rounds * chunk_rows(s)) + 20 * rounds + (s > 1 ? 100 : 0);
+            if (rows < least) { least = rows; best = s; }
+        }
     }
-    return best;
+    return (L + chunk_rows(best) - 1) / chunk_rows(best);
 }
 
 }  // namespace

@@ -283,10 +283,10 @@ int launch_gqa_decode(const void* q, const void* k, const void* v, void* o, floa
                       void* workspace, const int* kv_lens, int window, hipStream_t stream) {
     using namespace dec;
     const int G = Hq / Hkv;
-    const int S = num_splits;
     const int span = window > 0 ? (window < L ? window : L) : L;     // longest range any sequence reads
-    int chunk = (span + S - 1) / S;
+    int chunk = (span + num_splits - 1) / num_splits;
     chunk = (chunk + STEP - 1) / STEP * STEP;
+    const int S = (span + chunk - 1) / chunk;                        // chunks of whole steps: no workgroup without rows
 
     float* part_o = static_cast<float*>(workspace);
     float* part_m = part_o + (size_t)B * Hq * S * D;
@@ -296,7 +296,6 @@ int launch_gqa_decode(const void* q, const void* k, const void* v, void* o, floa
 #define TYR_DEC_LAUNCH(DD, WAVES)                                                                    \
     do {                                                                                             \
         const size_t lds = (size_t)(WAVES * G * DD + 2 * WAVES * QPAD) * sizeof(float);              \
-                                                                                                 \
         static const hipError_t attr = hipFuncSetAttribute(                                          \
             reinterpret_cast<const void*>(&gqa_decode_split_kernel<WAVES, DD>),                      \
             hipFuncAttributeMaxDynamicSharedMemorySize,                                              \
