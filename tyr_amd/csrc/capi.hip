@@ -26,8 +26,8 @@ constexpr uint64_t kMaxSplits = 64;
 // of a step).  A second pass costs 2.5 us, what a CU reads of 100 rows, and more than one workgroup's 384 rows take.  A CU
 // with one workgroup reads 20-40 GB/s (K and V go from the L2 to registers in 64-byte pieces), so fewer groups than CUs are
 // cut towards a workgroup on every CU, in chunks of 64 rows or more; rounding a chunk up to whole steps leaves some CUs
-// without one (8 groups of 1500 rows: 16 chunks of 96; both passes take 7.6 us, one split 16.5).  More groups than 128 are cut where that
-// fills the last round of workgroups: 320 groups of 3000 rows 110 us whole, 87 with 4 splits.
+// without one (8 groups of 1500 rows: 16 chunks of 96; both passes take 7.6 us, one split 16.5).  More groups than 128 are
+// cut where that fills the last round of workgroups: 320 groups of 3000 rows 110 us whole, 87 with 4 splits.
 uint64_t auto_splits(uint64_t B, uint64_t Hkv, uint64_t L) {
     const uint64_t groups = B * Hkv;
     if (groups == 0 || L <= 384) return 1;
