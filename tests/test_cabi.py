@@ -3,6 +3,7 @@ validation rejects bad arguments before touching a GPU (so these run without one
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -87,6 +88,42 @@ def test_automatic_decode_splits_all_hold_rows():
                 chunk = -(-(-(-rows // s)) // 32) * 32
                 assert 1 <= s <= 64 and -(-rows // chunk) == s, (B, Hkv, rows, s, chunk)
                 assert L.tyr_hip_gqa_decode_workspace_bytes(B, Hkv, Hkv, rows, 128, 0) == B * Hkv * s * 130 * 4
+
+
+def test_nothing_throws_when_the_heap_is_exhausted(tmp_path):
+    """The header promises that no entry point throws.  Host-side planning runs here with an operator new that fails: an
+    exception would leave a C function and end the process."""
+    src = tmp_path / "no_heap.cpp"
+    src.write_text(r"""
+#include <dlfcn.h>
+#include <stdint.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <new>
+static bool fail;
+void* operator new(size_t n) { if (fail) throw std::bad_alloc(); return malloc(n); }
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
+int main(int, char** argv) {
+    void* h = dlopen(argv[1], RTLD_NOW);
+    if (!h) { puts(dlerror()); return 2; }
+    auto bwd = (size_t(*)(uint64_t, uint64_t, uint64_t, uint64_t, uint64_t, int, uint64_t))dlsym(h, "tyr_hip_flash_attn_bwd_full_workspace_bytes");
+    auto gemm = (size_t(*)(uint64_t, uint64_t, uint64_t, uint64_t, int, int))dlsym(h, "tyr_hip_gemm_workspace_bytes");
+    auto dec = (size_t(*)(uint64_t, uint64_t, uint64_t, uint64_t, uint64_t, uint64_t))dlsym(h, "tyr_hip_gqa_decode_workspace_bytes");
+    fail = true;
+    size_t sum = 0;
+    for (uint64_t n = 1; n <= 8192; n = n * 3 / 2 + 1)
+        for (uint64_t hkv = 1; hkv <= 32; hkv *= 2)
+            for (int causal = 0; causal < 2; ++causal)
+                sum += bwd(1, 32, hkv, n, 128, causal, 0) + bwd(3, 32, hkv, n, 64, 1, 100) + gemm(1, n, 8 * n, 16 * n, 2, 1) + dec(2, 32, hkv, n, 128, 0);
+    fail = false;
+    printf("ok %d\n", sum != 0);
+}
+""")
+    exe = tmp_path / "no_heap"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-rdynamic", str(src), "-o", str(exe), "-ldl"])
+    r = subprocess.run([str(exe), _lib.LIB_PATH], capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout == "ok 1\n", (r.returncode, r.stdout, r.stderr[-500:])
 
 
 def test_python_mirror_refuses_cpu_tensors_without_a_gpu():

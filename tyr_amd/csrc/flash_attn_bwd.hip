@@ -40,7 +40,6 @@
 #include <algorithm>
 #include <functional>
 #include <type_traits>
-#include <vector>
 
 #include "common.hpp"
 #include "launch.hpp"
@@ -977,7 +976,8 @@ fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window)
         most = std::max(most, whole.steps(kt));
     }
     double least = 1e300;
-    std::vector<int> sizes;
+    int sizes[768];                                  // of the parts of one kv head: at most 256 x 3, or 64 whole tiles; no heap, the C entry must not throw
+    int listed = 0;
     for (int round = 0; round <= 3; ++round) {
         fab::Parts p = whole;
         auto count = [&](int chunk) {
@@ -996,21 +996,21 @@ fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window)
             p.chunk = lo;
         }
         int64_t cut = 0;
-        sizes.clear();
+        listed = 0;
         for (int kt = 0; kt < ntk; ++kt) {
             const int n = p.parts(kt);
             if (n > 1) cut += n;
-            for (int i = 0; i < n; ++i) sizes.push_back(p.chunk ? p.part_steps(kt) : p.steps(kt));
+            for (int i = 0; i < n; ++i) sizes[listed++] = p.chunk ? p.part_steps(kt) : p.steps(kt);
         }
         if (round && cut == 0) continue;
-        std::sort(sizes.begin(), sizes.end(), std::greater<int>());
+        std::sort(sizes, sizes + listed, std::greater<int>());
         // every size BHkv times, longest first over 256 CUs
-        const int64_t n = (int64_t)sizes.size() * BHkv;
+        const int64_t n = (int64_t)listed * BHkv;
         double steps = sizes[0];
         if (n > 256 && n <= 512) {
             for (int64_t j = 0; j < n - 256; ++j) steps = std::max(steps, (double)sizes[(255 - j) / BHkv] + sizes[(256 + j) / BHkv]);
         } else if (n > 512) {
-            steps = std::max(steps, (double)total * BHkv / 256 + 0.5 * total / sizes.size());
+            steps = std::max(steps, (double)total * BHkv / 256 + 0.5 * total / listed);
         }
         const double heads = std::max(1.0, std::min((double)G, (double)sizes[0] / std::max(1, p.last(0) - p.first(0))));
         double us = step * steps + 1.5 * (heads + std::max(0.0, (double)n / 256 - 1));
