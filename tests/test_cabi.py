@@ -90,6 +90,20 @@ def test_automatic_decode_splits_all_hold_rows():
                 assert L.tyr_hip_gqa_decode_workspace_bytes(B, Hkv, Hkv, rows, 128, 0) == B * Hkv * s * 130 * 4
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,cut", [
+    (9, 16, 4, 1944, 128, True),       # 36 kv heads: whole key tiles 832 us, in parts 573
+    (5, 32, 8, 1325, 128, True),       # 331, 296
+    (2, 32, 8, 4601, 64, True),        # with a key mask 607, 507
+    (4, 16, 4, 3000, 128, False),      # whole 534, in parts 555: the long first tiles run while other CUs are idle
+    (16, 16, 16, 4096, 128, False),    # 8192 key tiles fill the device
+    (1, 32, 8, 2000, 128, True)])      # 254, 149
+def test_backward_cuts_key_tiles_where_that_is_faster(B, Hq, Hkv, N, D, cut):
+    """The workspace says whether dK / dV of a causal backward are cut into parts; the times are of an MI355X."""
+    L = _lib.load()
+    least = L.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D)
+    assert (L.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, 1, 0) > least) == cut
+
+
 def test_nothing_throws_when_the_heap_is_exhausted(tmp_path):
     """The header promises that no entry point throws.  Host-side planning runs here with an operator new that fails: an
     exception would leave a C function and end the process."""

@@ -38,7 +38,6 @@
 #include <limits.h>
 
 #include <algorithm>
-#include <functional>
 #include <type_traits>
 
 #include "common.hpp"
@@ -960,15 +959,44 @@ size_t flash_attn_bwd_workspace_bytes(int B, int H, int N) {
 }
 
 namespace {
-// How the dK / dV work is cut.  A workgroup has a CU to itself; a step (64 queries x 128 keys) takes 1.55 us at D = 128, 0.9
-// at 64, a segment (one head's range) 1.5 us to start and end, the sum of the parts 4 us and the traffic of its partials
-// (written and read at 4 TB/s).  Tried: whole key tiles, and the finest cut with at most 256, 512 or 768 workgroups.
+// Steps until the last of 32 CUs (those of an XCD; 256 where heads are not dealt to XCDs) is done when workgroups go to free
+// CUs in the launch's order (bwd_dkv): head after head for whole key tiles, part after part of all heads where they are cut.
+int last_cu_steps(const fab::Parts& p, int ntk, int BHkv) {
+    const int cus = BHkv % 8 == 0 ? 32 : 256, heads = BHkv % 8 == 0 ? BHkv / 8 : BHkv;
+    int busy[256], n = 0, last = 0;                  // a heap, the CU that is free first on top
+    auto later = [](int x, int y) { return x > y; };
+    auto job = [&](int steps) {
+        if (n == cus) {
+            std::pop_heap(busy, busy + n, later);
+            busy[n - 1] += steps;
+        } else {
+            busy[n++] = steps;
+        }
+        last = std::max(last, busy[n - 1]);
+        std::push_heap(busy, busy + n, later);
+    };
+    if (p.chunk) {
+        for (int kt = 0; kt < ntk; ++kt)
+            for (int i = p.parts(kt) * heads; i > 0; --i) job(p.part_steps(kt));
+    } else {
+        for (int h = 0; h < heads; ++h)
+            for (int kt = 0; kt < ntk; ++kt) job(p.steps(kt));
+    }
+    return last;
+}
+// How the dK / dV work is cut.  A workgroup has a CU to itself.  A step (64 queries x 128 keys) takes 1.7 us at D = 128 (1.1
+// at 64) while other CUs are idle and a quarter more with all of them busy (measured: 1.65-1.75 with the last key tiles of
+// a head alone on the device, 2.0-2.2 with 256 equal workgroups, 1.95 in the large launches), a workgroup 2 us to start and
+// end, the sum of the parts 3 us and the traffic of its partials (written and read at 6 TB/s).  Tried: whole key tiles, and
+// the finest cut with at most 256, 512 or 768 workgroups.  On 235 shapes (1 to 16 sequences of 64 to 8192 rows, every mask)
+// the choice is 0.2 % slower than the best of the four, at worst 11 % (B6 Hq32 Hkv8 N92).  With 1.55 us for every step and
+// whole tiles taken longest first it was 1.7 %, at worst 45 %: B9 Hq16 Hkv4 N1944 ran whole, 832 us for 573 in parts.
 fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window) {
     const int ntk = (N + 127) / 128, nq = (N + 63) / 64;
     const fab::Parts whole{G, nq, causal, window, 0};
     fab::Parts best = whole;
-    if (ntk > 64) return best;
-    const double step = D == 128 ? 1.55 : 0.9;
+    if (ntk > 64 || (int64_t)ntk * BHkv > 768) return best;
+    const double step = D == 128 ? 1.7 : 1.1;
     int64_t total = 0;
     int most = 1;
     for (int kt = 0; kt < ntk; ++kt) {
@@ -976,8 +1004,6 @@ fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window)
         most = std::max(most, whole.steps(kt));
     }
     double least = 1e300;
-    int sizes[768];                                  // of the parts of one kv head: at most 256 x 3, or 64 whole tiles; no heap, the C entry must not throw
-    int listed = 0;
     for (int round = 0; round <= 3; ++round) {
         fab::Parts p = whole;
         auto count = [&](int chunk) {
@@ -986,6 +1012,7 @@ fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window)
             for (int kt = 0; kt < ntk; ++kt) n += p.parts(kt);
             return n * BHkv;
         };
+        int64_t n = (int64_t)ntk * BHkv, cut = 0;
         if (round) {
             int lo = std::max<int64_t>(2, total * BHkv / (256 * round)), hi = most;     // least chunk with few enough parts
             if (lo >= hi || count(hi) > 256 * round) continue;
@@ -993,28 +1020,13 @@ fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window)
                 const int mid = (lo + hi) / 2;
                 if (count(mid) <= 256 * round) hi = mid; else lo = mid + 1;
             }
-            p.chunk = lo;
+            n = count(lo);
+            for (int kt = 0; kt < ntk; ++kt) cut += p.parts(kt) > 1 ? p.parts(kt) : 0;
+            if (cut == 0) continue;
         }
-        int64_t cut = 0;
-        listed = 0;
-        for (int kt = 0; kt < ntk; ++kt) {
-            const int n = p.parts(kt);
-            if (n > 1) cut += n;
-            for (int i = 0; i < n; ++i) sizes[listed++] = p.chunk ? p.part_steps(kt) : p.steps(kt);
-        }
-        if (round && cut == 0) continue;
-        std::sort(sizes, sizes + listed, std::greater<int>());
-        // every size BHkv times, longest first over 256 CUs
-        const int64_t n = (int64_t)listed * BHkv;
-        double steps = sizes[0];
-        if (n > 256 && n <= 512) {
-            for (int64_t j = 0; j < n - 256; ++j) steps = std::max(steps, (double)sizes[(255 - j) / BHkv] + sizes[(256 + j) / BHkv]);
-        } else if (n > 512) {
-            steps = std::max(steps, (double)total * BHkv / 256 + 0.5 * total / listed);
-        }
-        const double heads = std::max(1.0, std::min((double)G, (double)sizes[0] / std::max(1, p.last(0) - p.first(0))));
-        double us = step * steps + 1.5 * (heads + std::max(0.0, (double)n / 256 - 1));
-        if (round) us += 4.0 + cut * BHkv * (128.0 * D * 8 * 2) / 4.0e6;
+        const double mean = (double)total * BHkv / 256;       // steps of a CU if all were equally busy
+        double us = step * std::max((double)last_cu_steps(p, ntk, BHkv), 1.25 * mean) + 2.0 * std::max(1.0, n / 256.0);
+        if (round) us += 3.0 + cut * BHkv * (128.0 * D * 8 * 2) / 6.0e6;
         if (us < least) { least = us; best = p; }
     }
     return best;
