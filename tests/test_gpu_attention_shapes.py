@@ -109,3 +109,55 @@ def test_tiles_hidden_by_the_key_mask_are_skipped(Hq, Hkv, N, D, causal):
     for got, ref, alive in zip(grads, want, (seen, used, used)):
         assert rel_fro(got, ref) <= 1e-2
         assert not bool(got[~alive].any())
+
+
+@pytest.mark.parametrize("mask", ["causal", "full", "window", "lens", "keys"])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 4, 1, 700, 128), (1, 8, 2, 1000, 64), (2, 16, 4, 1500, 128), (1, 8, 2, 2049, 64)])
+def test_backward_with_the_least_workspace(B, Hq, Hkv, N, D, mask):
+    """Shapes whose dK / dV are cut into parts where there is scratch for them (the first two beside dQ in one launch): with
+    the minimum, and with all but 16 bytes of what parts need, whole key tiles run and nothing else of the buffer is touched."""
+    from tyr_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    q, k, v, g = (torch.randn(B, h, N, D, device="cuda", generator=gen).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    i = torch.arange(N, device="cuda")
+    causal, window, lens, keys = int(mask != "full"), 0, None, None
+    visible = (i[None, :] <= i[:, None] if causal else torch.ones(N, N, dtype=torch.bool, device="cuda"))[None, None].expand(B, 1, N, N)
+    if mask == "window":
+        window = N // 2 + 1
+        visible = visible & (i[:, None] - i[None, :] < window)
+    if mask == "lens":
+        lens = torch.tensor([N - b * (N // (2 * B)) for b in range(B)], dtype=torch.int32, device="cuda")
+        visible = visible & (i[None, None, None, :] < lens[:, None, None, None])
+    if mask == "keys":
+        keys = (torch.rand(B, N, device="cuda", generator=gen) > 0.3).to(torch.uint8)
+        keys[:, 0] = 1
+        visible = visible & (keys != 0)[:, None, None, :]
+    want_o, want_lse, *want = reference(q, k, v, g, visible)
+    o, lse = want_o.bfloat16(), want_lse.contiguous()
+    least = lib.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D)
+    full = lib.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window)
+    assert full > least
+    buf = torch.empty(full + 4096, dtype=torch.uint8, device="cuda")
+    results = []
+    for nbytes in (least, full - 16, least, full):
+        buf.fill_(0xA5)
+        grads = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        ptrs = [t.data_ptr() for t in (q, k, v, o, g, lse, *grads)]
+        if keys is not None:
+            rc = lib.tyr_hip_flash_attn_bwd_mask(*ptrs, B, Hq, Hkv, N, D, causal, keys.data_ptr(), D ** -0.5, buf.data_ptr(), nbytes,
+                                                 torch.cuda.current_stream().cuda_stream)
+        else:
+            rc = lib.tyr_hip_flash_attn_bwd_gqa(*ptrs, B, Hq, Hkv, N, D, causal, window, lens.data_ptr() if lens is not None else None,
+                                                D ** -0.5, buf.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, lib.tyr_hip_strerror(rc)
+        assert bool((buf[least if nbytes < full else full:] == 0xA5).all())
+        results.append(grads)
+    for other in results[1:3]:
+        assert all(torch.equal(a, b) for a, b in zip(results[0], other))
+    for got, ref, parts in zip(results[0], want, results[3]):
+        assert rel_fro(got, ref) <= 1e-2
+        # row by row against the parts: f32 sums of the same terms in another order, each rounded to bf16, i.e. elements one
+        # unit apart at most (2^-8 of them; twice that allowed, and 1e-5 of a mean row where all terms cancel)
+        n = parts.float().norm(dim=-1)
+        assert bool(((got.float() - parts.float()).norm(dim=-1) <= 2 ** -7 * n + 1e-5 * n.mean()).all())

@@ -57,6 +57,22 @@ def test_every_lean_extern_is_defined_by_the_shim_with_matching_arity():
         assert len(params) == n_lean + 1, (sym, n_lean, len(params))
 
 
+def test_the_shim_passes_all_the_scratch_a_call_can_use():
+    """dK / dV are cut into parts, and K of a GEMM is split, only with scratch for the partial sums: the wrappers size it with
+    the queries that say so and call the forms that take it, as the Python mirror does."""
+    shim = re.sub(r"//[^\n]*", "", open(SHIM).read())
+    assert not re.findall(r"tyr_hip_flash_attn_bwd_workspace_bytes|tyr_hip_gemm_bf16\(|tyr_hip_gemm_bf16_batched\(|tyr_hip_gemm_fp8\(|tyr_hip_gemm_fp8_ex\(", shim)
+    bodies = dict(re.findall(r"lean_object\*\s+(lean_tyr_gpu_\w+)\s*\(.*?\)\s*\{(.*?)\n\}", shim, flags=re.S))
+    bwd = [n for n in bodies if "flash_attn_bwd" in n]
+    gemm = [n for n in bodies if "gemm" in n or "matmul" in n]
+    assert len(bwd) == 4 and len(gemm) == 6
+    for n in bwd + gemm:
+        body = " ".join(bodies[n].split())
+        query, call = ("tyr_hip_flash_attn_bwd_full_workspace_bytes(", r"tyr_hip_flash_attn_bwd\w*\(") if n in bwd else ("tyr_hip_gemm_workspace_bytes(", r"tyr_hip_gemm_\w+_ws\(")
+        assert "Scratch ws(" + query in body, n
+        assert re.search(r"rc = " + call + r"[^;]*ws\.ptr\(\), ws\.bytes, reinterpret_cast<void\*>\(stream\)\);", body), n
+
+
 def test_emitted_lean_launchers_type_check(tmp_path):
     from tyr_amd.dsl import kernels
     from tyr_amd.dsl.emit import LEAN_PREAMBLE, _Emitter

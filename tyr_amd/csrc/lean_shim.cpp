@@ -74,6 +74,17 @@ lean_object* pair_result(torch::Tensor a, torch::Tensor b) {
     return lean_io_result_mk_ok(p);
 }
 
+// Device scratch on the launch stream.  Every wrapper passes what its call can use, so that it runs the plan that was
+// measured: with the minimum, dK / dV are not cut into parts and K of a GEMM is not split.
+struct Scratch {
+    size_t bytes;
+    torch::Tensor block;
+    Scratch(size_t n, const torch::Tensor& like) : bytes(n) {
+        if (n) block = torch::empty({(int64_t)n}, like.options().dtype(torch::kUInt8));
+    }
+    void* ptr() const { return bytes ? block.data_ptr() : nullptr; }
+};
+
 lean_object* status_error(const char* what, int rc) {
     return io_error(std::string(what) + ": " + tyr_hip_strerror(rc));
 }
@@ -173,12 +184,11 @@ lean_object* lean_tyr_gpu_flash_attn_bwd(uint64_t B, uint64_t H, uint64_t N, uin
             return io_error(err);
         LaunchStreamScope on_stream(stream, q_);   // outputs and scratch belong to the launch stream
         auto dq = torch::empty_like(q_), dk = torch::empty_like(q_), dv = torch::empty_like(q_);
-        const size_t ws_bytes = tyr_hip_flash_attn_bwd_workspace_bytes(B, H, N, D);
-        auto ws = torch::empty({(int64_t)(ws_bytes ? ws_bytes : 16)}, q_.options().dtype(torch::kUInt8));
+        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, H, H, N, D, causal, 0), q_);
         const int rc = tyr_hip_flash_attn_bwd(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(),
                                               g_.data_ptr(), lse_.data_ptr<float>(), dq.data_ptr(),
                                               dk.data_ptr(), dv.data_ptr(), B, H, N, D, causal, (float)scale,
-                                              ws.data_ptr(), ws_bytes, reinterpret_cast<void*>(stream));
+                                              ws.ptr(), ws.bytes, reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("flashAttnBwd", rc);
         lean_object* inner = lean_alloc_ctor(0, 2, 0);
         lean_ctor_set(inner, 0, giveTensor(std::move(dk)));
@@ -209,12 +219,11 @@ lean_object* lean_tyr_gpu_flash_attn_bwd_gqa(uint64_t B, uint64_t Hq, uint64_t H
             return io_error(err);
         LaunchStreamScope on_stream(stream, q_);   // outputs and scratch belong to the launch stream
         auto dq = torch::empty_like(q_), dk = torch::empty_like(k_), dv = torch::empty_like(k_);
-        const size_t ws_bytes = tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D);
-        auto ws = torch::empty({(int64_t)(ws_bytes ? ws_bytes : 16)}, q_.options().dtype(torch::kUInt8));
+        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window), q_);
         const int rc = tyr_hip_flash_attn_bwd_gqa(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(),
                                                   g_.data_ptr(), lse_.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(),
                                                   dv.data_ptr(), B, Hq, Hkv, N, D, causal, window,
-                                                  n_.data_ptr<int32_t>(), (float)scale, ws.data_ptr(), ws_bytes,
+                                                  n_.data_ptr<int32_t>(), (float)scale, ws.ptr(), ws.bytes,
                                                   reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("flashAttnBwdGQA", rc);
         lean_object* inner = lean_alloc_ctor(0, 2, 0);
@@ -245,12 +254,11 @@ lean_object* lean_tyr_gpu_flash_attn_bwd_gqa_full(uint64_t B, uint64_t Hq, uint6
             return io_error(err);
         LaunchStreamScope on_stream(stream, q_);   // outputs and scratch belong to the launch stream
         auto dq = torch::empty_like(q_), dk = torch::empty_like(k_), dv = torch::empty_like(k_);
-        const size_t ws_bytes = tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D);
-        auto ws = torch::empty({(int64_t)(ws_bytes ? ws_bytes : 16)}, q_.options().dtype(torch::kUInt8));
+        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window), q_);
         const int rc = tyr_hip_flash_attn_bwd_gqa(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(),
                                                   g_.data_ptr(), lse_.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(),
                                                   dv.data_ptr(), B, Hq, Hkv, N, D, causal, window,
-                                                  nullptr, (float)scale, ws.data_ptr(), ws_bytes,
+                                                  nullptr, (float)scale, ws.ptr(), ws.bytes,
                                                   reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("flashAttnBwdGQA", rc);
         lean_object* inner = lean_alloc_ctor(0, 2, 0);
@@ -310,12 +318,11 @@ lean_object* lean_tyr_gpu_flash_attn_bwd_mask(uint64_t B, uint64_t Hq, uint64_t 
         if ((uint64_t)m_.numel() != B * N) return io_error("flashAttnBwdMask: keyMask must hold B*N bytes");
         LaunchStreamScope on_stream(stream, q_);   // outputs and scratch belong to the launch stream
         auto dq = torch::empty_like(q_), dk = torch::empty_like(k_), dv = torch::empty_like(k_);
-        const size_t ws_bytes = tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D);
-        auto ws = torch::empty({(int64_t)(ws_bytes ? ws_bytes : 16)}, q_.options().dtype(torch::kUInt8));
+        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, 0), q_);
         const int rc = tyr_hip_flash_attn_bwd_mask(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(),
                                                    g_.data_ptr(), lse_.data_ptr<float>(), dq.data_ptr(),
                                                    dk.data_ptr(), dv.data_ptr(), B, Hq, Hkv, N, D, causal,
-                                                   m_.data_ptr<uint8_t>(), (float)scale, ws.data_ptr(), ws_bytes,
+                                                   m_.data_ptr<uint8_t>(), (float)scale, ws.ptr(), ws.bytes,
                                                    reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("flashAttnBwdMask", rc);
         lean_object* inner = lean_alloc_ctor(0, 2, 0);
@@ -480,8 +487,9 @@ lean_object* lean_tyr_gpu_gemm_bf16(uint64_t M, uint64_t N, uint64_t K, b_lean_o
             return io_error(err);
         LaunchStreamScope on_stream(stream, a_);   // outputs and scratch belong to the launch stream
         auto c = torch::empty({(int64_t)M, (int64_t)N}, a_.options());
-        const int rc = tyr_hip_gemm_bf16(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), M, N, K, 0,
-                                         reinterpret_cast<void*>(stream));
+        const Scratch ws(tyr_hip_gemm_workspace_bytes(1, M, N, K, 2, 0), a_);
+        const int rc = tyr_hip_gemm_bf16_batched_ws(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), 1, M, N, K, 0, 0, 0, 0,
+                                                    ws.ptr(), ws.bytes, reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("gemmBf16", rc);
         return lean_io_result_mk_ok(giveTensor(std::move(c)));
     } catch (const std::exception& e) {
@@ -499,8 +507,9 @@ lean_object* lean_tyr_gpu_gemm_bf16_nt(uint64_t M, uint64_t N, uint64_t K, b_lea
             return io_error(err);
         LaunchStreamScope on_stream(stream, a_);   // outputs and scratch belong to the launch stream
         auto c = torch::empty({(int64_t)M, (int64_t)N}, a_.options());
-        const int rc = tyr_hip_gemm_bf16(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), M, N, K, 1,
-                                         reinterpret_cast<void*>(stream));
+        const Scratch ws(tyr_hip_gemm_workspace_bytes(1, M, N, K, 2, 1), a_);
+        const int rc = tyr_hip_gemm_bf16_batched_ws(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), 1, M, N, K, 0, 0, 0, 1,
+                                                    ws.ptr(), ws.bytes, reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("gemmBf16NT", rc);
         return lean_io_result_mk_ok(giveTensor(std::move(c)));
     } catch (const std::exception& e) {
@@ -519,8 +528,10 @@ lean_object* lean_tyr_gpu_gemm_fp8(uint64_t M, uint64_t N, uint64_t K, b_lean_ob
             return io_error(err);
         LaunchStreamScope on_stream(stream, a_);   // outputs and scratch belong to the launch stream
         auto c = torch::empty({(int64_t)M, (int64_t)N}, a_.options().dtype(torch::kBFloat16));
-        const int rc = tyr_hip_gemm_fp8(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), M, N, K, (float)scale_a,
-                                        (float)scale_b, 0, reinterpret_cast<void*>(stream));
+        const Scratch ws(tyr_hip_gemm_workspace_bytes(1, M, N, K, 1, 0), a_);
+        const int rc = tyr_hip_gemm_fp8_ws(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), M, N, K, (float)scale_a * (float)scale_b,
+                                           nullptr, nullptr, TYR_HIP_OUT_BF16, 0, ws.ptr(), ws.bytes,
+                                           reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("gemmFp8", rc);
         return lean_io_result_mk_ok(giveTensor(std::move(c)));
     } catch (const std::exception& e) {
@@ -538,8 +549,9 @@ lean_object* lean_tyr_gpu_matmul_bf16(uint64_t Bt, uint64_t M, uint64_t N, uint6
             return io_error(err);
         LaunchStreamScope on_stream(stream, a_);   // outputs and scratch belong to the launch stream
         auto c = torch::empty({(int64_t)Bt, (int64_t)M, (int64_t)N}, a_.options());
-        const int rc = tyr_hip_gemm_bf16_batched(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), Bt, M, N, K, M * K, K * N,
-                                                 M * N, 0, reinterpret_cast<void*>(stream));
+        const Scratch ws(tyr_hip_gemm_workspace_bytes(Bt, M, N, K, 2, 0), a_);
+        const int rc = tyr_hip_gemm_bf16_batched_ws(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), Bt, M, N, K, M * K, K * N,
+                                                    M * N, 0, ws.ptr(), ws.bytes, reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("matmulBf16", rc);
         return lean_io_result_mk_ok(giveTensor(std::move(c)));
     } catch (const std::exception& e) {
@@ -559,8 +571,10 @@ lean_object* lean_tyr_gpu_gemm_fp8_scaled(uint64_t M, uint64_t N, uint64_t K, b_
             return io_error(err);
         LaunchStreamScope on_stream(stream, a_);   // outputs and scratch belong to the launch stream
         auto c = torch::empty({(int64_t)M, (int64_t)N}, a_.options().dtype(torch::kFloat32));
-        const int rc = tyr_hip_gemm_fp8_ex(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), M, N, K, 1.0f, r_.data_ptr<float>(),
-                                           c_.data_ptr<float>(), TYR_HIP_OUT_F32, 0, reinterpret_cast<void*>(stream));
+        const Scratch ws(tyr_hip_gemm_workspace_bytes(1, M, N, K, 1, 0), a_);
+        const int rc = tyr_hip_gemm_fp8_ws(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), M, N, K, 1.0f, r_.data_ptr<float>(),
+                                           c_.data_ptr<float>(), TYR_HIP_OUT_F32, 0, ws.ptr(), ws.bytes,
+                                           reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("gemmFp8Scaled", rc);
         return lean_io_result_mk_ok(giveTensor(std::move(c)));
     } catch (const std::exception& e) {
@@ -578,8 +592,9 @@ lean_object* lean_tyr_gpu_gemm_fp8_e4m3(uint64_t M, uint64_t N, uint64_t K, b_le
             return io_error(err);
         LaunchStreamScope on_stream(stream, a_);   // outputs and scratch belong to the launch stream
         auto c = torch::empty({(int64_t)M, (int64_t)N}, a_.options());
-        const int rc = tyr_hip_gemm_fp8_ex(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), M, N, K, (float)scale, nullptr,
-                                           nullptr, TYR_HIP_OUT_E4M3, 0, reinterpret_cast<void*>(stream));
+        const Scratch ws(tyr_hip_gemm_workspace_bytes(1, M, N, K, 1, 0), a_);
+        const int rc = tyr_hip_gemm_fp8_ws(a_.data_ptr(), b_.data_ptr(), c.data_ptr(), M, N, K, (float)scale, nullptr,
+                                           nullptr, TYR_HIP_OUT_E4M3, 0, ws.ptr(), ws.bytes, reinterpret_cast<void*>(stream));
         if (rc != TYR_HIP_OK) return status_error("gemmFp8E4M3", rc);
         return lean_io_result_mk_ok(giveTensor(std::move(c)));
     } catch (const std::exception& e) {
