@@ -4,6 +4,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sys
 
 import pytest
 
@@ -138,6 +139,22 @@ int main(int, char** argv) {
     subprocess.check_call(["g++", "-O1", "-std=c++17", "-rdynamic", str(src), "-o", str(exe), "-ldl"])
     r = subprocess.run([str(exe), _lib.LIB_PATH], capture_output=True, text=True)
     assert r.returncode == 0 and r.stdout == "ok 1\n", (r.returncode, r.stdout, r.stderr[-500:])
+
+
+def test_import_opens_no_kernel_library(tmp_path):
+    """Importing the package opens nothing; the library is opened by the first call, and one that lacks functions (an older
+    build) is no error before a call needs them."""
+    src = tmp_path / "few.c"
+    src.write_text('const char* tyr_hip_strerror(int s) { return s ? "bad" : "ok"; }\n')
+    few = tmp_path / "libfew.so"
+    subprocess.check_call(["gcc", "-shared", "-fPIC", str(src), "-o", str(few)])
+    code = ("import tyr_amd, torch\nfrom tyr_amd import gpu\nmaps = open('/proc/self/maps').read()\n"
+            "assert '_tyr_torch' in maps and 'libfew' not in maps and 'libtyr_hip' not in maps\n"
+            "try: tyr_amd.copy(torch.zeros(4))\nexcept tyr_amd.TyrGpuError as e: assert 'CUDA tensor' in str(e), e\n"
+            "assert 'libfew' not in open('/proc/self/maps').read()\nprint('ok')\n")
+    for lib in (str(few), str(tmp_path / "absent.so"), _lib.LIB_PATH):
+        r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT, env=dict(os.environ, TYR_HIP_LIBRARY=lib))
+        assert r.returncode == 0 and r.stdout == "ok\n", (lib, r.stdout, r.stderr[-800:])
 
 
 def test_python_mirror_refuses_cpu_tensors_without_a_gpu():

@@ -37,13 +37,12 @@ class _Unbuilt:
 
     def __getattr__(self, name):
         _require(BINDING_PATH)
-        _require(LIB_PATH)
-        raise RuntimeError("the libraries were built after tyr_amd was imported: import it again in a new process")
+        raise RuntimeError("the binding was built after tyr_amd was imported: import it again in a new process")
 
 
 def load_binding(error: type):
-    """The native host layer (csrc/torch_binding.cpp), bound to the C ABI of LIB_PATH; it raises ``error``."""
-    if not (os.path.exists(BINDING_PATH) and os.path.exists(LIB_PATH)):
+    """The native host layer (csrc/torch_binding.cpp); it raises ``error`` and opens LIB_PATH when an entry point is called."""
+    if not os.path.exists(BINDING_PATH):
         return _Unbuilt()
     spec = importlib.util.spec_from_file_location("_tyr_torch", BINDING_PATH)
     binding = importlib.util.module_from_spec(spec)

@@ -19,6 +19,7 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <atomic>
 #include <cmath>
 #include <string>
 
@@ -26,25 +27,51 @@
 
 namespace {
 
-// The C ABI, resolved from the library the package loads (it can be another build, so it is not linked in).
+struct Failure {                      // becomes TyrGpuError
+    std::string what;
+};
+[[noreturn]] void fail(std::string what) { throw Failure{std::move(what)}; }
+
+// The C ABI.  It is not linked in: the library can be another build, and is opened by the first call of one of its
+// functions, not by the import of the package.  A build without some of them serves the calls that need only the others.
+std::string g_library;                // path, from load()
+PyObject* g_error = nullptr;          // tyr_amd.gpu.TyrGpuError
+
+void* library() {
+    static void* const handle = [] {  // a failed attempt throws and is repeated by the next call
+        void* h = dlopen(g_library.c_str(), RTLD_NOW | RTLD_LOCAL);
+        if (!h) fail(std::string(dlerror()) + " (build it with `make -C tyr_amd/csrc`; tyr_amd has no CPU or PyTorch fallback)");
+        return h;
+    }();
+    return handle;
+}
+template <class F> class Symbol;
+template <class R, class... A> class Symbol<R (*)(A...)> {
+    const char* name_;
+    mutable std::atomic<R (*)(A...)> f_{nullptr};
+public:
+    explicit Symbol(const char* name) : name_(name) {}
+    R operator()(A... a) const {
+        R (*f)(A...) = f_.load(std::memory_order_relaxed);
+        if (!f) {
+            f = reinterpret_cast<R (*)(A...)>(dlsym(library(), name_));
+            if (!f) fail(g_library + " does not export " + name_);
+            f_.store(f, std::memory_order_relaxed);
+        }
+        return f(a...);
+    }
+};
 #define TYR_ENTRY_POINTS(X)                                                                                                  \
     X(tyr_hip_strerror) X(tyr_hip_flash_attn_fwd_gqa) X(tyr_hip_flash_attn_fwd_mask) X(tyr_hip_flash_attn_bwd_full_workspace_bytes) \
     X(tyr_hip_flash_attn_bwd_gqa) X(tyr_hip_flash_attn_bwd_mask) X(tyr_hip_gqa_decode_workspace_bytes)                        \
     X(tyr_hip_gqa_decode_varlen) X(tyr_hip_decode_rope_append) X(tyr_hip_rope_fwd) X(tyr_hip_layernorm_residual)             \
     X(tyr_hip_copy) X(tyr_hip_gemm_workspace_bytes) X(tyr_hip_gemm_bf16_batched_ws) X(tyr_hip_gemm_fp8_ws)                    \
     X(tyr_hip_mse_loss_grad_workspace_bytes) X(tyr_hip_mse_loss_grad) X(tyr_hip_sgd_step)
-struct Api {
-#define X(f) decltype(&::f) f = nullptr;
+const struct Api {
+#define X(f) Symbol<decltype(&::f)> f{#f};
     TYR_ENTRY_POINTS(X)
 #undef X
 } api;
-
-PyObject* g_error = nullptr;          // tyr_amd.gpu.TyrGpuError
-
-struct Failure {                      // becomes TyrGpuError
-    std::string what;
-};
-[[noreturn]] void fail(std::string what) { throw Failure{std::move(what)}; }
 
 void check_status(int rc, const char* what) {
     if (rc != 0)
@@ -469,18 +496,12 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// load(path of libtyr_hip.so, exception class)
+// load(path of libtyr_hip.so, exception class): remembers both
 PyObject* load(PyObject*, PyObject* args) {
     const char* path = nullptr;
     PyObject* error = nullptr;
     if (!PyArg_ParseTuple(args, "sO", &path, &error)) return nullptr;
-    void* h = dlopen(path, RTLD_NOW | RTLD_LOCAL);
-    if (!h) return PyErr_Format(PyExc_RuntimeError, "%s", dlerror());
-#define X(f)                                                                                             \
-    api.f = reinterpret_cast<decltype(api.f)>(dlsym(h, #f));                                             \
-    if (!api.f) return PyErr_Format(PyExc_RuntimeError, "%s does not export %s", path, #f);
-    TYR_ENTRY_POINTS(X)
-#undef X
+    g_library = path;
     Py_INCREF(error);
     Py_XDECREF(g_error);
     g_error = error;
