@@ -84,3 +84,55 @@ def test_tiles_write_only_c(M, N, K, trans_b):
         assert bool((buf[:guard] == -7.0).all()) and bool((buf[guard + M * N:] == -7.0).all())
         assert bool((ws[need // 4:] == 5.0).all())
         assert rel_fro(buf[guard:guard + M * N].view(M, N).cpu(), a.float() @ b.float()) <= TOL_FRO
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (15, 4096, 144), (33, 272, 528), (65, 1296, 3088), (95, 4096, 2064), (127, 1024, 4112),
+                                   (129, 528, 1296), (3, 512, 8192), (333, 1408, 6608), (385, 2560, 2048), (1000, 2576, 1024), (2050, 1040, 1552)])
+def test_e4m3_output_of_the_tiles(M, N, K, trans_b):
+    """The bytes are the f32 output of the same product (same tile, same sums), clamped and rounded to nearest even; scaled so
+    that part of them saturate."""
+    import tyr_amd
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    aq, sa = tyr_amd.quantize_e4m3(torch.randn(M, K, generator=g, device="cuda"))
+    bq, sb = tyr_amd.quantize_e4m3(torch.randn(K, N, generator=g, device="cuda"))
+    rs = (torch.rand(M, generator=g, device="cuda") + 0.5) * 300.0
+    cs = torch.rand(N, generator=g, device="cuda") + 0.5
+    scale = sa * sb * K ** -0.5
+    bqb = bq.t().contiguous() if trans_b else bq
+    f = tyr_amd.gemm_fp8_scaled(aq, bqb, rs, cs, scale=scale, trans_b=trans_b)
+    want = (aq.float() @ bq.float()) * scale * rs[:, None] * cs[None, :]
+    assert rel_fro(f, want) <= 1e-4 and worst_line(f, want) <= 1e-3
+    if M * N > 1000:
+        assert float((f.abs() > 448.0).float().mean()) > 0.01
+    got = tyr_amd.gemm_fp8_scaled(aq, bqb, rs, cs, scale=scale, out_dtype=torch.float8_e4m3fn, trans_b=trans_b)
+    assert torch.equal(got.view(torch.uint8), f.clamp(-448.0, 448.0).to(torch.float8_e4m3fn).view(torch.uint8))
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("batch,M,N,K", [(2, 15, 4096, 144), (3, 33, 272, 528), (5, 65, 48, 80), (7, 1, 1040, 2048), (2, 129, 528, 1296),
+                                         (3, 200, 16, 4096), (4, 333, 1408, 1608), (2, 1000, 2576, 264)])
+def test_batches_of_tiles(batch, M, N, K, trans_b):
+    """Every entry has the bits of a product of its own without scratch (K in the same order), and nothing is written between
+    the entries of C."""
+    from tyr_amd import _lib
+    import tyr_amd
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(batch + M + N + K)
+    a = (torch.randn(batch, M, K, generator=g, device="cuda") * K ** -0.25).bfloat16()
+    b = (torch.randn(batch, *((N, K) if trans_b else (K, N)), generator=g, device="cuda") * K ** -0.25).bfloat16()
+    gap = 64
+    c = torch.full((batch, M * N + gap), -7.0, dtype=torch.bfloat16, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    rc = lib.tyr_hip_gemm_bf16_batched(a.data_ptr(), b.data_ptr(), c.data_ptr(), batch, M, N, K, M * K, N * K, M * N + gap, int(trans_b), stream)
+    assert rc == 0
+    assert bool((c[:, M * N:] == -7.0).all())
+    shared = tyr_amd.matmul_bf16(a, b[0].contiguous(), trans_b=trans_b)
+    assert torch.equal(tyr_amd.matmul_bf16(a, b, trans_b=trans_b), c[:, :M * N].view(batch, M, N))
+    one = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    for i in range(batch):
+        for got, bi in ((c[i, :M * N].view(M, N), b[i]), (shared[i], b[0])):
+            want = a[i].float() @ (bi.float().t() if trans_b else bi.float())
+            assert rel_fro(got, want) <= 3e-3 and worst_line(got, want) <= TOL_FRO
+            assert lib.tyr_hip_gemm_bf16(a[i].data_ptr(), bi.data_ptr(), one.data_ptr(), M, N, K, int(trans_b), stream) == 0
+            assert torch.equal(got, one)

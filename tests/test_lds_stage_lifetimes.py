@@ -1,10 +1,12 @@
 """Stage lifetimes of the kernels that fill LDS by global->LDS requests (no registers in between).
 
-Every such kernel keeps tiles in a small ring of LDS stages.  Two things must hold for every stage, whatever the
+Every such kernel keeps tiles in a small ring of LDS stages.  Three things must hold for every stage, whatever the
 relative speed of the waves of a workgroup:
 
   read-after-write   a fragment read of tile v from a stage comes after a workgroup barrier that every wave reached
                      after waiting for its own share of the requests of tile v (a wave only waits for its own requests);
+  write-after-write  two requests of a wave into one stage have a wait of that wave between them (whole tiles: the shares of a
+                     tile that several waves or instructions request go to different places of the stage);
   write-after-read   a request that overwrites a stage is issued after a workgroup barrier that follows, in every
                      wave's program order, the last read of the tile the stage held (LDS reads have returned at a
                      barrier: the compiler waits for them in front of it).
@@ -19,6 +21,9 @@ in an interval > i.
 The forward kernel once lacked the barrier between its prologue's reads of K stage 0 and the first step's request into
 that stage; `test_the_checker_catches_the_forward_kernels_old_race` runs that event order and demands a violation.
 """
+import os
+import re
+
 import pytest
 
 
@@ -29,9 +34,13 @@ class Trace:
         self.interval = 0
         self.events = []          # (kind, interval, stage, version)
         self.pending = []         # requests of this wave not yet waited for: indices into self.requests
+        self.collisions = []
         self.requests = []        # [stage, version, issued_interval, completed_barrier or None]
 
     def dma(self, stage, version):
+        for i in self.pending:                # two tiles on their way into one stage: either may land last
+            if self.requests[i][0] == stage and self.requests[i][1] != version:
+                self.collisions.append(f"{version} is requested into {stage} while {self.requests[i][1]} is in flight")
         self.requests.append([stage, version, self.interval, None])
         self.pending.append(len(self.requests) - 1)
 
@@ -58,7 +67,7 @@ class Trace:
 
 def violations(traces):
     """traces: one Trace per wave of a workgroup.  Returns a list of human-readable violations."""
-    out = []
+    out = [c for t in traces for c in t.collisions]
     skeleton = [(r[0], r[1], r[2], r[3]) for r in traces[0].requests]
     for t in traces[1:]:
         if [(r[0], r[1], r[2], r[3]) for r in t.requests] != skeleton:
@@ -86,13 +95,22 @@ def violations(traces):
 
 
 # ------------------------------------------------------------------ flash_attn_fwd_kernel (tyr_amd/csrc/flash_attn_fwd.hip)
-def forward_wave(passes, wave, barrier_after_prologue=True):
-    """passes: list of (nkv, nkv_w per wave, overlap_next).  Stages K0 K1 V0 V1; tile j of pass p is version (p, 'K'|'V', j).
+def forward_wave(passes, wave, barrier_after_prologue=True, restart=None, restart_waits=True):
+    """passes: list of (nkv, nkv_w per wave, overlap_next).  restart: tiles the prologue of a key-mask launch believed in before
+    it had read the mask; where the first of them is hidden it waits for what it requested and requests its first tiles again
+    (key-mask launches hand nothing over to a next tile).  Stages K0 K1 V0 V1; tile j of pass p is version (p, 'K'|'V', j).
     The epilogue stages O through the V stages (each wave its own quarter of them)."""
     t = Trace()
     preloaded = False
     for p, (nkv, nkv_ws, overlap_next) in enumerate(passes):
         nkv_w = nkv_ws[wave]
+        if restart is not None:
+            t.dma("K0", (p, "K", "before the mask"))
+            t.dma("V0", (p, "V", "before the mask"))
+            if restart > 1:
+                t.dma("K1", (p, "K", "before the mask"))
+            if restart_waits:
+                t.wait()
         if not preloaded:
             t.dma("K0", (p, "K", 0))
             t.dma("V0", (p, "V", 0))
@@ -152,12 +170,30 @@ def test_the_checker_catches_the_forward_kernels_old_race():
     assert v and all("K0" in x for x in v), v
 
 
+def key_mask_passes(nkvs):
+    return [(nkv, nkv_w, False) for nkv, nkv_w, _ in forward_passes(nkvs)]
+
+
+@pytest.mark.parametrize("before", [1, 2, 7])
+@pytest.mark.parametrize("nkvs", [[1], [2], [5], [4, 1], [3, 6]])
+def test_forward_kernel_with_hidden_first_tiles(nkvs, before):
+    assert violations([forward_wave(key_mask_passes(nkvs), w, restart=before) for w in range(4)]) == []
+
+
+def test_the_second_request_of_a_key_mask_prologue_needs_its_wait():
+    v = violations([forward_wave(key_mask_passes([3]), w, restart=4, restart_waits=False) for w in range(4)])
+    assert v and all("in flight" in x for x in v), v
+
+
 # ------------------------------------------------------------------ flash_attn_bwd_dq_kernel (tyr_amd/csrc/flash_attn_bwd.hip)
-def dq_wave(passes, wave):
-    """Stages KV0 KV1 (K and V of a tile are requested together); the epilogue stages dQ through the front of the LDS
+def dq_wave(passes, wave, restart=False):
+    """restart: as in the forward kernel, for a first tile that the key mask hides.  Stages KV0 KV1 (K and V of a tile are requested together); the epilogue stages dQ through the front of the LDS
     block, which overlaps both stages."""
     t = Trace()
     for p, (nkv, nkv_ws) in enumerate(passes):
+        if restart:
+            t.dma("KV0", (p, "before the mask"))
+            t.wait()
         t.dma("KV0", (p, 0))
         t.wait()
         t.bar()
@@ -180,6 +216,7 @@ def dq_wave(passes, wave):
 def test_backward_dq_kernel(nkvs):
     passes = [(n, [max(1, n - 1), max(1, n - 1), n, n]) for n in nkvs]
     assert violations([dq_wave(passes, w) for w in range(4)]) == []
+    assert violations([dq_wave(passes, w, restart=True) for w in range(4)]) == []
 
 
 # ------------------------------------------------------------------ flash_attn_bwd_dkv_kernel
@@ -273,3 +310,76 @@ def gemm_wave(KT, ksteps):
 @pytest.mark.parametrize("KT", [1, 2, 3, 4, 63, 64])
 def test_gemm_fast_kernels(KT, ksteps, waves):
     assert violations([gemm_wave(KT, ksteps) for _ in range(waves)]) == []
+
+
+# ------------------------------------------------------------------ gemm_tile_kernel (tyr_amd/csrc/gemm_tile.hpp)
+def tile_configs():
+    """(waves of a k-group, k-groups, stages) of every tile, read from the source."""
+    text = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tyr_amd", "csrc", "gemm_tile.hpp")).read()
+    found = re.findall(r"TYR_TILE\(T\d+x\d+, (\d+), (\d+), (\d+), (\d+), (\d+), (\d+)\)", text)
+    assert len(found) == 11
+    return sorted({((int(bm) // int(wtm)) * (int(bn) // int(wtn)), int(kg), int(st)) for bm, bn, wtm, wtn, kg, st in found})
+
+
+def tile_wave(np, kg, groups, stages, kept=2):
+    """A wave of k-group kg whose waves share a ring of `stages`: pieces kg, kg + groups, ... of np, one barrier per piece for the
+    whole workgroup, `stages` pieces requested ahead.  A step waits for piece i + 1 (all but the newest stages - `kept` requests;
+    everything once no full ring is in flight), synchronises, refills the stage of piece i and reads piece i + 1.  A group with
+    a piece less reads a stage at its last step that nobody filled, and drops it (not modelled).  The accumulators then go
+    through the whole ring."""
+    t = Trace()
+    n_own = max(0, -(-(np - kg) // groups))
+    n_iter = -(-np // groups)
+    for i in range(min(stages, n_own)):
+        t.dma(f"S{i}", i)
+    t.wait(keep_newest=stages - 1 if stages <= n_own else 0)
+    t.bar()
+    if n_own > 0:
+        t.read("S0", 0)
+    for i in range(n_iter - 1):
+        t.wait(keep_newest=stages - kept if i + stages <= n_own else 0)
+        t.bar()
+        if i + stages < n_own:
+            t.dma(f"S{i % stages}", i + stages)
+        if i + 1 < n_own:
+            t.read(f"S{(i + 1) % stages}", i + 1)
+    t.bar()
+    assert not t.pending                     # nothing lands in the ring any more when the accumulators do
+    for i in range(stages):
+        t.store(f"S{i}", "sums")
+    t.bar()
+    for i in range(stages):
+        t.read(f"S{i}", "sums")
+    return t
+
+
+@pytest.mark.parametrize("np", [1, 2, 3, 4, 5, 6, 7, 8, 9, 31, 32, 33])
+def test_gemm_tile_rings_shared_by_waves(np):
+    for waves, groups, stages in tile_configs():
+        if waves > 1:
+            for kg in range(groups):
+                assert violations([tile_wave(np, kg, groups, stages) for _ in range(waves)]) == [], (waves, groups, stages, kg)
+
+
+def test_a_gemm_tile_step_that_waited_for_one_piece_less_would_be_caught():
+    assert any("before its request completed" in v for v in violations([tile_wave(9, 0, 1, 3, kept=1) for _ in range(4)]))
+
+
+@pytest.mark.parametrize("np", [1, 2, 3, 4, 5, 6, 7, 8, 9, 31, 32, 33])
+def test_gemm_tile_rings_of_one_wave(np):
+    """A k-group of one wave has no barrier: its own waits order everything.  Piece i is waited for, read into registers
+    (lgkmcnt(0)) and only then is its stage requested again."""
+    alone = [c for c in tile_configs() if c[0] == 1]
+    assert alone
+    for _, groups, stages in alone:
+        for kg in range(groups):
+            t, n_own = Trace(), max(0, -(-(np - kg) // groups))
+            for i in range(min(stages, n_own)):
+                t.dma(f"S{i}", i)
+            for i in range(n_own):
+                t.wait(keep_newest=stages - 1 if i + stages <= n_own else 0)
+                holds = [r for r in t.requests if r[0] == f"S{i % stages}"][-1]
+                assert holds[1] == i and holds[3] == "waited", (groups, stages, kg, i)
+                if i + stages < n_own:
+                    t.dma(f"S{i % stages}", i + stages)
+            assert not t.pending and not t.collisions
