@@ -105,6 +105,22 @@ def test_backward_cuts_key_tiles_where_that_is_faster(B, Hq, Hkv, N, D, cut):
     assert (L.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, 1, 0) > least) == cut
 
 
+@pytest.mark.parametrize("bh,N,D,causal,window,rows", [
+    (96, 382, 128, 0, 0, 128),         # whole backward 60.6 us with 128-row tiles for dQ, 67.6 with 64
+    (40, 8160, 128, 1, 103, 128),      # 261, 285
+    (384, 810, 128, 1, 613, 128),      # 392, 416
+    (12, 3472, 128, 1, 0, 64),         # 181, 170
+    (8, 3545, 128, 1, 763, 64),        # 66.2, 64.4: few jobs under a window
+    (192, 150, 64, 0, 0, 128)])        # 23.8, 25.1
+def test_dq_takes_the_form_that_is_faster_for_it(bh, N, D, causal, window, rows):
+    """The dQ kernel's tiles are chosen by its own step times (internal function; the times are of an MI355X)."""
+    class Shape(ctypes.Structure):
+        _fields_ = [("rows", ctypes.c_int), ("pair", ctypes.c_int), ("single", ctypes.c_int)]
+    shape = ctypes.CDLL(_lib.LIB_PATH)["_ZN3tyr10attn_shapeEliibib"]
+    shape.restype, shape.argtypes = Shape, [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_bool, ctypes.c_int, ctypes.c_bool]
+    assert shape(bh, N, D, bool(causal), window, True).rows == rows
+
+
 def test_nothing_throws_when_the_heap_is_exhausted(tmp_path):
     """The header promises that no entry point throws.  Host-side planning runs here with an operator new that fails: an
     exception would leave a C function and end the process."""

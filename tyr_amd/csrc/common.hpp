@@ -374,8 +374,8 @@ struct AttnOrder {
     }
 };
 // What one job of a launch is: `rows` query rows (128, or 64 with the keys of every tile shared by two waves), and for
-// causal launches paired tiles or single ones.
+// causal launches paired tiles or single ones.  dq: for the dQ kernel, whose steps take other times than the forward's.
 struct AttnShape { int rows, pair, single; };
-AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window);
+AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window, bool dq);
 
 }  // namespace tyr

@@ -1075,7 +1075,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     const int BH = B * Hq, BHkv = B * Hkv, G = Hq / Hkv;
     const int ntk = (N + 127) / 128, npad = ntk * 128;
     const bool limits = window > 0 || kv_lens != nullptr;     // never together with a key mask
-    const AttnShape shape = attn_shape(BH, N, D, causal != 0, window);
+    const AttnShape shape = attn_shape(BH, N, D, causal != 0, window, true);
     const int ntq = (N + shape.rows - 1) / shape.rows;
     const int pair = shape.pair, single = shape.single;
     dim3 grid_q((unsigned)(BH * (pair ? (ntq + 1) / 2 : ntq))), block(THREADS);

@@ -485,10 +485,7 @@ __global__ __launch_bounds__(fa::THREADS, 2) void flash_attn_fwd_kernel(
     }
 }
 
-// The jobs of a launch and the time of its busiest CU.  Times are microseconds on an MI355X, measured on 150 shapes (4 to
-// 256 heads, 64 to 4096 rows): a key-tile step of a 128-row workgroup takes 1.0 us at D = 128 (0.64 at D = 64) with the device
-// busy, of a 64-row one 0.61 (0.38); a launch costs 5.6-6.1 us besides, a second workgroup of a CU and the second tile of
-// a pair 1-2.  The choice is 1.3 % slower on those shapes than the best of the three forms.
+// The jobs of a launch and the time of its busiest CU.
 namespace {
 struct AttnJobs {
     int ntq, steps0;             // tiles per head; steps of the longest
@@ -503,7 +500,26 @@ struct AttnJobs {
     }
     int ranks() const { return paired ? (ntq + 1) / 2 : ntq; }
 };
-double busiest_cu_us(const AttnJobs& jobs, int64_t bh, double step, double alone, double fixed, double extra) {
+// Microseconds on an MI355X: a key-tile step with two workgroups on the CU; by how much more a step costs a workgroup alone
+// on it; the launch; a second workgroup of a CU (or the second tile of a pair).
+struct FormTimes { double step, alone, fixed, extra; };
+enum Form { PAIRS, SINGLES, ROWS64, FORMS };
+// Under a window two tiles of a job are masked, and a 128-row workgroup alone on its CU hides none of that (forward, B1 Hq16
+// N1800 window 600: 1.25 us a step, 20.3 us, 19.1 with 64 rows; dQ with up to 256 jobs of 128 rows 3-10 % slower than 64).
+// Forward: on 150 shapes (4 to 256 heads, 64 to 4096 rows) the choice is 1.3 % slower than the best of the three forms.
+// dQ: three products a step for two, and one workgroup on a CU leaves more of it idle (128 rows, D = 128: 1.65 us a step
+// alone, 1.36-1.41 beside another; 64 rows 0.87).  On 471 shapes the choice is 0.7 % slower than the best form, with the
+// forward's times 1.4 %: B3 H32 N382 not causal 67.6 us for 60.6 (whole backward), B5 Hq8 Hkv2 N8160 window 103 285 for 261.
+FormTimes form_times(bool dq, int D, int form, bool edges) {
+    if (dq)
+        return D == 128 ? (form == ROWS64 ? FormTimes{0.87, 1.1, 8.0, 1.5} : FormTimes{1.36, edges ? 1.5 : form == PAIRS ? 1.1 : 1.2, 6.0, 1.3})
+                        : (form == ROWS64 ? FormTimes{0.45, 1.1, 6.5, 1.5} : FormTimes{0.80, edges ? 1.5 : 1.25, 6.0, 1.3});
+    return D == 128 ? (form == ROWS64 ? FormTimes{edges ? 0.56 : 0.61, 0.97, 6.1, 1.0} : FormTimes{1.0, edges ? 1.25 : 0.95, 5.6, 1.3})
+                    : (form == ROWS64 ? FormTimes{edges ? 0.36 : 0.38, 1.3, 5.0, 0.8} : FormTimes{0.64, edges ? 1.4 : 1.1, 4.7, 1.0});
+}
+// uneven: by how much more each step costs that the longer one of two workgroups of a CU has alone
+double busiest_cu_us(const AttnJobs& jobs, int64_t bh, const FormTimes& t, double uneven) {
+    const double step = t.step, alone = t.alone, fixed = t.fixed, extra = t.extra;
     const int64_t n = bh * jobs.ranks();
     if (n <= 256) return fixed + step * alone * jobs.work(0);
     if (n <= 512) {
@@ -511,7 +527,8 @@ double busiest_cu_us(const AttnJobs& jobs, int64_t bh, double step, double alone
         double worst = alone * jobs.work(0);
         for (int64_t j = 0; j < n - 256;) {
             const int64_t a = 255 - j, b = 256 + j;
-            worst = std::max(worst, jobs.work((int)(a / bh)) + jobs.work((int)(b / bh)));
+            const double first = jobs.work((int)(a / bh)), second = jobs.work((int)(b / bh));
+            worst = std::max(worst, first + second + uneven * (first - second));
             j += std::min(a % bh + 1, bh - b % bh);
         }
         return fixed + step * worst + extra;
@@ -525,25 +542,21 @@ double busiest_cu_us(const AttnJobs& jobs, int64_t bh, double step, double alone
 }
 }  // namespace
 
-AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window) {
+AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window, bool dq) {
     const bool ordered = causal && window <= 0;      // a window makes the tiles equal
     AttnShape best{128, 0, 0};
     double least = 1e300;
-    for (int form = 0; form < 3; ++form) {           // 0 = pairs, 1 = single tiles, 2 = 64-row tiles
-        const int rows = form == 2 ? 64 : 128, ntq = (N + rows - 1) / rows;
-        if (form == 0 && (!ordered || ntq == 1)) continue;
+    for (int form = PAIRS; form < FORMS; ++form) {   // pairs, single tiles, single tiles of 64 rows
+        const int rows = form == ROWS64 ? 64 : 128, ntq = (N + rows - 1) / rows;
+        if (form == PAIRS && (!ordered || ntq == 1)) continue;
         // many single tiles, longest first, walk all heads at once: their K / V do not fit an L2 (the backward of 256 heads
         // of 4096 rows was 14 % slower that way than with pairs, head after head)
-        if (form != 0 && ordered && ntq > 1 && bh * ntq > 2048) continue;
+        if (form != PAIRS && ordered && ntq > 1 && bh * ntq > 2048) continue;
         const int all = (N + 63) / 64, seen = window > 0 ? std::min<int64_t>(all, ((int64_t)window + rows) / 64 + 1) : all;
-        const AttnJobs jobs{ntq, seen, ordered, form == 0, rows, N};
-        // under a window two tiles of a job are masked, and a 128-row workgroup alone on its CU hides none of that (1.25 us a
-        // step; B1 Hq16 N1800 window 600: 20.3 us, 19.1 with 64 rows)
-        const bool edges = window > 0 && window < N;
-        const double us =
-            D == 128 ? (form == 2 ? busiest_cu_us(jobs, bh, edges ? 0.56 : 0.61, 0.97, 6.1, 1.0) : busiest_cu_us(jobs, bh, 1.0, edges ? 1.25 : 0.95, 5.6, 1.3))
-                     : (form == 2 ? busiest_cu_us(jobs, bh, edges ? 0.36 : 0.38, 1.3, 5.0, 0.8) : busiest_cu_us(jobs, bh, 0.64, edges ? 1.4 : 1.1, 4.7, 1.0));
-        if (us < least) { least = us; best = {rows, form == 0, form != 0 && ordered}; }
+        const AttnJobs jobs{ntq, seen, ordered, form == PAIRS, rows, N};
+        const FormTimes times = form_times(dq, D, form, window > 0 && window < N);
+        const double us = busiest_cu_us(jobs, bh, times, dq ? times.alone - 1.0 : 0.0);
+        if (us < least) { least = us; best = {rows, form == PAIRS, form != PAIRS && ordered}; }
     }
     return best;
 }
@@ -557,7 +570,7 @@ int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, 
     const int G = Hq / Hkv;
     const bool limits = window > 0 || kv_lens != nullptr;     // never together with a key mask
     // a window makes the tiles equal; lengths and key masks keep tile 0 starting at key 0
-    const AttnShape shape = attn_shape(BH, N, D, causal != 0, window);
+    const AttnShape shape = attn_shape(BH, N, D, causal != 0, window, false);
     const int ntq = (N + shape.rows - 1) / shape.rows;
     const int pair = shape.pair, single = shape.single;
     const int total_ids = BH * (pair ? (ntq + 1) / 2 : ntq);
