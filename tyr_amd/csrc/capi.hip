@@ -334,7 +334,8 @@ int tyr_hip_gqa_decode_static(const void* q, const void* k, const void* v, void*
         return TYR_HIP_ERR_BAD_SHAPE;
     if (num_splits == 0) {
         // A call with one split does not touch the array, so such calls may overlap on the device; from 256 groups on and
-        // below 1024 rows callers can rely on it.  Elsewhere as many splits as the array holds.
+        // below 1024 rows callers can rely on it (8 groups of 1000 rows: 12.4 us, 7.5 with 11 splits).  Elsewhere as many
+        // splits as the array holds.
         const uint64_t most = B * Hkv >= 256 || L < 1024 ? 1 : auto_splits(B, Hkv, L);
         num_splits = std::max<uint64_t>(1, std::min<uint64_t>(most, kStaticScratchBytes / (B * Hq * (D + 2) * sizeof(float))));
     }

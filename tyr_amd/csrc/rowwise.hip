@@ -92,8 +92,8 @@ __global__ __launch_bounds__(rw::THREADS) void copy_kernel(const u32x4* __restri
 }
 
 // x, y: [B*S*H][D].  One thread rotates one piece pair; a row takes per_row = D / (2E) consecutive threads.  I = uint32_t
-// unless there are more threads than that counts: with 64-bit divisions a thread spent as long on its indices as on its
-// 64 bytes (together with plain loads 2222 x 32 heads of 128: 8.4 -> 7.0 us, 36 MB).
+// unless there are more threads than that counts (x from 137 GB on): with 64-bit divisions a thread spent as long on its
+// indices as on its 64 bytes (together with plain loads 2222 x 32 heads of 128: 8.4 -> 7.0 us, 36 MB).
 template <typename T, bool CACHED, typename I>
 __global__ __launch_bounds__(rw::THREADS) void rope_kernel(const T* __restrict__ x, const float* __restrict__ cosp,
                                                            const float* __restrict__ sinp, T* __restrict__ y,
