@@ -206,8 +206,9 @@ int tyr_hip_flash_attn_bwd_gqa(const void* q, const void* k, const void* v, cons
                                void* workspace, size_t workspace_bytes, void* stream);
 
 /* Workspace with which the call is fastest.  dK / dV of few (or, causal, very unequal) key tiles leave most of the device
- * idle; with this much scratch their work is cut over more workgroups whose f32 partial sums a last kernel adds.  Anything
- * between tyr_hip_flash_attn_bwd_workspace_bytes and this is accepted and simply not cut.  Same bytes with a key mask
+ * idle; with this much scratch their work is cut over more workgroups whose f32 partial sums a last kernel adds.  For few
+ * heads (D = 128) it also holds dS in bf16, at most 288 MiB, from which dQ is one product instead of three.  Anything between
+ * tyr_hip_flash_attn_bwd_workspace_bytes and this is accepted and runs as with the minimum.  Same bytes with a key mask
  * (window = 0).  Results are reproducible either way and agree to the rounding of f32 sums. */
 size_t tyr_hip_flash_attn_bwd_full_workspace_bytes(uint64_t B, uint64_t Hq, uint64_t Hkv, uint64_t N, uint64_t D, int causal,
                                                    uint64_t window);

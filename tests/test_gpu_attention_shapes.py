@@ -159,3 +159,73 @@ def test_backward_with_the_least_workspace(B, Hq, Hkv, N, D, mask):
         # unit apart at most (2^-8 of them; twice that allowed, and 1e-5 of a mean row where all terms cancel)
         n = parts.float().norm(dim=-1)
         assert bool(((got.float() - parts.float()).norm(dim=-1) <= 2 ** -7 * n + 1e-5 * n.mean()).all())
+
+
+@pytest.mark.parametrize("mask", ["causal", "full", "window", "lens", "keys"])
+@pytest.mark.parametrize("B,Hq,Hkv,N", [(4, 16, 4, 577), (4, 16, 16, 640), (2, 32, 8, 1153), (4, 8, 1, 1025)])
+def test_backward_that_keeps_ds(B, Hq, Hkv, N, mask):
+    """Few heads at D = 128, where dK / dV leave dS for dQ: rows one past a tile, whole tiles, whole and cut key tiles.  Hidden keys
+    come first, in the middle (more than one block of 128) and last, with values that would outweigh every visible one."""
+    import tyr_amd
+    from tyr_amd import _lib
+    lib, D = _lib.load(), 128
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    q, k, v, g = (torch.randn(B, h, N, D, device="cuda", generator=gen).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    i = torch.arange(N, device="cuda")
+    visible = (i[None, :] <= i[:, None] if mask != "full" else torch.ones(N, N, dtype=torch.bool, device="cuda"))[None, None].expand(B, 1, N, N)
+    opt, window = dict(causal=mask != "full"), 0
+    shown = torch.ones(B, N, dtype=torch.bool, device="cuda")
+    if mask == "window":
+        opt["window"] = window = N - 37
+        visible = visible & (i[:, None] - i[None, :] < window)
+    if mask == "lens":
+        opt["kv_lens"] = torch.tensor([N, 0, N // 2 + 1, 129][:B], dtype=torch.int32, device="cuda")
+        shown = i[None, :] < opt["kv_lens"][:, None]
+    if mask == "keys":
+        shown = torch.rand(B, N, device="cuda", generator=gen) > 0.3
+        shown[:, :70] = shown[:, 130:400] = shown[0, -140:] = shown[-1] = False
+        opt["key_mask"] = shown
+    visible = visible & shown[:, None, None, :]
+    loud = torch.where(shown[:, None, :, None], 1.0, 300.0).bfloat16()
+    k, v = k * loud, v * loud
+    least = lib.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D)
+    assert lib.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, int(opt["causal"]), window) - least >= B * Hq * N * N
+    o, lse = tyr_amd.flash_attn_fwd(q, k, v, **opt)
+    grads = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)
+    *_, wq, wk, wv = reference(q, k, v, g, visible)
+    for got, ref in zip(grads, (wq, wk, wv)):
+        assert rel_fro(got, ref) <= 1e-2
+        err, n = (got.float() - ref).norm(dim=-1), ref.norm(dim=-1)
+        assert float((err / n.clamp_min(float(n[n > 0].mean()))).max()) <= 4e-2
+    assert all(torch.equal(a, b) for a, b in zip(grads, tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)))
+    # with the least scratch dQ makes dS itself, from the same bf16 operands: what may differ is the order of f32 sums, and
+    # with it one rounding to bf16 (2^-8 of an element) here and there
+    ws, plain = torch.empty(least, dtype=torch.uint8, device="cuda"), [torch.empty_like(t) for t in (q, k, v)]
+    ptrs = [t.data_ptr() for t in (q, k, v, o, g, lse, *plain)]
+    tail = (D ** -0.5, ws.data_ptr(), least, torch.cuda.current_stream().cuda_stream)
+    if mask == "keys":
+        rc = lib.tyr_hip_flash_attn_bwd_mask(*ptrs, B, Hq, Hkv, N, D, 1, opt["key_mask"].data_ptr(), *tail)
+    else:
+        lens = opt["kv_lens"].data_ptr() if mask == "lens" else None
+        rc = lib.tyr_hip_flash_attn_bwd_gqa(*ptrs, B, Hq, Hkv, N, D, int(opt["causal"]), window, lens, *tail)
+    assert rc == 0
+    assert all(rel_fro(a, b.float()) <= 1e-3 for a, b in zip(grads, plain))
+
+
+def test_backward_without_memory_for_ds():
+    """Where the full scratch cannot be had, the call runs with the least."""
+    import tyr_amd
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    q, g = (torch.randn(1, 32, 2000, 128, device="cuda", generator=gen).bfloat16() for _ in range(2))
+    k, v = (torch.randn(1, 8, 2000, 128, device="cuda", generator=gen).bfloat16() for _ in range(2))
+    o, lse = tyr_amd.flash_attn_fwd(q, k, v, causal=True)
+    want = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, causal=True)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (96 << 20)) / total)
+    try:
+        got = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, causal=True)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert all(rel_fro(a, b.float()) <= 1e-3 for a, b in zip(got, want))

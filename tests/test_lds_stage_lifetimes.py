@@ -276,6 +276,59 @@ def test_three_stages_would_not_be_enough_for_the_dkv_kernel():
     assert violations([dkv_wave(6, 1, w, True, stages=3) for w in range(4)])
 
 
+def dkv_waits(ntile, wave, with_stores=17):
+    """The counted waits of a dK/dV wave that also stores dS: `s_waitcnt vmcnt(n)` leaves the newest n of its loads (9 a tile) and
+    stores (2 a step) in flight.  Yields, per wait, whether the tile that is read next has landed."""
+    queue, u0 = [], wave
+    for k in range(3):
+        queue += [("load", k)] * 9
+    queue = queue[len(queue) - 18:]
+    for u in range(2 * ntile):
+        if u % 2 == 0 and u // 2 + 1 < ntile:
+            keep = with_stores if u - u0 >= 4 else 9
+            queue = queue[max(0, len(queue) - keep):]
+            yield ("load", u // 2 + 1) not in queue
+            queue += [("load", u // 2 + 3)] * 9
+        if u >= u0:
+            queue += [("store", u)] * 2
+
+
+@pytest.mark.parametrize("ntile", [1, 2, 3, 4, 5, 9, 64])
+def test_dkv_waits_count_the_ds_stores(ntile):
+    assert all(all(dkv_waits(ntile, w)) for w in range(4))
+
+
+def test_a_dkv_wait_that_left_one_more_in_flight_would_be_caught():
+    assert not all(all(dkv_waits(9, w, with_stores=18)) for w in range(4))
+
+
+# ------------------------------------------------------------------ flash_attn_bwd_dq_product_kernel
+def dq_product_wave(n, wave, causal=True, stages=5):
+    """Stages S0..S4 (32 keys of dS and K), four in flight; stages past the last are requested as well (zeros).  A causal wave
+    reads the stages up to its own rows'."""
+    t = Trace()
+    for i in range(stages - 1):
+        t.dma(f"S{i}", i)
+    for j in range(n):
+        t.wait(keep_newest=stages - 2)
+        t.bar()
+        t.dma(f"S{(j - 1) % stages}", j + stages - 1)
+        if not causal or j < n - 3 + wave:
+            t.read(f"S{j % stages}", j)
+    t.wait()
+    t.bar()
+    for s in range(stages):
+        t.store(f"S{s}", "dQ")
+        t.read(f"S{s}", "dQ")
+    return t
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 6, 63])
+def test_backward_dq_product_kernel(n, causal):
+    assert violations([dq_product_wave(n, w, causal) for w in range(4)]) == []
+
+
 # ------------------------------------------------------------------ gemm_bf16_fast_kernel / gemm_fp8_fast_kernel
 def gemm_wave(KT, ksteps):
     """Two stages S0 S1, each an A and a B slice.  Slice kt+1 is requested during the first k-steps of slice kt; the

@@ -32,6 +32,9 @@
 // Both recompute S (7 matrix products for an algorithm that needs 5): the price of writing dQ
 // without a float atomic accumulation buffer and a conversion pass.
 //
+// Few heads (keeps_ds) run the 5 products: flash_attn_bwd_stats_kernel makes the pairs, dK/dV goes first and leaves
+// its bf16 dS in the workspace, and flash_attn_bwd_dq_product_kernel adds dQ = dS K from there.  Same operands and roundings.
+//
 // LDS tiles are row-major with 16-byte chunks XOR-swizzled by a function of the row that is
 // conflict-free both for row fragments (16-byte reads, lane = row) and for transposed fragments
 // (ds_read_b64_tr_b16 over 4 rows x 64 bytes per lane-group pair).
@@ -435,18 +438,36 @@ struct Parts {
         part = __builtin_amdgcn_readfirstlane(item - (kt > 0 ? __shfl(upto, kt > 0 ? kt - 1 : 0, 64) : 0));
     }
 };
+// dS as the dK / dV workgroups leave it for flash_attn_bwd_dq_product_kernel: bf16 blocks of 32 query rows x 32 keys, 2 KB, as
+// a wave holds them (store_ds), so that every store of the one and every request of the other is a whole kilobyte.  The
+// blocks of 128 query rows are adjacent, ordered by key and then by query row: what a dQ workgroup reads is one stream.
+// Only blocks that the causal rule or a window lets be visible have a place.
+struct DsBlocks {
+    int ntk, causal, window;                         // ntk = tiles of 128 rows (of queries and of keys)
+    __host__ __device__ int width() const {          // key tiles that have a place for a query tile (causal without a window: qt + 1)
+        const int w = causal && window > 0 ? (window - 1 + 127) / 128 + 1 : ntk;
+        return w < ntk ? w : ntk;
+    }
+    __host__ __device__ bool triangle() const { return causal && window <= 0; }
+    // first key tile with a place; first block of the query tile
+    __host__ __device__ int first(int qt) const { const int f = qt + 1 - width(); return causal && window > 0 && f > 0 ? f : 0; }
+    __host__ __device__ int64_t at(int qt) const { return triangle() ? 8 * (int64_t)qt * (qt + 1) : 16 * (int64_t)width() * qt; }
+    __host__ __device__ int tiles(int qt) const { return triangle() ? qt + 1 : width(); }
+    __host__ __device__ int64_t head_bytes() const { return at(ntk) * 2048; }
+};
 }  // namespace fab
 
 // CUT: the launch has parts.  (Whole key tiles keep their own instantiation: with the bookkeeping of the parts in the same
 // code the pipeline below, which has no register to spare, is 4-8 % slower.)
 // OWN_STATS: nothing ran before this kernel, so the workgroup makes the (lse2, delta) pairs of its query rows itself.
-template <int D, bool CAUSAL, AttnMask MASK, bool CUT, bool OWN_STATS>
+// SPILL: dS also goes to `ds`, for the dQ launch after this one.
+template <int D, bool CAUSAL, AttnMask MASK, bool CUT, bool OWN_STATS, bool SPILL>
 __device__ __forceinline__ void bwd_dkv(int block,
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE, float2* stats,
     uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int BHkv, int N, int ntk, int npad, float scale, float scale_log2,
     int Hq, int window, const int* __restrict__ kv_lens, const uint8_t* __restrict__ key_mask, fab::Parts plan, int items,
-    float* __restrict__ partial) {
+    float* __restrict__ partial, unsigned char* __restrict__ ds) {
     constexpr bool WINDOW = MASK == AttnMask::Limits, PER_KEY = MASK != AttnMask::None;
     if (WINDOW && OWN_STATS && window <= 0) window = INT_MAX;      // lengths alone have no instantiation of their own there
     const int G = plan.G;
@@ -519,6 +540,22 @@ __device__ __forceinline__ void bwd_dkv(int block,
             kf[i] = __builtin_bit_cast(bf16x8, ld_global_16(Kp + off + i * 16));
             vf[i] = __builtin_bit_cast(bf16x8, ld_global_16(Vp + off + i * 16));
         }
+    }
+    // SPILL: the dS of a hidden key has to be 0, not only what it adds up to here.  Its K and V are taken as 0 and its scores
+    // start from -inf instead of 0 (the accumulator operand of their first product), so P and dS are 0 without an instruction
+    // in the steps.  Causal launches without a mask have no such key: the ones past N are above every query's diagonal.
+    constexpr bool KEY_BIAS = SPILL && (MASK != AttnMask::None || !CAUSAL);
+    f32x16 bias;
+    if constexpr (KEY_BIAS) {
+        const bool hidden = kvpos >= Nk || (key_mask != nullptr && key_mask[(size_t)(bh / hkv) * N + min(kvpos, N - 1)] == 0);
+#pragma unroll
+        for (int i = 0; i < C::KSTEPS; ++i) {
+            const bf16x8 zero = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
+            kf[i] = hidden ? zero : kf[i];
+            vf[i] = hidden ? zero : vf[i];
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) bias[e] = hidden ? -INFINITY : 0.0f;
     }
 
     // ---- Q / dO / pair tile loaders
@@ -619,7 +656,7 @@ __device__ __forceinline__ void bwd_dkv(int block,
     // S = Q K_w^T and dP = dO V_w^T of one sub-tile from its row fragments
     auto scores = [&](const bf16x8 (&qa)[C::KSTEPS], const bf16x8 (&da)[C::KSTEPS], f32x16& s, f32x16& dp) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) { s[e] = 0.0f; dp[e] = 0.0f; }
+        for (int e = 0; e < 16; ++e) { s[e] = KEY_BIAS ? bias[e] : 0.0f; dp[e] = 0.0f; }
 #pragma unroll
         for (int i = 0; i < C::KSTEPS; ++i) {
             s = mfma_32x32x16_bf16(qa[i], kf[i], s);
@@ -695,6 +732,17 @@ __device__ __forceinline__ void bwd_dkv(int block,
     auto rows_are_masked = [&](int qs0) {
         return (CAUSAL && qs0 < nw0 + 32) || (window > 0 && qs0 + 63 - nw0 >= window);
     };
+    // dS of half sh of the sub-tile at query row qs0: registers 8 sh .. 8 sh + 7 are query rows 16 sh + 4 g + {0..3} and 8 more.
+    // The 16-byte pieces are dealt to the kilobyte so that the transposing reads of the dQ workgroup, which take the same key
+    // of both halves and both g at once, find them in different banks.
+    const fab::DsBlocks place{ntk, CAUSAL, WINDOW ? window : 0};
+    unsigned char* ds_head = nullptr;
+    const uint32_t ds_lane[2] = {(uint32_t)(g * 32 + (r ^ (4 * g))) * 16u, (uint32_t)(g * 32 + (r ^ (4 * g + 8))) * 16u + 1024u};
+    auto store_ds = [&](int sh, int qs0, bf16x8 v) {
+        const int qt = qs0 >> 7;
+        unsigned char* to = ds_head + (place.at(qt) + (4 * (kt - place.first(qt)) + w) * 4 + ((qs0 >> 5) & 3)) * 2048;
+        st_global_16(to + ds_lane[sh], __builtin_bit_cast(u32x4, v));
+    };
     bf16x8 rq[C::KSTEPS], rd[C::KSTEPS];              // row fragments of the next sub-tile, read one step ahead
     bf16x8 pf0, dsf0;                                 // P, dS of the first half of the current sub-tile
     f32x4 st1[4];                                     // pairs of its second half
@@ -717,6 +765,7 @@ __device__ __forceinline__ void bwd_dkv(int block,
         using Stg2 = std::integral_constant<int, (STG + 1) & 3>;                        // stage of u+2
         bf16x8 dot0[C::DT], qt0[C::DT], dot1[C::DT], qt1[C::DT];
         f32x4 st0[4];
+        if constexpr (SPILL) store_ds(0, qs0, dsf0);
         read_transposed(stg, 2 * T, dot0, qt0);
         read_pairs(Stg1{}, Sub1{}, Half0{}, st0);
         read_transposed(stg, 2 * T + 1, dot1, qt1);
@@ -724,6 +773,7 @@ __device__ __forceinline__ void bwd_dkv(int block,
         bf16x8 pf1, dsf1;
         const bool apply = decltype(masked)::value && rows_are_masked(qs0);       // rows qs0 .. qs0 + 63
         probabilities(masked, Half1{}, st1, qs0, sc, dpc, pf1, dsf1, apply);
+        if constexpr (SPILL) store_ds(1, qs0, dsf1);
         read_pairs(Stg1{}, Sub1{}, Half1{}, st1);          // ahead of the row fragments: LDS answers in order
         read_rows(Stg2{}, sub, rq, rd);
 #pragma unroll
@@ -790,6 +840,20 @@ __device__ __forceinline__ void bwd_dkv(int block,
     for (int i = 0; i < C::KSTEPS; ++i) { pin_registers(kf[i]); pin_registers(vf[i]); }
     // this part's steps of the block; a block that no query sees has none (its rows are 0)
     const int per_head = jq_last - jq_first, per_part = CUT ? plan.part_steps(kt) : 0;
+    if constexpr (SPILL && MASK == AttnMask::Keys) {
+        // all 128 keys hidden between visible ones: the dQ workgroups walk from the first visible key to the last
+        if (block_hidden && key_mask != nullptr) {
+            const TileSpan span = visible_tiles(key_mask + (size_t)(bh / hkv) * N, N, lane);
+            const int all = G * per_head, end = CUT ? min(all, (part + 1) * per_part) : all;
+            if (span.first < 2 * kt + 2 && span.last > 2 * kt)
+                for (int at = CUT ? part * per_part : 0; at < end; ++at) {
+                    ds_head = ds + (size_t)(qh0 + at / per_head) * place.head_bytes();
+                    for (int qs0 = (jq_first + at % per_head) * C::BQ, T = 0; T < 2; ++T, qs0 += 32)
+                        if (!CAUSAL || qs0 >= nw0)
+                            for (int sh = 0; sh < 2; ++sh) store_ds(sh, qs0, __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0}));
+                }
+        }
+    }
     const int step_end = block_hidden ? 0 : CUT ? min(G * per_head, (part + 1) * per_part) : G;
     for (int step_at = CUT ? part * per_part : 0; step_at < step_end;) {
     if constexpr (CUT) {
@@ -800,6 +864,7 @@ __device__ __forceinline__ void bwd_dkv(int block,
     } else {
         hq = step_at++;
     }
+    if constexpr (SPILL) ds_head = ds + (size_t)(qh0 + hq) * place.head_bytes();
     const int ntile = jq_end - jq0;
     const int nsub = 2 * ntile;                       // 32-row sub-tiles, numbered from the segment's first tile
     // First sub-tile with a visible (query, key) pair for this wave.  Causal: the block's first
@@ -814,9 +879,12 @@ __device__ __forceinline__ void bwd_dkv(int block,
 
     // Tile t+1 is awaited, and tile t+3 requested into the stage tile t-1 has left, before the
     // first sub-tile of tile t (whose steps already read fragments of tile t+1): four stages.
+    // SPILL: a step's two stores count as well; tile t+1 was requested before the stores of the last two tiles, if these
+    // were steps of this wave (it skips the first u0), and before tile t+2.
     auto tile_boundary = [&](int u) {
         if (!(u & 1) && (u >> 1) + 1 < ntile) {
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::LOADS_PER_TILE) : "memory");
+            if (SPILL && u - u0 >= 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::LOADS_PER_TILE + 8) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::LOADS_PER_TILE) : "memory");
             __syncthreads();
             issue_tile(((u >> 1) + 3) & (C::NST - 1), jq0 + (u >> 1) + 3);
         }
@@ -890,14 +958,14 @@ pipeline_done:
     store_transposed_bf16<D>(dk, scale, scratch, dK + head_off + (size_t)nw0 * D, N - nw0, lane);
 }
 
-template <int D, bool CAUSAL, AttnMask MASK, bool CUT>
+template <int D, bool CAUSAL, AttnMask MASK, bool CUT, bool SPILL>
 __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     const uint16_t* __restrict__ dO, float2* stats, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int BHkv, int N,
     int ntk, int npad, float scale, float scale_log2, int Hq, int window, const int* __restrict__ kv_lens,
-    const uint8_t* __restrict__ key_mask, fab::Parts plan, int items, float* __restrict__ partial) {
-    bwd_dkv<D, CAUSAL, MASK, CUT, false>(blockIdx.x, Q, Kp, Vp, nullptr, dO, nullptr, stats, dK, dV, BHkv, N, ntk, npad, scale, scale_log2,
-                                         Hq, window, kv_lens, key_mask, plan, items, partial);
+    const uint8_t* __restrict__ key_mask, fab::Parts plan, int items, float* __restrict__ partial, unsigned char* __restrict__ ds) {
+    bwd_dkv<D, CAUSAL, MASK, CUT, false, SPILL>(blockIdx.x, Q, Kp, Vp, nullptr, dO, nullptr, stats, dK, dV, BHkv, N, ntk, npad, scale, scale_log2,
+                                         Hq, window, kv_lens, key_mask, plan, items, partial, ds);
 }
 
 // Both at once for launches that leave CUs idle anyway (rule at one_launch): the first `ndkv` workgroups are dK/dV's, the
@@ -912,23 +980,154 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_both_kernel(
     const uint8_t* __restrict__ key_mask, int single, fab::Parts plan, int items, float* __restrict__ partial, int ndkv) {
     const int at = blockIdx.x;
     if (at < ndkv) {
-        bwd_dkv<D, CAUSAL, MASK, CUT, true>(at, Q, Kp, Vp, O, dO, LSE, stats, dK, dV, BH / plan.G, N, ntk, npad, scale, scale_log2, Hq,
-                                         window, kv_lens, key_mask, plan, items, partial);
+        bwd_dkv<D, CAUSAL, MASK, CUT, true, false>(at, Q, Kp, Vp, O, dO, LSE, stats, dK, dV, BH / plan.G, N, ntk, npad, scale, scale_log2, Hq,
+                                         window, kv_lens, key_mask, plan, items, partial, nullptr);
     } else {
         bwd_dq<D, CAUSAL, MASK, true>(at - ndkv, Q, Kp, Vp, O, dO, LSE, dQ, nullptr, BH, N, ntq, npad, scale, scale_log2, Hq, plan.G,
                                       window, kv_lens, key_mask, 0, single);
     }
 }
 
+// ------------------------------------------------------------------------------------------
+// (lse * log2 e, delta) of every query row for dK/dV launches that no dQ launch precedes: delta = dO . O, rows of the padding
+// up to npad get (+inf, 0).  16 bytes a lane of each operand; bound by HBM.
+template <int D>
+__global__ __launch_bounds__(256) void flash_attn_bwd_stats_kernel(const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO,
+                                                                  const float* __restrict__ LSE, float2* __restrict__ stats, int N,
+                                                                  int npad, int masked) {
+    constexpr int LANES = D / 8, ROWS = 256 / LANES;
+    const int per_head = npad / ROWS;
+    const int bh = blockIdx.x / per_head, qpos = blockIdx.x % per_head * ROWS + threadIdx.x / LANES, qrow = min(qpos, N - 1);
+    const size_t off = ((size_t)bh * N + qrow) * D + threadIdx.x % LANES * 8;
+    float delta = fab::dot8_bf16(ld_global_16(dO + off), ld_global_16(O + off));
+    float lse2 = LSE[(size_t)bh * N + qrow] * fab::LOG2E;
+#pragma unroll
+    for (int x = 1; x < LANES; x <<= 1) delta += __shfl_xor(delta, x, 64);
+    if (masked && lse2 == -INFINITY) lse2 = INFINITY;                // a row that saw no key: every probability is 0
+    if (threadIdx.x % LANES == 0) stats[(size_t)bh * npad + qpos] = qpos < N ? make_float2(lse2, delta) : make_float2(INFINITY, 0.0f);
+}
+
+// dQ = dS K of the dS that the dK/dV launch left: one workgroup = 128 query rows (4 waves x 32), a ring of stages of 32 keys
+// (four 2 KB blocks of dS, 32 rows of K) filled by global -> LDS requests, products transposed as in flash_attn_bwd_dq_kernel:
+//    dQ^T (D x 32 q) += K_tile^T x dS^T
+// both operands by transposing reads.  Bound by the L2 -> LDS requests (B1 Hq32 Hkv8 N2000: 29 us for 142 MB of dS and as much of K; without
+// its products the kernel takes as long).  256 rows a workgroup halve the K part and take 36 us there: the longest has a CU to
+// itself.  Fragments read ahead of their products, across the stages: 30 us.
+namespace fab {
+template <int D>
+struct CfgP {
+    static constexpr int BM = 128, BN = 32, NST = 5; // two workgroups a CU share its 160 KB
+    static constexpr int ROW = D * 2, KCH = D / 8;
+    static constexpr int DS = 4 * 2048, STAGE = DS + BN * ROW, LDS = NST * STAGE;
+    static constexpr int PT = BN * KCH / THREADS;    // 16-byte chunks of K per thread and stage
+    static constexpr int LOADS = 2 + PT, DT = D / 32;
+};
+}  // namespace fab
+template <int D, bool CAUSAL, AttnMask MASK>
+__device__ __forceinline__ void bwd_dq_product(int block, const uint16_t* __restrict__ Kp, const unsigned char* __restrict__ ds,
+                                               uint16_t* __restrict__ dQ, int BH, int N, int ntq, float scale, int Hq, int G,
+                                               int window, const int* __restrict__ kv_lens, const uint8_t* __restrict__ key_mask,
+                                               int single) {
+    using namespace fab;
+    using C = CfgP<D>;
+    constexpr bool LIMITS = MASK == AttnMask::Limits, KEYS = MASK == AttnMask::Keys;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int t = threadIdx.x;
+    const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+
+    int bh, rank, kvbh;
+    AttnOrder{BH, Hq, G, ntq, single}.decode(block, bh, rank, kvbh);
+    const int qt = CAUSAL ? ntq - 1 - rank : rank;
+    const int q0 = qt * C::BM, qw0 = q0 + w * 32;
+    const int Nk = (LIMITS && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / Hq])) : N;
+    int kv_end = CAUSAL ? min(Nk, q0 + C::BM) : Nk;
+    int begin = (LIMITS && window > 0) ? max(0, q0 - window + 1) / C::BN : 0;      // stages = 32 keys
+    if constexpr (KEYS) {
+        const TileSpan span = visible_tiles(key_mask + (size_t)(bh / Hq) * N, kv_end, lane);
+        begin = 2 * span.first;
+        kv_end = min(kv_end, 64 * span.last);
+    }
+    const int end = (kv_end + C::BN - 1) / C::BN;
+    // the stages that hold a visible pair for this wave's rows: only those blocks are written for certain
+    const int wave_end = CAUSAL ? min(end, qw0 / C::BN + 1) : end;
+    const int wave_begin = (LIMITS && window > 0) ? max(0, qw0 - window + 1) / C::BN : begin;
+
+    const DsBlocks place{ntq, CAUSAL, LIMITS ? window : 0};
+    const int tile_bytes = place.tiles(qt) * 16 * 2048, s_first = 4 * place.first(qt);
+    const u32x4 s_rsrc = make_raw_rsrc(ds + (size_t)bh * place.head_bytes() + place.at(qt) * 2048, (uint32_t)tile_bytes);
+    const u32x4 k_rsrc = make_raw_rsrc(Kp + (size_t)kvbh * N * D, (uint32_t)N * D * 2u);
+    constexpr int ROWS_PER_INST = 1024 / C::ROW;
+    int s_voff[2], k_voff[C::PT];                    // request m carries 1024 m as its immediate offset
+    s_voff[0] = s_voff[1] = w * 2048 + lane * 16;
+#pragma unroll
+    for (int m = 0; m < C::PT; ++m) {
+        const int row = (w * C::PT + m) * ROWS_PER_INST + lane / C::KCH;
+        k_voff[m] = row * C::ROW + swz<D>(row, lane % C::KCH) * 16 - 1024 * m;
+    }
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
+    const uint32_t s_dst = __builtin_amdgcn_readfirstlane(lds_base + (uint32_t)w * 2048u);
+    const uint32_t k_dst = __builtin_amdgcn_readfirstlane(lds_base + C::DS + (uint32_t)w * C::PT * 1024u);
+    // stages past the end are requested beyond the buffers (zeros, no traffic), so that the wait count below is constant
+    auto issue = [&](uint32_t at, int j) {
+        load_global_to_lds_16xN<2>(s_rsrc, s_dst + at, s_voff, j < end ? (j - s_first) * C::DS : tile_bytes);
+        load_global_to_lds_16xN<C::PT>(k_rsrc, k_dst + at, k_voff, j < end ? j * C::BN * C::ROW : N * C::ROW);
+    };
+    // transposing reads: keys 16 c + 4 (lane / 32) + {0..3} and 8 more, in the same order of both operands
+    int tr_lo[C::DT], tr_hi[C::DT], s_lo, s_hi;
+    {
+        const int i16 = lane & 15, b16 = lane >> 4, row = 4 * (b16 >> 1) + (i16 >> 2);
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt) {
+            const int dcol = 32 * dt + 16 * (b16 & 1) + 4 * (i16 & 3);
+            tr_lo[dt] = C::DS + row * C::ROW + swz<D>(row, dcol >> 3) * 16 + (dcol & 7) * 2;
+            tr_hi[dt] = C::DS + (row + 8) * C::ROW + swz<D>(row + 8, dcol >> 3) * 16 + (dcol & 7) * 2;
+        }
+        // dS pieces as store_ds deals them: half sh = b16 & 1, its g = lane & 1, rows + 8 in the upper 8 bytes
+        const int sh = b16 & 1, gp = i16 & 1, x = 4 * gp + 8 * sh;
+        s_lo = w * 2048 + sh * 1024 + (gp * 32 + (row ^ x)) * 16 + ((i16 >> 1) & 1) * 8;
+        s_hi = w * 2048 + sh * 1024 + (gp * 32 + ((row + 8) ^ x)) * 16 + ((i16 >> 1) & 1) * 8;
+    }
+    f32x16 dq[C::DT];
+#pragma unroll
+    for (int i = 0; i < C::DT; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dq[i][e] = 0.0f;
+
+#pragma unroll
+    for (int i = 0; i < C::NST - 1; ++i) issue(i * C::STAGE, begin + i);
+    uint32_t at = 0;                                 // the stage's place in the ring
+    for (int j = begin; j < end; ++j) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((C::NST - 2) * C::LOADS) : "memory");
+        __syncthreads();                             // stage j is here; the one before it has been read by every wave
+        issue(at == 0 ? (C::NST - 1) * C::STAGE : at - C::STAGE, j + C::NST - 1);
+        if (j >= wave_begin && j < wave_end) {
+            const unsigned char* St = lds + at;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const bf16x4 dl = ds_read_tr16(St + s_lo + c * 256), dh = ds_read_tr16(St + s_hi + c * 256);
+                const bf16x8 dsf = __builtin_shufflevector(dl, dh, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+                for (int dt = 0; dt < C::DT; ++dt) {
+                    const bf16x4 lo = ds_read_tr16(St + tr_lo[dt] + c * 16 * C::ROW), hi = ds_read_tr16(St + tr_hi[dt] + c * 16 * C::ROW);
+                    dq[dt] = mfma_32x32x16_bf16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), dsf, dq[dt]);
+                }
+            }
+        }
+        at = at == (C::NST - 1) * C::STAGE ? 0 : at + C::STAGE;
+    }
+    wait_vmcnt0();
+    __syncthreads();
+    store_transposed_bf16<D>(dq, scale, lds + w * (32 * (D * 2 + 16)), dQ + ((size_t)bh * N + qw0) * D, N - qw0, lane);
+}
+
 // dK and dV of the key tiles that were cut into parts: the parts' f32 sums added in order, 8 elements of a row per thread.
 template <int D>
-__global__ __launch_bounds__(256) void flash_attn_bwd_sum_kernel(const float* __restrict__ partial, uint16_t* __restrict__ dK,
-                                                                uint16_t* __restrict__ dV, int N, int ntk, int items, float scale,
-                                                                fab::Parts plan) {
+__device__ __forceinline__ void bwd_sum(int block, const float* __restrict__ partial, uint16_t* __restrict__ dK,
+                                        uint16_t* __restrict__ dV, int N, int ntk, int items, float scale, fab::Parts plan) {
     constexpr int CH = D / 8, DT = D / 32, TILE16 = 2 * 4 * DT * 4 * 64;      // 16-byte pieces of one part
-    const int id = blockIdx.x * 256 + threadIdx.x;
+    const int id = block * 256 + threadIdx.x;
     constexpr int PER_TILE = 2 * 128 * CH;
-    const int tile = (blockIdx.x * 256) / PER_TILE;                          // a workgroup stays inside one tile
+    const int tile = (block * 256) / PER_TILE;                          // a workgroup stays inside one tile
     const int bh = tile / ntk, kt = tile % ntk;
     const int parts = plan.parts(kt);
     if (parts == 1) return;
@@ -951,6 +1150,24 @@ __global__ __launch_bounds__(256) void flash_attn_bwd_sum_kernel(const float* __
     v[2] = pack_bf16(hi[0] * mul, hi[1] * mul);
     v[3] = pack_bf16(hi[2] * mul, hi[3] * mul);
     st_global_16((which ? dK : dV) + ((size_t)bh * N + kt * 128 + row) * D + c * 8, v);
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void flash_attn_bwd_sum_kernel(const float* __restrict__ partial, uint16_t* __restrict__ dK,
+                                                                uint16_t* __restrict__ dV, int N, int ntk, int items, float scale,
+                                                                fab::Parts plan) {
+    bwd_sum<D>(blockIdx.x, partial, dK, dV, N, ntk, items, scale, plan);
+}
+// The launch after a dK/dV launch that left dS: the first `ndq` workgroups are dQ's, the rest add the parts, on the CUs that
+// short dQ tiles leave (B1 Hq32 Hkv8 N2000: 28 + 8 us in two launches).
+template <int D, bool CAUSAL, AttnMask MASK>
+__global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_product_kernel(
+    const uint16_t* __restrict__ Kp, const unsigned char* __restrict__ ds, uint16_t* __restrict__ dQ, int BH, int N, int ntq,
+    float scale, int Hq, int window, const int* __restrict__ kv_lens, const uint8_t* __restrict__ key_mask, int single, int ndq,
+    const float* __restrict__ partial, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int items, fab::Parts plan) {
+    const int at = blockIdx.x;
+    if (at < ndq) bwd_dq_product<D, CAUSAL, MASK>(at, Kp, ds, dQ, BH, N, ntq, scale, Hq, plan.G, window, kv_lens, key_mask, single);
+    else bwd_sum<D>(at - ndq, partial, dK, dV, N, ntq, items, scale, plan);
 }
 
 size_t flash_attn_bwd_workspace_bytes(int B, int H, int N) {
@@ -1059,11 +1276,47 @@ bool one_launch(int N, int64_t dq_blocks, int64_t dkv_blocks) {
 size_t dkv_partial_bytes(const fab::Parts& p, int BHkv, int N, int D) {
     return p.chunk ? (size_t)BHkv * dkv_items(p, N) * 128 * D * 8 : 0;
 }
+size_t ds_bytes(int BH, int N, bool causal, int window) {
+    return (size_t)BH * fab::DsBlocks{(N + 127) / 128, causal, window}.head_bytes();
+}
+// Whether dK/dV leave dS for dQ: five products in three launches (pairs, dK/dV, dQ) in place of seven in two.  Worth it while dS
+// stays in the 256 MB last-level cache and the heads are few: beyond, dS costs its traffic to HBM, and many short tiles
+// fill the device in the other form as well.  With G >= 4 query heads a K / V, dQ's share of the requests hits the L2.
+// Measured (us, without -> with, whole backward, D = 128): B1 Hq32 Hkv8 N2000 147.5 -> 131.5, B1 Hq4 N6083 201 -> 163, B9 Hq8
+// Hkv2 N900 full 176 -> 145; on the other side of the line B12 H16 N555 109 -> 117, B7 Hq32 Hkv8 N812 202 -> 206, B5 Hq8
+// Hkv2 N2724 (331 MB) 300 -> 307, B16 H16 N4096 (4.4 GB) 3640 -> 3530 with 18 times the scratch.
+bool keeps_ds(int BH, int G, int N, int D, bool causal, int window) {
+    const fab::DsBlocks place{(N + 127) / 128, causal, window};
+    return D == 128 && place.ntk >= 5 && place.width() >= std::min(place.ntk, 8) && BH <= (G >= 4 ? 128 : 64) &&
+           ds_bytes(BH, N, causal, window) <= (size_t)288 << 20;
+}
+// What a call does with all the scratch it can use, and the parts of that scratch, in this order.
+struct BwdPlan {
+    fab::Parts parts;
+    int items;
+    int64_t dq_blocks, dkv_blocks;                   // dq_blocks: of the 64-row form, beside dK/dV's in one launch
+    bool both, ds;
+    size_t stat_bytes, partial_bytes, ds_bytes;
+    size_t bytes() const { return stat_bytes + partial_bytes + ds_bytes; }
+};
+BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int D, bool causal, int window, bool least) {
+    BwdPlan p;
+    p.parts = dkv_plan(B * Hkv, Hq / Hkv, N, D, causal, window);
+    if (least) p.parts.chunk = 0;
+    p.items = dkv_items(p.parts, N);
+    p.dq_blocks = (int64_t)B * Hq * ((N + 63) / 64);
+    p.dkv_blocks = (int64_t)B * Hkv * p.items;
+    p.both = one_launch(N, p.dq_blocks, p.dkv_blocks);
+    p.ds = !least && !p.both && keeps_ds(B * Hq, Hq / Hkv, N, D, causal, window);
+    p.stat_bytes = flash_attn_bwd_workspace_bytes(B, Hq, N);
+    p.partial_bytes = dkv_partial_bytes(p.parts, B * Hkv, N, D);
+    p.ds_bytes = p.ds ? ds_bytes(B * Hq, N, causal, window) : 0;
+    return p;
+}
 }  // namespace
 
 size_t flash_attn_bwd_full_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int causal, int window) {
-    const fab::Parts p = dkv_plan(B * Hkv, Hq / Hkv, N, D, causal != 0, window);
-    return flash_attn_bwd_workspace_bytes(B, Hq, N) + dkv_partial_bytes(p, B * Hkv, N, D);
+    return bwd_plan(B, Hq, Hkv, N, D, causal != 0, window, false).bytes();
 }
 
 int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
@@ -1079,14 +1332,13 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     const int ntq = (N + shape.rows - 1) / shape.rows;
     const int pair = shape.pair, single = shape.single;
     dim3 grid_q((unsigned)(BH * (pair ? (ntq + 1) / 2 : ntq))), block(THREADS);
-    const size_t stat_bytes = flash_attn_bwd_workspace_bytes(B, Hq, N);
-    Parts plan = dkv_plan(BHkv, G, N, D, causal != 0, window);
-    if (workspace_bytes < stat_bytes + dkv_partial_bytes(plan, BHkv, N, D)) plan.chunk = 0;
-    const int items = dkv_items(plan, N);
-    dim3 grid_k((unsigned)(BHkv * items));
-    const int64_t dq_blocks = (int64_t)BH * ((N + 63) / 64);
-    const bool both = one_launch(N, dq_blocks, grid_k.x);
-    float* partial = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + stat_bytes);
+    BwdPlan how = bwd_plan(B, Hq, Hkv, N, D, causal != 0, window, false);
+    if (workspace_bytes < how.bytes()) how = bwd_plan(B, Hq, Hkv, N, D, causal != 0, window, true);
+    const Parts plan = how.parts;
+    const int items = how.items;
+    const dim3 grid_k((unsigned)how.dkv_blocks);
+    float* partial = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + how.stat_bytes);
+    unsigned char* ds = static_cast<unsigned char*>(workspace) + how.stat_bytes + how.partial_bytes;
     const float scale_log2 = scale * LOG2E;
     auto Qp = static_cast<const uint16_t*>(q);
     auto Kp = static_cast<const uint16_t*>(k);
@@ -1104,21 +1356,33 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
                            Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st, BH, N, ntq, npad, \
                            scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single);        \
     } while (0)
-#define TYR_FAB_DKV(DD, CC, EE, UU)                                                                   \
+#define TYR_FAB_DKV(DD, CC, EE, UU, PP)                                                               \
     do {                                                                                              \
         static const hipError_t a2 = hipFuncSetAttribute(                                             \
-            reinterpret_cast<const void*>(&flash_attn_bwd_dkv_kernel<DD, CC, EE, UU>),                \
+            reinterpret_cast<const void*>(&flash_attn_bwd_dkv_kernel<DD, CC, EE, UU, PP>),            \
             hipFuncAttributeMaxDynamicSharedMemorySize, CfgK<DD>::LDS);                               \
         if (a2 != hipSuccess) return -1;                                                              \
-        hipLaunchKernelGGL((flash_attn_bwd_dkv_kernel<DD, CC, EE, UU>), grid_k, block, CfgK<DD>::LDS, stream, \
-                           Qp, Kp, Vp, dOp, st, static_cast<uint16_t*>(dk),                           \
+        hipLaunchKernelGGL((flash_attn_bwd_dkv_kernel<DD, CC, EE, UU, PP>), grid_k, block, CfgK<DD>::LDS, \
+                           stream, Qp, Kp, Vp, dOp, st, static_cast<uint16_t*>(dk),                   \
                            static_cast<uint16_t*>(dv), BHkv, N, ntk, npad, scale, scale_log2, Hq,     \
-                           window, kv_lens, key_mask, plan, items, partial);                          \
+                           window, kv_lens, key_mask, plan, items, partial, ds);                      \
     } while (0)
-#define TYR_FAB_DKV_MASK(DD, CC, EE, UU)      /* lengths alone are a mask of keys here */             \
+#define TYR_FAB_DKV_MASK(DD, CC, EE, UU, PP)  /* lengths alone are a mask of keys here */             \
     do {                                                                                              \
-        if (EE == AttnMask::Limits && window <= 0) TYR_FAB_DKV(DD, CC, AttnMask::Keys, UU);           \
-        else TYR_FAB_DKV(DD, CC, EE, UU);                                                             \
+        if (EE == AttnMask::Limits && window <= 0) TYR_FAB_DKV(DD, CC, AttnMask::Keys, UU, PP);       \
+        else TYR_FAB_DKV(DD, CC, EE, UU, PP);                                                         \
+    } while (0)
+#define TYR_FAB_DQ_PRODUCT(DD, CC, EE)                                                                \
+    do {                                                                                              \
+        static const hipError_t a4 = hipFuncSetAttribute(                                             \
+            reinterpret_cast<const void*>(&flash_attn_bwd_dq_product_kernel<DD, CC, EE>),             \
+            hipFuncAttributeMaxDynamicSharedMemorySize, CfgP<DD>::LDS);                               \
+        if (a4 != hipSuccess) return -1;                                                              \
+        const int ndq = BH * ntk, nsum = plan.chunk ? BHkv * ntk * (DD / 8) : 0;                      \
+        hipLaunchKernelGGL((flash_attn_bwd_dq_product_kernel<DD, CC, EE>), dim3((unsigned)(ndq + nsum)), block, CfgP<DD>::LDS, stream, \
+                           Kp, ds, static_cast<uint16_t*>(dq), BH, N, ntk, scale, Hq, window, kv_lens, key_mask, \
+                           causal && window <= 0, ndq, partial, static_cast<uint16_t*>(dk),           \
+                           static_cast<uint16_t*>(dv), items, plan);                                  \
     } while (0)
 #define TYR_FAB_SUM(DD)                                                                               \
     hipLaunchKernelGGL(flash_attn_bwd_sum_kernel<DD>, dim3((unsigned)(BHkv * ntk * (DD / 8))), dim3(256), 0, stream, \
@@ -1129,25 +1393,35 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
             reinterpret_cast<const void*>(&flash_attn_bwd_both_kernel<DD, CC, EE, UU>),               \
             hipFuncAttributeMaxDynamicSharedMemorySize, CfgK<DD>::LDS);                               \
         if (a3 != hipSuccess) return -1;                                                              \
-        hipLaunchKernelGGL((flash_attn_bwd_both_kernel<DD, CC, EE, UU>), dim3(grid_k.x + (unsigned)dq_blocks), block, CfgK<DD>::LDS, \
+        hipLaunchKernelGGL((flash_attn_bwd_both_kernel<DD, CC, EE, UU>), dim3(grid_k.x + (unsigned)how.dq_blocks), block, CfgK<DD>::LDS, \
                            stream, Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st,          \
                            static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), BH, N, (N + 63) / 64, ntk, \
                            npad, scale, scale_log2, Hq, window, kv_lens, key_mask, causal && window <= 0, plan, items, partial, (int)grid_k.x); \
     } while (0)
 #define TYR_FAB_LAUNCH(DD, CC, EE)                                                                    \
     do {                                                                                              \
-        if (both) {                                                                                   \
+        if (how.both) {                                                                               \
             if (!plan.chunk) { TYR_FAB_BOTH(DD, CC, EE, false); break; }                              \
             TYR_FAB_BOTH(DD, CC, EE, true);                                                           \
             TYR_FAB_SUM(DD);                                                                          \
             break;                                                                                    \
         }                                                                                             \
+        if constexpr (DD == 128) {                                                                               \
+            if (how.ds) {                                                                             \
+                hipLaunchKernelGGL(flash_attn_bwd_stats_kernel<DD>, dim3((unsigned)(BH * (npad / (2048 / DD)))), dim3(256), 0, \
+                                   stream, Op, dOp, lse, st, N, npad, EE != AttnMask::None);          \
+                if (plan.chunk) TYR_FAB_DKV_MASK(DD, CC, EE, true, true);                             \
+                else TYR_FAB_DKV_MASK(DD, CC, EE, false, true);                                       \
+                TYR_FAB_DQ_PRODUCT(DD, CC, EE);                                                       \
+                break;                                                                                \
+            }                                                                                         \
+        }                                                                                             \
         if (shape.rows == 64) TYR_FAB_DQ(DD, CC, EE, true); else TYR_FAB_DQ(DD, CC, EE, false);       \
         if (plan.chunk) {                                                                             \
-            TYR_FAB_DKV_MASK(DD, CC, EE, true);                                                            \
+            TYR_FAB_DKV_MASK(DD, CC, EE, true, false);                                                \
             TYR_FAB_SUM(DD);                                                                          \
         } else {                                                                                      \
-            TYR_FAB_DKV_MASK(DD, CC, EE, false);                                                           \
+            TYR_FAB_DKV_MASK(DD, CC, EE, false, false);                                               \
         }                                                                                             \
     } while (0)
 #define TYR_FAB_PICK(DD, MM)                                                                          \
@@ -1164,6 +1438,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
 #undef TYR_FAB_LAUNCH
 #undef TYR_FAB_BOTH
 #undef TYR_FAB_SUM
+#undef TYR_FAB_DQ_PRODUCT
 #undef TYR_FAB_DKV_MASK
 #undef TYR_FAB_DKV
 #undef TYR_FAB_DQ

@@ -80,7 +80,16 @@ struct Scratch {
     size_t bytes;
     torch::Tensor block;
     Scratch(size_t n, const torch::Tensor& like) : bytes(n) {
-        if (n) block = torch::empty({(int64_t)n}, like.options().dtype(torch::kUInt8));
+        auto take = [&] { block = torch::empty({(int64_t)bytes}, like.options().dtype(torch::kUInt8)); };
+        try {
+            if (n) take();
+        } catch (const c10::OutOfMemoryError&) {
+            // What is more than the first operand is an attention backward that would keep dS (up to 0.4 GB) or a split K: both
+            // run with less, and the backward's minimum is 8 bytes a row of q.
+            if (n <= like.nbytes()) throw;
+            bytes = like.nbytes();
+            take();
+        }
     }
     void* ptr() const { return bytes ? block.data_ptr() : nullptr; }
 };
