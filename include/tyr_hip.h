@@ -334,8 +334,9 @@ int tyr_hip_gemm_bf16_batched(const void* a, const void* b, void* c, uint64_t ba
 /* The same products with device scratch.  A product with few output tiles and a long K leaves most of the device idle
  * unless K is split over workgroups; the f32 partial sums then pass through `workspace` (16-byte aligned device memory of
  * tyr_hip_gemm_workspace_bytes bytes; a smaller one, or NULL, only means that K is not split).  elem_bytes: 2 = bf16,
- * 1 = e4m3; 0 bytes = this shape is never split.  Results are reproducible launch to launch either way; splitting sums
- * K in another order, so the two forms may differ in the last bit of the output. */
+ * 1 = e4m3; 0 bytes = this shape does the same without.  Results are reproducible launch to launch either way; with scratch
+ * K may be summed in another order (16 bytes: only within a workgroup, nothing is written there), so the two forms may
+ * differ in the last bit of the output. */
 size_t tyr_hip_gemm_workspace_bytes(uint64_t batch, uint64_t M, uint64_t N, uint64_t K, int elem_bytes, int trans_b);
 int tyr_hip_gemm_bf16_batched_ws(const void* a, const void* b, void* c, uint64_t batch,
                                  uint64_t M, uint64_t N, uint64_t K,

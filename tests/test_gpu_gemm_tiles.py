@@ -136,3 +136,26 @@ def test_batches_of_tiles(batch, M, N, K, trans_b):
             assert rel_fro(got, want) <= 3e-3 and worst_line(got, want) <= TOL_FRO
             assert lib.tyr_hip_gemm_bf16(a[i].data_ptr(), bi.data_ptr(), one.data_ptr(), M, N, K, int(trans_b), stream) == 0
             assert torch.equal(got, one)
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (15, 264, 8192), (31, 4104, 2056), (33, 4096, 1024), (63, 4088, 2048), (65, 4096, 200),
+                                   (250, 4080, 1040), (257, 2048, 4096), (333, 4096, 4096), (512, 4088, 656)])
+def test_tiles_whose_k_range_twice_the_waves_share(M, N, K, trans_b):
+    """One workgroup a CU: eight waves on a tile instead of four.  Around the tiles' edges, with fewer pieces than waves and with
+    rows that start on cache lines or not; bf16 takes these tiles with scratch only, so the product without sums in another order."""
+    from tyr_amd import _lib
+    lib = _lib.load()
+    test_tiles_match_the_f32_product(M, N - N % 16, K - K % 16, trans_b)      # whole chunks of e4m3
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a = (torch.randn(M, K, generator=g, device="cuda") * K ** -0.25).bfloat16()
+    b = (torch.randn(*((N, K) if trans_b else (K, N)), generator=g, device="cuda") * K ** -0.25).bfloat16()
+    want = a.float() @ (b.float().t() if trans_b else b.float())
+    need = lib.tyr_hip_gemm_workspace_bytes(1, M, N, K, 2, int(trans_b))
+    ws = torch.full((need + 64,), 3, dtype=torch.uint8, device="cuda")
+    for w, nbytes in ((ws.data_ptr(), need), (ws.data_ptr(), max(0, need - 1)), (None, 0)):
+        c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert lib.tyr_hip_gemm_bf16_batched_ws(a.data_ptr(), b.data_ptr(), c.data_ptr(), 1, M, N, K, 0, 0, 0, int(trans_b), w, nbytes, 0) == 0
+        torch.cuda.synchronize()
+        assert rel_fro(c, want) <= 3e-3 and worst_line(c, want) <= TOL_FRO
+    assert bool((ws[need:] == 3).all()) and (need != 16 or bool((ws == 3).all()))

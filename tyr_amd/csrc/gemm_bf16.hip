@@ -394,7 +394,7 @@ __global__ __launch_bounds__(gemm2::THREADS, 1) void gemm_bf16_fast_kernel(
 size_t gemm_workspace_bytes(int M, int N, int K, int elem_bytes, int trans_b, int batch) {
     if (gemm_general_only() || !gt::offsets_fit(N, K, elem_bytes, trans_b != 0)) return 0;
     const gt::Plan p = gt::plan(M, N, K, elem_bytes, trans_b != 0, batch, true);
-    return p.splits > 1 ? (size_t)p.splits * batch * M * N * sizeof(float) : 0;
+    return gt::scratch_bytes(p, M, N, elem_bytes, batch);
 }
 
 int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K, int trans_b,
@@ -414,7 +414,7 @@ int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K,
     const bool fast_ok = !gemm_general_only() && (K % 8 == 0) && gt::offsets_fit(N, K, 2, trans_b != 0);
     if (fast_ok) {
         gt::Plan p = gt::plan(M, N, K, 2, trans_b != 0, batch, workspace != nullptr);
-        if (workspace_bytes < (size_t)(p.splits > 1 ? p.splits : 0) * batch * M * N * sizeof(float))
+        if (workspace_bytes < gt::scratch_bytes(p, M, N, 2, batch))
             p = gt::plan(M, N, K, 2, trans_b != 0, batch, false);
         if (p.tile != gt::T256x256) {
             const GemmEpilogue ep{1.0f, nullptr, nullptr, 0};

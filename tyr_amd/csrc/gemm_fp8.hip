@@ -425,7 +425,7 @@ int launch_gemm_fp8(const void* aq, const void* bq, void* c, int M, int N, int K
     const bool fast_ok = !gemm_general_only() && (K % 16 == 0) && gt::offsets_fit(N, K, 1, trans_b != 0);
     if (fast_ok) {
         gt::Plan p = gt::plan(M, N, K, 1, trans_b != 0, 1, workspace != nullptr);
-        if (workspace_bytes < (size_t)(p.splits > 1 ? p.splits : 0) * M * N * sizeof(float))
+        if (workspace_bytes < gt::scratch_bytes(p, M, N, 1, 1))
             p = gt::plan(M, N, K, 1, trans_b != 0, 1, false);
         if (p.tile != gt::T256x256) {
             auto part = static_cast<float*>(workspace);

@@ -400,23 +400,36 @@ __global__ __launch_bounds__(256) void gemm_tile_reduce_kernel(const float* __re
 // on an MI355X).  The plan takes the tile and the number of K splits with the least sum; on those shapes that is 2.6 %
 // slower than the best of 38 tiles tried one by one, and 3.3 times as fast as 256x256 tiles alone.
 namespace gt {
-struct TileCost { int bm, bn, kg, mf; float fixed, piece; };
-enum Tile { T16x16, T16x32, T16x64, T32x32, T64x32, T64x64, T64x128, T96x64, T128x128, T192x128, T128x256, T256x256, TILES };
+// The W tiles are those with the K range shared by twice as many waves, whose rings then take a CU's whole LDS: with one
+// workgroup a CU (ALONE) eight waves keep twice the pieces in flight (M = 256, N = K = 4096: fp8 10.1 -> 8.1 us, bf16 17.5 ->
+// 14.6 with 64x64; M = 333 fp8 12.4 -> 10.9 with 64x128), with more the next workgroup cannot start beside the last one (M =
+// 1000 28 -> 31 us).  16x16 over eight k-groups: from about 22 pieces on (M = 1, N = K = 4096 bf16 4.9 -> 4.4).
+enum Wide : uint8_t { NO, WIDE, ALONE };             // ALONE: WIDE, and one workgroup a CU
+struct TileCost { int bm, bn, kg, mf; float fixed, piece; Wide wide = NO; };
+enum Tile { T16x16, T16x16W, T16x32, T16x64, T32x32, T32x64W, T64x32, T64x32W, T64x64, T64x64W, T64x128, T64x128W, T96x64, T128x128,
+            T192x128, T128x256, T256x256, TILES };
 constexpr TileCost kTileCost[TILES] = {
-    {16, 16, 4, 16, 2.4f, 0.19f},   {16, 32, 4, 16, 2.3f, 0.29f},    {16, 64, 4, 16, 2.3f, 0.43f},    {32, 32, 4, 32, 2.4f, 0.34f},
-    {64, 32, 2, 32, 2.6f, 0.29f},   {64, 64, 1, 32, 3.1f, 0.255f},   {64, 128, 1, 32, 3.85f, 0.34f},  {96, 64, 2, 16, 3.2f, 0.71f},
-    {128, 128, 1, 32, 4.5f, 0.525f}, {192, 128, 1, 32, 5.5f, 0.665f}, {128, 256, 1, 32, 6.6f, 0.77f}, {256, 256, 1, 32, 3.9f, 1.17f}};
+    {16, 16, 4, 16, 2.4f, 0.19f},    {16, 16, 8, 16, 2.7f, 0.30f, WIDE},   {16, 32, 4, 16, 2.3f, 0.29f},   {16, 64, 4, 16, 2.3f, 0.43f},
+    {32, 32, 4, 32, 2.4f, 0.34f},    {32, 64, 4, 32, 2.7f, 0.52f, ALONE},  {64, 32, 2, 32, 2.6f, 0.29f},   {64, 32, 4, 32, 2.7f, 0.50f, ALONE},
+    {64, 64, 1, 32, 3.1f, 0.255f},   {64, 64, 2, 32, 2.9f, 0.36f, ALONE},  {64, 128, 1, 32, 3.85f, 0.34f}, {64, 128, 2, 32, 3.7f, 0.50f, ALONE},
+    {96, 64, 2, 16, 3.2f, 0.71f},    {128, 128, 1, 32, 4.5f, 0.525f}, {192, 128, 1, 32, 5.5f, 0.665f}, {128, 256, 1, 32, 6.6f, 0.77f},
+    {256, 256, 1, 32, 3.9f, 1.17f}};
 
 struct Plan { int tile, splits; };
 
 // A [K,N] B is fetched in rows of BN elements: at least 64 bytes of each.
 inline bool tile_takes(int tile, int es, bool tb) { return tb || kTileCost[tile].bn * es >= 64; }
 
-inline double tile_cost(int tile, int splits, int M, int N, int K, int es, int batch) {
+inline double tile_cost(int tile, int splits, int M, int N, int K, int es, bool tb, int batch) {
     const TileCost& t = kTileCost[tile];
     const int64_t pieces = ((int64_t)K * es + KB - 1) / KB, per_split = (pieces + splits - 1) / splits;
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * splits * batch;
-    double us = t.fixed + (double)t.piece * ((per_split + t.kg - 1) / t.kg) * ((tiles + 255) / 256);
+    if (t.wide == ALONE && tiles > 256) return 1e30;
+    // Rows that do not start on cache lines: every piece of one touches two.  A CU's requests are what bounds an ALONE tile
+    // (64x64W, 44 pieces of 126 x 6992 x 5544 bf16: 0.57 us each for 0.36), the others wait as much for other things (1.16 x).
+    const bool lines = (int64_t)K * es % KB == 0 && (tb || (int64_t)N * es % KB == 0);
+    const double piece = t.wide == ALONE && !lines ? 1.4 * t.piece : t.piece;
+    double us = t.fixed + piece * ((per_split + t.kg - 1) / t.kg) * ((tiles + 255) / 256);
     // the second kernel, and f32 partials written and read at 5 TB/s
     if (splits > 1) us += 2.6 + (double)M * N * batch * 8.0 * splits / 5.0e6;
     // no tile is faster than memory; among those that reach it the one with the least to do still wins
@@ -425,26 +438,27 @@ inline double tile_cost(int tile, int splits, int M, int N, int K, int es, int b
 }
 
 // `may_split`: the caller has scratch memory for partials.  The order in which K is summed depends on the MFMA shape, the
-// k-groups and the splits, not on the rest of the tile: a batch keeps the order its entries would have one by one
-// (except that it never splits), so that it gives the same bits, and picks the tile among those.
+// k-groups and the splits, not on the rest of the tile: a batch keeps the order its entries would have one by one without
+// scratch, so that it gives the same bits, and picks the tile among those.  The W tiles are therefore not for bf16 products
+// without scratch: a large batch would be left with one small tile of their order.  (There are no batches of e4m3.)
 inline Plan make_plan(int M, int N, int K, int es, bool tb, int batch, bool may_split) {
     Plan best{T256x256, 1};
-    double least = tile_cost(T256x256, 1, M, N, K, es, 1);
+    double least = tile_cost(T256x256, 1, M, N, K, es, tb, 1);
     const int64_t pieces = ((int64_t)K * es + KB - 1) / KB;
     for (int tile = 0; tile < T256x256; ++tile) {
-        if (!tile_takes(tile, es, tb)) continue;
+        if (!tile_takes(tile, es, tb) || (kTileCost[tile].wide && es == 2 && !(may_split && batch == 1))) continue;
         for (int splits = 1; splits <= 8; ++splits) {
             if (splits > 1 && (!may_split || batch > 1 || pieces < 4 * splits)) break;
-            const double us = tile_cost(tile, splits, M, N, K, es, 1);
+            const double us = tile_cost(tile, splits, M, N, K, es, tb, 1);
             if (us < least) { least = us; best = {tile, splits}; }
         }
     }
     if (batch > 1) {
         const TileCost order = kTileCost[best.tile];
-        least = tile_cost(best.tile, 1, M, N, K, es, batch);
+        least = tile_cost(best.tile, 1, M, N, K, es, tb, batch);
         for (int tile = 0; tile < TILES; ++tile) {
-            if (!tile_takes(tile, es, tb) || kTileCost[tile].kg != order.kg || kTileCost[tile].mf != order.mf) continue;
-            const double us = tile_cost(tile, 1, M, N, K, es, batch);
+            if (!tile_takes(tile, es, tb) || kTileCost[tile].wide || kTileCost[tile].kg != order.kg || kTileCost[tile].mf != order.mf) continue;
+            const double us = tile_cost(tile, 1, M, N, K, es, tb, batch);
             if (us < least) { least = us; best.tile = tile; }
         }
     }
@@ -452,6 +466,13 @@ inline Plan make_plan(int M, int N, int K, int es, bool tb, int batch, bool may_
     const int64_t per_split = (pieces + best.splits - 1) / best.splits;
     best.splits = (int)((pieces + per_split - 1) / per_split);
     return best;
+}
+
+// Scratch without which this plan is not taken.  A wide tile touches none of it: with any, the caller has no claim to the
+// order of sums of a product without.
+inline size_t scratch_bytes(const Plan& p, int M, int N, int es, int batch) {
+    if (p.splits > 1) return (size_t)p.splits * batch * M * N * sizeof(float);
+    return es == 2 && p.tile != T256x256 && kTileCost[p.tile].wide ? 16 : 0;
 }
 
 // make_plan costs about a microsecond of host time; a program repeats few shapes, so each thread keeps its last plans.
@@ -503,12 +524,17 @@ int launch_plan(const Plan& p, const void* a, const void* b, void* c, int M, int
         return -1;
     switch (p.tile) {
         TYR_TILE(T16x16, 16, 16, 16, 16, 4, 4)
+        TYR_TILE(T16x16W, 16, 16, 16, 16, 8, 2)
         TYR_TILE(T16x32, 16, 32, 16, 32, 4, 3)
         TYR_TILE(T16x64, 16, 64, 16, 64, 4, 2)
         TYR_TILE(T32x32, 32, 32, 32, 32, 4, 2)
+        TYR_TILE(T32x64W, 32, 64, 32, 32, 4, 3)
         TYR_TILE(T64x32, 64, 32, 32, 32, 2, 3)
+        TYR_TILE(T64x32W, 64, 32, 32, 32, 4, 3)
         TYR_TILE(T64x64, 64, 64, 32, 32, 1, 5)
+        TYR_TILE(T64x64W, 64, 64, 32, 32, 2, 3)
         TYR_TILE(T64x128, 64, 128, 64, 32, 1, 3)
+        TYR_TILE(T64x128W, 64, 128, 64, 32, 2, 3)
         TYR_TILE(T96x64, 96, 64, 48, 32, 2, 4)
         TYR_TILE(T128x128, 128, 128, 64, 32, 1, 5)
         TYR_TILE(T192x128, 192, 128, 96, 32, 1, 4)
