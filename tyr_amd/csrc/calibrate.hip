@@ -96,10 +96,10 @@ extern "C" int tyr_hip_mfma_sustain(const void* operands, size_t operand_bytes, 
     if (flop_per_launch) *flop_per_launch = 2.0 * 32 * 32 * k * NF * NF * (double)iters * 4.0 * (double)workgroups;
     auto ops = static_cast<const unsigned char*>(operands);
     if (dtype == TYR_HIP_MFMA_BF16)
-        hipLaunchKernelGGL(mfma_sustain_kernel<0>, dim3((unsigned)workgroups), dim3(256), 0,
+        launch_kernel(mfma_sustain_kernel<0>, dim3((unsigned)workgroups), dim3(256), 0,
                            static_cast<hipStream_t>(stream), ops, operand_bytes, (int)iters, sink);
     else
-        hipLaunchKernelGGL(mfma_sustain_kernel<1>, dim3((unsigned)workgroups), dim3(256), 0,
+        launch_kernel(mfma_sustain_kernel<1>, dim3((unsigned)workgroups), dim3(256), 0,
                            static_cast<hipStream_t>(stream), ops, operand_bytes, (int)iters, sink);
     return hipGetLastError() == hipSuccess ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }

@@ -1352,7 +1352,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
             reinterpret_cast<const void*>(&flash_attn_bwd_dq_kernel<DD, CC, EE, SS>),                 \
             hipFuncAttributeMaxDynamicSharedMemorySize, CfgQ<DD>::LDS);                               \
         if (a1 != hipSuccess) return -1;                                                              \
-        hipLaunchKernelGGL((flash_attn_bwd_dq_kernel<DD, CC, EE, SS>), grid_q, block, CfgQ<DD>::LDS, stream, \
+        launch_kernel((flash_attn_bwd_dq_kernel<DD, CC, EE, SS>), grid_q, block, CfgQ<DD>::LDS, stream, \
                            Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st, BH, N, ntq, npad, \
                            scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single);        \
     } while (0)
@@ -1362,7 +1362,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
             reinterpret_cast<const void*>(&flash_attn_bwd_dkv_kernel<DD, CC, EE, UU, PP>),            \
             hipFuncAttributeMaxDynamicSharedMemorySize, CfgK<DD>::LDS);                               \
         if (a2 != hipSuccess) return -1;                                                              \
-        hipLaunchKernelGGL((flash_attn_bwd_dkv_kernel<DD, CC, EE, UU, PP>), grid_k, block, CfgK<DD>::LDS, \
+        launch_kernel((flash_attn_bwd_dkv_kernel<DD, CC, EE, UU, PP>), grid_k, block, CfgK<DD>::LDS, \
                            stream, Qp, Kp, Vp, dOp, st, static_cast<uint16_t*>(dk),                   \
                            static_cast<uint16_t*>(dv), BHkv, N, ntk, npad, scale, scale_log2, Hq,     \
                            window, kv_lens, key_mask, plan, items, partial, ds);                      \
@@ -1379,13 +1379,13 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
             hipFuncAttributeMaxDynamicSharedMemorySize, CfgP<DD>::LDS);                               \
         if (a4 != hipSuccess) return -1;                                                              \
         const int ndq = BH * ntk, nsum = plan.chunk ? BHkv * ntk * (DD / 8) : 0;                      \
-        hipLaunchKernelGGL((flash_attn_bwd_dq_product_kernel<DD, CC, EE>), dim3((unsigned)(ndq + nsum)), block, CfgP<DD>::LDS, stream, \
+        launch_kernel((flash_attn_bwd_dq_product_kernel<DD, CC, EE>), dim3((unsigned)(ndq + nsum)), block, CfgP<DD>::LDS, stream, \
                            Kp, ds, static_cast<uint16_t*>(dq), BH, N, ntk, scale, Hq, window, kv_lens, key_mask, \
                            causal && window <= 0, ndq, partial, static_cast<uint16_t*>(dk),           \
                            static_cast<uint16_t*>(dv), items, plan);                                  \
     } while (0)
 #define TYR_FAB_SUM(DD)                                                                               \
-    hipLaunchKernelGGL(flash_attn_bwd_sum_kernel<DD>, dim3((unsigned)(BHkv * ntk * (DD / 8))), dim3(256), 0, stream, \
+    launch_kernel(flash_attn_bwd_sum_kernel<DD>, dim3((unsigned)(BHkv * ntk * (DD / 8))), dim3(256), 0, stream, \
                        partial, static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), N, ntk, items, scale, plan)
 #define TYR_FAB_BOTH(DD, CC, EE, UU)                                                                  \
     do {                                                                                              \
@@ -1393,7 +1393,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
             reinterpret_cast<const void*>(&flash_attn_bwd_both_kernel<DD, CC, EE, UU>),               \
             hipFuncAttributeMaxDynamicSharedMemorySize, CfgK<DD>::LDS);                               \
         if (a3 != hipSuccess) return -1;                                                              \
-        hipLaunchKernelGGL((flash_attn_bwd_both_kernel<DD, CC, EE, UU>), dim3(grid_k.x + (unsigned)how.dq_blocks), block, CfgK<DD>::LDS, \
+        launch_kernel((flash_attn_bwd_both_kernel<DD, CC, EE, UU>), dim3(grid_k.x + (unsigned)how.dq_blocks), block, CfgK<DD>::LDS, \
                            stream, Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st,          \
                            static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), BH, N, (N + 63) / 64, ntk, \
                            npad, scale, scale_log2, Hq, window, kv_lens, key_mask, causal && window <= 0, plan, items, partial, (int)grid_k.x); \
@@ -1408,7 +1408,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
         }                                                                                             \
         if constexpr (DD == 128) {                                                                               \
             if (how.ds) {                                                                             \
-                hipLaunchKernelGGL(flash_attn_bwd_stats_kernel<DD>, dim3((unsigned)(BH * (npad / (2048 / DD)))), dim3(256), 0, \
+                launch_kernel(flash_attn_bwd_stats_kernel<DD>, dim3((unsigned)(BH * (npad / (2048 / DD)))), dim3(256), 0, \
                                    stream, Op, dOp, lse, st, N, npad, EE != AttnMask::None);          \
                 if (plan.chunk) TYR_FAB_DKV_MASK(DD, CC, EE, true, true);                             \
                 else TYR_FAB_DKV_MASK(DD, CC, EE, false, true);                                       \

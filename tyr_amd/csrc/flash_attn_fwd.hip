@@ -603,7 +603,7 @@ int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, 
             reinterpret_cast<const void*>(&flash_attn_fwd_kernel<DD, CC, EE, SS>),               \
             hipFuncAttributeMaxDynamicSharedMemorySize, Cfg<DD>::LDS);                           \
         if (attr != hipSuccess) return -1;                                                       \
-        hipLaunchKernelGGL((flash_attn_fwd_kernel<DD, CC, EE, SS>), grid, block, Cfg<DD>::LDS, stream, \
+        launch_kernel((flash_attn_fwd_kernel<DD, CC, EE, SS>), grid, block, Cfg<DD>::LDS, stream, \
                            Qp, Kp, Vp, Op, lse, BH, N, ntq, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single, total_ids); \
     } while (0)
 #define TYR_FA_SHAPE(DD, CC, EE)                                                                 \

@@ -430,7 +430,7 @@ int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K,
                 reinterpret_cast<const void*>(&gemm_bf16_fast_kernel<TB, KT>),                    \
                 hipFuncAttributeMaxDynamicSharedMemorySize, gemm2::LDS_BYTES);                    \
             if (attr != hipSuccess) return -1;                                                    \
-            hipLaunchKernelGGL((gemm_bf16_fast_kernel<TB, KT>), grid, dim3(gemm2::THREADS), gemm2::LDS_BYTES, stream, \
+            launch_kernel((gemm_bf16_fast_kernel<TB, KT>), grid, dim3(gemm2::THREADS), gemm2::LDS_BYTES, stream, \
                                A, Bp, Cp, M, N, K, tiles_m, tiles_n, (long)stride_a, (long)stride_b,  \
                                (long)stride_c);                                                   \
         } while (0)
@@ -446,7 +446,7 @@ int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K,
             reinterpret_cast<const void*>(&gemm_bf16_kernel<TB, ED>),                             \
             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);                               \
         if (attr != hipSuccess) return -1;                                                        \
-        hipLaunchKernelGGL((gemm_bf16_kernel<TB, ED>), grid, block, LDS_BYTES, stream, A, Bp, Cp, \
+        launch_kernel((gemm_bf16_kernel<TB, ED>), grid, block, LDS_BYTES, stream, A, Bp, Cp, \
                            M, N, K, tiles_m, tiles_n, (long)stride_a, (long)stride_b,             \
                            (long)stride_c);                                                       \
     } while (0)

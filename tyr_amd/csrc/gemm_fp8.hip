@@ -440,7 +440,7 @@ int launch_gemm_fp8(const void* aq, const void* bq, void* c, int M, int N, int K
                 reinterpret_cast<const void*>(&gemm_fp8_fast_kernel<TB, KT>),                     \
                 hipFuncAttributeMaxDynamicSharedMemorySize, gemm8f::LDS_BYTES);                   \
             if (attr != hipSuccess) return -1;                                                    \
-            hipLaunchKernelGGL((gemm_fp8_fast_kernel<TB, KT>), grid, dim3(gemm8f::THREADS), gemm8f::LDS_BYTES, stream, \
+            launch_kernel((gemm_fp8_fast_kernel<TB, KT>), grid, dim3(gemm8f::THREADS), gemm8f::LDS_BYTES, stream, \
                                A, Bp, Cp, M, N, K, tiles_m, tiles_n, ep);                         \
         } while (0)
         const bool k_tail = K % gemm8f::BK != 0;
@@ -455,7 +455,7 @@ int launch_gemm_fp8(const void* aq, const void* bq, void* c, int M, int N, int K
             reinterpret_cast<const void*>(&gemm_fp8_kernel<TB, ED>),                              \
             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);                               \
         if (attr != hipSuccess) return -1;                                                        \
-        hipLaunchKernelGGL((gemm_fp8_kernel<TB, ED>), grid, block, LDS_BYTES, stream, A, Bp, Cp,  \
+        launch_kernel((gemm_fp8_kernel<TB, ED>), grid, block, LDS_BYTES, stream, A, Bp, Cp,  \
                            M, N, K, tiles_m, tiles_n, ep);                                        \
     } while (0)
     if (trans_b) { if (edge) TYR_GEMM8_LAUNCH(true, true); else TYR_GEMM8_LAUNCH(true, false); }

@@ -500,12 +500,12 @@ int launch(const void* a, const void* b, void* c, int M, int N, int K, int split
     int group_m = (int)lround(sqrt((double)tiles_m * tiles_n / 8 * C::BN / C::BM));
     group_m = group_m < 1 ? 1 : group_m > tiles_m ? tiles_m : group_m;
     const int pieces = (int)(((int64_t)K * C::ES + KB - 1) / KB), per_split = (pieces + splits - 1) / splits;
-    hipLaunchKernelGGL((gemm_tile_kernel<C>), dim3((unsigned)wgs, (unsigned)batch), dim3(C::THREADS), C::LDS, stream,
+    launch_kernel((gemm_tile_kernel<C>), dim3((unsigned)wgs, (unsigned)batch), dim3(C::THREADS), C::LDS, stream,
                        static_cast<const unsigned char*>(a), static_cast<const unsigned char*>(b), static_cast<unsigned char*>(c), part, M, N,
                        K, tiles_m, tiles_n, group_m, splits, pieces, per_split, (long)stride_a, (long)stride_b, (long)stride_c, ep);
     if (hipGetLastError() != hipSuccess) return -1;
     if (splits > 1) {
-        hipLaunchKernelGGL(gemm_tile_reduce_kernel<C::ES>, dim3((unsigned)(((size_t)M * (N / 4) + 255) / 256), (unsigned)batch), dim3(256), 0,
+        launch_kernel(gemm_tile_reduce_kernel<C::ES>, dim3((unsigned)(((size_t)M * (N / 4) + 255) / 256), (unsigned)batch), dim3(256), 0,
                            stream, part, static_cast<unsigned char*>(c), M, N, splits, (long)stride_c, ep);
         if (hipGetLastError() != hipSuccess) return -1;
     }

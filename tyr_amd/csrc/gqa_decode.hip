@@ -301,14 +301,14 @@ int launch_gqa_decode(const void* q, const void* k, const void* v, void* o, floa
             hipFuncAttributeMaxDynamicSharedMemorySize,                                              \
             (WAVES * QPAD * DD + 2 * WAVES * QPAD) * (int)sizeof(float));                            \
         if (attr != hipSuccess) return -1;                                                           \
-        hipLaunchKernelGGL((gqa_decode_split_kernel<WAVES, DD>), grid, dim3(64 * WAVES), lds, stream,          \
+        launch_kernel((gqa_decode_split_kernel<WAVES, DD>), grid, dim3(64 * WAVES), lds, stream,          \
                            static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),         \
                            static_cast<const uint16_t*>(v), part_o, part_m, part_l,                  \
                            static_cast<uint16_t*>(o), lse, Hq, Hkv, G, L, (long)kv_stride, S, chunk, \
                            scale * LOG2E, kv_lens, window);                                          \
         if (hipGetLastError() != hipSuccess) return -1;                                              \
         if (S > 1) {                                                                                 \
-            hipLaunchKernelGGL(gqa_decode_combine_kernel<DD>, dim3((unsigned)(B * Hq)), dim3(256), 0, \
+            launch_kernel(gqa_decode_combine_kernel<DD>, dim3((unsigned)(B * Hq)), dim3(256), 0, \
                                stream, part_o, part_m, part_l, static_cast<uint16_t*>(o), lse, S);   \
             if (hipGetLastError() != hipSuccess) return -1;                                          \
         }                                                                                            \

@@ -255,7 +255,7 @@ int launch_copy(const void* src, void* dst, size_t bytes, hipStream_t stream) {
     size_t blocks = (n16 + rw::STREAM_THREADS - 1) / rw::STREAM_THREADS;
     if (blocks == 0) blocks = 1;
     if (blocks > 0x7fffffffull) return -1;             // 2^31 workgroups of 1 KiB: 2 TiB
-    hipLaunchKernelGGL((2 * bytes <= kStreamCached ? copy_kernel<true> : copy_kernel<false>), dim3((unsigned)blocks), dim3(rw::STREAM_THREADS), 0, stream,
+    launch_kernel((2 * bytes <= kStreamCached ? copy_kernel<true> : copy_kernel<false>), dim3((unsigned)blocks), dim3(rw::STREAM_THREADS), 0, stream,
                        static_cast<const u32x4*>(src), static_cast<u32x4*>(dst), n16,
                        static_cast<const unsigned char*>(src) + n16 * 16, static_cast<unsigned char*>(dst) + n16 * 16,
                        tail);
@@ -269,7 +269,7 @@ int launch_rope_fwd(const void* x, const float* cosp, const float* sinp, void* y
     auto go = [&](auto elem, auto cached, auto index) {
         using T = decltype(elem);
         using I = decltype(index);
-        hipLaunchKernelGGL((rope_kernel<T, cached(), I>), dim3((unsigned)((threads + rw::THREADS - 1) / rw::THREADS)), dim3(rw::THREADS), 0,
+        launch_kernel((rope_kernel<T, cached(), I>), dim3((unsigned)((threads + rw::THREADS - 1) / rw::THREADS)), dim3(rw::THREADS), 0,
                            stream, static_cast<const T*>(x), cosp, sinp, static_cast<T*>(y), (I)threads, (unsigned)S, (unsigned)H, per_row);
     };
     auto pick = [&](auto elem) {
@@ -287,7 +287,7 @@ int launch_decode_rope_append(const void* q, const void* k_new, const void* v_ne
     const int nq = B * Hq, nkv = B * Hkv;
     const size_t threads = (size_t)(nq + 2 * nkv) * (D / 16);
     const size_t blocks = (threads + rw::THREADS - 1) / rw::THREADS;
-    hipLaunchKernelGGL(decode_rope_append_kernel, dim3((unsigned)blocks), dim3(rw::THREADS), 0, stream,
+    launch_kernel(decode_rope_append_kernel, dim3((unsigned)blocks), dim3(rw::THREADS), 0, stream,
                        static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k_new),
                        static_cast<const uint16_t*>(v_new), cosp, sinp, static_cast<uint16_t*>(q_out),
                        static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), nq, nkv, D, kv_stride, pos);
@@ -299,7 +299,7 @@ int launch_layernorm_residual(const void* x, const void* residual, const void* w
     auto go = [&](auto wpr, auto p) {
         constexpr int W = wpr(), RPB = W > 4 ? 1 : 4 / W;       // rows per workgroup
         auto kernel = rows * d_model * 8 <= kStreamCached ? &layernorm_residual_kernel<W, p(), true> : &layernorm_residual_kernel<W, p(), false>;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(W > 4 ? 64 * W : 256), 0, stream,
+        launch_kernel(kernel, dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(W > 4 ? 64 * W : 256), 0, stream,
                            static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(residual), static_cast<const uint16_t*>(weight),
                            static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(out), static_cast<uint16_t*>(out_resid), rows,
                            d_model, eps);

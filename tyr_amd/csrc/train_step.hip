@@ -178,15 +178,15 @@ int tyr_hip_mse_loss_grad(const void* out, const void* target, void* d_out, floa
     if (reinterpret_cast<uintptr_t>(workspace) & 3u) return TYR_HIP_ERR_MISALIGNED;
     auto s = static_cast<hipStream_t>(stream);
     if (pieces <= ONE_PASS) {
-        hipLaunchKernelGGL(mse_grad_loss_kernel, dim3(1), dim3(1024), 0, s, static_cast<const uint16_t*>(out),
+        launch_kernel(mse_grad_loss_kernel, dim3(1), dim3(1024), 0, s, static_cast<const uint16_t*>(out),
                            static_cast<const uint16_t*>(target), static_cast<uint16_t*>(d_out), loss, (int)pieces, (float)n);
         return hipGetLastError() == hipSuccess ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
     }
     float* partial = static_cast<float*>(workspace);
-    hipLaunchKernelGGL((6 * n <= kStreamCached ? mse_grad_kernel<true> : mse_grad_kernel<false>), dim3((unsigned)blocks), dim3(THREADS), 0, s, static_cast<const uint16_t*>(out),
+    launch_kernel((6 * n <= kStreamCached ? mse_grad_kernel<true> : mse_grad_kernel<false>), dim3((unsigned)blocks), dim3(THREADS), 0, s, static_cast<const uint16_t*>(out),
                        static_cast<const uint16_t*>(target), static_cast<uint16_t*>(d_out), partial, (size_t)pieces, (float)n);
     if (hipGetLastError() != hipSuccess) return TYR_HIP_ERR_LAUNCH;
-    hipLaunchKernelGGL(mse_loss_kernel, dim3(1), dim3(1024), 0, s, partial, (size_t)blocks, (double)n, loss);
+    launch_kernel(mse_loss_kernel, dim3(1), dim3(1024), 0, s, partial, (size_t)blocks, (double)n, loss);
     return hipGetLastError() == hipSuccess ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }
 
@@ -200,7 +200,7 @@ int tyr_hip_sgd_step(const float* param, const void* grad, float lr, float* para
     if (blocks > (uint64_t)INT_MAX) return TYR_HIP_ERR_BAD_SHAPE;
     if (!aligned16(param) || !aligned16(grad) || !aligned16(param_out) || !aligned16(param_out_bf16))
         return TYR_HIP_ERR_MISALIGNED;
-    hipLaunchKernelGGL((12 * n <= kStreamCached ? sgd_kernel<true> : sgd_kernel<false>), dim3((unsigned)blocks), dim3(THREADS), 0, static_cast<hipStream_t>(stream), param,
+    launch_kernel((12 * n <= kStreamCached ? sgd_kernel<true> : sgd_kernel<false>), dim3((unsigned)blocks), dim3(THREADS), 0, static_cast<hipStream_t>(stream), param,
                        static_cast<const uint16_t*>(grad), lr, param_out, static_cast<uint16_t*>(param_out_bf16), (size_t)n);
     return hipGetLastError() == hipSuccess ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }

@@ -26,6 +26,9 @@ class TyrGpuError(RuntimeError):
 # Checks, allocation and the C ABI call of every entry point below are native code (csrc/torch_binding.cpp): in Python
 # they took longer than most of the kernels they launch.
 _n = _lib.load_binding(TyrGpuError)
+_flash_attn_fwd, _flash_attn_bwd, _gqa_decode, _decode_rope_append = _n.flash_attn_fwd, _n.flash_attn_bwd, _n.gqa_decode, _n.decode_rope_append
+_rope_fwd, _layernorm_residual, _copy, _matmul_bf16, _gemm_bf16 = _n.rope_fwd, _n.layernorm_residual, _n.copy, _n.matmul_bf16, _n.gemm_bf16
+_gemm_fp8, _gemm_fp8_scaled, _mse_loss_grad, _sgd_step = _n.gemm_fp8, _n.gemm_fp8_scaled, _n.mse_loss_grad, _n.sgd_step
 
 
 def library_path() -> str:
@@ -51,9 +54,7 @@ def _launch_stream(stream):
         yield
 
 
-def _call(fn, stream, *args):
-    if stream is None:
-        return fn(*args)
+def _on_stream(stream, fn, *args):
     with _launch_stream(stream):
         return fn(*args)
 
@@ -77,7 +78,9 @@ def flash_attn_fwd(q, k, v, causal: bool = True, scale: float | None = None, win
     ``window`` > 0 (causal only) lets query i see keys (i - window, i]; ``kv_lens`` (int32 [B] on the device)
     masks the keys at or beyond each sequence's length; ``key_mask`` (bool / uint8 [B,N] on the device, nonzero =
     visible) hides any set of keys per sequence instead.  -> (bf16 [B,Hq,N,D], f32 [B,Hq,N])."""
-    return _call(_n.flash_attn_fwd, stream, q, k, v, causal, scale, window, kv_lens, key_mask)
+    if stream is None:
+        return _flash_attn_fwd(q, k, v, causal, scale, window, kv_lens, key_mask)
+    return _on_stream(stream, _flash_attn_fwd, q, k, v, causal, scale, window, kv_lens, key_mask)
 
 
 def flash_attn_bwd(q, k, v, o, lse, d_o, causal: bool = True, scale: float | None = None, window: int = 0,
@@ -87,7 +90,9 @@ def flash_attn_bwd(q, k, v, o, lse, d_o, causal: bool = True, scale: float | Non
     q, o, d_o bf16 [B,Hq,N,D]; k, v bf16 [B,Hkv,N,D]; lse f32 [B,Hq,N]; o and lse as returned by
     flash_attn_fwd for the same q, k, v, causal, scale, window, kv_lens and key_mask.  Returns dQ [B,Hq,N,D] and
     dK, dV [B,Hkv,N,D] (summed over the query heads of each kv head), bf16."""
-    return _call(_n.flash_attn_bwd, stream, q, k, v, o, lse, d_o, causal, scale, window, kv_lens, key_mask)
+    if stream is None:
+        return _flash_attn_bwd(q, k, v, o, lse, d_o, causal, scale, window, kv_lens, key_mask)
+    return _on_stream(stream, _flash_attn_bwd, q, k, v, o, lse, d_o, causal, scale, window, kv_lens, key_mask)
 
 
 def gqa_decode(q, k, v, scale: float | None = None, num_splits: int = 0, kv_len: int | None = None,
@@ -99,7 +104,9 @@ def gqa_decode(q, k, v, scale: float | None = None, num_splits: int = 0, kv_len:
     gives every sequence its own length in [0, kv_len] (a length of 0 yields O = 0, LSE = -inf); ``window`` > 0 restricts each sequence to its last
     ``window`` rows.  -> (bf16 [B,Hq,1,D], f32 [B,Hq]).
     """
-    return _call(_n.gqa_decode, stream, q, k, v, scale, num_splits, kv_len, kv_lens, window)
+    if stream is None:
+        return _gqa_decode(q, k, v, scale, num_splits, kv_len, kv_lens, window)
+    return _on_stream(stream, _gqa_decode, q, k, v, scale, num_splits, kv_len, kv_lens, window)
 
 
 def decode_rope_append(q, k_new, v_new, cos, sin, k_cache, v_cache, pos: int, stream=None):
@@ -108,39 +115,53 @@ def decode_rope_append(q, k_new, v_new, cos, sin, k_cache, v_cache, pos: int, st
     q bf16 [B,Hq,1,D] (or [B,1,Hq,D]); k_new, v_new bf16 [B,Hkv,1,D]; cos, sin f32 [1,D/2] (or [D/2]) for
     position ``pos``; caches bf16 [B,Hkv,maxLen,D], row ``pos`` of each is overwritten in place.  Returns the
     rotated q with q's shape."""
-    return _call(_n.decode_rope_append, stream, q, k_new, v_new, cos, sin, k_cache, v_cache, pos)
+    if stream is None:
+        return _decode_rope_append(q, k_new, v_new, cos, sin, k_cache, v_cache, pos)
+    return _on_stream(stream, _decode_rope_append, q, k_new, v_new, cos, sin, k_cache, v_cache, pos)
 
 
 def rope_fwd(x, cos, sin, stream=None):
     """y = applyRotaryEmb x cos sin.  x f32 or bf16 [B,S,H,D]; cos, sin f32 [S,D/2]."""
-    return _call(_n.rope_fwd, stream, x, cos, sin)
+    if stream is None:
+        return _rope_fwd(x, cos, sin)
+    return _on_stream(stream, _rope_fwd, x, cos, sin)
 
 
 def layernorm_residual(x, residual, weight, bias, eps: float = 1e-5, stream=None):
     """(out, outResid) = fusedLayerNormResidual x residual weight bias.  bf16; x, residual [..., d]; weight, bias [d]."""
-    return _call(_n.layernorm_residual, stream, x, residual, weight, bias, eps)
+    if stream is None:
+        return _layernorm_residual(x, residual, weight, bias, eps)
+    return _on_stream(stream, _layernorm_residual, x, residual, weight, bias, eps)
 
 
 def copy(src, stream=None):
     """out = copy src (any dtype, contiguous)."""
-    return _call(_n.copy, stream, src)
+    if stream is None:
+        return _copy(src)
+    return _on_stream(stream, _copy, src)
 
 
 def matmul_bf16(a, b, trans_b: bool = False, stream=None):
     """C = matmul a b for operands of rank > 2 (`lean_torch_matmul`): a bf16 [..., M, K]; b bf16 [..., K, N] with
     the same leading extents, or a plain [K, N] matrix used for every batch entry (b is [..., N, K] / [N, K] with
     trans_b) -> bf16 [..., M, N]."""
-    return _call(_n.matmul_bf16, stream, a, b, trans_b)
+    if stream is None:
+        return _matmul_bf16(a, b, trans_b)
+    return _on_stream(stream, _matmul_bf16, a, b, trans_b)
 
 
 def gemm_bf16(a, b, trans_b: bool = False, stream=None):
     """C = gemmBf16 a b.  a bf16 [M,K]; b bf16 [K,N] (or [N,K] with trans_b) -> bf16 [M,N]."""
-    return _call(_n.gemm_bf16, stream, a, b, trans_b)
+    if stream is None:
+        return _gemm_bf16(a, b, trans_b)
+    return _on_stream(stream, _gemm_bf16, a, b, trans_b)
 
 
 def gemm_fp8(aq, bq, scale_a: float, scale_b: float, trans_b: bool = False, stream=None):
     """C = gemmFp8 aq bq scaleA scaleB.  aq e4m3 [M,K]; bq e4m3 [K,N] (or [N,K]) -> bf16 [M,N]."""
-    return _call(_n.gemm_fp8, stream, aq, bq, scale_a, scale_b, trans_b)
+    if stream is None:
+        return _gemm_fp8(aq, bq, scale_a, scale_b, trans_b)
+    return _on_stream(stream, _gemm_fp8, aq, bq, scale_a, scale_b, trans_b)
 
 
 def gemm_fp8_scaled(aq, bq, row_scale=None, col_scale=None, scale: float = 1.0, out_dtype=torch.float32,
@@ -150,20 +171,26 @@ def gemm_fp8_scaled(aq, bq, row_scale=None, col_scale=None, scale: float = 1.0, 
     The per-row / per-column dequantisation epilogue of `tkH100Fp8ScaledGemmFwd` (f32 out) and, with no scales and
     out_dtype = torch.float8_e4m3fn, the E4M3 epilogue of `tkH100Fp8E4M3GemmFwd`.  aq e4m3 [M,K]; bq e4m3 [K,N] (or
     [N,K] with trans_b); row_scale f32 [M], col_scale f32 [N] or None."""
-    return _call(_n.gemm_fp8_scaled, stream, aq, bq, row_scale, col_scale, scale, out_dtype, trans_b)
+    if stream is None:
+        return _gemm_fp8_scaled(aq, bq, row_scale, col_scale, scale, out_dtype, trans_b)
+    return _on_stream(stream, _gemm_fp8_scaled, aq, bq, row_scale, col_scale, scale, out_dtype, trans_b)
 
 
 def mse_loss_grad(out, target, stream=None):
     """(loss, dO) = lossAndGradOut out target: loss = 0.5 mean((out - target)^2) as an f32 scalar tensor,
     dO = bf16((out - target) / numel).  out, target bf16, same shape, numel % 8 == 0."""
-    return _call(_n.mse_loss_grad, stream, out, target)
+    if stream is None:
+        return _mse_loss_grad(out, target)
+    return _on_stream(stream, _mse_loss_grad, out, target)
 
 
 def sgd_step(param, grad, lr: float, in_place: bool = False, stream=None):
     """(param', bf16 param') = sgdUpdate param grad lr: param' = param - f32(grad) * lr for an f32 master and a bf16
     gradient of the same shape, together with the bf16 cast the next step's kernels take.  ``in_place`` overwrites
     ``param`` instead of allocating."""
-    return _call(_n.sgd_step, stream, param, grad, lr, in_place)
+    if stream is None:
+        return _sgd_step(param, grad, lr, in_place)
+    return _on_stream(stream, _sgd_step, param, grad, lr, in_place)
 
 
 def quantize_e4m3(x: torch.Tensor):
