@@ -162,7 +162,7 @@ def test_backward_with_the_least_workspace(B, Hq, Hkv, N, D, mask):
 
 
 @pytest.mark.parametrize("mask", ["causal", "full", "window", "lens", "keys"])
-@pytest.mark.parametrize("B,Hq,Hkv,N", [(4, 16, 4, 577), (4, 16, 16, 640), (2, 32, 8, 1153), (4, 8, 1, 1025)])
+@pytest.mark.parametrize("B,Hq,Hkv,N", [(4, 16, 4, 577), (4, 16, 4, 640), (4, 16, 16, 769), (2, 32, 8, 1153), (4, 8, 1, 1025), (9, 16, 4, 129)])
 def test_backward_that_keeps_ds(B, Hq, Hkv, N, mask):
     """Few heads at D = 128, where dK / dV leave dS for dQ: rows one past a tile, whole tiles, whole and cut key tiles.  Hidden keys
     come first, in the middle (more than one block of 128) and last, with values that would outweigh every visible one."""
@@ -179,7 +179,7 @@ def test_backward_that_keeps_ds(B, Hq, Hkv, N, mask):
         opt["window"] = window = N - 37
         visible = visible & (i[:, None] - i[None, :] < window)
     if mask == "lens":
-        opt["kv_lens"] = torch.tensor([N, 0, N // 2 + 1, 129][:B], dtype=torch.int32, device="cuda")
+        opt["kv_lens"] = torch.tensor(([N, 0, N // 2 + 1, 129] * B)[:B], dtype=torch.int32, device="cuda")
         shown = i[None, :] < opt["kv_lens"][:, None]
     if mask == "keys":
         shown = torch.rand(B, N, device="cuda", generator=gen) > 0.3
@@ -196,7 +196,9 @@ def test_backward_that_keeps_ds(B, Hq, Hkv, N, mask):
     for got, ref in zip(grads, (wq, wk, wv)):
         assert rel_fro(got, ref) <= 1e-2
         err, n = (got.float() - ref).norm(dim=-1), ref.norm(dim=-1)
-        assert float((err / n.clamp_min(float(n[n > 0].mean()))).max()) <= 4e-2
+        # a dQ row with one heavy key takes delta's error whole: sum of g o r over D = 128, |r| <= 2^-8 the rounding of o, about
+        # 0.4 * 2^-8 rms, so 11.3 * 0.0016 = 0.018 times |scale K| = 1; five such are 0.09, and a mean row is 1.2 or more
+        assert float((err / n.clamp_min(float(n[n > 0].mean()))).max()) <= 8e-2
     assert all(torch.equal(a, b) for a, b in zip(grads, tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)))
     # with the least scratch dQ makes dS itself, from the same bf16 operands: what may differ is the order of f32 sums, and
     # with it one rounding to bf16 (2^-8 of an element) here and there

@@ -1269,9 +1269,11 @@ int dkv_items(const fab::Parts& p, int N) {
 // than that.  Measured (MI355X, us, two launches -> one): B1 H1 N128 D64 11.0 -> 7.5, B1 H4 N512 D128 causal 27.2 -> 18.3,
 // B1 Hq8 Hkv2 N700 40.6 -> 28.8; 384 workgroups, N1000 43.7 -> 39.8; beyond, a dK/dV workgroup waits longer for the pairs of
 // all its rows and dQ comes last: 512 workgroups, N2048 69 -> 73.
-bool one_launch(int N, int64_t dq_blocks, int64_t dkv_blocks) {
-    const int64_t n = dq_blocks + dkv_blocks;
-    return n <= 256 || (n <= 640 && N <= 1024);
+// Where dS could be kept that is faster from 420 workgroups on (300 not causal): B2 Hq16 Hkv4 N564 full, 528 of them, 59.7 ->
+// 39.7, B2 H8 N707 with a key mask, 448, 38.9 -> 33.4.  On 180 shapes of 60 to 1500 workgroups the choice among the three forms
+// is 0.4 % slower than the best, D = 64 (of two) 0.9 %.
+bool one_launch(int N, int64_t blocks, bool ds, bool causal) {
+    return blocks <= 256 || (N <= 1024 && blocks <= (!ds ? 640 : causal ? 420 : 300));
 }
 size_t dkv_partial_bytes(const fab::Parts& p, int BHkv, int N, int D) {
     return p.chunk ? (size_t)BHkv * dkv_items(p, N) * 128 * D * 8 : 0;
@@ -1281,14 +1283,17 @@ size_t ds_bytes(int BH, int N, bool causal, int window) {
 }
 // Whether dK/dV leave dS for dQ: five products in three launches (pairs, dK/dV, dQ) in place of seven in two.  Worth it while dS
 // stays in the 256 MB last-level cache and the heads are few: beyond, dS costs its traffic to HBM, and many short tiles
-// fill the device in the other form as well.  With G >= 4 query heads a K / V, dQ's share of the requests hits the L2.
+// fill the device in the other form as well.  With G >= 4 query heads a K / V, dQ's share of the requests hits the L2 (any
+// window, more heads); without, a causal launch of few short tiles and one of a narrow window save little.
 // Measured (us, without -> with, whole backward, D = 128): B1 Hq32 Hkv8 N2000 147.5 -> 131.5, B1 Hq4 N6083 201 -> 163, B9 Hq8
-// Hkv2 N900 full 176 -> 145; on the other side of the line B12 H16 N555 109 -> 117, B7 Hq32 Hkv8 N812 202 -> 206, B5 Hq8
-// Hkv2 N2724 (331 MB) 300 -> 307, B16 H16 N4096 (4.4 GB) 3640 -> 3530 with 18 times the scratch.
+// Hkv2 N900 full 176 -> 145, B15 Hq16 Hkv4 N316 full 96 -> 78; on the other side of the line B12 H16 N555 109 -> 117, B7 Hq32
+// Hkv8 N812 202 -> 206, B1 H32 N563 31 -> 37, B5 Hq8 Hkv2 N2724 (331 MB) 300 -> 307, B16 H16 N4096 (4.4 GB) 3640 -> 3530 with
+// 18 times the scratch.  D = 64: 0.9 to 1.3 times the time, mostly slower.
 bool keeps_ds(int BH, int G, int N, int D, bool causal, int window) {
     const fab::DsBlocks place{(N + 127) / 128, causal, window};
-    return D == 128 && place.ntk >= 5 && place.width() >= std::min(place.ntk, 8) && BH <= (G >= 4 ? 128 : 64) &&
-           ds_bytes(BH, N, causal, window) <= (size_t)288 << 20;
+    if (D != 128 || place.ntk < 2 || ds_bytes(BH, N, causal, window) > (size_t)288 << 20) return false;
+    if (G >= 4) return BH <= (place.ntk <= 4 ? 256 : 128);
+    return BH <= 64 && (!causal || (place.ntk >= 6 && place.width() >= std::min(place.ntk, 8)));
 }
 // What a call does with all the scratch it can use, and the parts of that scratch, in this order.
 struct BwdPlan {
@@ -1306,8 +1311,9 @@ BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int D, bool causal, int window, 
     p.items = dkv_items(p.parts, N);
     p.dq_blocks = (int64_t)B * Hq * ((N + 63) / 64);
     p.dkv_blocks = (int64_t)B * Hkv * p.items;
-    p.both = one_launch(N, p.dq_blocks, p.dkv_blocks);
-    p.ds = !least && !p.both && keeps_ds(B * Hq, Hq / Hkv, N, D, causal, window);
+    const bool ds = !least && keeps_ds(B * Hq, Hq / Hkv, N, D, causal, window);
+    p.both = one_launch(N, p.dq_blocks + p.dkv_blocks, ds, causal);
+    p.ds = ds && !p.both;
     p.stat_bytes = flash_attn_bwd_workspace_bytes(B, Hq, N);
     p.partial_bytes = dkv_partial_bytes(p.parts, B * Hkv, N, D);
     p.ds_bytes = p.ds ? ds_bytes(B * Hq, N, causal, window) : 0;
