@@ -248,6 +248,13 @@ __device__ __forceinline__ void store_quadrant_bf16(const f32x16 (&acc)[4][NJ], 
     }
 }
 
+// Four f32 to e4m3, round to nearest even, saturating at +-448; NaN stays.
+__device__ __forceinline__ uint32_t pack_e4m3(f32x4 v) {
+#pragma unroll
+    for (int x = 0; x < 4; ++x) v[x] = v[x] != v[x] ? v[x] : fminf(fmaxf(v[x], -448.0f), 448.0f);
+    const int w = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], w, true);
+}
 // Epilogue variants of the fp8 GEMM beyond "one scalar, bf16 out": per-row and per-column scales and the
 // output element type.  The common case (no vectors, bf16) takes store_quadrant_bf16 above.
 struct GemmEpilogue {
@@ -257,11 +264,21 @@ struct GemmEpilogue {
     int out;                     // 0 = bf16, 1 = f32, 2 = e4m3 (round to nearest even, saturating at +-448)
     __device__ __host__ bool plain_bf16() const { return out == 0 && row_scale == nullptr && col_scale == nullptr; }
 };
+// Four scaled elements of C (row pitch N) from column gn on.
+__device__ __forceinline__ void store_scaled4(const GemmEpilogue& ep, void* C, int N, int gm, int gn, f32x4 v) {
+    const size_t at = (size_t)gm * N + gn;
+    if (ep.out == 1) {
+        *reinterpret_cast<f32x4*>(static_cast<float*>(C) + at) = v;
+    } else if (ep.out == 2) {
+        *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(C) + at) = pack_e4m3(v);
+    } else {
+        st_global_8(static_cast<uint16_t*>(C) + at, u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])});
+    }
+}
 // One wave's 128x128 accumulator quadrant (layout as in store_quadrant_bf16) written straight from registers:
 // a lane stores the 4 consecutive n of a register group of its row.  gm0 / gn0 = global row / column of the
 // quadrant's first element; M, N = extents of C (row pitch N elements).
-template <int NJ>
-__device__ __forceinline__ void store_quadrant_ex(const f32x16 (&acc)[4][NJ], const GemmEpilogue& ep, void* C, int M, int N,
+__device__ __forceinline__ void store_quadrant_ex(const f32x16 (&acc)[4][4], const GemmEpilogue& ep, void* C, int M, int N,
                                                   int gm0, int gn0, int lane) {
     const int r = lane & 31, g = lane >> 5;
 #pragma unroll
@@ -270,32 +287,63 @@ __device__ __forceinline__ void store_quadrant_ex(const f32x16 (&acc)[4][NJ], co
         if (gm >= M) continue;
         const float rs = ep.scale * (ep.row_scale ? ep.row_scale[gm] : 1.0f);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int q4 = 0; q4 < 4; ++q4) {
                 const int gn = gn0 + j * 32 + q4 * 8 + g * 4;
                 if (gn >= N) continue;                       // N is a multiple of 16: a group of 4 is inside or outside
-                float v[4];
+                f32x4 v = f32x4{acc[i][j][q4 * 4], acc[i][j][q4 * 4 + 1], acc[i][j][q4 * 4 + 2], acc[i][j][q4 * 4 + 3]} * rs;
+                if (ep.col_scale) v *= *reinterpret_cast<const f32x4*>(ep.col_scale + gn);
+                store_scaled4(ep, C, N, gm, gn, v);
+            }
+    }
+}
+// One wave's 128x64 block the same way, but through the wave's LDS scratch: each 32-row band as f32 (rows of 64 + 4), read back
+// along the rows, so that a store is 16 bytes a lane and whole rows of the block (64 to 256 bytes) whatever the element, and
+// the row and column scales are read once a lane.  Straight from registers a store touches 64 lines: M = 1065, N = 7136,
+// K = 448 bf16 out 20.9 us, 12.2 this way (11.0 without vectors); 4096^3 60.5 -> 51.0, 8192^3 402 -> 375.
+template <int OUT>
+__device__ __forceinline__ void store_block_scaled(const f32x16 (&acc)[4][2], const GemmEpilogue& ep, unsigned char* scratch, void* C,
+                                                   int M, int N, int gm0, int gn0, int lane) {
+    constexpr int ES = OUT == 0 ? 2 : OUT == 1 ? 4 : 1, W = 16 / ES, LPR = 64 / W;      // columns a lane, lanes a row
+    const int r = lane & 31, g = lane >> 5;
+    const int gn = gn0 + (lane % LPR) * W;                   // N is a multiple of 16: inside or outside as a whole
+    float rs[4];
+    f32x4 cs[W / 4];
 #pragma unroll
-                for (int x = 0; x < 4; ++x) v[x] = acc[i][j][q4 * 4 + x] * rs;
-                if (ep.col_scale) {
-                    const f32x4 cs = *reinterpret_cast<const f32x4*>(ep.col_scale + gn);
+    for (int i = 0; i < 4; ++i) rs[i] = ep.scale * (ep.row_scale ? ep.row_scale[min(gm0 + i * 32 + r, M - 1)] : 1.0f);
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) v[x] *= cs[x];
-                }
-                const size_t at = (size_t)gm * N + gn;
-                if (ep.out == 1) {
-                    *reinterpret_cast<f32x4*>(static_cast<float*>(C) + at) = f32x4{v[0], v[1], v[2], v[3]};
-                } else if (ep.out == 2) {
+    for (int x = 0; x < W / 4; ++x)
+        cs[x] = ep.col_scale && gn < N ? *reinterpret_cast<const f32x4*>(ep.col_scale + gn + 4 * x) : f32x4{1.0f, 1.0f, 1.0f, 1.0f};
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) v[x] = v[x] != v[x] ? v[x] : fminf(fmaxf(v[x], -448.0f), 448.0f);
-                    int w = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
-                    w = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], w, true);
-                    *reinterpret_cast<int*>(static_cast<uint8_t*>(C) + at) = w;
-                } else {
-                    st_global_8(static_cast<uint16_t*>(C) + at, u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])});
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4)
+                *reinterpret_cast<f32x4*>(scratch + r * 272 + (j * 32 + q4 * 8 + g * 4) * 4) =
+                    f32x4{acc[i][j][q4 * 4], acc[i][j][q4 * 4 + 1], acc[i][j][q4 * 4 + 2], acc[i][j][q4 * 4 + 3]} * rs[i];
+#pragma unroll
+        for (int k = 0; k < 32 / W; ++k) {
+            const int row = lane / LPR + W * k, gm = gm0 + i * 32 + row;
+            const unsigned char* from = scratch + row * 272 + (lane % LPR) * (W * 4);
+            u32x4 out;
+            if constexpr (OUT == 1) {
+                out = __builtin_bit_cast(u32x4, *reinterpret_cast<const f32x4*>(from) * cs[0]);
+            } else {
+#pragma unroll
+                for (int x = 0; x < W / 4; ++x) {
+                    const f32x4 v = *reinterpret_cast<const f32x4*>(from + 16 * x) * cs[x];
+                    if constexpr (OUT == 0) {
+                        out[2 * x] = pack_bf16(v[0], v[1]);
+                        out[2 * x + 1] = pack_bf16(v[2], v[3]);
+                    } else {
+                        out[x] = pack_e4m3(v);
+                    }
                 }
             }
+            if (gm < M && gn < N) st_global_16(static_cast<unsigned char*>(C) + ((size_t)gm * N + gn) * ES, out);
+        }
     }
 }
 

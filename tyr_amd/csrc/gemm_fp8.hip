@@ -402,7 +402,11 @@ __global__ __launch_bounds__(gemm8f::THREADS, 1) void gemm_fp8_fast_kernel(
 #undef TYR_FENCE
 
     if (!ep.plain_bf16()) {
-        store_quadrant_ex<2>(acc, ep, C, M, N, m0 + wm * 128, n0 + wn * 64, lane);
+        unsigned char* scratch = lds + w * kEpilogueScratchBytes;
+        const int gm0 = m0 + wm * 128, gn0 = n0 + wn * 64;
+        if (ep.out == 1)      store_block_scaled<1>(acc, ep, scratch, C, M, N, gm0, gn0, lane);
+        else if (ep.out == 2) store_block_scaled<2>(acc, ep, scratch, C, M, N, gm0, gn0, lane);
+        else                  store_block_scaled<0>(acc, ep, scratch, C, M, N, gm0, gn0, lane);
         return;
     }
     store_quadrant_bf16<2>(acc, scale, lds + w * kEpilogueScratchBytes,

@@ -108,21 +108,9 @@ __device__ __forceinline__ i32x8 join(u32x4 a, u32x4 b) {
 
 // four consecutive columns of C at (gm, gn), N % 4 == 0
 __device__ __forceinline__ void store4(const GemmEpilogue& ep, void* C, int N, int gm, int gn, f32x4 v) {
-    const float rs = ep.scale * (ep.row_scale ? ep.row_scale[gm] : 1.0f);
-    v *= rs;
+    v *= ep.scale * (ep.row_scale ? ep.row_scale[gm] : 1.0f);
     if (ep.col_scale) v *= *reinterpret_cast<const f32x4*>(ep.col_scale + gn);
-    const size_t at = (size_t)gm * N + gn;
-    if (ep.out == 1) {
-        *reinterpret_cast<f32x4*>(static_cast<float*>(C) + at) = v;
-    } else if (ep.out == 2) {
-#pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] = v[x] != v[x] ? v[x] : fminf(fmaxf(v[x], -448.0f), 448.0f);
-        int w = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
-        w = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], w, true);
-        *reinterpret_cast<int*>(static_cast<uint8_t*>(C) + at) = w;
-    } else {
-        st_global_8(static_cast<uint16_t*>(C) + at, u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])});
-    }
+    store_scaled4(ep, C, N, gm, gn, v);
 }
 
 // Consecutive workgroup ids go round-robin to the 8 XCDs; this gives every XCD one contiguous range of logical ids.
