@@ -280,6 +280,21 @@ __global__ __launch_bounds__(C::THREADS, (160 * 1024 / C::LDS) >= 2 ? 2 : 1) voi
 #pragma unroll
     for (int i = 0; i < C::ST; ++i)
         if (i < n_own) issue(i, i);
+    // The epilogue's scales, while the first pieces are on their way: read there, each would cost its latency again (M = 1065,
+    // N = 7136, K = 1024 with both vectors 15.7 us, 14.0 this way, 13.5 without any).  Products of bf16 have no vectors.
+    constexpr int QPR = C::BN / 4, ROW_STEP = C::THREADS / QPR, QUADS = (C::BM + ROW_STEP - 1) / ROW_STEP;
+    static_assert(C::THREADS % QPR == 0, "a lane keeps its columns");
+    const int row0 = t / QPR, col = (t % QPR) * 4;
+    float row_scale[QUADS];
+    f32x4 col_scale{1.0f, 1.0f, 1.0f, 1.0f};
+    if constexpr (ES == 1) {
+#pragma unroll
+        for (int i = 0; i < QUADS; ++i) row_scale[i] = 1.0f;
+        if (ep.row_scale != nullptr)
+#pragma unroll
+            for (int i = 0; i < QUADS; ++i) row_scale[i] = ep.row_scale[min(m0 + row0 + i * ROW_STEP, M - 1)];
+        if (ep.col_scale != nullptr && n0 + col < N) col_scale = *reinterpret_cast<const f32x4*>(ep.col_scale + n0 + col);
+    }
     if constexpr (C::WPG == 1) {
         // the wave's own ring: no barrier.  A stage is refilled as soon as its fragments are in registers.
         Frags f;
@@ -351,18 +366,21 @@ __global__ __launch_bounds__(C::THREADS, (160 * 1024 / C::LDS) >= 2 ? 2 : 1) voi
                     f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
             }
     __syncthreads();
-    constexpr int QPR = C::BN / 4;
-    for (int q = t; q < C::BM * QPR; q += C::THREADS) {
-        const int row = q / QPR, col = (q % QPR) * 4;
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) {
+        const int row = row0 + i * ROW_STEP;
         const int gm = m0 + row, gn = n0 + col;
-        if (gm >= M || gn >= N) continue;
+        if (row >= C::BM || gm >= M || gn >= N) continue;
         f32x4 v = *reinterpret_cast<const f32x4*>(red + (size_t)row * C::RED_PITCH + col);
 #pragma unroll
         for (int k = 1; k < C::KG; ++k) v += *reinterpret_cast<const f32x4*>(red + ((size_t)k * C::BM + row) * C::RED_PITCH + col);
-        if (splits > 1)
+        if (splits > 1) {
             *reinterpret_cast<f32x4*>(part + (((size_t)z * gridDim.y + blockIdx.y) * M + gm) * N + gn) = v;
-        else
-            store4(ep, Cp + (size_t)blockIdx.y * stride_c * (ep.out == 1 ? 4 : ep.out == 2 ? 1 : 2), N, gm, gn, v);
+        } else {
+            if constexpr (ES == 1) v = v * (ep.scale * row_scale[i]) * col_scale;
+            else                   v *= ep.scale;
+            store_scaled4(ep, Cp + (size_t)blockIdx.y * stride_c * (ep.out == 1 ? 4 : ep.out == 2 ? 1 : 2), N, gm, gn, v);
+        }
     }
 }
 
