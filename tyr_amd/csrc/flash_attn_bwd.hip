@@ -968,10 +968,281 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
                                          Hq, window, kv_lens, key_mask, plan, items, partial, ds);
 }
 
+// dK and dV of 64 keys for small launches: waves w and w + 2 own the same 32 keys, one the first and one the second 32 rows of
+// every query tile, and exchange at the end (one finishes dV, the other dK).  Half the work a step and twice the workgroups of
+// bwd_dkv.  The query tiles of all G heads are one run of steps, three requested ahead into a ring of four stages; the pairs
+// of all of them are made first and stay in LDS, so nothing is written that another workgroup reads.  Bound by latencies: a
+// step is 32 products of 32 cycles a wave and takes 1.6 us (1.0 at D = 64), of which the pairs are a third.  Tried: one
+// product, then its share of the other instructions by scheduling groups (4 % slower), pairs a step ahead instead of first (as slow).
+template <int D, bool CAUSAL, AttnMask MASK>
+__device__ __forceinline__ void bwd_dkv_half(int block,
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
+    const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
+    uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int BHkv, int N, float scale, float scale_log2, int Hq, int G, int window, const int* __restrict__ kv_lens, const uint8_t* __restrict__ key_mask) {
+    using namespace fab;
+    using C = CfgK<D>;
+    constexpr bool WINDOW = MASK == AttnMask::Limits, PER_KEY = MASK != AttnMask::None;
+    constexpr int BNK = 64, STAGE = 2 * C::TILE;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int t = threadIdx.x;
+    const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int r = lane & 31, g = lane >> 5, T = w >> 1;
+
+    int bh, kt;                           // causal: key tile 0 meets every query tile, so heavy first
+    if ((BHkv & 7) == 0) {
+        const int slot = block >> 3, heads = BHkv >> 3;
+        bh = slot % heads * 8 + (block & 7);
+        kt = slot / heads;
+    } else {
+        bh = block % BHkv;
+        kt = block / BHkv;
+    }
+    const int n0 = kt * BNK, nw0 = n0 + (w & 1) * 32, kvpos = nw0 + r;
+    const size_t head_off = (size_t)bh * N * D;
+    const int hkv = Hq / G;
+    const size_t qh0 = (size_t)(bh / hkv) * Hq + (size_t)(bh % hkv) * G;
+    const int Nk = (PER_KEY && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / hkv])) : N;
+    bool block_hidden = PER_KEY && n0 >= Nk;
+    if (PER_KEY && key_mask != nullptr && !block_hidden) {
+        const TileSpan span = visible_tiles(key_mask + (size_t)(bh / hkv) * N + n0, min(BNK, Nk - n0), lane);
+        block_hidden = span.first >= span.last;
+    }
+    // query tiles [jq0, jq1) of each head see keys of the block
+    const int nq = (N + C::BQ - 1) / C::BQ, jq0 = CAUSAL ? kt : 0;
+    int jq1 = nq;
+    if (WINDOW && window > 0) jq1 = (int)min((int64_t)nq, ((int64_t)n0 + BNK - 2 + window) / C::BQ + 1);
+    const int per_head = jq1 - jq0, steps = block_hidden ? 0 : G * per_head;
+
+    const uint32_t head_bytes = (uint32_t)N * D * 2u;
+    const u32x4 q_rsrc = make_raw_rsrc(Q + qh0 * N * D, head_bytes * (uint32_t)G);
+    const u32x4 do_rsrc = make_raw_rsrc(dO + qh0 * N * D, head_bytes * (uint32_t)G);
+    constexpr int ROWS_PER_INST = 1024 / C::ROW;
+    int g_voff[C::PT];
+#pragma unroll
+    for (int m = 0; m < C::PT; ++m) {
+        const int row = (w * C::PT + m) * ROWS_PER_INST + lane / C::KCH;
+        g_voff[m] = row * C::ROW + swz<D>(row, lane % C::KCH) * 16 - 1024 * m;   // request m carries 1024 m as its immediate offset
+    }
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
+    const uint32_t wave_dst = __builtin_amdgcn_readfirstlane(lds_base + (uint32_t)w * C::PT * 1024u);
+    // steps past the last one are requested beyond the buffers (zeros, no traffic)
+    struct Place { int hq, jq; };                    // of a step: its head, its query tile
+    auto next = [&](Place& p) {
+        if (++p.jq == jq1) { p.jq = jq0; ++p.hq; }
+    };
+    auto issue_rows = [&](int at, const Place& p) {
+        const uint32_t dst = wave_dst + (uint32_t)(at & (C::NST - 1)) * STAGE;
+        const int soff = at < steps ? p.hq * (int)head_bytes + p.jq * C::BQ * C::ROW : (int)(head_bytes * (uint32_t)G);
+        load_global_to_lds_16xN<C::PT>(q_rsrc, dst, g_voff, soff);
+        load_global_to_lds_16xN<C::PT>(do_rsrc, dst + C::TILE, g_voff, soff);
+    };
+    Place ahead{0, jq0};                             // of the next step to request
+#pragma unroll
+    for (int at = 0; at < 3; ++at) {
+        issue_rows(at, ahead);
+        next(ahead);
+    }
+    bf16x8 kf[C::KSTEPS], vf[C::KSTEPS];
+    {
+        const size_t off = head_off + (size_t)min(kvpos, N - 1) * D + g * 8;
+#pragma unroll
+        for (int i = 0; i < C::KSTEPS; ++i) {
+            kf[i] = __builtin_bit_cast(bf16x8, ld_global_16(Kp + off + i * 16));
+            vf[i] = __builtin_bit_cast(bf16x8, ld_global_16(Vp + off + i * 16));
+        }
+    }
+    // The (lse2, delta = dO . O) pairs of all steps, in LDS behind the stages.  A row is 16 bytes a lane of D / 8 adjacent lanes and
+    // the loads of four tiles are in flight.  (A row a lane, as the products want them, and through memory, as bwd_dkv makes them:
+    // 1 us a tile, as much as its step.)
+    float2* pairs = reinterpret_cast<float2*>(lds + C::NST * STAGE);
+    {
+        constexpr int LPR = D / 8, ROWS = THREADS / LPR, PASSES = C::BQ / ROWS, TILES = 4;
+        const int row = t / LPR, c = t % LPR;
+        Place p{0, jq0};
+        for (int s0 = 0; s0 < steps; s0 += TILES) {
+            u32x4 o[TILES][PASSES], d[TILES][PASSES];
+            float lse[TILES][PASSES];
+            int qpos[TILES];
+#pragma unroll
+            for (int i = 0; i < TILES; ++i)
+                if (s0 + i < steps) {
+                    qpos[i] = p.jq * C::BQ + row;
+#pragma unroll
+                    for (int k = 0; k < PASSES; ++k) {
+                        const size_t at = (qh0 + p.hq) * N + min(qpos[i] + k * ROWS, N - 1);
+                        o[i][k] = ld_global_16(O + at * D + c * 8);
+                        d[i][k] = ld_global_16(dO + at * D + c * 8);
+                        lse[i][k] = LSE[at];
+                    }
+                    next(p);
+                }
+#pragma unroll
+            for (int i = 0; i < TILES; ++i)
+                if (s0 + i < steps) {
+#pragma unroll
+                    for (int k = 0; k < PASSES; ++k) {
+                        float delta = dot8_bf16(d[i][k], o[i][k]);
+                        // lanes xor 1, xor 2, then the mirrored half row and row: sums of 4, 8 and 16 lanes
+                        auto add = [&](auto ctrl) {
+                            delta += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, delta), decltype(ctrl)::value, 0xf, 0xf, true));
+                        };
+                        add(std::integral_constant<int, 0xb1>{});
+                        add(std::integral_constant<int, 0x4e>{});
+                        add(std::integral_constant<int, 0x141>{});
+                        if (LPR == 16) add(std::integral_constant<int, 0x140>{});
+                        float lse2 = lse[i][k] * LOG2E;
+                        if (MASK != AttnMask::None && lse2 == -INFINITY) lse2 = INFINITY;    // a row that saw no key: every probability is 0
+                        if (c == 0) pairs[(s0 + i) * C::BQ + row + k * ROWS] = qpos[i] + k * ROWS < N ? make_float2(lse2, delta) : make_float2(INFINITY, 0.0f);
+                    }
+                }
+        }
+    }
+    Place now{0, jq0};
+#pragma unroll
+    for (int i = 0; i < C::KSTEPS; ++i) { pin_registers(kf[i]); pin_registers(vf[i]); }
+    wait_vmcnt0();
+    __syncthreads();
+
+    // fragment addresses inside a stage, of this wave's 32 rows
+    int row_off[C::KSTEPS], tr_lo[C::DT], tr_hi[C::DT];
+#pragma unroll
+    for (int i = 0; i < C::KSTEPS; ++i) row_off[i] = (32 * T + r) * C::ROW + swz<D>(r, 2 * i + g) * 16;
+    {
+        const int i16 = lane & 15, b16 = lane >> 4, row = 4 * (b16 >> 1) + (i16 >> 2);
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt) {
+            const int dcol = 32 * dt + 16 * (b16 & 1) + 4 * (i16 & 3);
+            tr_lo[dt] = (32 * T + row) * C::ROW + swz<D>(row, dcol >> 3) * 16 + (dcol & 7) * 2;
+            tr_hi[dt] = (32 * T + row + 8) * C::ROW + swz<D>(row + 8, dcol >> 3) * 16 + (dcol & 7) * 2;
+        }
+    }
+    f32x16 dk[C::DT], dv[C::DT];
+#pragma unroll
+    for (int i = 0; i < C::DT; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) { dk[i][e] = 0.0f; dv[i][e] = 0.0f; }
+
+    auto scores = [&](int at, f32x16& s, f32x16& dp) {
+        const unsigned char* St = lds + (at & (C::NST - 1)) * STAGE;
+        bf16x8 qa[C::KSTEPS], da[C::KSTEPS];
+#pragma unroll
+        for (int i = 0; i < C::KSTEPS; ++i) {
+            qa[i] = *reinterpret_cast<const bf16x8*>(St + row_off[i]);
+            da[i] = *reinterpret_cast<const bf16x8*>(St + C::TILE + row_off[i]);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < C::KSTEPS; ++i) {
+            s = mfma_32x32x16_bf16(qa[i], kf[i], s);
+            dp = mfma_32x32x16_bf16(da[i], vf[i], dp);
+        }
+    };
+    // The products of the next step's scores stand beside this step's exponentials: tile at + 1 is awaited a step early.
+    auto step = [&](int at, const f32x16& s, const f32x16& dp, f32x16& s_next, f32x16& dp_next) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * C::PT) : "memory");
+        __syncthreads();
+        issue_rows(at + 3, ahead);                   // into the stage of the step before
+        next(ahead);
+        const int qs0 = now.jq * C::BQ + 32 * T;
+        next(now);
+        const unsigned char* St = lds + (at & (C::NST - 1)) * STAGE;
+        // register e of a product <-> query row qs0 + 8 (e / 4) + 4 g + e % 4
+        f32x4 pair[8];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float2* p = pairs + at * C::BQ + 32 * T + 4 * g + 8 * k;
+            pair[2 * k] = *reinterpret_cast<const f32x4*>(p);
+            pair[2 * k + 1] = *reinterpret_cast<const f32x4*>(p + 2);
+        }
+        scores(at + 1, s_next, dp_next);
+        bf16x8 dot[2][C::DT], qt[2][C::DT];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt) {
+                const unsigned char* lo = St + tr_lo[dt] + c * 16 * C::ROW;
+                const unsigned char* hi = St + tr_hi[dt] + c * 16 * C::ROW;
+                dot[c][dt] = __builtin_shufflevector(ds_read_tr16(lo + C::TILE), ds_read_tr16(hi + C::TILE), 0, 1, 2, 3, 4, 5, 6, 7);
+                qt[c][dt] = __builtin_shufflevector(ds_read_tr16(lo), ds_read_tr16(hi), 0, 1, 2, 3, 4, 5, 6, 7);
+            }
+        // selected, not branched over: a branch would end the block that the products and this are interleaved in
+        const int row_lo = CAUSAL && qs0 < nw0 + 32 ? kvpos - qs0 - 4 * g : INT_MIN;                 // rows below are hidden
+        const int row_hi = WINDOW && window > 0 && qs0 + 31 - nw0 >= window ? kvpos + window - qs0 - 4 * g : INT_MAX;       // and from here on
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            u32x4 ppk, dpk;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int k = 2 * c + h;
+                float p[4], ds[4];
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    p[x] = fast_exp2(fmaf(s[4 * k + x], scale_log2, -pair[2 * k + x / 2][2 * (x & 1)]));
+                    if (CAUSAL) p[x] = 8 * k + x < row_lo ? 0.0f : p[x];
+                    if (WINDOW) p[x] = 8 * k + x >= row_hi ? 0.0f : p[x];
+                    ds[x] = p[x] * (dp[4 * k + x] - pair[2 * k + x / 2][2 * (x & 1) + 1]);
+                }
+                ppk[2 * h] = pack_bf16(p[0], p[1]);
+                ppk[2 * h + 1] = pack_bf16(p[2], p[3]);
+                dpk[2 * h] = pack_bf16(ds[0], ds[1]);
+                dpk[2 * h + 1] = pack_bf16(ds[2], ds[3]);
+            }
+            const bf16x8 pf = __builtin_bit_cast(bf16x8, ppk), dsf = __builtin_bit_cast(bf16x8, dpk);
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt) {
+                dv[dt] = mfma_32x32x16_bf16(dot[c][dt], pf, dv[dt]);
+                dk[dt] = mfma_32x32x16_bf16(qt[c][dt], dsf, dk[dt]);
+            }
+        }
+    };
+    f32x16 sA, dpA, sB, dpB;
+    if (steps > 0) scores(0, sA, dpA);
+    for (int at = 0; at < steps; at += 2) {
+        step(at, sA, dpA, sB, dpB);
+        if (at + 1 < steps) step(at + 1, sB, dpB, sA, dpA);
+    }
+    wait_vmcnt0();
+    __syncthreads();                                 // the stages are free
+    if constexpr (PER_KEY) {
+        if (kvpos >= Nk || (key_mask != nullptr && key_mask[(size_t)(bh / hkv) * N + min(kvpos, N - 1)] == 0)) {
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) dv[dt][e] = dk[dt][e] = 0.0f;
+        }
+    }
+    // waves 0, 1 give dK away and finish dV, waves 2, 3 the other way round
+    f32x4* give = reinterpret_cast<f32x4*>(lds) + w * (C::DT * 4 * 64) + lane;
+    const f32x4* take = reinterpret_cast<const f32x4*>(lds) + (w ^ 2) * (C::DT * 4 * 64) + lane;
+    unsigned char* scratch = lds + 4 * C::DT * 4 * 64 * 16 + w * (32 * (D * 2 + 16));
+    static_assert(4 * C::DT * 4 * 64 * 16 + 4 * 32 * (D * 2 + 16) <= C::NST * STAGE, "exchange and transposition");
+    auto hand_over = [&](const f32x16 (&v)[C::DT]) {
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) give[(dt * 4 + q4) * 64] = f32x4{v[dt][4 * q4], v[dt][4 * q4 + 1], v[dt][4 * q4 + 2], v[dt][4 * q4 + 3]};
+    };
+    auto finish = [&](f32x16 (&v)[C::DT], float mul, uint16_t* out) {
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+                const f32x4 other = take[(dt * 4 + q4) * 64];
+#pragma unroll
+                for (int x = 0; x < 4; ++x) v[dt][4 * q4 + x] += other[x];
+            }
+        store_transposed_bf16<D>(v, mul, scratch, out + head_off + (size_t)nw0 * D, N - nw0, lane);
+    };
+    if (T == 0) hand_over(dk); else hand_over(dv);
+    __syncthreads();
+    if (T == 0) finish(dv, 1.0f, dV); else finish(dk, scale, dK);
+}
+
 // Both at once for launches that leave CUs idle anyway (rule at one_launch): the first `ndkv` workgroups are dK/dV's, the
-// rest dQ's (64-row form).  The dQ kernel then need not end before dK/dV starts -- a launch, a prologue and a drain, 3.5 us
+// rest dQ's (64-row form).  HALF: dK/dV by bwd_dkv_half (rule at half_steps).  The dQ kernel then need not end before dK/dV starts -- a launch, a prologue and a drain, 3.5 us
 // of 11 for one head of 128 rows, 12 of 41 for 8 heads of 700.
-template <int D, bool CAUSAL, AttnMask MASK, bool CUT>
+template <int D, bool CAUSAL, AttnMask MASK, bool CUT, bool HALF>
 __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_both_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
@@ -979,7 +1250,10 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_both_kernel(
     int ntk, int npad, float scale, float scale_log2, int Hq, int window, const int* __restrict__ kv_lens,
     const uint8_t* __restrict__ key_mask, int single, fab::Parts plan, int items, float* __restrict__ partial, int ndkv) {
     const int at = blockIdx.x;
-    if (at < ndkv) {
+    if (HALF && at < ndkv) {
+        bwd_dkv_half<D, CAUSAL, MASK>(at, Q, Kp, Vp, O, dO, LSE, dK, dV, BH / plan.G, N, scale, scale_log2, Hq, plan.G,
+                                      window, kv_lens, key_mask);
+    } else if (at < ndkv) {
         bwd_dkv<D, CAUSAL, MASK, CUT, true, false>(at, Q, Kp, Vp, O, dO, LSE, stats, dK, dV, BH / plan.G, N, ntk, npad, scale, scale_log2, Hq,
                                          window, kv_lens, key_mask, plan, items, partial, nullptr);
     } else {
@@ -1275,6 +1549,27 @@ int dkv_items(const fab::Parts& p, int N) {
 bool one_launch(int N, int64_t blocks, bool ds, bool causal) {
     return blocks <= 256 || (N <= 1024 && blocks <= (!ds ? 640 : causal ? 420 : 300));
 }
+// Steps of the longest 64-key tile of a launch that takes bwd_dkv_half, 0 = the launch does not.  One launch, no scratch, half
+// the steps' length; against bwd_dkv a workgroup has twice the parts of a query's K / V to itself and the queries are read
+// twice as often, so it is for tiles of few steps, and with G > 1 (all heads of the group are one tile's steps) for fewer.
+// Measured (us, whole backward, before -> with): D = 128 B2 H16 N218 18.4 -> 14.6, B3 H8 N473 28.1 -> 21.3, B1 H8 N700 full 41.7
+// -> 25.6, B3 H4 N231 window 83 21.7 -> 13.0, B10 H1 N763 34.2 -> 28.0, B5 Hq32 Hkv8 N83 window 65 35.0 -> 22.4; D = 64 B1 H1
+// N128 7.7 -> 6.3, B2 H16 N218 13.5 -> 9.1, B14 H4 N448 19.3 -> 13.3.  On the other side: D = 128 B1 H1 N1024 24.3 -> 33.1 (16
+// steps on 32 workgroups, which parts share better), B2 H4 N1204 full 41.9 -> 47.8, B6 H16 N116 15.4 -> 16.8 (one 128-key tile
+// a head), B1 Hq8 Hkv2 N300 20.2 -> 39.8.  On 432 shapes of up to 1600 workgroups the choice is 0.8 % slower than the best.
+int half_steps(int BH, int BHkv, int N, int D, bool causal, int window) {
+    const int G = BH / BHkv, nq = (N + 63) / 64;
+    const int64_t blocks = (int64_t)(BH + BHkv) * nq;
+    const int seen = causal && window > 0 ? (int)std::min<int64_t>(nq, ((int64_t)window + 62) / 64 + 1) : nq;
+    const int64_t most = (int64_t)G * seen;
+    bool take;
+    if (G > 1) take = blocks <= 1600 && most <= (D == 128 ? (blocks <= 256 ? 4 : 12) : (blocks <= 256 ? 8 : 16));
+    else if (N <= 128) take = blocks <= (D == 128 ? 256 : 400);
+    else if (D == 128) take = blocks <= 400 && most <= std::min<int64_t>(15, std::max<int64_t>(6, blocks / 16));
+    else take = blocks <= 512 && most <= (blocks <= 40 ? 10 : 32);
+    return take ? (int)most : 0;
+}
+size_t half_lds(int D, int steps) { return (size_t)4 * 2 * 64 * D * 2 + (size_t)steps * 64 * sizeof(float2); }
 size_t dkv_partial_bytes(const fab::Parts& p, int BHkv, int N, int D) {
     return p.chunk ? (size_t)BHkv * dkv_items(p, N) * 128 * D * 8 : 0;
 }
@@ -1301,18 +1596,20 @@ struct BwdPlan {
     int items;
     int64_t dq_blocks, dkv_blocks;                   // dq_blocks: of the 64-row form, beside dK/dV's in one launch
     bool both, ds;
+    int half;                                        // half_steps
     size_t stat_bytes, partial_bytes, ds_bytes;
     size_t bytes() const { return stat_bytes + partial_bytes + ds_bytes; }
 };
 BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int D, bool causal, int window, bool least) {
     BwdPlan p;
-    p.parts = dkv_plan(B * Hkv, Hq / Hkv, N, D, causal, window);
+    p.half = half_steps(B * Hq, B * Hkv, N, D, causal, window);
+    p.parts = p.half ? fab::Parts{Hq / Hkv, (N + 63) / 64, causal, window, 0} : dkv_plan(B * Hkv, Hq / Hkv, N, D, causal, window);
     if (least) p.parts.chunk = 0;
     p.items = dkv_items(p.parts, N);
     p.dq_blocks = (int64_t)B * Hq * ((N + 63) / 64);
-    p.dkv_blocks = (int64_t)B * Hkv * p.items;
-    const bool ds = !least && keeps_ds(B * Hq, Hq / Hkv, N, D, causal, window);
-    p.both = one_launch(N, p.dq_blocks + p.dkv_blocks, ds, causal);
+    p.dkv_blocks = (int64_t)B * Hkv * (p.half ? (N + 63) / 64 : p.items);
+    const bool ds = !p.half && !least && keeps_ds(B * Hq, Hq / Hkv, N, D, causal, window);
+    p.both = p.half || one_launch(N, p.dq_blocks + p.dkv_blocks, ds, causal);
     p.ds = ds && !p.both;
     p.stat_bytes = flash_attn_bwd_workspace_bytes(B, Hq, N);
     p.partial_bytes = dkv_partial_bytes(p.parts, B * Hkv, N, D);
@@ -1393,22 +1690,23 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
 #define TYR_FAB_SUM(DD)                                                                               \
     launch_kernel(flash_attn_bwd_sum_kernel<DD>, dim3((unsigned)(BHkv * ntk * (DD / 8))), dim3(256), 0, stream, \
                        partial, static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), N, ntk, items, scale, plan)
-#define TYR_FAB_BOTH(DD, CC, EE, UU)                                                                  \
+#define TYR_FAB_BOTH(DD, CC, EE, UU, HH)                                                               \
     do {                                                                                              \
         static const hipError_t a3 = hipFuncSetAttribute(                                             \
-            reinterpret_cast<const void*>(&flash_attn_bwd_both_kernel<DD, CC, EE, UU>),               \
-            hipFuncAttributeMaxDynamicSharedMemorySize, CfgK<DD>::LDS);                               \
+            reinterpret_cast<const void*>(&flash_attn_bwd_both_kernel<DD, CC, EE, UU, HH>),               \
+            hipFuncAttributeMaxDynamicSharedMemorySize, HH ? 160 * 1024 : CfgK<DD>::LDS);                               \
         if (a3 != hipSuccess) return -1;                                                              \
-        launch_kernel((flash_attn_bwd_both_kernel<DD, CC, EE, UU>), dim3(grid_k.x + (unsigned)how.dq_blocks), block, CfgK<DD>::LDS, \
+        launch_kernel((flash_attn_bwd_both_kernel<DD, CC, EE, UU, HH>), dim3((unsigned)(how.dkv_blocks + how.dq_blocks)), block, HH ? half_lds(DD, how.half) : CfgK<DD>::LDS, \
                            stream, Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st,          \
                            static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), BH, N, (N + 63) / 64, ntk, \
-                           npad, scale, scale_log2, Hq, window, kv_lens, key_mask, causal && window <= 0, plan, items, partial, (int)grid_k.x); \
+                           npad, scale, scale_log2, Hq, window, kv_lens, key_mask, causal && window <= 0, plan, items, partial, (int)how.dkv_blocks); \
     } while (0)
 #define TYR_FAB_LAUNCH(DD, CC, EE)                                                                    \
     do {                                                                                              \
         if (how.both) {                                                                               \
-            if (!plan.chunk) { TYR_FAB_BOTH(DD, CC, EE, false); break; }                              \
-            TYR_FAB_BOTH(DD, CC, EE, true);                                                           \
+            if (how.half) { TYR_FAB_BOTH(DD, CC, EE, false, true); break; }                           \
+            if (!plan.chunk) { TYR_FAB_BOTH(DD, CC, EE, false, false); break; }                       \
+            TYR_FAB_BOTH(DD, CC, EE, true, false);                                                    \
             TYR_FAB_SUM(DD);                                                                          \
             break;                                                                                    \
         }                                                                                             \
