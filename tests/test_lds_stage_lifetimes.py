@@ -302,6 +302,37 @@ def test_a_dkv_wait_that_left_one_more_in_flight_would_be_caught():
     assert not all(all(dkv_waits(9, w, with_stores=18)) for w in range(4))
 
 
+def dkv_half_wave(steps, stages=4):
+    """64-key tiles: T0..T3 hold Q and dO of 64 query rows, three requested ahead (zeros past the last).  Step t reads the row
+    fragments of tile t+1 and the transposed ones of tile t; the exchange and the output go through the stages."""
+    t = Trace()
+    for k in range(3):
+        t.dma(f"T{k}", k)
+    t.wait()
+    t.bar()
+    if steps:
+        t.read("T0", 0)
+    for i in range(steps):
+        t.wait(keep_newest=1)
+        t.bar()
+        t.dma(f"T{(i + 3) % stages}", i + 3)
+        t.read(f"T{(i + 1) % stages}", i + 1)
+        t.read(f"T{i % stages}", i)
+    t.wait()
+    t.bar()
+    for s in range(stages):
+        t.store(f"T{s}", "dKdV")
+    t.bar()
+    for s in range(stages):
+        t.read(f"T{s}", "dKdV")
+    return t
+
+
+@pytest.mark.parametrize("steps", [0, 1, 2, 3, 4, 5, 12, 32])
+def test_backward_of_64_key_tiles(steps):
+    assert violations([dkv_half_wave(steps) for _ in range(4)]) == []
+
+
 # ------------------------------------------------------------------ flash_attn_bwd_dq_product_kernel
 def dq_product_wave(n, wave, causal=True, stages=5):
     """Stages S0..S4 (32 keys of dS and K), four in flight; stages past the last are requested as well (zeros).  A causal wave
