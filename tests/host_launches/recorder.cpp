@@ -1,0 +1,68 @@
+// A HIP runtime that launches nothing, for the host code of the library on a machine without a GPU: one line of stdin is one call
+// of the C ABI, one line of stdout its result and the kernels it would launch, in order.
+//   bytes B Hq Hkv N D causal window          scratch of the backward: least and full
+//   bwd   B Hq Hkv N D causal window mask ws  status, then "kernel<arguments>:workgroups" each; mask = none | lens | keys
+#include <cxxabi.h>
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <iostream>
+#include <map>
+#include <sstream>
+#include <string>
+
+#include "../../include/tyr_hip.h"
+
+static std::map<const void*, std::string>& kernels() {
+    static std::map<const void*, std::string> m;
+    return m;
+}
+static std::string launched;
+
+extern "C" {
+void** __hipRegisterFatBinary(const void*) { return nullptr; }
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {
+    int bad = 0;
+    char* plain = abi::__cxa_demangle(name, nullptr, nullptr, &bad);
+    std::string s = bad ? name : plain;
+    free(plain);
+    s = s.substr(0, s.find(">(") == std::string::npos ? s.find('(') : s.find(">(") + 1);
+    for (const char* drop : {"void ", "tyr::", "(AttnMask)", " "})
+        for (size_t at; (at = s.find(drop)) != std::string::npos;) s.erase(at, std::string(drop).size());
+    kernels()[host] = s;
+}
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void**, size_t, hipStream_t) {
+    launched += " " + kernels()[f] + ":" + std::to_string(grid.x);
+    return hipSuccess;
+}
+}
+
+int main() {
+    alignas(16) static char p[16];               // stands for every tensor: nothing reads them
+    float* f = reinterpret_cast<float*>(p);
+    for (std::string line; std::getline(std::cin, line);) {
+        std::istringstream in(line);
+        std::string what, mask;
+        uint64_t B, Hq, Hkv, N, D, window;
+        int causal;
+        size_t ws = 0;
+        in >> what >> B >> Hq >> Hkv >> N >> D >> causal >> window >> mask >> ws;
+        launched.clear();
+        if (what == "bytes") {
+            printf("%zu %zu\n", tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D),
+                   tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window));
+        } else {
+            const int rc = mask == "keys" ? tyr_hip_flash_attn_bwd_mask(p, p, p, p, p, f, p, p, p, B, Hq, Hkv, N, D, causal, reinterpret_cast<uint8_t*>(p),
+                                                                        0.125f, p, ws, nullptr)
+                                          : tyr_hip_flash_attn_bwd_gqa(p, p, p, p, p, f, p, p, p, B, Hq, Hkv, N, D, causal, window,
+                                                                       mask == "lens" ? reinterpret_cast<int32_t*>(p) : nullptr, 0.125f, p, ws, nullptr);
+            printf("%d%s\n", rc, launched.c_str());
+        }
+        fflush(stdout);
+    }
+}

@@ -1,0 +1,50 @@
+"""What the C ABI's host code decides, on the CPU: the kernel files are compiled for the host alone, with every signed overflow
+an abort, and linked with a HIP runtime that records the launches instead of making them (tests/host_launches)."""
+import os
+import subprocess
+from concurrent.futures import ThreadPoolExecutor
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CHECKED = ["-Xarch_host", "-fsanitize=signed-integer-overflow", "-Xarch_host", "-fsanitize-minimal-runtime", "-Xarch_host",
+           "-fno-sanitize-recover=signed-integer-overflow"]
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("host")
+    hipcc = "/opt/rocm/bin/hipcc"
+
+    def compile_(name):
+        obj = str(tmp / (os.path.basename(name) + ".o"))
+        subprocess.check_call([hipcc, "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17", "-w", *CHECKED, "-c",
+                               os.path.join(ROOT, name), "-o", obj])
+        return obj
+    with ThreadPoolExecutor() as pool:
+        objs = list(pool.map(compile_, ["tyr_amd/csrc/capi.hip", "tyr_amd/csrc/flash_attn_fwd.hip", "tyr_amd/csrc/flash_attn_bwd.hip"]))
+    main, exe = str(tmp / "recorder.o"), str(tmp / "recorder")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-isystem", "/opt/rocm/include", "-c",
+                           os.path.join(ROOT, "tests", "host_launches", "recorder.cpp"), "-o", main])
+    # what the other kernel files and the fat binaries would define is never reached
+    subprocess.check_call(["/opt/rocm/llvm/bin/clang++", main, *objs, "-fsanitize=signed-integer-overflow", "-fsanitize-minimal-runtime",
+                           "-Wl,--unresolved-symbols=ignore-all", "-o", exe])
+
+    def run(lines):
+        r = subprocess.run([exe], input="\n".join(lines) + "\n", capture_output=True, text=True)
+        got = r.stdout.splitlines()
+        assert r.returncode == 0 and len(got) == len(lines), (lines[min(len(got), len(lines) - 1)], r.returncode, r.stderr[-300:])
+        return got
+    return run
+
+
+def test_a_window_of_any_size_is_one_of_all_rows(ask):
+    """The sums that the plan and the places of dS make with a window stay in 32 bits: the last 126 values below 2^31 did not."""
+    for B, Hq, Hkv, N in ((1, 32, 8, 2000), (4, 16, 16, 769), (9, 16, 4, 200), (2, 4, 4, 100), (16, 16, 16, 4096)):
+        whole = None
+        for window in (N, N + 1, 2 ** 30, 2 ** 31 - 127, 2 ** 31 - 126, 2 ** 31 - 1, 2 ** 31, 2 ** 64 - 1):
+            size, = ask([f"bytes {B} {Hq} {Hkv} {N} 128 1 {window}"])
+            ws = int(size.split()[1])
+            got = [size] + ask([f"bwd {B} {Hq} {Hkv} {N} 128 1 {window} {mask} {w}" for mask in ("none", "lens") for w in (ws, int(size.split()[0]))])
+            whole = whole or got
+            assert got == whole and got[1].startswith("0 flash_attn_bwd"), (window, got, whole)

@@ -19,6 +19,8 @@ namespace {
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline bool fits_int(uint64_t v) { return v <= (uint64_t)INT_MAX; }
+// A window of all `rows` hides nothing that a larger one does not, and leaves the sums that plans and kernels make with it in 32 bits.
+inline int window_rows(uint64_t window, uint64_t rows) { return (int)std::min(window, rows); }
 
 constexpr uint64_t kMaxSplits = 64;
 
@@ -189,7 +191,7 @@ static int attn_fwd_checked(const void* q, const void* k, const void* v, void* o
     if (lse && (reinterpret_cast<uintptr_t>(lse) & 3u)) return TYR_HIP_ERR_MISALIGNED;
     if (kv_lens && (reinterpret_cast<uintptr_t>(kv_lens) & 3u)) return TYR_HIP_ERR_MISALIGNED;
     const int rc = tyr::launch_flash_attn_fwd(q, k, v, o, lse, (int)B, (int)Hq, (int)Hkv, (int)N, (int)D,
-                                              causal != 0, (int)(window > (uint64_t)INT_MAX ? INT_MAX : window),
+                                              causal != 0, window_rows(window, N),
                                               kv_lens, key_mask, scale, static_cast<hipStream_t>(stream));
     return rc == 0 ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }
@@ -219,7 +221,7 @@ size_t tyr_hip_flash_attn_bwd_full_workspace_bytes(uint64_t B, uint64_t Hq, uint
     if (B == 0 || Hq == 0 || Hkv == 0 || N == 0 || Hq % Hkv != 0 || (D != 64 && D != 128)) return 0;
     if (!fits_int(N) || !fits_int(B * Hq) || B * Hq > (uint64_t)INT_MAX / ((N + 127) / 128)) return 0;
     return tyr::flash_attn_bwd_full_workspace_bytes((int)B, (int)Hq, (int)Hkv, (int)N, (int)D, causal != 0,
-                                                    (int)(window > (uint64_t)INT_MAX ? INT_MAX : window));
+                                                    window_rows(window, N));
 }
 
 int tyr_hip_flash_attn_bwd(const void* q, const void* k, const void* v, const void* o,
@@ -254,7 +256,7 @@ static int attn_bwd_checked(const void* q, const void* k, const void* v, const v
     if (!aligned16(workspace)) return TYR_HIP_ERR_MISALIGNED;
     const int rc = tyr::launch_flash_attn_bwd(q, k, v, o, d_o, lse, dq, dk, dv, (int)B, (int)Hq, (int)Hkv, (int)N,
                                               (int)D, causal != 0,
-                                              (int)(window > (uint64_t)INT_MAX ? INT_MAX : window), kv_lens, key_mask,
+                                              window_rows(window, N), kv_lens, key_mask,
                                               scale, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
     return rc == 0 ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }
@@ -318,7 +320,7 @@ int tyr_hip_gqa_decode_varlen(const void* q, const void* k, const void* v, void*
     if (!aligned16(workspace)) return TYR_HIP_ERR_MISALIGNED;
     const int rc = tyr::launch_gqa_decode(q, k, v, o, lse, (int)B, (int)Hq, (int)Hkv, (int)L, (int)D,
                                           (int64_t)kv_stride, scale, (int)num_splits, workspace, kv_lens,
-                                          (int)(window > (uint64_t)INT_MAX ? INT_MAX : window),
+                                          window_rows(window, L),
                                           static_cast<hipStream_t>(stream));
     return rc == 0 ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;
 }

@@ -443,7 +443,7 @@ struct Parts {
 // blocks of 128 query rows are adjacent, ordered by key and then by query row: what a dQ workgroup reads is one stream.
 // Only blocks that the causal rule or a window lets be visible have a place.
 struct DsBlocks {
-    int ntk, causal, window;                         // ntk = tiles of 128 rows (of queries and of keys)
+    int ntk, causal, window;                         // ntk = tiles of 128 rows (of queries and of keys); window <= rows
     __host__ __device__ int width() const {          // key tiles that have a place for a query tile (causal without a window: qt + 1)
         const int w = causal && window > 0 ? (window - 1 + 127) / 128 + 1 : ntk;
         return w < ntk ? w : ntk;
