@@ -48,3 +48,16 @@ def test_a_window_of_any_size_is_one_of_all_rows(ask):
             got = [size] + ask([f"bwd {B} {Hq} {Hkv} {N} 128 1 {window} {mask} {w}" for mask in ("none", "lens") for w in (ws, int(size.split()[0]))])
             whole = whole or got
             assert got == whole and got[1].startswith("0 flash_attn_bwd"), (window, got, whole)
+
+
+def test_scratch_queries_take_any_length(ask):
+    """Beyond the lengths a call accepts, the largest scratch is 0 (nothing uses it); no query overflows."""
+    for N in (2 ** 22, 2 ** 23 - 1, 2 ** 23, 2 ** 25, 2 ** 30, 2 ** 31 - 129, 2 ** 31 - 127, 2 ** 31 - 1, 2 ** 31, 2 ** 40):
+        for window in (0, 1, 2 ** 31 - 1, 2 ** 40):
+            for D in (64, 128):
+                got, = ask([f"bytes 1 1 1 {N} {D} 1 {window}"])
+                least, full = map(int, got.split())
+                assert least == (0 if N >= 2 ** 31 else (N + 127) // 128 * 1024)
+                assert (full == 0) if N * D * 2 >= 2 ** 31 else full >= least
+                call, = ask([f"bwd 1 1 1 {N} {D} 1 {window} none {least}"])
+                assert (call == "-3" if N < 2 ** 31 else call == "-2") if full == 0 else call.startswith("0 flash_attn_bwd")

@@ -216,10 +216,14 @@ size_t tyr_hip_flash_attn_bwd_workspace_bytes(uint64_t B, uint64_t H, uint64_t N
     return tyr::flash_attn_bwd_workspace_bytes((int)B, (int)H, (int)N);
 }
 
+// the backward's 32-bit offsets inside the G query heads of one kv head (and inside their pairs)
+static bool heads_fit(uint64_t G, uint64_t N, uint64_t D) { return G * N * D * 2 < ((uint64_t)1 << 31); }
+
 size_t tyr_hip_flash_attn_bwd_full_workspace_bytes(uint64_t B, uint64_t Hq, uint64_t Hkv, uint64_t N, uint64_t D, int causal,
                                                    uint64_t window) {
     if (B == 0 || Hq == 0 || Hkv == 0 || N == 0 || Hq % Hkv != 0 || (D != 64 && D != 128)) return 0;
     if (!fits_int(N) || !fits_int(B * Hq) || B * Hq > (uint64_t)INT_MAX / ((N + 127) / 128)) return 0;
+    if (!heads_fit(Hq / Hkv, N, D)) return 0;
     return tyr::flash_attn_bwd_full_workspace_bytes((int)B, (int)Hq, (int)Hkv, (int)N, (int)D, causal != 0,
                                                     window_rows(window, N));
 }
@@ -244,8 +248,7 @@ static int attn_bwd_checked(const void* q, const void* k, const void* v, const v
     if (!(scale > 0.0f) || scale > 3.0e38f) return TYR_HIP_ERR_UNSUPPORTED;
     if (!fits_int(N) || !fits_int(B * Hq) || B * Hq > (uint64_t)INT_MAX / ((N + 127) / 128))
         return TYR_HIP_ERR_BAD_SHAPE;
-    // 32-bit offsets inside the G query heads of one kv head (and inside their pairs)
-    if ((Hq / Hkv) * N * D * 2 >= ((uint64_t)1 << 31)) return TYR_HIP_ERR_UNSUPPORTED;
+    if (!heads_fit(Hq / Hkv, N, D)) return TYR_HIP_ERR_UNSUPPORTED;
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o) || !aligned16(d_o) ||
         !aligned16(dq) || !aligned16(dk) || !aligned16(dv))
         return TYR_HIP_ERR_MISALIGNED;

@@ -1445,7 +1445,7 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_product_ker
 }
 
 size_t flash_attn_bwd_workspace_bytes(int B, int H, int N) {
-    const size_t npad = (size_t)((N + 127) / 128) * 128;
+    const size_t npad = ((size_t)N + 127) / 128 * 128;
     return (size_t)B * H * npad * sizeof(float2);
 }
 
