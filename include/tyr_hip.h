@@ -206,10 +206,13 @@ int tyr_hip_flash_attn_bwd_gqa(const void* q, const void* k, const void* v, cons
                                void* workspace, size_t workspace_bytes, void* stream);
 
 /* Workspace with which the call is fastest.  dK / dV of few (or, causal, very unequal) key tiles leave most of the device
- * idle; with this much scratch their work is cut over more workgroups whose f32 partial sums a last kernel adds.  For few
- * heads (D = 128) it also holds dS in bf16, at most 288 MiB, from which dQ is one product instead of three.  Anything between
- * tyr_hip_flash_attn_bwd_workspace_bytes and this is accepted and runs as with the minimum.  Same bytes with a key mask
- * (window = 0).  Results are reproducible either way and agree to the rounding of f32 sums. */
+ * idle; with tyr_hip_flash_attn_bwd_parts_workspace_bytes their work is cut over more workgroups whose f32 partial sums a last
+ * kernel adds.  For few heads (D = 128) tyr_hip_flash_attn_bwd_full_workspace_bytes also holds dS in bf16, at most 288 MiB, from
+ * which dQ is one product instead of three.  A call runs the fastest of the three forms that its workspace is large enough for.
+ * Same bytes with a key mask (window = 0); 0 = sizes that every call refuses.  Results are reproducible in each form and agree
+ * to the rounding of f32 sums between them. */
+size_t tyr_hip_flash_attn_bwd_parts_workspace_bytes(uint64_t B, uint64_t Hq, uint64_t Hkv, uint64_t N, uint64_t D, int causal,
+                                                    uint64_t window);
 size_t tyr_hip_flash_attn_bwd_full_workspace_bytes(uint64_t B, uint64_t Hq, uint64_t Hkv, uint64_t N, uint64_t D, int causal,
                                                    uint64_t window);
 

@@ -1,6 +1,6 @@
 // A HIP runtime that launches nothing, for the host code of the library on a machine without a GPU: one line of stdin is one call
 // of the C ABI, one line of stdout its result and the kernels it would launch, in order.
-//   bytes B Hq Hkv N D causal window          scratch of the backward: least and full
+//   bytes B Hq Hkv N D causal window          scratch of the backward: least, with parts, full
 //   bwd   B Hq Hkv N D causal window mask ws  status, then "kernel<arguments>:workgroups" each; mask = none | lens | keys
 #include <cxxabi.h>
 #include <hip/hip_runtime_api.h>
@@ -54,7 +54,8 @@ int main() {
         in >> what >> B >> Hq >> Hkv >> N >> D >> causal >> window >> mask >> ws;
         launched.clear();
         if (what == "bytes") {
-            printf("%zu %zu\n", tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D),
+            printf("%zu %zu %zu\n", tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D),
+                   tyr_hip_flash_attn_bwd_parts_workspace_bytes(B, Hq, Hkv, N, D, causal, window),
                    tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window));
         } else {
             const int rc = mask == "keys" ? tyr_hip_flash_attn_bwd_mask(p, p, p, p, p, f, p, p, p, B, Hq, Hkv, N, D, causal, reinterpret_cast<uint8_t*>(p),

@@ -99,10 +99,10 @@ def test_automatic_decode_splits_all_hold_rows():
     (16, 16, 16, 4096, 128, False),    # 8192 key tiles fill the device
     (1, 32, 8, 2000, 128, True)])      # 254, 149
 def test_backward_cuts_key_tiles_where_that_is_faster(B, Hq, Hkv, N, D, cut):
-    """The workspace says whether dK / dV of a causal backward are cut into parts; the times are of an MI355X."""
+    """The workspace of the parts says whether dK / dV of a causal backward are cut into them; the times are of an MI355X."""
     L = _lib.load()
     least = L.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D)
-    assert (L.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, 1, 0) > least) == cut
+    assert (L.tyr_hip_flash_attn_bwd_parts_workspace_bytes(B, Hq, Hkv, N, D, 1, 0) > least) == cut
 
 
 @pytest.mark.parametrize("bh,N,D,causal,window,rows", [

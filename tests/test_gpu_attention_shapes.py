@@ -134,7 +134,7 @@ def test_backward_with_the_least_workspace(B, Hq, Hkv, N, D, mask):
     want_o, want_lse, *want = reference(q, k, v, g, visible)
     o, lse = want_o.bfloat16(), want_lse.contiguous()
     least = lib.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D)
-    full = lib.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window)
+    full = lib.tyr_hip_flash_attn_bwd_parts_workspace_bytes(B, Hq, Hkv, N, D, causal, window)
     assert full > least
     buf = torch.empty(full + 4096, dtype=torch.uint8, device="cuda")
     results = []
@@ -257,8 +257,10 @@ def test_backward_of_64_key_tiles(B, Hq, Hkv, N, D, mask):
 
 
 def test_backward_without_memory_for_ds():
-    """Where the full scratch cannot be had, the call runs with the least."""
+    """Where the full scratch cannot be had, the call runs with parts, and does not make the allocator empty its cache to find out."""
     import tyr_amd
+    from tyr_amd import _lib
+    lib = _lib.load()
     gen = torch.Generator(device="cuda").manual_seed(0)
     q, g = (torch.randn(1, 32, 2000, 128, device="cuda", generator=gen).bfloat16() for _ in range(2))
     k, v = (torch.randn(1, 8, 2000, 128, device="cuda", generator=gen).bfloat16() for _ in range(2))
@@ -268,8 +270,16 @@ def test_backward_without_memory_for_ds():
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(0).total_memory
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (96 << 20)) / total)
+    before = torch.cuda.memory_stats()
     try:
         got = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, causal=True)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+    after = torch.cuda.memory_stats()
+    assert all(after[n] == before[n] for n in ("num_alloc_retries", "num_ooms", "num_device_free"))
     assert all(rel_fro(a, b.float()) <= 1e-3 for a, b in zip(got, want))
+    parts = lib.tyr_hip_flash_attn_bwd_parts_workspace_bytes(1, 32, 8, 2000, 128, 1, 0)
+    ws, cut = torch.empty(parts, dtype=torch.uint8, device="cuda"), [torch.empty_like(t) for t in (q, k, v)]
+    assert 0 == lib.tyr_hip_flash_attn_bwd_gqa(*(t.data_ptr() for t in (q, k, v, o, g, lse, *cut)), 1, 32, 8, 2000, 128, 1, 0, None, 128 ** -0.5,
+                                               ws.data_ptr(), parts, torch.cuda.current_stream().cuda_stream)
+    assert all(torch.equal(a, b) for a, b in zip(got, cut))

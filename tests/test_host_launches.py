@@ -44,8 +44,7 @@ def test_a_window_of_any_size_is_one_of_all_rows(ask):
         whole = None
         for window in (N, N + 1, 2 ** 30, 2 ** 31 - 127, 2 ** 31 - 126, 2 ** 31 - 1, 2 ** 31, 2 ** 64 - 1):
             size, = ask([f"bytes {B} {Hq} {Hkv} {N} 128 1 {window}"])
-            ws = int(size.split()[1])
-            got = [size] + ask([f"bwd {B} {Hq} {Hkv} {N} 128 1 {window} {mask} {w}" for mask in ("none", "lens") for w in (ws, int(size.split()[0]))])
+            got = [size] + ask([f"bwd {B} {Hq} {Hkv} {N} 128 1 {window} {mask} {ws}" for mask in ("none", "lens") for ws in size.split()])
             whole = whole or got
             assert got == whole and got[1].startswith("0 flash_attn_bwd"), (window, got, whole)
 
@@ -56,8 +55,30 @@ def test_scratch_queries_take_any_length(ask):
         for window in (0, 1, 2 ** 31 - 1, 2 ** 40):
             for D in (64, 128):
                 got, = ask([f"bytes 1 1 1 {N} {D} 1 {window}"])
-                least, full = map(int, got.split())
+                least, parts, full = map(int, got.split())
                 assert least == (0 if N >= 2 ** 31 else (N + 127) // 128 * 1024)
-                assert (full == 0) if N * D * 2 >= 2 ** 31 else full >= least
+                assert (full == parts == 0) if N * D * 2 >= 2 ** 31 else full >= parts >= least
                 call, = ask([f"bwd 1 1 1 {N} {D} 1 {window} none {least}"])
                 assert (call == "-3" if N < 2 ** 31 else call == "-2") if full == 0 else call.startswith("0 flash_attn_bwd")
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal,window", [(1, 32, 8, 2000, 128, 1, 0), (2, 16, 4, 1500, 128, 0, 0), (1, 8, 8, 3000, 128, 1, 1500),
+                                                        (1, 4, 4, 700, 128, 1, 0), (1, 8, 2, 2049, 64, 1, 0), (2, 4, 4, 100, 64, 0, 0),
+                                                        (16, 16, 16, 4096, 128, 1, 0)])
+@pytest.mark.parametrize("mask", ["none", "lens", "keys"])
+def test_backward_runs_the_largest_form_that_its_scratch_holds(ask, B, Hq, Hkv, N, D, causal, window, mask):
+    """dS kept, else key tiles cut into parts, else whole key tiles: one byte less than a form needs gives the next one."""
+    if mask == "keys" and window:
+        pytest.skip("refused")
+    shape = f"{B} {Hq} {Hkv} {N} {D} {causal} {window}"
+    least, parts, full = map(int, ask([f"bytes {shape}"])[0].split())
+    sizes = [least - 1, least, parts - 1, parts, full - 1, full, 1 << 40]
+    got = dict(zip(sizes, ask([f"bwd {shape} {mask} {n}" for n in sizes])))
+    assert got[least - 1] == "-5" and got[full] == got[1 << 40]
+    assert not any(k in got[least] for k in ("_sum_", "_product_"))
+    if parts > least:
+        assert got[parts - 1] == got[least] and "_sum_kernel" in got[parts] and "_product_" not in got[parts]
+    if full > parts:
+        assert got[full - 1] == got[parts] and "_stats_kernel" in got[full] and "_product_kernel" in got[full]
+    assert (full > parts, parts > least) == {2000: (True, True), 1500: (True, True), 3000: (True, False), 700: (False, True), 2049: (False, True),
+                                             100: (False, False), 4096: (False, False)}[N]

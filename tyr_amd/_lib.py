@@ -12,7 +12,8 @@ LIB_PATH = os.environ.get("TYR_HIP_LIBRARY") or os.path.join(_HERE, "lib", "libt
 # every symbol include/tyr_hip.h declares
 SYMBOLS = (
     "tyr_hip_strerror", "tyr_hip_version", "tyr_hip_device_info", "tyr_hip_check_device_pointer",
-    "tyr_hip_flash_attn_fwd", "tyr_hip_flash_attn_fwd_gqa", "tyr_hip_flash_attn_bwd_workspace_bytes", "tyr_hip_flash_attn_bwd_full_workspace_bytes", "tyr_hip_flash_attn_bwd",
+    "tyr_hip_flash_attn_fwd", "tyr_hip_flash_attn_fwd_gqa", "tyr_hip_flash_attn_bwd_workspace_bytes", "tyr_hip_flash_attn_bwd_parts_workspace_bytes",
+    "tyr_hip_flash_attn_bwd_full_workspace_bytes", "tyr_hip_flash_attn_bwd",
     "tyr_hip_flash_attn_bwd_gqa", "tyr_hip_flash_attn_fwd_mask", "tyr_hip_flash_attn_bwd_mask",
     "tyr_hip_gqa_decode_workspace_bytes", "tyr_hip_gqa_decode_auto_splits",
     "tyr_hip_gqa_decode", "tyr_hip_gqa_decode_varlen", "tyr_hip_gqa_decode_static", "tyr_hip_gemm_bf16", "tyr_hip_gemm_bf16_batched", "tyr_hip_gemm_bf16_batched_ws", "tyr_hip_gemm_workspace_bytes", "tyr_hip_gemm_force_general", "tyr_hip_flash_attn_fwd_persistent", "tyr_hip_gemm_fp8", "tyr_hip_gemm_fp8_ex", "tyr_hip_gemm_fp8_ws",
@@ -73,8 +74,8 @@ def load() -> ctypes.CDLL:
     L.tyr_hip_flash_attn_fwd_gqa.restype = ci
     L.tyr_hip_flash_attn_bwd_workspace_bytes.argtypes = [u64] * 4
     L.tyr_hip_flash_attn_bwd_workspace_bytes.restype = sz
-    L.tyr_hip_flash_attn_bwd_full_workspace_bytes.argtypes = [u64] * 5 + [ci, u64]
-    L.tyr_hip_flash_attn_bwd_full_workspace_bytes.restype = sz
+    for f in (L.tyr_hip_flash_attn_bwd_parts_workspace_bytes, L.tyr_hip_flash_attn_bwd_full_workspace_bytes):
+        f.argtypes, f.restype = [u64] * 5 + [ci, u64], sz
     L.tyr_hip_flash_attn_bwd.argtypes = [vp] * 9 + [u64] * 4 + [ci, f32, vp, sz, vp]
     L.tyr_hip_flash_attn_bwd.restype = ci
     L.tyr_hip_flash_attn_bwd_gqa.argtypes = [vp] * 9 + [u64] * 5 + [ci, u64, vp, f32, vp, sz, vp]

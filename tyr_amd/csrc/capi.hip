@@ -219,13 +219,22 @@ size_t tyr_hip_flash_attn_bwd_workspace_bytes(uint64_t B, uint64_t H, uint64_t N
 // the backward's 32-bit offsets inside the G query heads of one kv head (and inside their pairs)
 static bool heads_fit(uint64_t G, uint64_t N, uint64_t D) { return G * N * D * 2 < ((uint64_t)1 << 31); }
 
-size_t tyr_hip_flash_attn_bwd_full_workspace_bytes(uint64_t B, uint64_t Hq, uint64_t Hkv, uint64_t N, uint64_t D, int causal,
-                                                   uint64_t window) {
+typedef size_t (*BwdScratch)(int, int, int, int, int, int, int);
+static size_t bwd_scratch(BwdScratch of, uint64_t B, uint64_t Hq, uint64_t Hkv, uint64_t N, uint64_t D, int causal, uint64_t window) {
     if (B == 0 || Hq == 0 || Hkv == 0 || N == 0 || Hq % Hkv != 0 || (D != 64 && D != 128)) return 0;
     if (!fits_int(N) || !fits_int(B * Hq) || B * Hq > (uint64_t)INT_MAX / ((N + 127) / 128)) return 0;
     if (!heads_fit(Hq / Hkv, N, D)) return 0;
-    return tyr::flash_attn_bwd_full_workspace_bytes((int)B, (int)Hq, (int)Hkv, (int)N, (int)D, causal != 0,
-                                                    window_rows(window, N));
+    return of((int)B, (int)Hq, (int)Hkv, (int)N, (int)D, causal != 0, window_rows(window, N));
+}
+
+size_t tyr_hip_flash_attn_bwd_parts_workspace_bytes(uint64_t B, uint64_t Hq, uint64_t Hkv, uint64_t N, uint64_t D, int causal,
+                                                    uint64_t window) {
+    return bwd_scratch(tyr::flash_attn_bwd_parts_workspace_bytes, B, Hq, Hkv, N, D, causal, window);
+}
+
+size_t tyr_hip_flash_attn_bwd_full_workspace_bytes(uint64_t B, uint64_t Hq, uint64_t Hkv, uint64_t N, uint64_t D, int causal,
+                                                   uint64_t window) {
+    return bwd_scratch(tyr::flash_attn_bwd_full_workspace_bytes, B, Hq, Hkv, N, D, causal, window);
 }
 
 int tyr_hip_flash_attn_bwd(const void* q, const void* k, const void* v, const void* o,

@@ -30,7 +30,8 @@ int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, 
                           int Hq, int Hkv, int N, int D, int causal, int window, const int* kv_lens,
                           const uint8_t* key_mask, float scale, hipStream_t stream);
 size_t flash_attn_bwd_workspace_bytes(int B, int H, int N);          // what a call needs
-// what a call can use: with it the dK / dV work of few or unequal key tiles is cut over more workgroups
+// what a call can use: the dK / dV work of few or unequal key tiles is cut over more workgroups, and for few heads dS is kept for dQ
+size_t flash_attn_bwd_parts_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int causal, int window);       // without dS
 size_t flash_attn_bwd_full_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int causal, int window);
 int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                           const float* lse, void* dq, void* dk, void* dv, int B, int Hq, int Hkv, int N, int D,

@@ -29,10 +29,12 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
 
 #include "../../include/tyr_hip.h"
+#include "torch_scratch.hpp"
 
 // Provided by the reference's cc/src/tyr.cpp (same library).
 torch::Tensor borrowTensor(b_lean_obj_arg o);
@@ -75,21 +77,18 @@ lean_object* pair_result(torch::Tensor a, torch::Tensor b) {
 }
 
 // Device scratch on the launch stream.  Every wrapper passes what its call can use, so that it runs the plan that was
-// measured: with the minimum, dK / dV are not cut into parts and K of a GEMM is not split.
+// measured: with the minimum, dK / dV are not cut into parts and K of a GEMM is not split.  Where there is no memory for that, an
+// attention backward tries `parts`; then it is the first operand's size at most: a GEMM runs without any, and the backward's minimum
+// is 8 bytes a row of q.
 struct Scratch {
-    size_t bytes;
+    size_t bytes = 0;
     torch::Tensor block;
-    Scratch(size_t n, const torch::Tensor& like) : bytes(n) {
-        auto take = [&] { block = torch::empty({(int64_t)bytes}, like.options().dtype(torch::kUInt8)); };
-        try {
-            if (n) take();
-        } catch (const c10::OutOfMemoryError&) {
-            // What is more than the first operand is an attention backward that would keep dS (up to 0.4 GB) or a split K: both
-            // run with less, and the backward's minimum is 8 bytes a row of q.
-            if (n <= like.nbytes()) throw;
-            bytes = like.nbytes();
-            take();
-        }
+    Scratch(size_t n, const torch::Tensor& like, size_t parts = 0) {
+        const size_t least = std::min<size_t>(n, like.nbytes());
+        block = tyr_torch::take_largest(n, parts, least, like.device().index(), [&](size_t size) {
+            bytes = size;
+            return size ? torch::empty({(int64_t)size}, like.options().dtype(torch::kUInt8)) : torch::Tensor();
+        });
     }
     void* ptr() const { return bytes ? block.data_ptr() : nullptr; }
 };
@@ -193,7 +192,8 @@ lean_object* lean_tyr_gpu_flash_attn_bwd(uint64_t B, uint64_t H, uint64_t N, uin
             return io_error(err);
         LaunchStreamScope on_stream(stream, q_);   // outputs and scratch belong to the launch stream
         auto dq = torch::empty_like(q_), dk = torch::empty_like(q_), dv = torch::empty_like(q_);
-        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, H, H, N, D, causal, 0), q_);
+        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, H, H, N, D, causal, 0), q_,
+                         tyr_hip_flash_attn_bwd_parts_workspace_bytes(B, H, H, N, D, causal, 0));
         const int rc = tyr_hip_flash_attn_bwd(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(),
                                               g_.data_ptr(), lse_.data_ptr<float>(), dq.data_ptr(),
                                               dk.data_ptr(), dv.data_ptr(), B, H, N, D, causal, (float)scale,
@@ -228,7 +228,8 @@ lean_object* lean_tyr_gpu_flash_attn_bwd_gqa(uint64_t B, uint64_t Hq, uint64_t H
             return io_error(err);
         LaunchStreamScope on_stream(stream, q_);   // outputs and scratch belong to the launch stream
         auto dq = torch::empty_like(q_), dk = torch::empty_like(k_), dv = torch::empty_like(k_);
-        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window), q_);
+        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window), q_,
+                         tyr_hip_flash_attn_bwd_parts_workspace_bytes(B, Hq, Hkv, N, D, causal, window));
         const int rc = tyr_hip_flash_attn_bwd_gqa(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(),
                                                   g_.data_ptr(), lse_.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(),
                                                   dv.data_ptr(), B, Hq, Hkv, N, D, causal, window,
@@ -263,7 +264,8 @@ lean_object* lean_tyr_gpu_flash_attn_bwd_gqa_full(uint64_t B, uint64_t Hq, uint6
             return io_error(err);
         LaunchStreamScope on_stream(stream, q_);   // outputs and scratch belong to the launch stream
         auto dq = torch::empty_like(q_), dk = torch::empty_like(k_), dv = torch::empty_like(k_);
-        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window), q_);
+        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window), q_,
+                         tyr_hip_flash_attn_bwd_parts_workspace_bytes(B, Hq, Hkv, N, D, causal, window));
         const int rc = tyr_hip_flash_attn_bwd_gqa(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(),
                                                   g_.data_ptr(), lse_.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(),
                                                   dv.data_ptr(), B, Hq, Hkv, N, D, causal, window,
@@ -327,7 +329,8 @@ lean_object* lean_tyr_gpu_flash_attn_bwd_mask(uint64_t B, uint64_t Hq, uint64_t 
         if ((uint64_t)m_.numel() != B * N) return io_error("flashAttnBwdMask: keyMask must hold B*N bytes");
         LaunchStreamScope on_stream(stream, q_);   // outputs and scratch belong to the launch stream
         auto dq = torch::empty_like(q_), dk = torch::empty_like(k_), dv = torch::empty_like(k_);
-        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, 0), q_);
+        const Scratch ws(tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, 0), q_,
+                         tyr_hip_flash_attn_bwd_parts_workspace_bytes(B, Hq, Hkv, N, D, causal, 0));
         const int rc = tyr_hip_flash_attn_bwd_mask(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(),
                                                    g_.data_ptr(), lse_.data_ptr<float>(), dq.data_ptr(),
                                                    dk.data_ptr(), dv.data_ptr(), B, Hq, Hkv, N, D, causal,

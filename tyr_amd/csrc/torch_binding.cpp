@@ -24,6 +24,7 @@
 #include <string>
 
 #include "../../include/tyr_hip.h"
+#include "torch_scratch.hpp"
 
 namespace {
 
@@ -63,7 +64,7 @@ public:
 };
 #define TYR_ENTRY_POINTS(X)                                                                                                  \
     X(tyr_hip_strerror) X(tyr_hip_flash_attn_fwd_gqa) X(tyr_hip_flash_attn_fwd_mask) X(tyr_hip_flash_attn_bwd_full_workspace_bytes) \
-    X(tyr_hip_flash_attn_bwd_workspace_bytes)                                                                                \
+    X(tyr_hip_flash_attn_bwd_parts_workspace_bytes) X(tyr_hip_flash_attn_bwd_workspace_bytes)                                \
     X(tyr_hip_flash_attn_bwd_gqa) X(tyr_hip_flash_attn_bwd_mask) X(tyr_hip_gqa_decode_workspace_bytes)                        \
     X(tyr_hip_gqa_decode_varlen) X(tyr_hip_decode_rope_append) X(tyr_hip_rope_fwd) X(tyr_hip_layernorm_residual)             \
     X(tyr_hip_copy) X(tyr_hip_gemm_workspace_bytes) X(tyr_hip_gemm_bf16_batched_ws) X(tyr_hip_gemm_fp8_ws)                    \
@@ -212,12 +213,10 @@ PyObject* flash_attn_bwd(PyObject* const* a) {
         dq = empty_like(q);
         dk = empty_like(k);
         dv = empty_like(k);
-        at::Tensor ws;
-        try {
-            ws = scratch(api.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window), q);
-        } catch (const c10::OutOfMemoryError&) {         // the fastest form takes up to 0.4 GB; the call needs far less
-            ws = scratch(api.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D), q);
-        }
+        const at::Tensor ws = tyr_torch::take_largest(api.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, causal, window),
+                                                      api.tyr_hip_flash_attn_bwd_parts_workspace_bytes(B, Hq, Hkv, N, D, causal, window),
+                                                      api.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D), q.device().index(),
+                                                      [&](size_t bytes) { return scratch(bytes, q); });
         const float* lse_p = static_cast<const float*>(lse.data_ptr());
         rc = mask ? api.tyr_hip_flash_attn_bwd_mask(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse_p,
                                                     dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, Hq, Hkv, N, D, causal, mask, scale,
