@@ -1,6 +1,7 @@
 // A HIP runtime that launches nothing, for the host code of the library on a machine without a GPU: one line of stdin is one call
 // of the C ABI, one line of stdout its result and the kernels it would launch, in order.
 //   bytes B Hq Hkv N D causal window          scratch of the backward: least, with parts, full
+//   kernels                                   every kernel of the files linked
 //   bwd   B Hq Hkv N D causal window mask ws  status, then "kernel<arguments>:workgroups" each; mask = none | lens | keys
 #include <cxxabi.h>
 #include <hip/hip_runtime_api.h>
@@ -51,7 +52,14 @@ int main() {
         uint64_t B, Hq, Hkv, N, D, window;
         int causal;
         size_t ws = 0;
-        in >> what >> B >> Hq >> Hkv >> N >> D >> causal >> window >> mask >> ws;
+        in >> what;
+        if (what == "kernels") {
+            for (const auto& k : kernels()) printf("%s ", k.second.c_str());
+            printf("\n");
+            fflush(stdout);
+            continue;
+        }
+        in >> B >> Hq >> Hkv >> N >> D >> causal >> window >> mask >> ws;
         launched.clear();
         if (what == "bytes") {
             printf("%zu %zu %zu\n", tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D),

@@ -82,3 +82,13 @@ def test_backward_runs_the_largest_form_that_its_scratch_holds(ask, B, Hq, Hkv, 
         assert got[full - 1] == got[parts] and "_stats_kernel" in got[full] and "_product_kernel" in got[full]
     assert (full > parts, parts > least) == {2000: (True, True), 1500: (True, True), 3000: (True, False), 700: (False, True), 2049: (False, True),
                                              100: (False, False), 4096: (False, False)}[N]
+
+
+def test_every_backward_kernel_is_reached(ask):
+    built = {k for k in ask(["kernels"])[0].split() if k.startswith("flash_attn_bwd")}
+    calls = [f"bwd {B} {Hq} {Hkv} {N} {D} {causal} {window if mask != 'keys' else 0} {mask} {ws if ws else B * Hq * ((N + 127) // 128) * 1024}"
+             for B in (1, 4, 16) for Hq, Hkv in ((4, 4), (16, 4), (32, 8)) for N in (64, 300, 700, 1500, 4096) for D in (64, 128)
+             for causal, window in ((0, 0), (1, 0), (1, 50), (1, 600)) for mask in ("none", "lens", "keys") for ws in (0, 1 << 40)]
+    got = ask(calls)
+    assert all(g.startswith("0 ") for g in got)
+    assert built == {k.rsplit(":", 1)[0] for g in got for k in g.split()[1:]}

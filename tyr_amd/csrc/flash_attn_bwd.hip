@@ -460,7 +460,8 @@ struct DsBlocks {
 // CUT: the launch has parts.  (Whole key tiles keep their own instantiation: with the bookkeeping of the parts in the same
 // code the pipeline below, which has no register to spare, is 4-8 % slower.)
 // OWN_STATS: nothing ran before this kernel, so the workgroup makes the (lse2, delta) pairs of its query rows itself.
-// SPILL: dS also goes to `ds`, for the dQ launch after this one.
+// SPILL: dS also goes to `ds`, for the dQ launch after this one.  Under a window that takes 4 and 6 registers more than there are
+// (20 and 28 bytes a lane in scratch memory; 2 of CUT without it).
 template <int D, bool CAUSAL, AttnMask MASK, bool CUT, bool OWN_STATS, bool SPILL>
 __device__ __forceinline__ void bwd_dkv(int block,
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
@@ -1677,10 +1678,14 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
                            static_cast<uint16_t*>(dv), BHkv, N, ntk, npad, scale, scale_log2, Hq,     \
                            window, kv_lens, key_mask, plan, items, partial, ds);                      \
     } while (0)
-#define TYR_FAB_DKV_MASK(DD, CC, EE, UU, PP)  /* lengths alone are a mask of keys here */             \
+#define TYR_FAB_DKV_MASK(DD, CC, EE, UU, PP)  /* lengths alone are a mask of keys here; a window is causal */ \
     do {                                                                                              \
-        if (EE == AttnMask::Limits && window <= 0) TYR_FAB_DKV(DD, CC, AttnMask::Keys, UU, PP);       \
-        else TYR_FAB_DKV(DD, CC, EE, UU, PP);                                                         \
+        if constexpr (EE == AttnMask::Limits) {                                                       \
+            if (CC && window > 0) TYR_FAB_DKV(DD, true, EE, UU, PP);                                  \
+            else TYR_FAB_DKV(DD, CC, AttnMask::Keys, UU, PP);                                         \
+        } else {                                                                                      \
+            TYR_FAB_DKV(DD, CC, EE, UU, PP);                                                          \
+        }                                                                                             \
     } while (0)
 #define TYR_FAB_DQ_PRODUCT(DD, CC, EE)                                                                \
     do {                                                                                              \
