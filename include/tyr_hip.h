@@ -336,10 +336,11 @@ int tyr_hip_gemm_bf16_batched(const void* a, const void* b, void* c, uint64_t ba
 
 /* The same products with device scratch.  A product with few output tiles and a long K leaves most of the device idle
  * unless K is split over workgroups; the f32 partial sums then pass through `workspace` (16-byte aligned device memory of
- * tyr_hip_gemm_workspace_bytes bytes; a smaller one, or NULL, only means that K is not split).  elem_bytes: 2 = bf16,
- * 1 = e4m3; 0 bytes = this shape does the same without.  Results are reproducible launch to launch either way; with scratch
- * K may be summed in another order (16 bytes: only within a workgroup, nothing is written there), so the two forms may
- * differ in the last bit of the output. */
+ * tyr_hip_gemm_workspace_bytes bytes; with a smaller one K is not split).  elem_bytes: 2 = bf16, 1 = e4m3.
+ * The workspace also says which sums the caller accepts.  NULL: a bf16 product has the bits it has as an entry of a batch.  Otherwise
+ * K may be summed in another order, with which the last bit of the output may differ; where that needs no memory (0 bytes),
+ * TYR_HIP_ANY_ORDER takes the place of the pointer.  Results are reproducible launch to launch either way. */
+#define TYR_HIP_ANY_ORDER ((void*)16)
 size_t tyr_hip_gemm_workspace_bytes(uint64_t batch, uint64_t M, uint64_t N, uint64_t K, int elem_bytes, int trans_b);
 int tyr_hip_gemm_bf16_batched_ws(const void* a, const void* b, void* c, uint64_t batch,
                                  uint64_t M, uint64_t N, uint64_t K,
@@ -392,7 +393,7 @@ int tyr_hip_gemm_fp8_ex(const void* aq, const void* bq, void* c,
                         uint64_t M, uint64_t N, uint64_t K,
                         float scale, const float* row_scale, const float* col_scale, int out_dtype,
                         int trans_b, void* stream);
-/* tyr_hip_gemm_fp8_ex with scratch for split-K partials, as tyr_hip_gemm_bf16_batched_ws. */
+/* tyr_hip_gemm_fp8_ex with scratch for split-K partials, as tyr_hip_gemm_bf16_batched_ws (NULL only means that K is not split). */
 int tyr_hip_gemm_fp8_ws(const void* aq, const void* bq, void* c,
                         uint64_t M, uint64_t N, uint64_t K,
                         float scale, const float* row_scale, const float* col_scale, int out_dtype,

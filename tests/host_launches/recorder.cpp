@@ -1,6 +1,8 @@
 // A HIP runtime that launches nothing, for the host code of the library on a machine without a GPU: one line of stdin is one call
 // of the C ABI, one line of stdout its result and the kernels it would launch, in order.
 //   bytes B Hq Hkv N D causal window          scratch of the backward: least, with parts, full
+//   gemm  M N K trans_b bytes ws              a product of elements of 2 (bf16) or 1 (e4m3) bytes: as bwd; ws = bytes of scratch,
+//                                             0 = null, any = TYR_HIP_ANY_ORDER; its scratch follows the status
 //   kernels                                   every kernel of the files linked
 //   bwd   B Hq Hkv N D causal window mask ws  status, then "kernel<arguments>:workgroups" each; mask = none | lens | keys
 #include <cxxabi.h>
@@ -56,6 +58,20 @@ int main() {
         if (what == "kernels") {
             for (const auto& k : kernels()) printf("%s ", k.second.c_str());
             printf("\n");
+            fflush(stdout);
+            continue;
+        }
+        if (what == "gemm") {
+            uint64_t M, N, K;
+            int trans_b, bytes;
+            std::string scratch;
+            in >> M >> N >> K >> trans_b >> bytes >> scratch;
+            void* to = scratch == "any" ? TYR_HIP_ANY_ORDER : scratch == "0" ? nullptr : p;
+            const size_t size = scratch == "any" ? SIZE_MAX : strtoull(scratch.c_str(), nullptr, 10);
+            launched.clear();
+            const int rc = bytes == 2 ? tyr_hip_gemm_bf16_batched_ws(p, p, p, 1, M, N, K, 0, 0, 0, trans_b, to, size, nullptr)
+                                      : tyr_hip_gemm_fp8_ws(p, p, p, M, N, K, 1.0f, nullptr, nullptr, TYR_HIP_OUT_BF16, trans_b, to, size, nullptr);
+            printf("%d %zu%s\n", rc, tyr_hip_gemm_workspace_bytes(1, M, N, K, bytes, trans_b), launched.c_str());
             fflush(stdout);
             continue;
         }

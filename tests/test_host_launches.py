@@ -22,7 +22,7 @@ def ask(tmp_path_factory):
                                os.path.join(ROOT, name), "-o", obj])
         return obj
     with ThreadPoolExecutor() as pool:
-        objs = list(pool.map(compile_, ["tyr_amd/csrc/capi.hip", "tyr_amd/csrc/flash_attn_fwd.hip", "tyr_amd/csrc/flash_attn_bwd.hip"]))
+        objs = list(pool.map(compile_, [f"tyr_amd/csrc/{n}.hip" for n in ("capi", "flash_attn_fwd", "flash_attn_bwd", "gemm_bf16", "gemm_fp8")]))
     main, exe = str(tmp / "recorder.o"), str(tmp / "recorder")
     subprocess.check_call(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-isystem", "/opt/rocm/include", "-c",
                            os.path.join(ROOT, "tests", "host_launches", "recorder.cpp"), "-o", main])
@@ -92,3 +92,22 @@ def test_every_backward_kernel_is_reached(ask):
     got = ask(calls)
     assert all(g.startswith("0 ") for g in got)
     assert built == {k.rsplit(":", 1)[0] for g in got for k in g.split()[1:]}
+
+
+@pytest.mark.parametrize("M,N,K,trans_b,size", [(256, 4096, 4096, 0, 2), (1, 4096, 4096, 1, 2), (3, 512, 8192, 1, 2), (200, 16, 8192, 1, 2),
+                                                (4096, 4096, 4096, 0, 2), (333, 4096, 4096, 1, 1), (120, 1024, 8192, 0, 1)])
+def test_sums_in_any_order_need_no_memory(ask, M, N, K, trans_b, size):
+    """Without memory for partials, or with less than they take, K is not split, but still summed by as many waves as is fastest;
+    without a workspace in the order that a batch has.  The scratch of what is not split is none."""
+    def call(ws):
+        rc, need, *kernels = ask([f"gemm {M} {N} {K} {trans_b} {size} {ws}"])[0].split()
+        assert rc == "0"
+        return int(need), " ".join(kernels)
+    need, alone = call("any")
+    assert "_reduce_" not in alone and call(16)[1] == alone
+    if need:
+        assert "_reduce_" in call(need)[1] and call(need - 1)[1] == alone
+    else:
+        assert call(1 << 40)[1] == alone
+    assert (need > 0) == ((M, N) in ((3, 512), (200, 16), (120, 1024)))
+    assert (call(0)[1] == alone) == (size == 1 or M == 4096), (call(0), alone)

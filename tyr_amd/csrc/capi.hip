@@ -452,6 +452,7 @@ int tyr_hip_gemm_bf16_batched_ws(const void* a, const void* b, void* c, uint64_t
         if (stride_a > ((uint64_t)1 << 40) || stride_b > ((uint64_t)1 << 40) || stride_c > ((uint64_t)1 << 40))
             return TYR_HIP_ERR_BAD_SHAPE;
     }
+    if (workspace == TYR_HIP_ANY_ORDER) workspace_bytes = 0;         // no memory
     const int rc = tyr::launch_gemm_bf16(a, b, c, (int)M, (int)N, (int)K, trans_b != 0, (int)batch,
                                          (int64_t)stride_a, (int64_t)stride_b, (int64_t)stride_c, workspace,
                                          workspace_bytes, static_cast<hipStream_t>(stream));
@@ -486,6 +487,7 @@ int tyr_hip_gemm_fp8_ws(const void* aq, const void* bq, void* c, uint64_t M, uin
     if (!aligned16(aq) || !aligned16(bq) || !aligned16(c) || !aligned16(workspace)) return TYR_HIP_ERR_MISALIGNED;
     if ((row_scale && (reinterpret_cast<uintptr_t>(row_scale) & 3u)) || (col_scale && !aligned16(col_scale)))
         return TYR_HIP_ERR_MISALIGNED;
+    if (workspace == TYR_HIP_ANY_ORDER) workspace_bytes = 0;         // no memory
     const int rc = tyr::launch_gemm_fp8(aq, bq, c, (int)M, (int)N, (int)K, scale, trans_b != 0, row_scale, col_scale,
                                         out_dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
     return rc == 0 ? TYR_HIP_OK : TYR_HIP_ERR_LAUNCH;

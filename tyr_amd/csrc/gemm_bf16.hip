@@ -393,8 +393,8 @@ __global__ __launch_bounds__(gemm2::THREADS, 1) void gemm_bf16_fast_kernel(
 
 size_t gemm_workspace_bytes(int M, int N, int K, int elem_bytes, int trans_b, int batch) {
     if (gemm_general_only() || !gt::offsets_fit(N, K, elem_bytes, trans_b != 0)) return 0;
-    const gt::Plan p = gt::plan(M, N, K, elem_bytes, trans_b != 0, batch, true);
-    return gt::scratch_bytes(p, M, N, elem_bytes, batch);
+    const gt::Plan p = gt::plan(M, N, K, elem_bytes, trans_b != 0, batch, gt::SPLIT);
+    return gt::scratch_bytes(p, M, N, batch);
 }
 
 int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K, int trans_b,
@@ -413,9 +413,7 @@ int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K,
     // gemm_general_only() sends every shape there: a switch for tests and for comparing the paths.
     const bool fast_ok = !gemm_general_only() && (K % 8 == 0) && gt::offsets_fit(N, K, 2, trans_b != 0);
     if (fast_ok) {
-        gt::Plan p = gt::plan(M, N, K, 2, trans_b != 0, batch, workspace != nullptr);
-        if (workspace_bytes < gt::scratch_bytes(p, M, N, 2, batch))
-            p = gt::plan(M, N, K, 2, trans_b != 0, batch, false);
+        const gt::Plan p = gt::plan_within(M, N, K, 2, trans_b != 0, batch, workspace, workspace_bytes);
         if (p.tile != gt::T256x256) {
             const GemmEpilogue ep{1.0f, nullptr, nullptr, 0};
             auto part = static_cast<float*>(workspace);

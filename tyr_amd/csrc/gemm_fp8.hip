@@ -428,9 +428,7 @@ int launch_gemm_fp8(const void* aq, const void* bq, void* c, int M, int N, int K
     // As in launch_gemm_bf16: tiles or 256x256 tiles within the 32-bit offsets, the general kernels beyond them.
     const bool fast_ok = !gemm_general_only() && (K % 16 == 0) && gt::offsets_fit(N, K, 1, trans_b != 0);
     if (fast_ok) {
-        gt::Plan p = gt::plan(M, N, K, 1, trans_b != 0, 1, workspace != nullptr);
-        if (workspace_bytes < gt::scratch_bytes(p, M, N, 1, 1))
-            p = gt::plan(M, N, K, 1, trans_b != 0, 1, false);
+        const gt::Plan p = gt::plan_within(M, N, K, 1, trans_b != 0, 1, workspace, workspace_bytes);
         if (p.tile != gt::T256x256) {
             auto part = static_cast<float*>(workspace);
             return trans_b ? gt::launch_plan<1, true>(p, aq, bq, c, M, N, K, part, 1, 0, 0, 0, ep, stream)

@@ -443,18 +443,20 @@ inline double tile_cost(int tile, int splits, int M, int N, int K, int es, bool 
     return (us > memory ? us : memory) + 0.05 * us;
 }
 
-// `may_split`: the caller has scratch memory for partials.  The order in which K is summed depends on the MFMA shape, the
-// k-groups and the splits, not on the rest of the tile: a batch keeps the order its entries would have one by one without
-// scratch, so that it gives the same bits, and picks the tile among those.  The W tiles are therefore not for bf16 products
-// without scratch: a large batch would be left with one small tile of their order.  (There are no batches of e4m3.)
-inline Plan make_plan(int M, int N, int K, int es, bool tb, int batch, bool may_split) {
+// What a caller allows.  The order in which K is summed depends on the MFMA shape, the k-groups and the splits, not on the rest of the
+// tile.  BATCH: the order that the same product has as an entry of a batch, so that both give the same bits; a batch picks its tile
+// among those.  The W tiles are not for it (bf16; there are no batches of e4m3): a large batch would be left with one small tile of
+// their order.  ANY: without scratch for partials.  SPLIT: with.
+enum Sums : uint8_t { BATCH, ANY, SPLIT };
+inline Plan make_plan(int M, int N, int K, int es, bool tb, int batch, Sums sums) {
+    if (batch > 1) sums = BATCH;
     Plan best{T256x256, 1};
     double least = tile_cost(T256x256, 1, M, N, K, es, tb, 1);
     const int64_t pieces = ((int64_t)K * es + KB - 1) / KB;
     for (int tile = 0; tile < T256x256; ++tile) {
-        if (!tile_takes(tile, es, tb) || (kTileCost[tile].wide && es == 2 && !(may_split && batch == 1))) continue;
+        if (!tile_takes(tile, es, tb) || (kTileCost[tile].wide && es == 2 && sums == BATCH)) continue;
         for (int splits = 1; splits <= 8; ++splits) {
-            if (splits > 1 && (!may_split || batch > 1 || pieces < 4 * splits)) break;
+            if (splits > 1 && (sums != SPLIT || pieces < 4 * splits)) break;
             const double us = tile_cost(tile, splits, M, N, K, es, tb, 1);
             if (us < least) { least = us; best = {tile, splits}; }
         }
@@ -474,23 +476,25 @@ inline Plan make_plan(int M, int N, int K, int es, bool tb, int batch, bool may_
     return best;
 }
 
-// Scratch without which this plan is not taken.  A wide tile touches none of it: with any, the caller has no claim to the
-// order of sums of a product without.
-inline size_t scratch_bytes(const Plan& p, int M, int N, int es, int batch) {
-    if (p.splits > 1) return (size_t)p.splits * batch * M * N * sizeof(float);
-    return es == 2 && p.tile != T256x256 && kTileCost[p.tile].wide ? 16 : 0;
+inline size_t scratch_bytes(const Plan& p, int M, int N, int batch) {
+    return p.splits > 1 ? (size_t)p.splits * batch * M * N * sizeof(float) : 0;
 }
 
 // make_plan costs about a microsecond of host time; a program repeats few shapes, so each thread keeps its last plans.
-inline Plan plan(int M, int N, int K, int es, bool tb, int batch, bool may_split) {
+inline Plan plan(int M, int N, int K, int es, bool tb, int batch, Sums sums) {
     struct Entry { int M, N, K, batch, kind; Plan plan; };
     static thread_local Entry kept[64];
-    const int kind = 1 + es * 4 + tb * 2 + may_split;                // 0 = an unused entry
+    const int kind = 1 + (es * 2 + tb) * 3 + sums;                   // 0 = an unused entry
     const uint32_t h = ((uint32_t)M * 0x9e3779b1u ^ (uint32_t)N * 0x85ebca6bu ^ (uint32_t)K * 0xc2b2ae35u ^ (uint32_t)batch * 0x27d4eb2fu ^ (uint32_t)kind) * 0x9e3779b1u;
     Entry& e = kept[h >> 26];
     if (e.kind != kind || e.M != M || e.N != N || e.K != K || e.batch != batch)
-        e = {M, N, K, batch, kind, make_plan(M, N, K, es, tb, batch, may_split)};
+        e = {M, N, K, batch, kind, make_plan(M, N, K, es, tb, batch, sums)};
     return e.plan;
+}
+inline Plan plan_within(int M, int N, int K, int es, bool tb, int batch, const void* workspace, size_t workspace_bytes) {
+    if (workspace == nullptr) return plan(M, N, K, es, tb, batch, BATCH);
+    const Plan p = plan(M, N, K, es, tb, batch, SPLIT);
+    return scratch_bytes(p, M, N, batch) <= workspace_bytes ? p : plan(M, N, K, es, tb, batch, ANY);
 }
 
 template <class C>

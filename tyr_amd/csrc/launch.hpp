@@ -8,7 +8,8 @@
 namespace tyr {
 
 // `batch` independent products; strides in elements between consecutive batch entries (stride_b = 0
-// uses one B for every entry).  workspace (may be null): device scratch for split-K partials, gemm_workspace_bytes bytes.
+// uses one B for every entry).  workspace: device scratch for split-K partials, gemm_workspace_bytes bytes; null = sums in the order
+// of a batch.
 int launch_gemm_bf16(const void* a, const void* b, void* c, int M, int N, int K, int trans_b,
                      int batch, int64_t stride_a, int64_t stride_b, int64_t stride_c, void* workspace, size_t workspace_bytes,
                      hipStream_t stream);

@@ -90,7 +90,7 @@ struct Scratch {
             return size ? torch::empty({(int64_t)size}, like.options().dtype(torch::kUInt8)) : torch::Tensor();
         });
     }
-    void* ptr() const { return bytes ? block.data_ptr() : nullptr; }
+    void* ptr() const { return bytes ? block.data_ptr() : TYR_HIP_ANY_ORDER; }
 };
 
 lean_object* status_error(const char* what, int rc) {

@@ -361,7 +361,7 @@ struct Partials {
         : bytes(api.tyr_hip_gemm_workspace_bytes(batch, e.M, e.N, e.K, elem_bytes, trans_b)) {
         if (bytes) block = scratch(bytes, like);
     }
-    void* ptr() const { return bytes ? block.data_ptr() : nullptr; }
+    void* ptr() const { return bytes ? block.data_ptr() : TYR_HIP_ANY_ORDER; }
 };
 
 // (a, b, trans_b)
