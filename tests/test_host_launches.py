@@ -1,6 +1,7 @@
 """What the C ABI's host code decides, on the CPU: the kernel files are compiled for the host alone, with every signed overflow
 an abort, and linked with a HIP runtime that records the launches instead of making them (tests/host_launches)."""
 import os
+import re
 import subprocess
 from concurrent.futures import ThreadPoolExecutor
 
@@ -111,3 +112,19 @@ def test_sums_in_any_order_need_no_memory(ask, M, N, K, trans_b, size):
         assert call(1 << 40)[1] == alone
     assert (need > 0) == ((M, N) in ((3, 512), (200, 16), (120, 1024)))
     assert (call(0)[1] == alone) == (size == 1 or M == 4096), (call(0), alone)
+
+
+@pytest.mark.parametrize("M,N,K,trans_b,size,rows,cols,groups,split", [
+    (2719, 448, 1280, 0, 2, 96, 64, 2, False),      # 8.2 us; 64x128 over two k-groups 8.7
+    (1105, 1344, 832, 0, 2, 96, 64, 2, False),      # 6.9, 7.2
+    (173, 352, 4456, 1, 2, 16, 16, 4, False),       # 5.2; over eight k-groups 5.9
+    (401, 296, 3488, 1, 2, 32, 32, 4, False),       # 5.7; 16x16 over eight 7.0
+    (549, 736, 7936, 0, 1, 64, 128, 1, True),       # 13.3; 32x64 over four in one piece 17.9
+    (1, 4096, 4096, 1, 2, 16, 16, 8, False),        # 4.4; over four 4.9
+    (333, 4096, 4096, 1, 1, 64, 128, 2, False),     # 10.9; over one 12.4
+    (256, 4096, 4096, 0, 2, 64, 64, 2, False)])     # 14.6; over one 17.5
+def test_tiles_of_twice_the_waves_where_they_are_faster(ask, M, N, K, trans_b, size, rows, cols, groups, split):
+    """The tile of a product, the k-groups of its workgroups and whether K is split; the times are of an MI355X."""
+    got, = ask([f"gemm {M} {N} {K} {trans_b} {size} {1 << 40}"])
+    m = re.fullmatch(r"0 \d+ gemm_tile_kernel<gt::Cfg<(1|2),(true|false),(\d+),(\d+),\d+,\d+,(\d+),\d+>>:\d+( gemm_tile_reduce_kernel<\d>:\d+)?", got)
+    assert m and (int(m[1]), m[2] == "true", int(m[3]), int(m[4]), int(m[5]), bool(m[6])) == (size, bool(trans_b), rows, cols, groups, split), got

@@ -410,6 +410,8 @@ namespace gt {
 // workgroup a CU (ALONE) eight waves keep twice the pieces in flight (M = 256, N = K = 4096: fp8 10.1 -> 8.1 us, bf16 17.5 ->
 // 14.6 with 64x64; M = 333 fp8 12.4 -> 10.9 with 64x128), with more the next workgroup cannot start beside the last one (M =
 // 1000 28 -> 31 us).  16x16 over eight k-groups: from about 22 pieces on (M = 1, N = K = 4096 bf16 4.9 -> 4.4).
+// Of 18000 drawn shapes 1935 take another plan than without them, in 10 % less time in the mean; 59 are slower by more than 2 %, the
+// worst 37 % (33 x 1840 x 4928 NT bf16: 64x64W over 8 splits 8.2 us, 16x32 6.0).
 enum Wide : uint8_t { NO, WIDE, ALONE };             // ALONE: WIDE, and one workgroup a CU
 struct TileCost { int bm, bn, kg, mf; float fixed, piece; Wide wide = NO; };
 enum Tile { T16x16, T16x16W, T16x32, T16x64, T32x32, T32x64W, T64x32, T64x32W, T64x64, T64x64W, T64x128, T64x128W, T96x64, T128x128,
@@ -426,16 +428,31 @@ struct Plan { int tile, splits; };
 // A [K,N] B is fetched in rows of BN elements: at least 64 bytes of each.
 inline bool tile_takes(int tile, int es, bool tb) { return tb || kTileCost[tile].bn * es >= 64; }
 
-inline double tile_cost(int tile, int splits, int M, int N, int K, int es, bool tb, int batch) {
+// What a caller allows.  The order in which K is summed depends on the MFMA shape, the k-groups and the splits, not on the rest of the
+// tile.  BATCH: the order that the same product has as an entry of a batch, so that both give the same bits; a batch picks its tile
+// among those.  The W tiles are not for it (bf16; there are no batches of e4m3): a large batch would be left with one small tile of
+// their order.  ANY: without scratch for partials.  SPLIT: with.
+enum Sums : uint8_t { BATCH, ANY, SPLIT };
+
+inline double tile_cost(int tile, int splits, int M, int N, int K, int es, bool tb, int batch, Sums sums) {
     const TileCost& t = kTileCost[tile];
     const int64_t pieces = ((int64_t)K * es + KB - 1) / KB, per_split = (pieces + splits - 1) / splits;
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * splits * batch;
     if (t.wide == ALONE && tiles > 256) return 1e30;
-    // Rows that do not start on cache lines: every piece of one touches two.  A CU's requests are what bounds an ALONE tile
-    // (64x64W, 44 pieces of 126 x 6992 x 5544 bf16: 0.57 us each for 0.36), the others wait as much for other things (1.16 x).
-    const bool lines = (int64_t)K * es % KB == 0 && (tb || (int64_t)N * es % KB == 0);
-    const double piece = t.wide == ALONE && !lines ? 1.4 * t.piece : t.piece;
+    // Rows that do not start on cache lines, or are half a line: every piece of one touches two.  A CU's requests are what bounds an
+    // ALONE tile (64x64W, 44 pieces of 126 x 6992 x 5544 bf16: 0.57 us each for 0.36) and 16x16W with more than 16 rows on all CUs
+    // (173 x 352 x 4456 NT bf16 5.2 us with 16x16, 5.9 with 16x16W), the others wait as much for other things (1.16 x).
+    const bool half = !tb && t.bn * es < KB;
+    const bool lines = (int64_t)K * es % KB == 0 && (tb || ((int64_t)N * es % KB == 0 && !half));
+    double piece = !lines && (t.wide == ALONE || (t.wide == WIDE && tiles > 200 && M > t.bm)) ? 1.4 * t.piece : t.piece;
+    // The ring of 96x64 takes a CU's whole LDS too: its 0.71 us hold that every further round starts anew.  2719 x 448 x 1280 NN
+    // bf16, one round of 10 pieces a k-group, 8.2 us (64x128W 8.7).  Not where its order of sums would bind a batch, which has no
+    // other tile of that order.
+    if (tile == T96x64 && es == 2 && sums != BATCH && splits == 1 && tiles <= 256 && pieces <= 64) piece = 0.53;
     double us = t.fixed + piece * ((per_split + t.kg - 1) / t.kg) * ((tiles + 255) / 256);
+    // Half lines of a long [K,N] B, where K can be split instead (the other tiles that take it whole are slower still): 549 x 736 x
+    // 7936 e4m3 17.9 us with 32x64W, 13.3 with 64x128 over 4 splits.
+    if (t.wide == ALONE && half && sums == SPLIT && per_split > 40) us += 0.1 * (per_split - 40);
     // the second kernel, and f32 partials written and read at 5 TB/s
     if (splits > 1) us += 2.6 + (double)M * N * batch * 8.0 * splits / 5.0e6;
     // no tile is faster than memory; among those that reach it the one with the least to do still wins
@@ -443,30 +460,25 @@ inline double tile_cost(int tile, int splits, int M, int N, int K, int es, bool 
     return (us > memory ? us : memory) + 0.05 * us;
 }
 
-// What a caller allows.  The order in which K is summed depends on the MFMA shape, the k-groups and the splits, not on the rest of the
-// tile.  BATCH: the order that the same product has as an entry of a batch, so that both give the same bits; a batch picks its tile
-// among those.  The W tiles are not for it (bf16; there are no batches of e4m3): a large batch would be left with one small tile of
-// their order.  ANY: without scratch for partials.  SPLIT: with.
-enum Sums : uint8_t { BATCH, ANY, SPLIT };
 inline Plan make_plan(int M, int N, int K, int es, bool tb, int batch, Sums sums) {
     if (batch > 1) sums = BATCH;
     Plan best{T256x256, 1};
-    double least = tile_cost(T256x256, 1, M, N, K, es, tb, 1);
+    double least = tile_cost(T256x256, 1, M, N, K, es, tb, 1, sums);
     const int64_t pieces = ((int64_t)K * es + KB - 1) / KB;
     for (int tile = 0; tile < T256x256; ++tile) {
         if (!tile_takes(tile, es, tb) || (kTileCost[tile].wide && es == 2 && sums == BATCH)) continue;
         for (int splits = 1; splits <= 8; ++splits) {
             if (splits > 1 && (sums != SPLIT || pieces < 4 * splits)) break;
-            const double us = tile_cost(tile, splits, M, N, K, es, tb, 1);
+            const double us = tile_cost(tile, splits, M, N, K, es, tb, 1, sums);
             if (us < least) { least = us; best = {tile, splits}; }
         }
     }
     if (batch > 1) {
         const TileCost order = kTileCost[best.tile];
-        least = tile_cost(best.tile, 1, M, N, K, es, tb, batch);
+        least = tile_cost(best.tile, 1, M, N, K, es, tb, batch, BATCH);
         for (int tile = 0; tile < TILES; ++tile) {
             if (!tile_takes(tile, es, tb) || kTileCost[tile].wide || kTileCost[tile].kg != order.kg || kTileCost[tile].mf != order.mf) continue;
-            const double us = tile_cost(tile, 1, M, N, K, es, tb, batch);
+            const double us = tile_cost(tile, 1, M, N, K, es, tb, batch, BATCH);
             if (us < least) { least = us; best.tile = tile; }
         }
     }
