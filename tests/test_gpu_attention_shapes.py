@@ -162,7 +162,7 @@ def test_backward_with_the_least_workspace(B, Hq, Hkv, N, D, mask):
 
 
 @pytest.mark.parametrize("mask", ["causal", "full", "window", "lens", "keys"])
-@pytest.mark.parametrize("B,Hq,Hkv,N", [(4, 16, 4, 577), (4, 16, 4, 640), (4, 16, 16, 769), (2, 32, 8, 1153), (4, 8, 1, 1025), (9, 16, 4, 200)])
+@pytest.mark.parametrize("B,Hq,Hkv,N", [(4, 16, 4, 577), (4, 16, 4, 640), (4, 16, 16, 769), (2, 32, 8, 1153), (4, 8, 1, 1025), (4, 16, 4, 200)])
 def test_backward_that_keeps_ds(B, Hq, Hkv, N, mask):
     """Few heads at D = 128, where dK / dV leave dS for dQ: rows one past a tile, whole tiles, whole and cut key tiles.  Hidden keys
     come first, in the middle (more than one block of 128) and last, with values that would outweigh every visible one."""
@@ -216,7 +216,7 @@ def test_backward_that_keeps_ds(B, Hq, Hkv, N, mask):
 
 @pytest.mark.parametrize("mask", ["causal", "full", "window", "lens", "keys"])
 @pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 1, 1, 1, 64), (2, 4, 4, 64, 128), (2, 4, 4, 65, 64), (3, 4, 4, 130, 128), (6, 4, 4, 263, 128), (2, 4, 4, 449, 64),
-                                          (2, 8, 8, 685, 128), (9, 16, 4, 129, 128), (9, 8, 2, 193, 64), (6, 2, 1, 63, 128), (1, 2, 2, 2001, 64)])
+                                          (2, 8, 8, 685, 128), (9, 16, 4, 129, 128), (9, 8, 2, 193, 64), (6, 2, 1, 63, 128), (1, 4, 4, 2001, 64)])
 def test_backward_of_64_key_tiles(B, Hq, Hkv, N, D, mask):
     """Small launches: one to 32 steps a tile, rows one past a tile, all heads of a group in one run; hidden keys that would
     outweigh every visible one, a whole tile of them among others, and a sequence without any key."""
@@ -269,6 +269,13 @@ def test_backward_without_memory_for_ds():
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+    held, size = [], 1 << 30                 # what other tests left in the cache is not for this one
+    while size >= 1 << 20:
+        try:
+            held.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+        except torch.cuda.OutOfMemoryError:
+            size >>= 1
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (96 << 20)) / total)
     before = torch.cuda.memory_stats()
     try:

@@ -87,9 +87,10 @@ def test_backward_runs_the_largest_form_that_its_scratch_holds(ask, B, Hq, Hkv, 
 
 def test_every_backward_kernel_is_reached(ask):
     built = {k for k in ask(["kernels"])[0].split() if k.startswith("flash_attn_bwd")}
-    calls = [f"bwd {B} {Hq} {Hkv} {N} {D} {causal} {window if mask != 'keys' else 0} {mask} {ws if ws else B * Hq * ((N + 127) // 128) * 1024}"
-             for B in (1, 4, 16) for Hq, Hkv in ((4, 4), (16, 4), (32, 8)) for N in (64, 300, 700, 1500, 4096) for D in (64, 128)
-             for causal, window in ((0, 0), (1, 0), (1, 50), (1, 600)) for mask in ("none", "lens", "keys") for ws in (0, 1 << 40)]
+    shapes = [f"{B} {Hq} {Hkv} {N} {D} {opt}" for B in (1, 2, 4, 16) for Hq, Hkv in ((1, 1), (8, 2), (4, 4), (32, 8)) for N in (64, 300, 700, 1500, 4096)
+              for D in (64, 128) for opt in ("0 0", "1 0", "1 50", "1 600")]
+    calls = [f"bwd {shape} {mask} {ws}" for shape, sizes in zip(shapes, ask([f"bytes {s}" for s in shapes])) for ws in sizes.split()
+             for mask in ("none", "lens", "keys") if mask != "keys" or shape.endswith(" 0")]
     got = ask(calls)
     assert all(g.startswith("0 ") for g in got)
     assert built == {k.rsplit(":", 1)[0] for g in got for k in g.split()[1:]}
@@ -128,3 +129,25 @@ def test_tiles_of_twice_the_waves_where_they_are_faster(ask, M, N, K, trans_b, s
     got, = ask([f"gemm {M} {N} {K} {trans_b} {size} {1 << 40}"])
     m = re.fullmatch(r"0 \d+ gemm_tile_kernel<gt::Cfg<(1|2),(true|false),(\d+),(\d+),\d+,\d+,(\d+),\d+>>:\d+( gemm_tile_reduce_kernel<\d>:\d+)?", got)
     assert m and (int(m[1]), m[2] == "true", int(m[3]), int(m[4]), int(m[5]), bool(m[6])) == (size, bool(trans_b), rows, cols, groups, split), got
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,opt,form", [
+    (1, 32, 32, 315, 64, "0 0", "one"),         # two launches 17.2, one 14.4, 64-key tiles 15.4 us
+    (10, 32, 8, 222, 64, "0 0", "two"),         # 42.7, 53.1, 55.6
+    (9, 8, 8, 66, 64, "0 0", "one"),            # 11.6, 8.1, 10.4
+    (1, 2, 2, 2001, 64, "1 0", "one"),          # 39.8, 31.3, 37.3
+    (4, 8, 8, 310, 64, "1 0", "half"),          # 20.2, 16.1, 11.3
+    (1, 1, 1, 128, 64, "0 0", "half"),          # the train step of one head
+    (2, 8, 8, 685, 128, "0 0", "one"),          # 40.3, 34.5, 41.0; dS kept 38.6
+    (5, 8, 8, 217, 128, "0 0", "one"),          # 24.6, 17.5, 19.8; 22.5
+    (2, 8, 8, 685, 128, "1 0", "half"),         # 40.4, 38.1, 26.6; 31.9
+    (2, 16, 16, 764, 128, "1 0", "one"),        # 45.4, 40.7, 47.3; 46.0
+    (4, 16, 4, 544, 128, "1 0", "ds"),          # 52.5, 60.2, 68.3; 45.4
+    (1, 32, 8, 2000, 128, "1 0", "ds"),         # 148, -, -; 136
+    (16, 16, 16, 4096, 128, "1 0", "two")])     # dS would take 4.4 GB
+def test_the_form_of_a_backward_is_the_fastest(ask, B, Hq, Hkv, N, D, opt, form):
+    """By the launches of a call with all the scratch it can use; the times are of an MI355X, whole backward."""
+    got, = ask([f"bwd {B} {Hq} {Hkv} {N} {D} {opt} none {1 << 40}"])
+    first = got.split()[1]
+    kind = {"flash_attn_bwd_dq_kernel": "two", "flash_attn_bwd_stats_kernel": "ds", "flash_attn_bwd_both_kernel": "half" if first.split(":")[0].endswith("true>") else "one"}
+    assert kind[first.split("<")[0]] == form, got

@@ -438,5 +438,6 @@ struct AttnOrder {
 // causal launches paired tiles or single ones.  dq: for the dQ kernel, whose steps take other times than the forward's.
 struct AttnShape { int rows, pair, single; };
 AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window, bool dq);
+double attn_us(int64_t bh, int N, int D, bool causal, int window, bool dq);      // its launch, estimated
 
 }  // namespace tyr

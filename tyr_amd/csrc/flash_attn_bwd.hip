@@ -32,7 +32,7 @@
 // Both recompute S (7 matrix products for an algorithm that needs 5): the price of writing dQ
 // without a float atomic accumulation buffer and a conversion pass.
 //
-// Few heads (keeps_ds) run the 5 products: flash_attn_bwd_stats_kernel makes the pairs, dK/dV goes first and leaves
+// Where that is faster (launch_us), and dS fits, the 5 products run: flash_attn_bwd_stats_kernel makes the pairs, dK/dV goes first and leaves
 // its bf16 dS in the workspace, and flash_attn_bwd_dq_product_kernel adds dQ = dS K from there.  Same operands and roundings.
 //
 // LDS tiles are row-major with 16-byte chunks XOR-swizzled by a function of the row that is
@@ -1240,9 +1240,10 @@ __device__ __forceinline__ void bwd_dkv_half(int block,
     if (T == 0) finish(dv, 1.0f, dV); else finish(dk, scale, dK);
 }
 
-// Both at once for launches that leave CUs idle anyway (rule at one_launch): the first `ndkv` workgroups are dK/dV's, the
-// rest dQ's (64-row form).  HALF: dK/dV by bwd_dkv_half (rule at half_steps).  The dQ kernel then need not end before dK/dV starts -- a launch, a prologue and a drain, 3.5 us
-// of 11 for one head of 128 rows, 12 of 41 for 8 heads of 700.
+// Both at once for launches that leave CUs idle anyway (launch_us): the first `ndkv` workgroups are dK/dV's, the
+// rest dQ's (64-row form).  HALF: dK/dV by bwd_dkv_half.
+// The dQ kernel then need not end before dK/dV starts -- a launch, a prologue and a drain, 3.5 us of 11 for one head of 128 rows,
+// 12 of 41 for 8 heads of 700.
 template <int D, bool CAUSAL, AttnMask MASK, bool CUT, bool HALF>
 __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_both_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
@@ -1476,6 +1477,12 @@ int last_cu_steps(const fab::Parts& p, int ntk, int BHkv) {
     }
     return last;
 }
+// traffic of the f32 partials, written and read at 6 TB/s
+double partial_us(const fab::Parts& p, int BHkv, int N, int D) {
+    int64_t cut = 0;
+    for (int kt = 0; kt < (N + 127) / 128; ++kt) cut += p.parts(kt) > 1 ? p.parts(kt) : 0;
+    return cut * BHkv * (128.0 * D * 8 * 2) / 6.0e6;
+}
 // How the dK / dV work is cut.  A workgroup has a CU to itself.  A step (64 queries x 128 keys) takes 1.7 us at D = 128 (1.1
 // at 64) while other CUs are idle and a quarter more with all of them busy (measured: 1.65-1.75 with the last key tiles of
 // a head alone on the device, 2.0-2.2 with 256 equal workgroups, 1.95 in the large launches), a workgroup 2 us to start and
@@ -1483,11 +1490,14 @@ int last_cu_steps(const fab::Parts& p, int ntk, int BHkv) {
 // the finest cut with at most 256, 512 or 768 workgroups.  On 235 shapes (1 to 16 sequences of 64 to 8192 rows, every mask)
 // the choice is 0.2 % slower than the best of the four, at worst 11 % (B6 Hq32 Hkv8 N92).  With 1.55 us for every step and
 // whole tiles taken longest first it was 1.7 %, at worst 45 %: B9 Hq16 Hkv4 N1944 ran whole, 832 us for 573 in parts.
-fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window) {
+struct DkvPlan {
+    fab::Parts parts;
+    double us;
+};
+DkvPlan make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window, bool cut_tiles) {
     const int ntk = (N + 127) / 128, nq = (N + 63) / 64;
     const fab::Parts whole{G, nq, causal, window, 0};
-    fab::Parts best = whole;
-    if (ntk > 64 || (int64_t)ntk * BHkv > 768) return best;
+    DkvPlan best{whole, 1e300};
     const double step = D == 128 ? 1.7 : 1.1;
     int64_t total = 0;
     int most = 1;
@@ -1495,8 +1505,9 @@ fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window)
         total += whole.steps(kt);
         most = std::max(most, whole.steps(kt));
     }
-    double least = 1e300;
-    for (int round = 0; round <= 3; ++round) {
+    const double mean = (double)total * BHkv / 256;           // steps of a CU if all were equally busy
+    const bool few = ntk <= 64 && (int64_t)ntk * BHkv <= 768;
+    for (int round = 0; round <= (cut_tiles && few ? 3 : 0); ++round) {
         fab::Parts p = whole;
         auto count = [&](int chunk) {
             p.chunk = chunk;
@@ -1516,22 +1527,12 @@ fab::Parts make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window)
             for (int kt = 0; kt < ntk; ++kt) cut += p.parts(kt) > 1 ? p.parts(kt) : 0;
             if (cut == 0) continue;
         }
-        const double mean = (double)total * BHkv / 256;       // steps of a CU if all were equally busy
-        double us = step * std::max((double)last_cu_steps(p, ntk, BHkv), 1.25 * mean) + 2.0 * std::max(1.0, n / 256.0);
-        if (round) us += 3.0 + cut * BHkv * (128.0 * D * 8 * 2) / 6.0e6;
-        if (us < least) { least = us; best = p; }
+        const double last = n <= 2048 ? last_cu_steps(p, ntk, BHkv) : mean + 0.5 * most;
+        double us = step * std::max(last, 1.25 * mean) + 2.0 * std::max(1.0, n / 256.0);
+        if (round) us += 3.0 + partial_us(p, BHkv, N, D);
+        if (us < best.us) best = {p, us};
     }
     return best;
-}
-// some microseconds of host time: each thread keeps its last plans
-fab::Parts dkv_plan(int BHkv, int G, int N, int D, bool causal, int window) {
-    struct Entry { int BHkv, G, N, D, causal, window; fab::Parts plan; };
-    static thread_local Entry kept[16];
-    const uint32_t h = ((uint32_t)BHkv * 0x9e3779b1u ^ (uint32_t)N * 0x85ebca6bu ^ (uint32_t)(G * 131 + D) * 0xc2b2ae35u ^ (uint32_t)(window * 2 + causal) * 0x27d4eb2fu) * 0x9e3779b1u;
-    Entry& e = kept[h >> 28];
-    if (e.BHkv != BHkv || e.G != G || e.N != N || e.D != D || e.causal != causal || e.window != window)
-        e = {BHkv, G, N, D, causal, window, make_dkv_plan(BHkv, G, N, D, causal, window)};
-    return e.plan;
 }
 int dkv_items(const fab::Parts& p, int N) {
     const int ntk = (N + 127) / 128;
@@ -1540,36 +1541,6 @@ int dkv_items(const fab::Parts& p, int N) {
     for (int kt = 0; kt < ntk; ++kt) n += p.parts(kt);
     return n;
 }
-// dQ and dK/dV as one launch: where every workgroup gets a CU to itself, and up to 1024 rows while there are not many more
-// than that.  Measured (MI355X, us, two launches -> one): B1 H1 N128 D64 11.0 -> 7.5, B1 H4 N512 D128 causal 27.2 -> 18.3,
-// B1 Hq8 Hkv2 N700 40.6 -> 28.8; 384 workgroups, N1000 43.7 -> 39.8; beyond, a dK/dV workgroup waits longer for the pairs of
-// all its rows and dQ comes last: 512 workgroups, N2048 69 -> 73.
-// Where dS could be kept that is faster from 420 workgroups on (300 not causal): B2 Hq16 Hkv4 N564 full, 528 of them, 59.7 ->
-// 39.7, B2 H8 N707 with a key mask, 448, 38.9 -> 33.4.  On 180 shapes of 60 to 1500 workgroups the choice among the three forms
-// is 0.4 % slower than the best, D = 64 (of two) 0.9 %.
-bool one_launch(int N, int64_t blocks, bool ds, bool causal) {
-    return blocks <= 256 || (N <= 1024 && blocks <= (!ds ? 640 : causal ? 420 : 300));
-}
-// Steps of the longest 64-key tile of a launch that takes bwd_dkv_half, 0 = the launch does not.  One launch, no scratch, half
-// the steps' length; against bwd_dkv a workgroup has twice the parts of a query's K / V to itself and the queries are read
-// twice as often, so it is for tiles of few steps, and with G > 1 (all heads of the group are one tile's steps) for fewer.
-// Measured (us, whole backward, before -> with): D = 128 B2 H16 N218 18.4 -> 14.6, B3 H8 N473 28.1 -> 21.3, B1 H8 N700 full 41.7
-// -> 25.6, B3 H4 N231 window 83 21.7 -> 13.0, B10 H1 N763 34.2 -> 28.0, B5 Hq32 Hkv8 N83 window 65 35.0 -> 22.4; D = 64 B1 H1
-// N128 7.7 -> 6.3, B2 H16 N218 13.5 -> 9.1, B14 H4 N448 19.3 -> 13.3.  On the other side: D = 128 B1 H1 N1024 24.3 -> 33.1 (16
-// steps on 32 workgroups, which parts share better), B2 H4 N1204 full 41.9 -> 47.8, B6 H16 N116 15.4 -> 16.8 (one 128-key tile
-// a head), B1 Hq8 Hkv2 N300 20.2 -> 39.8.  On 432 shapes of up to 1600 workgroups the choice is 0.8 % slower than the best.
-int half_steps(int BH, int BHkv, int N, int D, bool causal, int window) {
-    const int G = BH / BHkv, nq = (N + 63) / 64;
-    const int64_t blocks = (int64_t)(BH + BHkv) * nq;
-    const int seen = causal && window > 0 ? (int)std::min<int64_t>(nq, ((int64_t)window + 62) / 64 + 1) : nq;
-    const int64_t most = (int64_t)G * seen;
-    bool take;
-    if (G > 1) take = blocks <= 1600 && most <= (D == 128 ? (blocks <= 256 ? 4 : 12) : (blocks <= 256 ? 8 : 16));
-    else if (N <= 128) take = blocks <= (D == 128 ? 256 : 400);
-    else if (D == 128) take = blocks <= 400 && most <= std::min<int64_t>(15, std::max<int64_t>(6, blocks / 16));
-    else take = blocks <= 512 && most <= (blocks <= 40 ? 10 : 32);
-    return take ? (int)most : 0;
-}
 size_t half_lds(int D, int steps) { return (size_t)4 * 2 * 64 * D * 2 + (size_t)steps * 64 * sizeof(float2); }
 size_t dkv_partial_bytes(const fab::Parts& p, int BHkv, int N, int D) {
     return p.chunk ? (size_t)BHkv * dkv_items(p, N) * 128 * D * 8 : 0;
@@ -1577,19 +1548,117 @@ size_t dkv_partial_bytes(const fab::Parts& p, int BHkv, int N, int D) {
 size_t ds_bytes(int BH, int N, bool causal, int window) {
     return (size_t)BH * fab::DsBlocks{(N + 127) / 128, causal, window}.head_bytes();
 }
-// Whether dK/dV leave dS for dQ: five products in three launches (pairs, dK/dV, dQ) in place of seven in two.  Worth it while dS
-// stays in the 256 MB last-level cache and the heads are few: beyond, dS costs its traffic to HBM, and many short tiles
-// fill the device in the other form as well.  With G >= 4 query heads a K / V, dQ's share of the requests hits the L2 (any
-// window, more heads); without, a causal launch of few short tiles and one of a narrow window save little.
-// Measured (us, without -> with, whole backward, D = 128): B1 Hq32 Hkv8 N2000 147.5 -> 131.5, B1 Hq4 N6083 201 -> 163, B9 Hq8
-// Hkv2 N900 full 176 -> 145, B15 Hq16 Hkv4 N316 full 96 -> 78; on the other side of the line B12 H16 N555 109 -> 117, B7 Hq32
-// Hkv8 N812 202 -> 206, B1 H32 N563 31 -> 37, B5 Hq8 Hkv2 N2724 (331 MB) 300 -> 307, B16 H16 N4096 (4.4 GB) 3640 -> 3530 with
-// 18 times the scratch.  D = 64: 0.9 to 1.3 times the time, mostly slower.
-bool keeps_ds(int BH, int G, int N, int D, bool causal, int window) {
-    const fab::DsBlocks place{(N + 127) / 128, causal, window};
-    if (D != 128 || place.ntk < 2 || ds_bytes(BH, N, causal, window) > (size_t)288 << 20) return false;
-    if (G >= 4) return BH <= (place.ntk <= 4 ? 256 : 128);
-    return BH <= 64 && (!causal || (place.ntk >= 6 && place.width() >= std::min(place.ntk, 8)));
+// The four forms of a backward: dQ and dK/dV one after the other (seven products); in one launch; dK/dV leaving dS for dQ (five
+// products, three launches); in one launch with 64-key tiles.
+enum Form { TWO, ONE, DS, HALF, FORMS };
+// One of the eight XCDs, which are alike: 32 CUs that take every eighth workgroup of a launch, in its order, as they get free.
+struct Xcd {
+    double free_at[32], last = 0;
+    int64_t at = 0;
+    int busy = 0;
+    void run(double us, int64_t workgroups) {
+        auto later = [](double x, double y) { return x > y; };
+        int64_t mine = (at + workgroups + 7) / 8 - (at + 7) / 8;
+        for (at += workgroups; mine > 0; --mine) {
+            if (busy == 32) std::pop_heap(free_at, free_at + busy, later); else free_at[busy++] = 0;
+            last = std::max(last, free_at[busy - 1] += us);
+            std::push_heap(free_at, free_at + busy, later);
+        }
+    }
+};
+constexpr size_t kMostDs = (size_t)288 << 20;        // the 256 MB last-level cache and what of it is read soon; beyond, 300 -> 307 us at 331 MB
+int half_steps(int G, int N, bool causal, int window) {                 // of the longest 64-key tile
+    const int nq = (N + 63) / 64;
+    return G * (causal && window > 0 ? (int)std::min<int64_t>(nq, ((int64_t)window + 62) / 64 + 1) : nq);
+}
+// What each form takes, in microseconds on an MI355X: the workgroups' times (start and end, and a step: 64 queries x 64 or 128 keys)
+// dealt to the CUs in the launch's order, or the estimates that dQ's and dK/dV's own plans are chosen by, weighted as they
+// follow one another.  Steps take longer with all CUs busy (`crowd`) and with the mask instructions of a window (`edges`).
+// Constants: least squares in the logarithm, weighed towards the choice, over 5100 shapes (heads 1 to 32, 64 to 8192 rows, every
+// mask; graphs of 12 calls), each form within 8 to 14 %.  On 3000 others the form chosen is 0.5 % slower than the best of the four.
+// Examples, two / one / dS / half:  D = 128 B1 Hq32 Hkv8 N2000 149 / - / 137 / -, B2 H16 N483 full 36 / 28 / 33 / 34, B5 H8 N217 full 25
+// / 18 / 22 / 20, B2 H8 N685 40 / 38 / 32 / 27; D = 64 B1 H1 N128 10.5 / 7.7 / - / 6.3, B9 H8 N66 full 11.6 / 8.1 / - / 10.4, B10
+// Hq32 Hkv8 N222 full 43 / 53 / - / 56, B1 H2 N2001 40 / 31 / - / 37.
+struct FormModel {
+    double half, half_wg, half_step;                 // launch; dK/dV workgroup and step
+    double dq_wg, dq_tile;                           // dQ's 64-row workgroups beside either
+    double one, part_wg, part_step, sum, traffic;    // launch; dK/dV; the addition of parts and its partials
+    double two, two_dq, two_dkv;
+    double crowd, edges;
+    double ds, ds_bytes, ds_dkv, ds_tile, ds_mean, ds_sum;      // pairs (and per microsecond of their traffic), dK/dV, product, parts
+};
+constexpr FormModel kModel128{3.1, 3.6, 1.86, 4.1, 0.87, 0.9, 8.4, 2.1, 2.6, 1.6, 6.5, 0.8, 1.31, 0.15, 1.28, 11.2, 0.36, 0.85, 0.23, 1.05, 1.8};
+constexpr FormModel kModel64{2.2, 2.6, 1.08, 2.9, 0.79, 1.5, 5.1, 1.87, 2.6, 0.9, 4.0, 1.06, 1.11, 0.12, 1.09, 0, 0, 0, 0, 0, 0};
+void launch_us(int BH, int BHkv, int N, int D, bool causal, int window, const DkvPlan& plan, double (&us)[FORMS]) {
+    const FormModel& m = D == 128 ? kModel128 : kModel64;
+    const int G = BH / BHkv, nq = (N + 63) / 64, ntk = (N + 127) / 128;
+    const bool edges = window > 0 && window < N, ordered = causal && window <= 0;
+    const int seen = window > 0 ? (int)std::min<int64_t>(nq, ((int64_t)window + 62) / 64 + 1) : nq;      // 64-key tiles of 64 queries
+    const fab::Parts& p = plan.parts;
+    auto step_scale = [&](int64_t workgroups) {
+        return (1.0 + m.crowd * std::min(1.0, std::max(0.0, (workgroups - 200) / 400.0))) * (edges ? m.edges : 1.0);
+    };
+    auto dq = [&](Xcd& x, double scale) {
+        // longest first over all heads, or head after head
+        for (int h = 0; h < (ordered || !causal ? 1 : BH); ++h)
+            for (int qt = nq; qt > 0; --qt)
+                x.run(m.dq_wg + m.dq_tile * scale * (causal ? std::min(qt, seen) : nq), ordered || !causal ? BH : 1);
+    };
+    us[TWO] = m.two + m.two_dq * attn_us(BH, N, D, causal, window, true) + m.two_dkv * plan.us;
+    const double sum = p.chunk ? partial_us(p, BHkv, N, D) : 0.0;
+    us[ONE] = us[DS] = us[HALF] = 1e300;
+    int64_t items = 0;
+    for (int kt = 0; kt < ntk; ++kt) items += p.parts(kt);
+    const int64_t one = items * BHkv + (int64_t)BH * nq, half = (int64_t)(BHkv + BH) * nq;
+    if (one <= 1024) {                               // never the fastest beyond
+        Xcd x;
+        const double scale = step_scale(one), step = m.part_step * scale;
+        if (p.chunk) {
+            for (int kt = 0; kt < ntk; ++kt) x.run(m.part_wg + step * p.part_steps(kt), (int64_t)p.parts(kt) * BHkv);
+        } else {
+            const int heads = BHkv % 8 == 0 ? BHkv / 8 : BHkv;
+            for (int h = 0; h < heads; ++h)
+                for (int kt = 0; kt < ntk; ++kt) x.run(m.part_wg + step * p.steps(kt), BHkv / heads);
+        }
+        dq(x, scale);
+        us[ONE] = m.one + x.last + (p.chunk ? m.sum + m.traffic * sum : 0.0);
+    }
+    if (half <= 1600 && half_lds(D, half_steps(G, N, causal, window)) <= 160 * 1024) {
+        Xcd x;
+        const double scale = step_scale(half), step = m.half_step * (edges ? scale / m.edges : scale);       // its mask is always on
+        for (int kt = 0; kt < nq; ++kt)
+            x.run(m.half_wg + step * G * (std::min(nq, (window > 0 ? kt : 0) + seen) - (causal ? kt : 0)), BHkv);
+        dq(x, scale);
+        us[HALF] = m.half + x.last;
+    }
+    if (D == 128 && ntk > 1 && ds_bytes(BH, N, causal, window) <= kMostDs) {
+        // product: stages of 32 keys, two workgroups a CU
+        const int longest = 2 * (window > 0 ? (int)std::min<int64_t>(nq, ((int64_t)window + 126) / 64 + 1) : nq);
+        double mean = 0;
+        for (int qt = 0; qt < ntk; ++qt) mean += causal ? std::min(longest, 4 * (qt + 1)) : longest;
+        mean *= BH / 512.0;
+        const double scale = edges ? m.edges : 1.0;
+        us[DS] = m.ds + m.ds_bytes * (double)BH * N * D * 4 / 1.0e6 + scale * (m.ds_dkv * plan.us + std::max(m.ds_tile * longest, m.ds_mean * mean)) +
+                 (p.chunk ? m.ds_sum : 0.0);
+    }
+}
+// some microseconds of host time (tens for hundreds of workgroups): each thread keeps its last plans
+struct Launches {
+    fab::Parts parts;
+    double us[FORMS];
+};
+Launches launches(int BH, int BHkv, int N, int D, bool causal, int window, bool cut_tiles) {
+    struct Entry { int BH, BHkv, N, D, causal, window, cut; Launches how; };
+    static thread_local Entry kept[32];
+    const int rule = causal * 2 + cut_tiles;
+    const uint32_t h = ((uint32_t)BHkv * 0x9e3779b1u ^ (uint32_t)N * 0x85ebca6bu ^ (uint32_t)(BH * 131 + D) * 0xc2b2ae35u ^ (uint32_t)(window * 4 + rule) * 0x27d4eb2fu) * 0x9e3779b1u;
+    Entry& e = kept[h >> 27];
+    if (e.BH != BH || e.BHkv != BHkv || e.N != N || e.D != D || e.causal != causal || e.window != window || e.cut != cut_tiles) {
+        const DkvPlan plan = make_dkv_plan(BHkv, BH / BHkv, N, D, causal, window, cut_tiles);
+        e = {BH, BHkv, N, D, causal, window, cut_tiles, {plan.parts, {}}};
+        launch_us(BH, BHkv, N, D, causal, window, plan, e.how.us);
+    }
+    return e.how;
 }
 // What a call does with the scratch it has, and the pieces of that scratch, in this order.  Three forms, each for callers without
 // the memory of the next: the pairs alone (whole key tiles), parts too, dS too.  B1 Hq32 Hkv8 N2000: 254 us with 0.5 MiB, 148
@@ -1606,15 +1675,18 @@ struct BwdPlan {
 };
 BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int D, bool causal, int window, Scratch form) {
     BwdPlan p;
-    p.half = half_steps(B * Hq, B * Hkv, N, D, causal, window);
-    p.parts = p.half ? fab::Parts{Hq / Hkv, (N + 63) / 64, causal, window, 0} : dkv_plan(B * Hkv, Hq / Hkv, N, D, causal, window);
-    if (form == Scratch::Pairs) p.parts.chunk = 0;
+    const int BH = B * Hq, BHkv = B * Hkv;
+    Launches how = launches(BH, BHkv, N, D, causal, window, form != Scratch::Pairs);
+    if (form != Scratch::Ds) how.us[DS] = 1e300;
+    const int pick = (int)(std::min_element(how.us, how.us + FORMS) - how.us);
+    p.parts = how.parts;
+    if (pick == HALF) p.parts.chunk = 0;
+    p.half = pick == HALF ? half_steps(Hq / Hkv, N, causal, window) : 0;
+    p.both = pick == HALF || pick == ONE;
+    p.ds = pick == DS;
     p.items = dkv_items(p.parts, N);
-    p.dq_blocks = (int64_t)B * Hq * ((N + 63) / 64);
-    p.dkv_blocks = (int64_t)B * Hkv * (p.half ? (N + 63) / 64 : p.items);
-    const bool ds = !p.half && form == Scratch::Ds && keeps_ds(B * Hq, Hq / Hkv, N, D, causal, window);
-    p.both = p.half || one_launch(N, p.dq_blocks + p.dkv_blocks, ds, causal);
-    p.ds = ds && !p.both;
+    p.dq_blocks = (int64_t)BH * ((N + 63) / 64);
+    p.dkv_blocks = (int64_t)BHkv * (p.half ? (N + 63) / 64 : p.items);
     p.stat_bytes = flash_attn_bwd_workspace_bytes(B, Hq, N);
     p.partial_bytes = dkv_partial_bytes(p.parts, B * Hkv, N, D);
     p.ds_bytes = p.ds ? ds_bytes(B * Hq, N, causal, window) : 0;

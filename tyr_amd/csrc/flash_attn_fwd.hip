@@ -542,10 +542,10 @@ double busiest_cu_us(const AttnJobs& jobs, int64_t bh, const FormTimes& t, doubl
 }
 }  // namespace
 
-AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window, bool dq) {
+static AttnShape attn_choice(int64_t bh, int N, int D, bool causal, int window, bool dq, double& least) {
     const bool ordered = causal && window <= 0;      // a window makes the tiles equal
     AttnShape best{128, 0, 0};
-    double least = 1e300;
+    least = 1e300;
     for (int form = PAIRS; form < FORMS; ++form) {   // pairs, single tiles, single tiles of 64 rows
         const int rows = form == ROWS64 ? 64 : 128, ntq = (N + rows - 1) / rows;
         if (form == PAIRS && (!ordered || ntq == 1)) continue;
@@ -559,6 +559,15 @@ AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window, bool dq)
         if (us < least) { least = us; best = {rows, form == PAIRS, form != PAIRS && ordered}; }
     }
     return best;
+}
+AttnShape attn_shape(int64_t bh, int N, int D, bool causal, int window, bool dq) {
+    double us;
+    return attn_choice(bh, N, D, causal, window, dq, us);
+}
+double attn_us(int64_t bh, int N, int D, bool causal, int window, bool dq) {
+    double us;
+    attn_choice(bh, N, D, causal, window, dq, us);
+    return us;
 }
 
 int launch_flash_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B,
