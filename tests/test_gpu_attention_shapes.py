@@ -214,6 +214,39 @@ def test_backward_that_keeps_ds(B, Hq, Hkv, N, mask):
     assert all(rel_fro(a, b.float()) <= 1e-3 for a, b in zip(grads, plain))
 
 
+@pytest.mark.parametrize("lengths", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,N,window", [(2, 8, 1, 1029, 68), (5, 4, 4, 927, 102), (7, 4, 4, 708, 321), (7, 4, 4, 768, 257), (3, 32, 8, 850, 389), (1, 8, 2, 2079, 390)])
+def test_kept_ds_of_a_narrow_window(B, Hq, Hkv, N, window, lengths):
+    """dS where a query tile has places for a few key tiles only: windows below and above one tile, whole and cut key tiles, and with
+    lengths (none, one row past a tile), whose hidden keys would outweigh every visible one."""
+    import tyr_amd
+    from tyr_amd import _lib
+    lib, D = _lib.load(), 128
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    q, k, v, g = (torch.randn(B, h, N, D, device="cuda", generator=gen).bfloat16() for h in (Hq, Hkv, Hkv, Hq))
+    i = torch.arange(N, device="cuda")
+    visible = ((i[None, :] <= i[:, None]) & (i[:, None] - i[None, :] < window))[None, None].expand(B, 1, N, N)
+    opt = dict(causal=True, window=window)
+    if lengths:
+        opt["kv_lens"] = torch.tensor(([N // 2 + 1, N, 0, 129, N - 1] * B)[:B], dtype=torch.int32, device="cuda")
+        shown = i[None, :] < opt["kv_lens"][:, None]
+        visible = visible & shown[:, None, None, :]
+        loud = torch.where(shown[:, None, :, None], 1.0, 300.0).bfloat16()
+        k, v = k * loud, v * loud
+    parts, full = (f(B, Hq, Hkv, N, D, 1, window) for f in (lib.tyr_hip_flash_attn_bwd_parts_workspace_bytes, lib.tyr_hip_flash_attn_bwd_full_workspace_bytes))
+    assert full - parts >= B * Hq * N * min(window, N) * 2
+    o, lse = tyr_amd.flash_attn_fwd(q, k, v, **opt)
+    grads = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)
+    *_, wq, wk, wv = reference(q, k, v, g, visible)
+    seen, used = visible.any(-1).expand(B, Hq, N), visible.any(-2).expand(B, Hkv, N)
+    for got, ref, alive in zip(grads, (wq, wk, wv), (seen, used, used)):
+        assert rel_fro(got, ref) <= 1e-2
+        err, n = (got.float() - ref).norm(dim=-1), ref.norm(dim=-1)
+        assert float((err / n.clamp_min(float(n[n > 0].mean()))).max()) <= 8e-2         # as in test_backward_that_keeps_ds
+        assert not bool(got[~alive].any())
+    assert all(torch.equal(a, b) for a, b in zip(grads, tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)))
+
+
 @pytest.mark.parametrize("mask", ["causal", "full", "window", "lens", "keys"])
 @pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 1, 1, 1, 64), (2, 4, 4, 64, 128), (2, 4, 4, 65, 64), (3, 4, 4, 130, 128), (6, 4, 4, 263, 128), (2, 4, 4, 449, 64),
                                           (2, 8, 8, 685, 128), (9, 16, 4, 129, 128), (9, 8, 2, 193, 64), (6, 2, 1, 63, 128), (1, 4, 4, 2001, 64)])
