@@ -125,7 +125,8 @@ __device__ __forceinline__ void store_transposed_bf16(const f32x16 (&acc)[D / 32
 // dQ (and the (lse2, delta) pairs)
 // MASK as in the forward kernel;
 // G = query heads per kv head.  SPLIT: 64 query rows per workgroup, the two 32-key sub-tiles of a tile on two waves whose
-// dQ are added through LDS at the end (same use as in the forward kernel: launches with few tiles).
+// dQ are added through LDS at the end (same use as in the forward kernel: launches with few tiles).  Not causal at D = 128, 39 to
+// 54 registers are too many for two waves a SIMD (160 to 220 bytes a lane in scratch memory; causal none).
 template <int D, bool CAUSAL, AttnMask MASK, bool SPLIT>
 __device__ __forceinline__ void bwd_dq(int block,
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
@@ -975,6 +976,7 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
 // of all of them are made first and stay in LDS, so nothing is written that another workgroup reads.  Bound by latencies: a
 // step is 32 products of 32 cycles a wave and takes 1.6 us (1.0 at D = 64), of which the pairs are a third.  Tried: one
 // product, then its share of the other instructions by scheduling groups (4 % slower), pairs a step ahead instead of first (as slow).
+// Not causal with lengths, six registers too many at D = 128 (28 bytes a lane in scratch memory).
 template <int D, bool CAUSAL, AttnMask MASK>
 __device__ __forceinline__ void bwd_dkv_half(int block,
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
