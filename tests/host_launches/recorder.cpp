@@ -39,7 +39,8 @@ void __hipRegisterFunction(void**, const void* host, char*, const char* name, un
 }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void**, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t lds, hipStream_t) {
+    if (lds > 160 * 1024 || grid.x == 0 || grid.x > 0x7fffffffu || block.x > 1024) abort();
     launched += " " + kernels()[f] + ":" + std::to_string(grid.x);
     return hipSuccess;
 }
