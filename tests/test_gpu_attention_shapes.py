@@ -162,7 +162,7 @@ def test_backward_with_the_least_workspace(B, Hq, Hkv, N, D, mask):
 
 
 @pytest.mark.parametrize("mask", ["causal", "full", "window", "lens", "keys"])
-@pytest.mark.parametrize("B,Hq,Hkv,N", [(4, 16, 4, 577), (4, 16, 4, 640), (4, 16, 16, 769), (2, 32, 8, 1153), (4, 8, 1, 1025), (4, 16, 4, 200)])
+@pytest.mark.parametrize("B,Hq,Hkv,N", [(4, 16, 4, 577), (4, 16, 4, 640), (4, 16, 16, 769), (2, 32, 8, 1153), (4, 8, 1, 1025), (9, 16, 4, 200), (4, 16, 4, 200)])
 def test_backward_that_keeps_ds(B, Hq, Hkv, N, mask):
     """Few heads at D = 128, where dK / dV leave dS for dQ: rows one past a tile, whole tiles, whole and cut key tiles.  Hidden keys
     come first, in the middle (more than one block of 128) and last, with values that would outweigh every visible one."""
@@ -189,7 +189,8 @@ def test_backward_that_keeps_ds(B, Hq, Hkv, N, mask):
     loud = torch.where(shown[:, None, :, None], 1.0, 300.0).bfloat16()
     k, v = k * loud, v * loud
     least = lib.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D)
-    assert lib.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, int(opt["causal"]), window) - least >= B * Hq * N * N
+    if (B, N, mask) != (9, 200, "window"):               # 64-key tiles, as fast (42.8 us, 42.9 with dS)
+        assert lib.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, int(opt["causal"]), window) - least >= B * Hq * N * N
     o, lse = tyr_amd.flash_attn_fwd(q, k, v, **opt)
     grads = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)
     *_, wq, wk, wv = reference(q, k, v, g, visible)
@@ -249,7 +250,7 @@ def test_kept_ds_of_a_narrow_window(B, Hq, Hkv, N, window, lengths):
 
 @pytest.mark.parametrize("mask", ["causal", "full", "window", "lens", "keys"])
 @pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 1, 1, 1, 64), (2, 4, 4, 64, 128), (2, 4, 4, 65, 64), (3, 4, 4, 130, 128), (6, 4, 4, 263, 128), (2, 4, 4, 449, 64),
-                                          (2, 8, 8, 685, 128), (9, 16, 4, 129, 128), (9, 8, 2, 193, 64), (6, 2, 1, 63, 128), (1, 4, 4, 2001, 64)])
+                                          (2, 8, 8, 685, 128), (9, 16, 4, 129, 128), (9, 8, 2, 193, 64), (6, 2, 1, 63, 128), (1, 2, 2, 2001, 64), (1, 4, 4, 2001, 64)])
 def test_backward_of_64_key_tiles(B, Hq, Hkv, N, D, mask):
     """Small launches: one to 32 steps a tile, rows one past a tile, all heads of a group in one run; hidden keys that would
     outweigh every visible one, a whole tile of them among others, and a sequence without any key."""
@@ -276,7 +277,8 @@ def test_backward_of_64_key_tiles(B, Hq, Hkv, N, D, mask):
     k, v = k * loud, v * loud
     lib = _lib.load()
     full = lib.tyr_hip_flash_attn_bwd_full_workspace_bytes(B, Hq, Hkv, N, D, int(opt["causal"]), opt.get("window", 0))
-    assert full == lib.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D)          # no parts, no dS
+    if (Hq, N) != (2, 2001) or mask in ("full", "window"):     # else key tiles in parts: 31.3 us causal, 37.3 with 64-key tiles
+        assert full == lib.tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D)      # no parts, no dS
     o, lse = tyr_amd.flash_attn_fwd(q, k, v, **opt)
     grads = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)
     *_, wq, wk, wv = reference(q, k, v, g, visible)
