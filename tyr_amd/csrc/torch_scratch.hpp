@@ -19,14 +19,16 @@ inline bool can_have(size_t bytes, c10::DeviceIndex device) {
     namespace alloc = c10::hip::HIPCachingAllocator;
     try {
         const auto stats = alloc::getDeviceStats(device);
-        const int64_t reserved = stats.reserved_bytes[0].current, cached = reserved - stats.active_bytes[0].current;
+        using c10::CachingAllocator::StatType;
+        constexpr size_t all = (size_t)StatType::AGGREGATE, large = (size_t)StatType::LARGE_POOL;
+        const int64_t cached = stats.reserved_bytes[large].current - stats.active_bytes[large].current;
         if (cached >= (int64_t)bytes || c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return true;
         size_t free = 0, total = 0;
         if (hipMemGetInfo(&free, &total) != hipSuccess) {
             (void)hipGetLastError();
             return true;
         }
-        const int64_t allowed = (int64_t)(alloc::getMemoryFraction(device) * (double)total) - reserved;
+        const int64_t allowed = (int64_t)(alloc::getMemoryFraction(device) * (double)total) - stats.reserved_bytes[all].current;
         return cached + std::min<int64_t>((int64_t)free, allowed) >= (int64_t)bytes;
     } catch (const c10::Error&) {                     // an allocator that does not tell
         return true;
