@@ -69,8 +69,7 @@ def test_scratch_queries_take_any_length(ask):
 @pytest.mark.parametrize("mask", ["none", "lens", "keys"])
 def test_backward_runs_the_largest_form_that_its_scratch_holds(ask, B, Hq, Hkv, N, D, causal, window, mask):
     """dS kept, else key tiles cut into parts, else whole key tiles: one byte less than a form needs gives the next one."""
-    if mask == "keys" and window:
-        pytest.skip("refused")
+    window = 0 if mask == "keys" else window
     shape = f"{B} {Hq} {Hkv} {N} {D} {causal} {window}"
     least, parts, full = map(int, ask([f"bytes {shape}"])[0].split())
     sizes = [least - 1, least, parts - 1, parts, full - 1, full, 1 << 40]
@@ -81,8 +80,9 @@ def test_backward_runs_the_largest_form_that_its_scratch_holds(ask, B, Hq, Hkv, 
         assert got[parts - 1] == got[least] and "_sum_kernel" in got[parts] and "_product_" not in got[parts]
     if full > parts:
         assert got[full - 1] == got[parts] and "_stats_kernel" in got[full] and "_product_kernel" in got[full]
-    assert (full > parts, parts > least) == {2000: (True, True), 1500: (True, True), 3000: (True, False), 700: (False, True), 2049: (False, True),
-                                             100: (False, False), 4096: (False, False)}[N]
+    kept, cut = {2000: (True, True), 1500: (True, True), 3000: (True, not window), 700: (False, True), 2049: (False, True),
+                 100: (False, False), 4096: (False, False)}[N]
+    assert (full > parts, parts > least) == (kept, cut)
 
 
 def test_every_backward_kernel_is_reached(ask):
