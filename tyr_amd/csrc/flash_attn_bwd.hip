@@ -1568,7 +1568,7 @@ struct Xcd {
         }
     }
 };
-constexpr size_t kMostDs = (size_t)288 << 20;        // the 256 MB last-level cache and what of it is read soon; beyond, 300 -> 307 us at 331 MB
+constexpr size_t kMostDs = (size_t)288 << 20;        // about the 256 MB last-level cache; with 331 MB B5 Hq8 Hkv2 N2724 300 -> 307 us
 int half_steps(int G, int N, bool causal, int window) {                 // of the longest 64-key tile
     const int nq = (N + 63) / 64;
     return G * (causal && window > 0 ? (int)std::min<int64_t>(nq, ((int64_t)window + 62) / 64 + 1) : nq);
@@ -1576,8 +1576,9 @@ int half_steps(int G, int N, bool causal, int window) {                 // of th
 // What each form takes, in microseconds on an MI355X: the workgroups' times (start and end, and a step: 64 queries x 64 or 128 keys)
 // dealt to the CUs in the launch's order, or the estimates that dQ's and dK/dV's own plans are chosen by, weighted as they
 // follow one another.  Steps take longer with all CUs busy (`crowd`) and with the mask instructions of a window (`edges`).
-// Constants: least squares in the logarithm, weighed towards the choice, over 5100 shapes (heads 1 to 32, 64 to 8192 rows, every
-// mask; graphs of 12 calls), each form within 8 to 14 %.  On 3000 others the form chosen is 0.5 % slower than the best of the four.
+// The constants are near what single workgroups measure and are fitted to make the choice, over 5100 shapes (heads 1 to 32, 64 to 8192
+// rows, every mask; graphs of 12 calls); a form's estimate is within 8 to 14 %.  On 3000 other shapes the form chosen is 0.5 %
+// slower than the best of the four.
 // Examples, two / one / dS / half:  D = 128 B1 Hq32 Hkv8 N2000 149 / - / 137 / -, B2 H16 N483 full 36 / 28 / 33 / 34, B5 H8 N217 full 25
 // / 18 / 22 / 20, B2 H8 N685 40 / 38 / 32 / 27; D = 64 B1 H1 N128 10.5 / 7.7 / - / 6.3, B9 H8 N66 full 11.6 / 8.1 / - / 10.4, B10
 // Hq32 Hkv8 N222 full 43 / 53 / - / 56, B1 H2 N2001 40 / 31 / - / 37.
@@ -1587,7 +1588,7 @@ struct FormModel {
     double one, part_wg, part_step, sum, traffic;    // launch; dK/dV; the addition of parts and its partials
     double two, two_dq, two_dkv;
     double crowd, edges;
-    double ds, ds_bytes, ds_dkv, ds_tile, ds_mean, ds_sum;      // pairs (and per microsecond of their traffic), dK/dV, product, parts
+    double ds, ds_bytes, ds_dkv, ds_tile, ds_mean, ds_sum;      // launches; pairs, per MB of O and dO; dK/dV; product: longest, mean; parts
 };
 constexpr FormModel kModel128{3.1, 3.6, 1.86, 4.1, 0.87, 0.9, 8.4, 2.1, 2.6, 1.6, 6.5, 0.8, 1.31, 0.15, 1.28, 11.2, 0.36, 0.85, 0.23, 1.05, 1.8};
 constexpr FormModel kModel64{2.2, 2.6, 1.08, 2.9, 0.79, 1.5, 5.1, 1.87, 2.6, 0.9, 4.0, 1.06, 1.11, 0.12, 1.09, 0, 0, 0, 0, 0, 0};
@@ -1612,7 +1613,7 @@ void launch_us(int BH, int BHkv, int N, int D, bool causal, int window, const Dk
     int64_t items = 0;
     for (int kt = 0; kt < ntk; ++kt) items += p.parts(kt);
     const int64_t one = items * BHkv + (int64_t)BH * nq, half = (int64_t)(BHkv + BH) * nq;
-    if (one <= 1024) {                               // never the fastest beyond
+    if (one <= 1024) {                               // hardly ever the fastest beyond (2 of 1650 shapes)
         Xcd x;
         const double scale = step_scale(one), step = m.part_step * scale;
         if (p.chunk) {
@@ -1653,7 +1654,7 @@ Launches launches(int BH, int BHkv, int N, int D, bool causal, int window, bool 
     struct Entry { int BH, BHkv, N, D, causal, window, cut; Launches how; };
     static thread_local Entry kept[32];
     const int rule = causal * 2 + cut_tiles;
-    const uint32_t h = ((uint32_t)BHkv * 0x9e3779b1u ^ (uint32_t)N * 0x85ebca6bu ^ (uint32_t)(BH * 131 + D) * 0xc2b2ae35u ^ (uint32_t)(window * 4 + rule) * 0x27d4eb2fu) * 0x9e3779b1u;
+    const uint32_t h = ((uint32_t)BHkv * 0x9e3779b1u ^ (uint32_t)N * 0x85ebca6bu ^ ((uint32_t)BH * 131u + (uint32_t)D) * 0xc2b2ae35u ^ (uint32_t)(window * 4 + rule) * 0x27d4eb2fu) * 0x9e3779b1u;
     Entry& e = kept[h >> 27];
     if (e.BH != BH || e.BHkv != BHkv || e.N != N || e.D != D || e.causal != causal || e.window != window || e.cut != cut_tiles) {
         const DkvPlan plan = make_dkv_plan(BHkv, BH / BHkv, N, D, causal, window, cut_tiles);
