@@ -426,6 +426,19 @@ struct Parts {
     __host__ __device__ int steps(int kt) const { return G * (last(kt) - first(kt)); }
     __host__ __device__ int parts(int kt) const { return chunk == 0 ? 1 : (steps(kt) + chunk - 1) / chunk; }
     __host__ __device__ int part_steps(int kt) const { const int n = parts(kt); return (steps(kt) + n - 1) / n; }
+    // Whole key tiles: the head (of those of an XCD, or of all) and the key tile of workgroup `slot`.  An XCD deals its workgroups
+    // to its four shader engines in turn, in order: one whose engine has no free CU holds up all behind it.  Causal tiles are of
+    // unequal length (the first meets every query tile, the last one two), so neighbours in the order are the same tile of eight
+    // heads.  Head after head instead, CUs stood idle for 5 to 25 %
+    // of the launch: dK/dV of B16 H16 N4096 2367 us, 2232 in this order, of B32 H32 N512 362 and 273, at D = 64 of B16 H32 N1024 324 and 266.
+    // Equal tiles go head after head: their Q / dO then share the L2.
+    __host__ __device__ int order(int slot, int heads, bool xcds, int tiles, int& kt) const {
+        const int unit = causal && window <= 0 ? (xcds ? 8 : 32) : 1;
+        const int first = slot / (unit * tiles) * unit, n = heads - first < unit ? heads - first : unit;
+        const int at = slot - first * tiles;
+        kt = at / n;
+        return first + at % n;
+    }
     // item = position in the list of all parts of a kv head (chunk > 0: there are at most 64 key tiles)
     __device__ void find(int item, int ntk, int& kt, int& part) const {
         const int lane = threadIdx.x & 63;
@@ -483,17 +496,16 @@ __device__ __forceinline__ void bwd_dkv(int block,
 
     int bh, item;                         // bh indexes (batch, kv head)
     {
-        const int id = block;
-        // causal: key tile 0 meets every query tile, so heavy first; parts of all kv heads of an XCD in that order, or
-        // head after head where whole key tiles are many (their Q / dO then share the L2)
-        if ((BHkv & 7) == 0) {
-            const int xcd = id & 7, slot = id >> 3, heads = BHkv >> 3;
-            bh = (CUT ? slot % heads : slot / items) * 8 + xcd;
-            item = CUT ? slot / heads : slot % items;
+        const bool xcds = (BHkv & 7) == 0;           // heads are dealt to XCDs
+        const int heads = xcds ? BHkv >> 3 : BHkv, slot = xcds ? block >> 3 : block;
+        if constexpr (CUT) {
+            // part after part of all heads, the heaviest first
+            bh = slot % heads;
+            item = slot / heads;
         } else {
-            bh = CUT ? id % BHkv : id / items;
-            item = CUT ? id / BHkv : id % items;
+            bh = plan.order(slot, heads, xcds, items, item);
         }
+        if (xcds) bh = bh * 8 + (block & 7);
     }
     int kt = item, part = 0;
     if constexpr (CUT) plan.find(item, ntk, kt, part);
@@ -1454,28 +1466,29 @@ size_t flash_attn_bwd_workspace_bytes(int B, int H, int N) {
 }
 
 namespace {
-// Steps until the last of 32 CUs (those of an XCD; 256 where heads are not dealt to XCDs) is done when workgroups go to free
-// CUs in the launch's order (bwd_dkv): head after head for whole key tiles, part after part of all heads where they are cut.
+// Steps until the last of an XCD's 32 CUs is done.  It gets every eighth workgroup of the launch and deals them to its four
+// engines of eight CUs in turn; the next one waits until the engine whose turn it is has a free CU (fab::Parts::order).
 int last_cu_steps(const fab::Parts& p, int ntk, int BHkv) {
-    const int cus = BHkv % 8 == 0 ? 32 : 256, heads = BHkv % 8 == 0 ? BHkv / 8 : BHkv;
-    int busy[256], n = 0, last = 0;                  // a heap, the CU that is free first on top
-    auto later = [](int x, int y) { return x > y; };
+    const bool xcds = BHkv % 8 == 0;
+    const int heads = xcds ? BHkv / 8 : BHkv, stride = xcds ? 1 : 8;
+    int busy[4][8] = {}, n = 0, started = 0, last = 0;
     auto job = [&](int steps) {
-        if (n == cus) {
-            std::pop_heap(busy, busy + n, later);
-            busy[n - 1] += steps;
-        } else {
-            busy[n++] = steps;
-        }
-        last = std::max(last, busy[n - 1]);
-        std::push_heap(busy, busy + n, later);
+        int* cu = std::min_element(busy[n & 3], busy[n & 3] + 8);
+        ++n;
+        started = std::max(started, *cu);
+        *cu = started + steps;
+        last = std::max(last, *cu);
     };
     if (p.chunk) {
-        for (int kt = 0; kt < ntk; ++kt)
-            for (int i = p.parts(kt) * heads; i > 0; --i) job(p.part_steps(kt));
+        for (int kt = 0, at = 0; kt < ntk; ++kt)
+            for (const int end = at + p.parts(kt) * heads; at < end; ++at)
+                if (at % stride == 0) job(p.part_steps(kt));
     } else {
-        for (int h = 0; h < heads; ++h)
-            for (int kt = 0; kt < ntk; ++kt) job(p.steps(kt));
+        for (int at = 0; at < heads * ntk; at += stride) {
+            int kt;
+            p.order(at, heads, xcds, ntk, kt);
+            job(p.steps(kt));
+        }
     }
     return last;
 }
@@ -1532,7 +1545,8 @@ DkvPlan make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window, bo
         const double last = n <= 2048 ? last_cu_steps(p, ntk, BHkv) : mean + 0.5 * most;
         double us = step * std::max(last, 1.25 * mean) + 2.0 * std::max(1.0, n / 256.0);
         if (round) us += 3.0 + partial_us(p, BHkv, N, D);
-        if (us < best.us) best = {p, us};
+        // (a tie goes to the parts at D = 128: B5 Hq32 Hkv8 N1325 294 us in parts, 296 whole, estimated 4 % apart the other way)
+        if (us < best.us * (best.parts.chunk == 0 && D == 128 ? 1.045 : 1.0)) best = {p, us};
     }
     return best;
 }
