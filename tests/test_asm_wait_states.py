@@ -1,0 +1,112 @@
+"""Wait states around the matrix products that flash_attn_bwd_dkv_wide_kernel issues in asm, where the compiler, which puts
+them in for its own products, does not see any.  The kernel file is compiled to gfx950 assembly (no GPU needed) and every product
+of those kernels is checked against the instructions around it, with the body of every loop entered twice:
+  * no operand is written by an ordinary vector instruction less than 2 wait states before the product,
+  * no result is read or written by another kind of instruction less than 8 (16x16x32) or 12 (32x32x16) wait states behind it,
+  * no accumulator operand of a product in flight is written.
+An instruction is one wait state, s_nop n is n + 1."""
+import os
+import re
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tyr_amd", "csrc")
+HIPCC = "/opt/rocm/bin/hipcc"
+
+
+def registers(text):
+    """(class, index) of every vector register that a list of operands names."""
+    out = set()
+    for c, lo, hi, one in re.findall(r"\b([va])(?:\[(\d+):(\d+)\]|(\d+)\b)", text):
+        out |= {(c, i) for i in (range(int(lo), int(hi) + 1) if lo else (int(one),))}
+    return out
+
+
+def operands(line):
+    name, _, rest = line.partition(" ")
+    ops, depth, cur = [], 0, ""
+    for ch in rest:
+        depth += (ch == "[") - (ch == "]")
+        if ch == "," and depth == 0:
+            ops.append(cur.strip())
+            cur = ""
+        else:
+            cur += ch
+    return name, [o for o in ops + [cur.strip()] if o]
+
+
+def straight(lines):
+    """Instructions with every backward branch taken once more."""
+    at = {m.group(1): i for i, l in enumerate(lines) if (m := re.match(r"(\.L\w+):", l))}
+    out = []
+    for i, l in enumerate(lines):
+        if not l.endswith(":"):
+            out.append(l)
+        m = re.match(r"s_c?branch\S*\s+(\.L\w+)", l)
+        if m and at.get(m.group(1), i + 1) <= i:
+            out += [x for x in lines[at[m.group(1)]:i + 1] if not x.endswith(":")]
+    return out
+
+
+def violations(code):
+    bad, now = [], 0
+    vector_write, result, source = {}, {}, {}     # register -> wait state of its last write; (wait state, needed) of a product's result, operand
+    for line in code:
+        name, ops = operands(line)
+        if name == "s_nop":
+            now += int(ops[0], 0) + 1
+            continue
+        now += 1
+        if name.startswith("v_mfma"):
+            need = 12 if "32x32" in name else 8
+            dst, a, b, c = (registers(o) for o in ops[:4])
+            bad += [line for r in a | b | c if now - vector_write.get(r, -99) <= 2]
+            bad += [line for r in (a | b) & result.keys() if now - result[r][0] <= result[r][1]]
+            for r in dst:
+                result[r] = (now, need)
+            for r in c:
+                source[r] = (now, need)
+            continue
+        used = registers(" ".join(ops))
+        bad += [line for r in used & result.keys() if now - result[r][0] <= result[r][1]]
+        stores = name.startswith(("global_store", "buffer_", "ds_write", "scratch_store", "s_"))
+        written = set() if stores or not ops else registers(ops[0]) | (registers(ops[1]) if "swap" in name else set())
+        bad += [line for r in written & source.keys() if now - source[r][0] <= source[r][1]]
+        for r in written:
+            result.pop(r, None)
+            if name.startswith("v_"):
+                vector_write[r] = now
+            else:
+                vector_write.pop(r, None)
+    return bad
+
+
+def wide_kernels(path):
+    with open(path) as f:
+        text = f.read()
+    for m in re.finditer(r"^(_ZN3tyr30flash_attn_bwd_dkv_wide_kernel\w+):(.*?)^\.Lfunc_end", text, re.S | re.M):
+        lines = [l.split(";")[0].split("//")[0].strip() for l in m.group(2).split("\n")]
+        yield m.group(1), [l for l in lines if l and (l.endswith(":") or not l.startswith("."))]
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+def test_products_in_asm_keep_their_distance(tmp_path):
+    out = str(tmp_path / "bwd.s")
+    subprocess.check_call([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                           "--cuda-device-only", "-S", os.path.join(CSRC, "flash_attn_bwd.hip"), "-o", out], stderr=subprocess.DEVNULL)
+    kernels = dict(wide_kernels(out))
+    assert kernels
+    for name, lines in kernels.items():
+        assert sum(l.startswith("v_mfma") for l in lines) >= 96, name
+        assert violations(straight(lines)) == [], name
+
+
+def test_what_comes_too_early_is_found():
+    mfma = "v_mfma_f32_16x16x32_bf16 v[0:3], v[4:7], v[8:11], v[0:3]"
+    assert violations(["v_mov_b32 v4, 0", mfma]) and not violations(["v_mov_b32 v4, 0", "s_nop 1", mfma])
+    assert violations([mfma, "s_nop 6", "v_mul_f32 v20, v1, v1"]) and not violations([mfma, "s_nop 7", "v_mul_f32 v20, v1, v1"])
+    assert violations([mfma, "ds_read_b128 v[0:3], v30"]) and not violations([mfma, mfma])
+    acc = "v_mfma_f32_32x32x16_bf16 a[0:15], v[4:7], v[8:11], a[0:15]"
+    assert violations([acc, "s_nop 7", "v_accvgpr_read_b32 v20, a3"])
+    assert violations(straight([".LBB0_1:", "v_mul_f32 v20, v1, v1", mfma, "s_cbranch_scc1 .LBB0_1"]))

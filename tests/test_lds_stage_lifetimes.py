@@ -302,6 +302,42 @@ def test_a_dkv_wait_that_left_one_more_in_flight_would_be_caught():
     assert not all(all(dkv_waits(9, w, with_stores=18)) for w in range(4))
 
 
+# ------------------------------------------------------------------ flash_attn_bwd_dkv_wide_kernel
+def dkv_wide_wave(ntile, stages=4):
+    """Tiles as above, sub-tile u = 4t + T.  A step on u reads the transposed fragments of u and, ahead, the last row fragments of u+1
+    and the others of u+2.  No wait for LDS reads in front of a barrier: what the last step before it read ahead may return behind it."""
+    t = Trace()
+
+    def rd(u):
+        if u < 4 * ntile:
+            t.read(f"T{u // 4 % stages}", u // 4)
+
+    for k in range(3):
+        t.dma(f"T{k % stages}", k)
+    t.wait(keep_newest=2)
+    t.bar()
+    for u in (0, 1):
+        rd(u)
+    for tile in range(ntile):
+        t.wait(keep_newest=1)
+        t.bar()
+        rd(4 * tile + 1)                                 # read ahead by the step before
+        t.dma(f"T{(tile + 3) % stages}", tile + 3)
+        for u in range(4 * tile, 4 * tile + 4):
+            for ahead in range(3):
+                rd(u + ahead)
+    return t
+
+
+@pytest.mark.parametrize("ntile", [1, 2, 3, 4, 5, 9, 64])
+def test_backward_dkv_wide_kernel(ntile):
+    assert violations([dkv_wide_wave(ntile) for _ in range(4)]) == []
+
+
+def test_three_stages_would_not_be_enough_for_the_wide_kernel():
+    assert violations([dkv_wide_wave(6, stages=3) for _ in range(4)])
+
+
 def dkv_half_wave(steps, stages=4):
     """64-key tiles: T0..T3 hold Q and dO of 64 query rows, three requested ahead (zeros past the last).  Step t reads the row
     fragments of tile t+1 and the transposed ones of tile t; the exchange and the output go through the stages."""

@@ -92,6 +92,18 @@ __device__ __forceinline__ float dot8_bf16(u32x4 a, u32x4 b) {
     return s;
 }
 
+// What the dK / dV workgroups need of a query row: (lse * log2 e, delta), or for the wide kernel, by groups of four rows, four
+// lse * log2 e and four -delta (16 bytes each: what a lane's scores need; its dP starts from -delta).
+__device__ __forceinline__ void store_stats(float2* head, int row, float lse2, float delta, int fours) {
+    if (fours) {
+        float* to = reinterpret_cast<float*>(head + (row & ~3)) + (row & 3);
+        to[0] = lse2;
+        to[4] = -delta;
+    } else {
+        head[row] = make_float2(lse2, delta);
+    }
+}
+
 // One wave's 32 columns x D rows accumulator (lane = column l%32, register e of tile dt <-> row
 // 32 dt + 8(e/4) + 4(l/32) + e%4), scaled, written as bf16 rows of length D: out row = column.
 // Goes through a private LDS scratch so the global stores are 16 bytes per lane along rows.
@@ -133,7 +145,7 @@ __device__ __forceinline__ void bwd_dq(int block,
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
     uint16_t* __restrict__ dQ, float2* __restrict__ stats, int BH, int N, int ntq, int npad, float scale,
     float scale_log2, int Hq, int G, int window, const int* __restrict__ kv_lens,
-    const uint8_t* __restrict__ key_mask, int pair, int single) {
+    const uint8_t* __restrict__ key_mask, int pair, int single, int fours) {
     using namespace fab;
     using C = CfgQ<D>;
     constexpr bool LIMITS = MASK == AttnMask::Limits, KEYS = MASK == AttnMask::Keys;
@@ -185,7 +197,7 @@ __device__ __forceinline__ void bwd_dq(int block,
         lse2 = LSE[(size_t)bh * N + qrow] * LOG2E;
         if (MASK != AttnMask::None && lse2 == -INFINITY) lse2 = INFINITY;      // a row that saw no key: every probability is 0
         if (stats != nullptr && g == 0 && T0 == 0) {
-            stats[(size_t)bh * npad + qpos] = qpos < N ? make_float2(lse2, delta) : make_float2(INFINITY, 0.0f);
+            store_stats(stats + (size_t)bh * npad, qpos, qpos < N ? lse2 : INFINITY, qpos < N ? delta : 0.0f, fours);
         }
     }
 
@@ -398,9 +410,9 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
     uint16_t* __restrict__ dQ, float2* __restrict__ stats, int BH, int N, int ntq, int npad, float scale,
     float scale_log2, int Hq, int G, int window, const int* __restrict__ kv_lens,
-    const uint8_t* __restrict__ key_mask, int pair, int single) {
+    const uint8_t* __restrict__ key_mask, int pair, int single, int fours) {
     bwd_dq<D, CAUSAL, MASK, SPLIT>(blockIdx.x, Q, Kp, Vp, O, dO, LSE, dQ, stats, BH, N, ntq, npad, scale, scale_log2, Hq, G, window,
-                                   kv_lens, key_mask, pair, single);
+                                   kv_lens, key_mask, pair, single, fours);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -416,11 +428,12 @@ __global__ __launch_bounds__(fab::THREADS, 2) void flash_attn_bwd_dq_kernel(
 namespace fab {
 struct Parts {
     int G, nq, causal, window, chunk;                // chunk = 0: one part per key tile
+    int keys;                                        // of a key tile: 128, or 256 (flash_attn_bwd_dkv_wide_kernel, chunk = 0)
     // 64-row query tiles that see key tile kt: [first(kt), last(kt))
-    __host__ __device__ int first(int kt) const { return causal ? 2 * kt : 0; }
+    __host__ __device__ int first(int kt) const { return causal ? keys / 64 * kt : 0; }
     __host__ __device__ int last(int kt) const {
-        if (window <= 0) return nq;                  // the last query that sees a key of the tile is 128 kt + 127 + window - 1
-        const int64_t e = ((int64_t)128 * kt + 126 + window) / 64 + 1;
+        if (window <= 0) return nq;                  // the last query that sees a key of the tile is keys (kt + 1) - 1 + window - 1
+        const int64_t e = ((int64_t)keys * kt + keys - 2 + window) / 64 + 1;
         return e < nq ? (int)e : nq;
     }
     __host__ __device__ int steps(int kt) const { return G * (last(kt) - first(kt)); }
@@ -982,6 +995,369 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_kernel(
                                          Hq, window, kv_lens, key_mask, plan, items, partial, ds);
 }
 
+// ------------------------------------------------------------------------------------------
+// dK, dV of 256 keys for launches of many whole key tiles (after a dQ launch that has left the statistics of the rows in groups
+// of four): 4 waves of 64 keys, each over all rows of every query tile.
+//
+// One wave a SIMD, so what a wave issues between two products is what bounds it, and LDS reads are the dearest of that (an
+// instruction every 5 ns and wave).  With 64 keys a wave instead of bwd_dkv's 32, each fragment read serves twice the products,
+// and what a workgroup takes to start and end (14 us) is paid half as often.  That takes all 512 registers: the 256
+// accumulation registers are dK and dV of 64 x 128, K and V fragments 128 of the others.  Scores come in sub-tiles of 16 query
+// rows by 16x16x32 products, whose results take half the registers of 32x32 ones; a row exchange (v_permlane16_swap)
+// makes P and dS of two of their 16-key blocks the column operand of a 32x32x16 product.  All products are in asm: the compiler has all results
+// of its own in accumulation registers here, or none, and copies the others back and forth.
+// dK/dV by bwd_dkv and by this: B16 H16 N4096 causal 2232 and 1850 us, at D = 64 1370 and 1170; B8 H16 N4096 not causal 2050 and 1600.
+namespace fab {
+// The bank swizzle for row fragments of 16 rows x 64 bytes.  A 16-byte LDS read serves lanes {0-3, 12-15, 20-27} at once, then
+// {4-11, 16-19, 28-31}: rows 0-3 and 12-15 of one chunk with rows 4-11 of the next (rows of the product; as query rows, bits 2 and 3
+// are exchanged).  The two low bits keep those apart (SQ_LDS_BANK_CONFLICT 0.3 of the LDS cycles with swz, none so); the upper ones are swz's.
+template <int D> __device__ __forceinline__ int swz16(int row, int c) {
+    const int low = (((row >> 3) ^ (row >> 2)) & 1) << 1 | ((row >> 2) & 1);
+    return c ^ ((D == 128 ? (row & 3) << 2 : ((row >> 1) & 1) << 2) | low);
+}
+// P and dS of a lane (slot j <-> query row 8 (j / 4) + j % 4) set to 0 where gap + that row is not below `seen`
+__device__ __forceinline__ void clear_hidden_pairs(uint32_t gap, uint32_t seen, bf16x8& p, bf16x8& d) {
+    u32x4 keep;
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+        const uint32_t row = 8 * (y >> 1) + 2 * (y & 1);
+        keep[y] = (gap + row < seen ? 0xffffu : 0u) | (gap + row + 1 < seen ? 0xffff0000u : 0u);
+    }
+    p = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, p) & keep);
+    d = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, d) & keep);
+}
+}  // namespace fab
+
+template <int D, bool CAUSAL, AttnMask MASK>
+__global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_wide_kernel(
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
+    const uint16_t* __restrict__ dO, const float2* __restrict__ stats, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int BHkv, int N,
+    int npad, float scale, float scale_log2, int Hq, int window, const int* __restrict__ kv_lens,
+    const uint8_t* __restrict__ key_mask, fab::Parts plan, int items) {
+    constexpr bool WINDOW = MASK == AttnMask::Limits, PER_KEY = MASK != AttnMask::None;
+    constexpr int BNK = 256, NSUB = 4;               // keys of the workgroup; 16-row sub-tiles of a query tile
+    const int G = plan.G;
+    using namespace fab;
+    using C = CfgK<D>;
+    constexpr int KS = D / 32;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+
+    const int t = threadIdx.x;
+    const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int l16 = lane & 15, g4 = lane >> 4;
+
+    const bool xcds = (BHkv & 7) == 0;               // heads are dealt to XCDs
+    int kt;
+    int bh = plan.order(xcds ? blockIdx.x >> 3 : blockIdx.x, xcds ? BHkv >> 3 : BHkv, xcds, items, kt);
+    bh = __builtin_amdgcn_readfirstlane(xcds ? bh * 8 + (int)(blockIdx.x & 7) : bh);        // of (batch, kv head)
+    kt = __builtin_amdgcn_readfirstlane(kt);
+    const int n0 = kt * BNK;
+    const int nw0 = n0 + 64 * w;                                      // this wave's first key
+    const size_t head_off = (size_t)bh * N * D;                       // of K, V, dK, dV
+    const int hkv = Hq / G;
+    const size_t qh0 = (size_t)(bh / hkv) * Hq + (size_t)(bh % hkv) * G;   // first query head of the group
+    const int Nk = (PER_KEY && kv_lens != nullptr) ? max(0, min(N, kv_lens[bh / hkv])) : N;
+    // no key of the block is seen by any query (beyond the length, or all hidden by the key mask)
+    bool block_hidden = PER_KEY && n0 >= Nk;
+    if (PER_KEY && key_mask != nullptr && !block_hidden) {
+        const TileSpan span = visible_tiles(key_mask + (size_t)(bh / hkv) * N + n0, min(BNK, Nk - n0), lane);
+        block_hidden = span.first >= span.last;
+    }
+    // the query tiles that see the block's keys, head after head of the group
+    const int jq_first = plan.first(kt), jq_last = __builtin_amdgcn_readfirstlane(plan.last(kt));
+    const int ntile = __builtin_amdgcn_readfirstlane(block_hidden ? 0 : G * (jq_last - jq_first));
+
+    // ---- Q / dO / statistics loaders
+    // The G query heads of the group are adjacent in memory: one buffer covers them, a head is a
+    // scalar offset.  (Rows past N of a head then alias the next head's first rows instead of
+    // reading as zero; their statistics are (+inf, 0), so their probabilities are exactly 0 either way.)
+    const uint32_t head_bytes = (uint32_t)N * D * 2u;
+    const u32x4 q_rsrc = make_raw_rsrc(Q + qh0 * N * D, head_bytes * (uint32_t)G);
+    const u32x4 do_rsrc = make_raw_rsrc(dO + qh0 * N * D, head_bytes * (uint32_t)G);
+    const uint32_t stat_bytes = (uint32_t)npad * 8u;
+    const u32x4 st_rsrc = make_raw_rsrc(stats + qh0 * npad, stat_bytes * (uint32_t)G);
+    // Request m of a wave fills the kilobyte at 4 KB m + 1 KB w of a tile: the rows of one swizzle, so that one register of
+    // per-lane offsets serves all of them.
+    static_assert(C::PT * 4096 == C::TILE, "a request of each of four waves is 4 KB");
+    int g_voff;
+    {
+        const int row = w * (1024 / C::ROW) + lane / C::KCH;
+        g_voff = row * C::ROW + swz16<D>(row, lane % C::KCH) * 16;
+    }
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
+    const uint32_t wave_dst = __builtin_amdgcn_readfirstlane(lds_base + (uint32_t)w * 1024u);
+    // Query tile `rq_jq` of head `rq_head`, piece by piece.  Tiles past the last are requested at an offset beyond the
+    // buffer (they read as zero), so that every iteration issues the same number of loads and the wait count below stays constant.
+    int rq_head = 0, rq_jq = jq_first, rq_left = ntile;
+    int rq_at = 0, rq_stats_at = 0;                  // offsets of the tile that is being requested
+    auto request_begin = [&] {
+        rq_at = __builtin_amdgcn_readfirstlane(rq_left > 0 ? rq_head * (int)head_bytes + rq_jq * C::BQ * C::ROW : (int)(head_bytes * (uint32_t)G));
+        rq_stats_at = __builtin_amdgcn_readfirstlane(rq_left > 0 ? (rq_head * npad + rq_jq * C::BQ) * 8 : (int)(stat_bytes * (uint32_t)G));
+        --rq_left;
+        if (++rq_jq == jq_last) { rq_jq = jq_first; ++rq_head; }
+    };
+    auto request_piece = [&](int stage, int m) {
+        const uint32_t dst = wave_dst + (uint32_t)stage * C::STAGE + 4096u * m;
+        load_global_to_lds_16(q_rsrc, dst, g_voff, rq_at + 4096 * m);
+        load_global_to_lds_16(do_rsrc, dst + C::TILE, g_voff, rq_at + 4096 * m);
+    };
+    // every wave requests the same kilobyte of statistics (identical bytes, one instruction)
+    auto request_stats = [&](int stage) {
+        load_global_to_lds_16(st_rsrc, lds_base + (uint32_t)stage * C::STAGE + 2 * C::TILE, lane * 16, rq_stats_at);
+    };
+    auto request_tile = [&](int stage) {
+        request_begin();
+#pragma unroll
+        for (int m = 0; m < C::PT; ++m) request_piece(stage, m);
+        request_stats(stage);
+    };
+
+    // The first query tile is on its way before K and V are, the others behind them; everything is waited for at once.
+    if (ntile > 0) request_tile(0);
+    // ---- this wave's K and V rows as column operands (lane = key row 16b + l%16, columns 32i + 8(l/16) + [0,8))
+    bf16x8 kf[4][KS], vf[4][KS];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const size_t off = head_off + (size_t)min(nw0 + 16 * b + l16, N - 1) * D + g4 * 8;
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            kf[b][i] = __builtin_bit_cast(bf16x8, ld_global_16(Kp + off + i * 32));
+            vf[b][i] = __builtin_bit_cast(bf16x8, ld_global_16(Vp + off + i * 32));
+        }
+    }
+    if (ntile > 0) {
+        request_tile(1);
+        request_tile(2);
+    }
+
+    // LDS addresses, of stage 0; the loop moves them from stage to stage.  Row i of a score product is query row pi(i) of
+    // the sub-tile, bits 2 and 3 of i exchanged: the row exchange then leaves P and dS with lane half g holding query rows
+    // 4g + {0..3} and 4g + 8 + {0..3}, which is what the transposing reads of Q and dO deliver.
+    // (A chunk of 64 columns further is a flip of bit 6 and up: swz16 and the rows' alignment.)
+    const int row16 = (l16 & 3) | ((l16 & 4) << 1) | ((l16 & 8) >> 1);
+    const int q4 = ((g4 & 1) << 3) | ((g4 & 2) << 1);              // first of the four query rows of a lane's scores
+    uint32_t rowp, trlo, trhi, statp;
+    {
+        const int trow = 4 * (g4 >> 1) + (l16 >> 2), tcol = 16 * (g4 & 1) + 4 * (l16 & 3);
+        rowp = lds_base + row16 * C::ROW + swz16<D>(row16, g4) * 16;
+        trlo = lds_base + trow * C::ROW + swz16<D>(trow, tcol >> 3) * 16 + (tcol & 7) * 2;
+        trhi = lds_base + (trow + 8) * C::ROW + swz16<D>(trow + 8, tcol >> 3) * 16 + (tcol & 7) * 2;
+        statp = lds_base + 2 * C::TILE + q4 * 8;
+    }
+    typedef __attribute__((address_space(3))) const unsigned char* lds_cptr;
+    auto read_row = [](uint32_t a) { return *reinterpret_cast<__attribute__((address_space(3))) const bf16x8*>((lds_cptr)(uintptr_t)a); };
+    auto read_stats = [](uint32_t a) { return *reinterpret_cast<__attribute__((address_space(3))) const f32x4*>((lds_cptr)(uintptr_t)a); };
+    auto tr16 = [](uint32_t a) {
+        typedef __attribute__((ext_vector_type(4))) short s16x4;
+        return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(uintptr_t)a));
+    };
+
+    f32x16 dk[C::DT][2], dv[C::DT][2];               // [32 columns of D][32 keys]
+#pragma unroll
+    for (int i = 0; i < C::DT; ++i)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) { dk[i][b][e] = 0.0f; dv[i][b][e] = 0.0f; }
+
+    f32x4 s[4], dp[4];                               // scores and dP - delta of 16 query rows x 16 keys, register x <-> query row q4 + x
+    bf16x8 pf[2], dsf[2];                            // P and dS of the sub-tile at hand as column operands of 32 keys
+    bf16x8 fq[KS], fd[KS];                           // row fragments of Q and dO, of the next sub-tile
+    f32x4 neg_delta;                                 // of the lane's rows of the next sub-tile: what dP starts from
+    auto read_rows = [&](int i, int off) {
+        fq[i] = read_row((rowp ^ (64 * i)) + off);
+        fd[i] = read_row((rowp ^ (64 * i)) + off + C::TILE);
+    };
+    // S = Q K^T and dP - delta = dO V^T - delta of a sub-tile: k-step i, keys 16b + {0..15}
+    auto scores = [&](int i, int b) {
+        if (i == 0) {
+            mfma_16x16x32_bf16_vgpr_begin(s[b], fq[i], kf[b][i]);
+            mfma_16x16x32_bf16_vgpr_begin(dp[b], fd[i], vf[b][i], neg_delta);
+        } else {
+            mfma_16x16x32_bf16_vgpr(s[b], fq[i], kf[b][i]);
+            mfma_16x16x32_bf16_vgpr(dp[b], fd[i], vf[b][i]);
+        }
+    };
+    // P and dS of the scores in 16 pieces of vector instructions, with slot(0) .. slot(15) behind them
+    auto probabilities = [&](const f32x4& lse2, bf16x8 (&p_out)[2], bf16x8 (&ds_out)[2], auto&& slot) {
+        u32x2 pp[2], dd[2];
+        u32x4 po, dso;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            float p[4], d[4];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) p[x] = fmaf(s[b][x], scale_log2, -lse2[x]);
+            slot(4 * b);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) p[x] = fast_exp2(p[x]);
+            slot(4 * b + 1);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) d[x] = p[x] * dp[b][x];
+            slot(4 * b + 2);
+            pp[b & 1] = u32x2{pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3])};
+            dd[b & 1] = u32x2{pack_bf16(d[0], d[1]), pack_bf16(d[2], d[3])};
+            if (b & 1) {
+                // lane groups (0, 1, 2, 3) of two 16-key blocks -> (0, 0', 2, 2') and (1, 1', 3, 3')
+#pragma unroll
+                for (int y = 0; y < 2; ++y) {
+                    const u32x2 sp = __builtin_amdgcn_permlane16_swap(pp[0][y], pp[1][y], false, false);
+                    const u32x2 sd = __builtin_amdgcn_permlane16_swap(dd[0][y], dd[1][y], false, false);
+                    po[y] = sp.x; po[2 + y] = sp.y;
+                    dso[y] = sd.x; dso[2 + y] = sd.y;
+                }
+                p_out[b >> 1] = __builtin_bit_cast(bf16x8, po);
+                ds_out[b >> 1] = __builtin_bit_cast(bf16x8, dso);
+            }
+            slot(4 * b + 3);
+        }
+    };
+    // Hidden pairs of the sub-tile at query row q0, if it has any (wave-uniform): P = dS = 0, whatever was computed for them.
+    // A pair is visible iff 0 <= query - key < window; `gap` is query - key of the lane's first query row at q0 = 0.
+    const uint32_t gap = (uint32_t)(4 * (lane >> 5) - nw0 - (lane & 31));
+    const uint32_t seen = WINDOW ? (uint32_t)window : 0x80000000u;
+    auto hide = [&](int q0, bf16x8 (&p)[2], bf16x8 (&d)[2]) {
+        if constexpr (CAUSAL) {
+            if (__builtin_expect(q0 < nw0 + 63 || (WINDOW && q0 + 15 - nw0 >= window), 0)) {
+                clear_hidden_pairs(gap + (uint32_t)q0, seen, p[0], d[0]);
+                clear_hidden_pairs(gap + (uint32_t)q0 - 32u, seen, p[1], d[1]);
+            }
+        }
+    };
+
+    if (ntile > 0) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int i = 0; i < KS; ++i) { pin_registers(kf[b][i]); pin_registers(vf[b][i]); }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * C::LOADS_PER_TILE) : "memory");
+    __syncthreads();
+
+    // Sub-tile 0 up to P and dS, and the row fragments of sub-tile 1: what a step finds of its predecessor.
+    neg_delta = read_stats(statp + 16);
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+        read_rows(i, 0);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) scores(i, b);
+        if (i == 1) asm volatile("" ::"v"(neg_delta));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_nop 7" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]), "+v"(dp[0]), "+v"(dp[1]), "+v"(dp[2]), "+v"(dp[3]));
+    probabilities(read_stats(statp), pf, dsf, [](int) { __builtin_amdgcn_sched_barrier(0); });
+    int jq = jq_first;                               // the tile at hand
+    hide(jq * C::BQ, pf, dsf);
+#pragma unroll
+    for (int i = 0; i < KS - 1; ++i) read_rows(i, 16 * C::ROW);
+    neg_delta = read_stats(statp + 128 + 16);
+
+    // A step on sub-tile u of a tile has two phases of as many matrix cycles:
+    //   A: S and dP of u + 1, beside the transposed fragments of u and a piece of the request for the tile after next but one
+    //   B: dV and dK of u, beside P and dS of u + 1 and the row fragments of u + 2
+    // The vector work of B fits between its 32x32x16 products; the fences keep the order that is written here (the compiler
+    // does not know that the asm is products).  `advance` moves an address to the next stage of the ring; q0 is the first row of u + 1.
+    auto step = [&](auto sub, int advance, int into, int q0) {
+        constexpr int SUB = decltype(sub)::value, NEXT = (SUB + 1) % NSUB, NEXT2 = (SUB + 2) % NSUB;
+        constexpr int OFF = SUB * 16 * C::ROW;
+        bf16x4 tr[C::DT][4];                         // of dO: query rows 4g + {0..3} and 8 more; of Q
+        auto read_transposed = [&](int piece) {
+            const int dt = piece >> 2, x = piece & 3;
+            tr[dt][x] = tr16((((x & 1) ? trhi : trlo) ^ (64 * dt)) + OFF + (x < 2 ? C::TILE : 0));
+        };
+        f32x4 lse2;
+        if (SUB == 0) request_begin();
+#pragma unroll
+        for (int i = 0; i < KS; ++i)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int at = 4 * i + b;            // two products, then their share of the rest
+                scores(i, b);
+                if (at < 4 * (C::DT - 1)) read_transposed(at);
+                if (at == 1) read_rows(KS - 1, NEXT * 16 * C::ROW);
+                if (at == 4 * KS - 5) lse2 = read_stats(statp + NEXT * 128);
+                if (at == 2 && SUB < C::PT) request_piece(into, SUB);
+                if (SUB == 0 && at == 4 * KS - 1) request_stats(into);
+                if (at == 7) asm volatile("" ::"v"(neg_delta));      // no other use of its registers while products read them
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        if (SUB == NSUB - 2) { rowp += advance; statp += advance; }
+        bf16x8 pn[2], dsn[2];
+        // product m: dV and dK in turn, columns m / 4 of D, keys (m / 2) % 2
+        auto product = [&](int m) {
+            const int dt = m >> 2, b = (m >> 1) & 1, x = 2 * (m & 1);
+            const bf16x8 f = __builtin_shufflevector(tr[dt][x], tr[dt][x + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+            if (m & 1) mfma_32x32x16_bf16_acc(dk[dt][b], f, dsf[b]); else mfma_32x32x16_bf16_acc(dv[dt][b], f, pf[b]);
+        };
+        // Wait states between an ordinary instruction and a product on its result (P, dS), and between a product and an ordinary
+        // instruction on its result: the first scores are used behind product(0), eight products and this after their own.
+        asm volatile("s_nop 1" : "+v"(pf[0]), "+v"(pf[1]), "+v"(dsf[0]), "+v"(dsf[1]), "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]),
+                     "+v"(dp[0]), "+v"(dp[1]), "+v"(dp[2]), "+v"(dp[3]));
+        product(0);
+        __builtin_amdgcn_sched_barrier(0);
+        probabilities(lse2, pn, dsn, [&](int k) {
+            if (k < 4) read_transposed(4 * (C::DT - 1) + k);
+            if (k + 1 < 4 * C::DT) product(k + 1);
+            if (k >= 8 && !(k & 1) && (k - 8) / 2 < KS - 1) read_rows((k - 8) / 2, NEXT2 * 16 * C::ROW);
+            if (k == 13) neg_delta = read_stats(statp + NEXT2 * 128 + 16);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        hide(q0, pn, dsn);
+        if (SUB == NSUB - 1) { trlo += advance; trhi += advance; }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) { pf[b] = pn[b]; dsf[b] = dsn[b]; }
+    };
+    // Tile t+1 is awaited, and tile t+3 requested into the stage tile t-1 has left, before and in the steps of tile t (which read
+    // row fragments of tile t+1): four stages.  (No wait for LDS reads in front of the barrier, as __syncthreads would have: the ones
+    // on their way are of tile t, those of tile t-1 have all been used.)
+    int stage = 0;
+    for (int tile = 0; tile < ntile; ++tile) {
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(C::LOADS_PER_TILE) : "memory");
+        const int into = (stage + 3) & (C::NST - 1);
+        const int advance = stage == C::NST - 1 ? -(C::NST - 1) * C::STAGE : C::STAGE;
+        const int q0 = jq * C::BQ;
+        step(std::integral_constant<int, 0>{}, advance, into, q0 + 16);
+        step(std::integral_constant<int, 1>{}, advance, into, q0 + 32);
+        step(std::integral_constant<int, 2>{}, advance, into, q0 + 48);
+        if (++jq == jq_last) jq = jq_first;
+        step(std::integral_constant<int, 3>{}, advance, into, jq * C::BQ);
+        stage = (stage + 1) & (C::NST - 1);
+    }
+    }
+    // (the wait states between a product and an ordinary instruction on its result)
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt)
+        asm volatile("" : "+a"(dk[dt][0]), "+a"(dk[dt][1]), "+a"(dv[dt][0]), "+a"(dv[dt][1])::"memory");
+
+    // ---- lane (key, g) holds columns 8 q + 4 g + {0..3}: a swap of the upper half of the one with the lower half of the next
+    // makes them 16 bytes of a row
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        const int key = nw0 + 32 * b + (lane & 31);
+        const bool hidden = PER_KEY && (key >= Nk || (key_mask != nullptr && key_mask[(size_t)(bh / hkv) * N + min(key, N - 1)] == 0));
+        const size_t row = head_off + (size_t)key * D + 8 * (lane >> 5);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float mul = i ? scale : 1.0f;
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int x = 0; x < 16; x += 8) {
+                    const f32x16& a = i ? dk[dt][b] : dv[dt][b];
+                    u32x4 v;
+#pragma unroll
+                    for (int y = 0; y < 2; ++y) {
+                        const u32x2 z = __builtin_amdgcn_permlane32_swap(pack_bf16(a[x + 2 * y] * mul, a[x + 2 * y + 1] * mul),
+                                                                         pack_bf16(a[x + 4 + 2 * y] * mul, a[x + 5 + 2 * y] * mul), false, false);
+                        v[y] = hidden ? 0u : z.x;
+                        v[2 + y] = hidden ? 0u : z.y;
+                    }
+                    if (key < N) st_global_16((i ? dK : dV) + row + 32 * dt + 2 * x, v);
+                }
+        }
+    }
+    wait_vmcnt0();                                   // the requests past the end write LDS, which is the next workgroup's then
+}
+
 // dK and dV of 64 keys for small launches: waves w and w + 2 own the same 32 keys, one the first and one the second 32 rows of
 // every query tile, and exchange at the end (one finishes dV, the other dK).  Half the work a step and twice the workgroups of
 // bwd_dkv.  The query tiles of all G heads are one run of steps, three requested ahead into a ring of four stages; the pairs
@@ -1274,7 +1650,7 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_both_kernel(
                                          window, kv_lens, key_mask, plan, items, partial, nullptr);
     } else {
         bwd_dq<D, CAUSAL, MASK, true>(at - ndkv, Q, Kp, Vp, O, dO, LSE, dQ, nullptr, BH, N, ntq, npad, scale, scale_log2, Hq, plan.G,
-                                      window, kv_lens, key_mask, 0, single);
+                                      window, kv_lens, key_mask, 0, single, 0);
     }
 }
 
@@ -1466,17 +1842,19 @@ size_t flash_attn_bwd_workspace_bytes(int B, int H, int N) {
 }
 
 namespace {
-// Steps until the last of an XCD's 32 CUs is done.  It gets every eighth workgroup of the launch and deals them to its four
-// engines of eight CUs in turn; the next one waits until the engine whose turn it is has a free CU (fab::Parts::order).
-int last_cu_steps(const fab::Parts& p, int ntk, int BHkv) {
+// When the last of an XCD's 32 CUs is done, with workgroups of wg + step * steps.  The XCD gets every eighth workgroup of the launch
+// and deals them to its four engines of eight CUs in turn; the next one waits until the engine whose turn it is has a
+// free CU (fab::Parts::order).
+double last_cu(const fab::Parts& p, int ntk, int BHkv, double wg, double step) {
     const bool xcds = BHkv % 8 == 0;
     const int heads = xcds ? BHkv / 8 : BHkv, stride = xcds ? 1 : 8;
-    int busy[4][8] = {}, n = 0, started = 0, last = 0;
+    double busy[4][8] = {}, started = 0, last = 0;
+    int n = 0;
     auto job = [&](int steps) {
-        int* cu = std::min_element(busy[n & 3], busy[n & 3] + 8);
+        double* cu = std::min_element(busy[n & 3], busy[n & 3] + 8);
         ++n;
         started = std::max(started, *cu);
-        *cu = started + steps;
+        *cu = started + wg + step * steps;
         last = std::max(last, *cu);
     };
     if (p.chunk) {
@@ -1511,7 +1889,7 @@ struct DkvPlan {
 };
 DkvPlan make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window, bool cut_tiles) {
     const int ntk = (N + 127) / 128, nq = (N + 63) / 64;
-    const fab::Parts whole{G, nq, causal, window, 0};
+    const fab::Parts whole{G, nq, causal, window, 0, 128};
     DkvPlan best{whole, 1e300};
     const double step = D == 128 ? 1.7 : 1.1;
     int64_t total = 0;
@@ -1542,16 +1920,35 @@ DkvPlan make_dkv_plan(int BHkv, int G, int N, int D, bool causal, int window, bo
             for (int kt = 0; kt < ntk; ++kt) cut += p.parts(kt) > 1 ? p.parts(kt) : 0;
             if (cut == 0) continue;
         }
-        const double last = n <= 2048 ? last_cu_steps(p, ntk, BHkv) : mean + 0.5 * most;
+        const double last = n <= 2048 ? last_cu(p, ntk, BHkv, 0, 1) : mean + 0.5 * most;
         double us = step * std::max(last, 1.25 * mean) + 2.0 * std::max(1.0, n / 256.0);
         if (round) us += 3.0 + partial_us(p, BHkv, N, D);
-        // (a tie goes to the parts at D = 128: B5 Hq32 Hkv8 N1325 294 us in parts, 296 whole, estimated 4 % apart the other way)
-        if (us < best.us * (best.parts.chunk == 0 && D == 128 ? 1.045 : 1.0)) best = {p, us};
+        // A tie goes to the parts at D = 128 where an XCD has several heads: B5 Hq32 Hkv8 N1325 294 us in parts, 296 whole, estimated 4 %
+        // apart the other way.  (One head: B8 H1 N7207 402 in parts, 386 whole.)
+        if (us < best.us * (best.parts.chunk == 0 && D == 128 && BHkv > 8 ? 1.045 : 1.0)) best = {p, us};
     }
     return best;
 }
+// What key tiles of 256 save a dQ launch and a dK/dV launch one after the other: a workgroup of them takes 13.5 us and 2.3 a step (64
+// queries x 256 keys) at D = 128, 8.3 and 1.6 at 64, in a launch that fills the device; plan.us against that, as the two were measured.
+// On 556 shapes (1 to 16 sequences of 64 to 8192 rows, 1 to 32 heads, every mask) the choice is 0.1 % slower than the better of the two
+// at D = 128 and 0.3 % at 64; there are 117 shapes where the wide tiles are the faster ones, by up to 23 %.
+double wide_saves(int BHkv, int G, int N, int D, bool causal, int window, const DkvPlan& plan) {
+    const int ntk = (N + 255) / 256;
+    const fab::Parts wide{G, (N + 63) / 64, causal, window, 0, 256};
+    const double wg = D == 128 ? 13.5 : 8.3, step = D == 128 ? 2.29 : 1.59;
+    double us;
+    if ((int64_t)ntk * BHkv <= 16384) {
+        us = last_cu(wide, ntk, BHkv, wg, step);
+    } else {
+        int64_t steps = 0;
+        for (int kt = 0; kt < ntk; ++kt) steps += wide.steps(kt);
+        us = (wg * ntk + step * (double)steps) * BHkv / 256;
+    }
+    return (D == 128 ? 0.89 * plan.us + 8.7 : 0.957 * plan.us + 5.1) - us;
+}
 int dkv_items(const fab::Parts& p, int N) {
-    const int ntk = (N + 127) / 128;
+    const int ntk = (N + p.keys - 1) / p.keys;
     if (p.chunk == 0) return ntk;
     int n = 0;
     for (int kt = 0; kt < ntk; ++kt) n += p.parts(kt);
@@ -1662,6 +2059,7 @@ void launch_us(int BH, int BHkv, int N, int D, bool causal, int window, const Dk
 // some microseconds of host time (tens for hundreds of workgroups): each thread keeps its last plans
 struct Launches {
     fab::Parts parts;
+    bool wide;                                       // TWO: key tiles of 256 instead
     double us[FORMS];
 };
 Launches launches(int BH, int BHkv, int N, int D, bool causal, int window, bool cut_tiles) {
@@ -1672,8 +2070,10 @@ Launches launches(int BH, int BHkv, int N, int D, bool causal, int window, bool 
     Entry& e = kept[h >> 27];
     if (e.BH != BH || e.BHkv != BHkv || e.N != N || e.D != D || e.causal != causal || e.window != window || e.cut != cut_tiles) {
         const DkvPlan plan = make_dkv_plan(BHkv, BH / BHkv, N, D, causal, window, cut_tiles);
-        e = {BH, BHkv, N, D, causal, window, cut_tiles, {plan.parts, {}}};
+        const double saved = wide_saves(BHkv, BH / BHkv, N, D, causal, window, plan);
+        e = {BH, BHkv, N, D, causal, window, cut_tiles, {plan.parts, saved > 0, {}}};
         launch_us(BH, BHkv, N, D, causal, window, plan, e.how.us);
+        e.how.us[TWO] -= std::max(0.0, saved);
     }
     return e.how;
 }
@@ -1698,6 +2098,10 @@ BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int D, bool causal, int window, 
     const int pick = (int)(std::min_element(how.us, how.us + FORMS) - how.us);
     p.parts = how.parts;
     if (pick == HALF) p.parts.chunk = 0;
+    if (pick == TWO && how.wide) {
+        p.parts.chunk = 0;
+        p.parts.keys = 256;
+    }
     p.half = pick == HALF ? half_steps(Hq / Hkv, N, causal, window) : 0;
     p.both = pick == HALF || pick == ONE;
     p.ds = pick == DS;
@@ -1754,7 +2158,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
         if (a1 != hipSuccess) return -1;                                                              \
         launch_kernel((flash_attn_bwd_dq_kernel<DD, CC, EE, SS>), grid_q, block, CfgQ<DD>::LDS, stream, \
                            Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st, BH, N, ntq, npad, \
-                           scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single);        \
+                           scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single, plan.keys == 256); \
     } while (0)
 #define TYR_FAB_DKV(DD, CC, EE, UU, PP)                                                               \
     do {                                                                                              \
@@ -1766,6 +2170,17 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
                            stream, Qp, Kp, Vp, dOp, st, static_cast<uint16_t*>(dk),                   \
                            static_cast<uint16_t*>(dv), BHkv, N, ntk, npad, scale, scale_log2, Hq,     \
                            window, kv_lens, key_mask, plan, items, partial, ds);                      \
+    } while (0)
+#define TYR_FAB_DKV_WIDE(DD, CC, EE)                                                                  \
+    do {                                                                                              \
+        static const hipError_t a5 = hipFuncSetAttribute(                                             \
+            reinterpret_cast<const void*>(&flash_attn_bwd_dkv_wide_kernel<DD, CC, EE>),               \
+            hipFuncAttributeMaxDynamicSharedMemorySize, CfgK<DD>::LDS);                               \
+        if (a5 != hipSuccess) return -1;                                                              \
+        launch_kernel((flash_attn_bwd_dkv_wide_kernel<DD, CC, EE>), grid_k, block, CfgK<DD>::LDS,     \
+                           stream, Qp, Kp, Vp, dOp, st, static_cast<uint16_t*>(dk),                   \
+                           static_cast<uint16_t*>(dv), BHkv, N, npad, scale, scale_log2, Hq,          \
+                           window, kv_lens, key_mask, plan, items);                                   \
     } while (0)
 #define TYR_FAB_DKV_MASK(DD, CC, EE, UU, PP)  /* lengths alone are a mask of keys here; a window is causal */ \
     do {                                                                                              \
@@ -1822,6 +2237,15 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
             }                                                                                         \
         }                                                                                             \
         if (shape.rows == 64) TYR_FAB_DQ(DD, CC, EE, true); else TYR_FAB_DQ(DD, CC, EE, false);       \
+        if (plan.keys == 256) {                                                                       \
+            if constexpr (EE == AttnMask::Limits) {                                                   \
+                if (CC && window > 0) TYR_FAB_DKV_WIDE(DD, true, EE);                                 \
+                else TYR_FAB_DKV_WIDE(DD, CC, AttnMask::Keys);                                        \
+            } else {                                                                                  \
+                TYR_FAB_DKV_WIDE(DD, CC, EE);                                                         \
+            }                                                                                         \
+            break;                                                                                    \
+        }                                                                                             \
         if (plan.chunk) {                                                                             \
             TYR_FAB_DKV_MASK(DD, CC, EE, true, false);                                                \
             TYR_FAB_SUM(DD);                                                                          \
@@ -1846,6 +2270,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
 #undef TYR_FAB_DQ_PRODUCT
 #undef TYR_FAB_DKV_MASK
 #undef TYR_FAB_DKV
+#undef TYR_FAB_DKV_WIDE
 #undef TYR_FAB_DQ
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
