@@ -1,6 +1,7 @@
 """Backward with dK / dV by key tiles of 256 (launches of many whole tiles): lengths around its 64-row query tiles, 64-key waves and
-256-key tiles, grouped queries, head counts that are no multiple of the XCDs, every mask.  Two (sequence, kv head) pairs of
-each launch against float64 gradients of the bf16 inputs; bounds as in test_gpu_attention_bwd."""
+256-key tiles, grouped queries, head counts that are no multiple of the XCDs, every mask; and by tiles of 64 where two workgroups share
+a CU.  Three (sequence, kv head) pairs of each launch against float64 gradients of the bf16 inputs; bounds as in
+test_gpu_attention_bwd."""
 import pytest
 import torch
 
@@ -27,6 +28,17 @@ def reference(q, k, v, g, visible):
     (16, 32, 8, 1100, 128, True, "keys", 0), (17, 12, 4, 600, 64, False, "keys", 0), (16, 32, 8, 700, 64, True, "keys", 0),
     (16, 32, 8, 1216, 128, True, None, 600), (16, 32, 8, 1153, 128, True, "lens", 600)])
 def test_wide_key_tiles_match_float64(B, Hq, Hkv, N, D, causal, mask, window):
+    compare(B, Hq, Hkv, N, D, causal, mask, window)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal,mask,window", [
+    (16, 8, 8, 130, 64, False, None, 0), (6, 8, 8, 320, 64, False, "lens", 0), (8, 16, 4, 385, 64, False, "keys", 0),
+    (3, 16, 16, 283, 64, True, None, 70), (5, 16, 4, 511, 64, True, "lens", 100), (2, 4, 4, 1400, 64, True, None, 129)])
+def test_two_workgroups_of_64_key_tiles_on_a_cu(B, Hq, Hkv, N, D, causal, mask, window):
+    compare(B, Hq, Hkv, N, D, causal, mask, window)
+
+
+def compare(B, Hq, Hkv, N, D, causal, mask, window):
     import tyr_amd
     gen = torch.Generator(device="cuda").manual_seed(N + D)
     q, g = (torch.randn(B, Hq, N, D, generator=gen, device="cuda").bfloat16() for _ in range(2))

@@ -1635,7 +1635,7 @@ __device__ __forceinline__ void bwd_dkv_half(int block,
 // The dQ kernel then need not end before dK/dV starts -- a launch, a prologue and a drain, 3.5 us of 11 for one head of 128 rows,
 // 12 of 41 for 8 heads of 700.
 template <int D, bool CAUSAL, AttnMask MASK, bool CUT, bool HALF>
-__global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_both_kernel(
+__global__ __launch_bounds__(fab::THREADS, D == 64 && HALF ? 2 : 1) void flash_attn_bwd_both_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
     const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO, const float* __restrict__ LSE,
     uint16_t* __restrict__ dQ, float2* stats, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int BH, int N, int ntq,
@@ -1954,7 +1954,17 @@ int dkv_items(const fab::Parts& p, int N) {
     for (int kt = 0; kt < ntk; ++kt) n += p.parts(kt);
     return n;
 }
-size_t half_lds(int D, int steps) { return (size_t)4 * 2 * 64 * D * 2 + (size_t)steps * 64 * sizeof(float2); }
+// At D = 64 two workgroups of 64-key tiles fit a CU, and do where there are more than CUs and all take as long (B1 H16 N514 not causal
+// 20.6 -> 16.0 us, B12 H4 N237 window 157 15.7 -> 11.2).  Causal ones are kept apart by the LDS they ask for: the longest must not share
+// its CU (B15 Hq16 Hkv4 N64 9.7 us, 10.5 beside others); nor must the dK/dV ones of grouped heads while they have one each (B2 Hq32
+// Hkv8 N257 window 79 20.3, 21.3).
+bool kept_apart(int G, int N, bool causal, int window, int64_t workgroups) {
+    return (causal && (window <= 0 || window > N / 2)) || (G > 1 && workgroups <= 512);
+}
+size_t half_lds(int D, int steps, bool apart) {
+    const size_t bytes = (size_t)4 * 2 * 64 * D * 2 + (size_t)steps * 64 * sizeof(float2);
+    return apart ? std::max<size_t>(bytes, 82 * 1024) : bytes;
+}
 size_t dkv_partial_bytes(const fab::Parts& p, int BHkv, int N, int D) {
     return p.chunk ? (size_t)BHkv * dkv_items(p, N) * 128 * D * 8 : 0;
 }
@@ -2037,13 +2047,16 @@ void launch_us(int BH, int BHkv, int N, int D, bool causal, int window, const Dk
         dq(x, scale);
         us[ONE] = m.one + x.last + (p.chunk ? m.sum + m.traffic * sum : 0.0);
     }
-    if (half <= 1600 && half_lds(D, half_steps(G, N, causal, window)) <= 160 * 1024) {
+    if (half <= 1600 && half_lds(D, half_steps(G, N, causal, window), false) <= 160 * 1024) {
         Xcd x;
         const double scale = step_scale(half), step = m.half_step * (edges ? scale / m.edges : scale);       // its mask is always on
         for (int kt = 0; kt < nq; ++kt)
             x.run(m.half_wg + step * G * (std::min(nq, (window > 0 ? kt : 0) + seen) - (causal ? kt : 0)), BHkv);
         dq(x, scale);
         us[HALF] = m.half + x.last;
+        // two workgroups of it on a CU (half_lds).  Smaller launches would take it more often with this too (B1 H32 N315 not causal 14.0 us in
+        // one launch of 128-key tiles, 11.3), but their choice is kept.
+        if (D == 64 && half >= 384 && !kept_apart(G, N, causal, window, half) && half_lds(D, half_steps(G, N, causal, window), false) <= 80 * 1024) us[HALF] *= 0.72;
     }
     if (D == 128 && ntk > 1 && ds_bytes(BH, N, causal, window) <= kMostDs) {
         // product: stages of 32 keys, two workgroups a CU
@@ -2212,7 +2225,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
             reinterpret_cast<const void*>(&flash_attn_bwd_both_kernel<DD, CC, EE, UU, HH>),               \
             hipFuncAttributeMaxDynamicSharedMemorySize, HH ? 160 * 1024 : CfgK<DD>::LDS);                               \
         if (a3 != hipSuccess) return -1;                                                              \
-        launch_kernel((flash_attn_bwd_both_kernel<DD, CC, EE, UU, HH>), dim3((unsigned)(how.dkv_blocks + how.dq_blocks)), block, HH ? half_lds(DD, how.half) : CfgK<DD>::LDS, \
+        launch_kernel((flash_attn_bwd_both_kernel<DD, CC, EE, UU, HH>), dim3((unsigned)(how.dkv_blocks + how.dq_blocks)), block, HH ? half_lds(DD, how.half, kept_apart(G, N, causal, window, how.dkv_blocks + how.dq_blocks)) : CfgK<DD>::LDS, \
                            stream, Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st,          \
                            static_cast<uint16_t*>(dk), static_cast<uint16_t*>(dv), BH, N, (N + 63) / 64, ntk, \
                            npad, scale, scale_log2, Hq, window, kv_lens, key_mask, causal && window <= 0, plan, items, partial, (int)how.dkv_blocks); \
