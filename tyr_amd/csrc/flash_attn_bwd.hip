@@ -27,7 +27,8 @@
 //     rows, four stages deep.  Every lane owns one key column:
 //        S  (32 q x 32 kv) = Q_tile x K_w^T        dP (32 q x 32 kv) = dO_tile x V_w^T
 //        dV^T (D x 32 kv) += dO_tile^T x P         dK^T (D x 32 kv) += Q_tile^T x dS
-//     with lse / delta of the 16 query rows a lane holds read from the staged pairs.
+//     with lse / delta of the 16 query rows a lane holds read from the staged pairs.  Launches of many key tiles take
+//     flash_attn_bwd_dkv_wide_kernel, 256 keys a workgroup; small ones bwd_dkv_half, 64 keys.
 //
 // Both recompute S (7 matrix products for an algorithm that needs 5): the price of writing dQ
 // without a float atomic accumulation buffer and a conversion pass.
