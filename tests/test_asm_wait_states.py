@@ -1,10 +1,14 @@
-"""Wait states around the matrix products that flash_attn_bwd_dkv_wide_kernel issues in asm, where the compiler, which puts
-them in for its own products, does not see any.  The kernel file is compiled to gfx950 assembly (no GPU needed) and every product
-of those kernels is checked against the instructions around it, with the body of every loop entered twice:
+"""What the gfx950 assembly of the attention backward has to show (compiled here, no GPU needed).
+
+Wait states around the matrix products that flash_attn_bwd_dkv_wide_kernel issues in asm, where the compiler, which puts
+them in for its own products, does not see any.  Every product of those kernels is checked against the instructions around it,
+with the body of every loop entered twice:
   * no operand is written by an ordinary vector instruction less than 2 wait states before the product,
   * no result is read or written by another kind of instruction less than 8 (16x16x32) or 12 (32x32x16) wait states behind it,
   * no accumulator operand of a product in flight is written.
-An instruction is one wait state, s_nop n is n + 1."""
+An instruction is one wait state, s_nop n is n + 1.
+
+Scalar offsets of the requests of query tiles: at most the size of the buffer, which is what their range check is known for."""
 import os
 import re
 import subprocess
@@ -90,16 +94,44 @@ def wide_kernels(path):
         yield m.group(1), [l for l in lines if l and (l.endswith(":") or not l.startswith("."))]
 
 
-@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
-def test_products_in_asm_keep_their_distance(tmp_path):
-    out = str(tmp_path / "bwd.s")
+@pytest.fixture(scope="module")
+def listing(tmp_path_factory):
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not installed")
+    out = str(tmp_path_factory.mktemp("asm") / "bwd.s")
     subprocess.check_call([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                            "--cuda-device-only", "-S", os.path.join(CSRC, "flash_attn_bwd.hip"), "-o", out], stderr=subprocess.DEVNULL)
-    kernels = dict(wide_kernels(out))
+    return out
+
+
+def test_products_in_asm_keep_their_distance(listing):
+    kernels = dict(wide_kernels(listing))
     assert kernels
     for name, lines in kernels.items():
         assert sum(l.startswith("v_mfma") for l in lines) >= 96, name
         assert violations(straight(lines)) == [], name
+
+
+def unbounded_requests(code):
+    """Buffers (registers of their descriptors) with a request whose scalar offset is not a minimum with a buffer's size."""
+    last, out = {}, {}
+    for line in code:
+        name, ops = operands(line)
+        if name == "buffer_load_dwordx4" and line.endswith(" lds"):
+            out.setdefault(ops[1], []).append(last.get(ops[2].split()[0]) == "s_min_u32")
+        elif name.startswith("s_") and ops and re.fullmatch(r"s\d+", ops[0]):
+            last[ops[0]] = name
+    return out, {d for d, bounded in out.items() if not all(bounded)}
+
+
+def test_no_request_of_a_query_tile_starts_beyond_its_buffer(listing):
+    """(the statistics' offset is a whole tile's and needs no minimum)"""
+    kernels = dict(wide_kernels(listing))
+    assert kernels
+    for name, lines in kernels.items():
+        buffers, unbounded = unbounded_requests(lines)
+        assert len(buffers) == 3 and len(unbounded) <= 1, (name, unbounded)
+        assert sorted(map(len, buffers.values()))[1:] == [16 if "Li128E" in name else 8] * 2, name      # four tiles in the code, PT pieces each
 
 
 def test_what_comes_too_early_is_found():

@@ -1,7 +1,7 @@
 """Backward with dK / dV by key tiles of 256 (launches of many whole tiles): lengths around its 64-row query tiles, 64-key waves and
 256-key tiles, grouped queries, head counts that are no multiple of the XCDs, every mask; and by tiles of 64 where two workgroups share
-a CU.  Three (sequence, kv head) pairs of each launch against float64 gradients of the bf16 inputs; bounds as in
-test_gpu_attention_bwd."""
+a CU.  Four (sequence, kv head) pairs of each launch against float64 gradients of the bf16 inputs, the last one among them: its rows end
+where Q and dO do, and the memory behind those holds NaN.  Bounds as in test_gpu_attention_bwd."""
 import pytest
 import torch
 
@@ -38,10 +38,17 @@ def test_two_workgroups_of_64_key_tiles_on_a_cu(B, Hq, Hkv, N, D, causal, mask, 
     compare(B, Hq, Hkv, N, D, causal, mask, window)
 
 
+def before_nan(x):
+    """The same values in front of 64 KB that read as NaN, in one allocation."""
+    room = torch.full((x.numel() + 32768,), float("nan"), dtype=x.dtype, device=x.device)
+    room[:x.numel()] = x.flatten()
+    return room[:x.numel()].view(x.shape)
+
+
 def compare(B, Hq, Hkv, N, D, causal, mask, window):
     import tyr_amd
     gen = torch.Generator(device="cuda").manual_seed(N + D)
-    q, g = (torch.randn(B, Hq, N, D, generator=gen, device="cuda").bfloat16() for _ in range(2))
+    q, g = (before_nan(torch.randn(B, Hq, N, D, generator=gen, device="cuda").bfloat16()) for _ in range(2))
     k, v = (torch.randn(B, Hkv, N, D, generator=gen, device="cuda").bfloat16() for _ in range(2))
     opt = dict(causal=causal)
     i = torch.arange(N, device="cuda")
@@ -62,7 +69,7 @@ def compare(B, Hq, Hkv, N, D, causal, mask, window):
     o, lse = tyr_amd.flash_attn_fwd(q, k, v, **opt)
     got = tyr_amd.flash_attn_bwd(q, k, v, o, lse, g, **opt)
     G = Hq // Hkv
-    for b, h in ((0, 0), (1, Hkv - 1), (B - 2, 1)):
+    for b, h in ((0, 0), (1, Hkv - 1), (B - 2, 1), (B - 1, Hkv - 1)):
         want = reference(q[b, h * G:(h + 1) * G], k[b, h], v[b, h], g[b, h * G:(h + 1) * G], visible & keys[b][None, :])
         for name, x, y in zip(("dq", "dk", "dv"), (got[0][b, h * G:(h + 1) * G], got[1][b, h], got[2][b, h]), want):
             assert bool(((x.double() - y).abs() <= 3e-2 + 3e-2 * y.abs()).all()), (name, b, h)

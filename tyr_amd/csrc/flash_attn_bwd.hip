@@ -1016,6 +1016,13 @@ template <int D> __device__ __forceinline__ int swz16(int row, int c) {
     const int low = (((row >> 3) ^ (row >> 2)) & 1) << 1 | ((row >> 2) & 1);
     return c ^ ((D == 128 ? (row & 3) << 2 : ((row >> 1) & 1) << 2) | low);
 }
+// Scalar offset of the request for piece m (4 KB) of the query tile at `tile` in a buffer of `bytes`: never beyond the buffer, like every
+// request's here.  (The range check is on the whole offset; the manual gives it as lane offset >= bytes - scalar offset, and does not
+// say what a scalar offset above bytes makes of the difference.)  A piece that would start there has no row of the buffer.
+__host__ __device__ inline uint32_t piece_at(uint32_t tile, int m, uint32_t bytes) {
+    const uint32_t at = tile + 4096u * m;            // (both below 2^31)
+    return at < bytes ? at : bytes;
+}
 // P and dS of a lane (slot j <-> query row 8 (j / 4) + j % 4) set to 0 where gap + that row is not below `seen`
 __device__ __forceinline__ void clear_hidden_pairs(uint32_t gap, uint32_t seen, bf16x8& p, bf16x8& d) {
     u32x4 keep;
@@ -1072,9 +1079,9 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_wide_kerne
     // The G query heads of the group are adjacent in memory: one buffer covers them, a head is a
     // scalar offset.  (Rows past N of a head then alias the next head's first rows instead of
     // reading as zero; their statistics are (+inf, 0), so their probabilities are exactly 0 either way.)
-    const uint32_t head_bytes = (uint32_t)N * D * 2u;
-    const u32x4 q_rsrc = make_raw_rsrc(Q + qh0 * N * D, head_bytes * (uint32_t)G);
-    const u32x4 do_rsrc = make_raw_rsrc(dO + qh0 * N * D, head_bytes * (uint32_t)G);
+    const uint32_t head_bytes = (uint32_t)N * D * 2u, group_bytes = head_bytes * (uint32_t)G;
+    const u32x4 q_rsrc = make_raw_rsrc(Q + qh0 * N * D, group_bytes);
+    const u32x4 do_rsrc = make_raw_rsrc(dO + qh0 * N * D, group_bytes);
     const uint32_t stat_bytes = (uint32_t)npad * 8u;
     const u32x4 st_rsrc = make_raw_rsrc(stats + qh0 * npad, stat_bytes * (uint32_t)G);
     // Request m of a wave fills the kilobyte at 4 KB m + 1 KB w of a tile: the rows of one swizzle, so that one register of
@@ -1087,20 +1094,21 @@ __global__ __launch_bounds__(fab::THREADS, 1) void flash_attn_bwd_dkv_wide_kerne
     }
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
     const uint32_t wave_dst = __builtin_amdgcn_readfirstlane(lds_base + (uint32_t)w * 1024u);
-    // Query tile `rq_jq` of head `rq_head`, piece by piece.  Tiles past the last are requested at an offset beyond the
-    // buffer (they read as zero), so that every iteration issues the same number of loads and the wait count below stays constant.
+    // Query tile `rq_jq` of head `rq_head`, piece by piece.  Tiles past the last are requested at the buffer's
+    // end (they read as zero), so that every iteration issues the same number of loads and the wait count below stays constant.
     int rq_head = 0, rq_jq = jq_first, rq_left = ntile;
     int rq_at = 0, rq_stats_at = 0;                  // offsets of the tile that is being requested
     auto request_begin = [&] {
-        rq_at = __builtin_amdgcn_readfirstlane(rq_left > 0 ? rq_head * (int)head_bytes + rq_jq * C::BQ * C::ROW : (int)(head_bytes * (uint32_t)G));
+        rq_at = __builtin_amdgcn_readfirstlane(rq_left > 0 ? rq_head * (int)head_bytes + rq_jq * C::BQ * C::ROW : (int)group_bytes);
         rq_stats_at = __builtin_amdgcn_readfirstlane(rq_left > 0 ? (rq_head * npad + rq_jq * C::BQ) * 8 : (int)(stat_bytes * (uint32_t)G));
         --rq_left;
         if (++rq_jq == jq_last) { rq_jq = jq_first; ++rq_head; }
     };
     auto request_piece = [&](int stage, int m) {
         const uint32_t dst = wave_dst + (uint32_t)stage * C::STAGE + 4096u * m;
-        load_global_to_lds_16(q_rsrc, dst, g_voff, rq_at + 4096 * m);
-        load_global_to_lds_16(do_rsrc, dst + C::TILE, g_voff, rq_at + 4096 * m);
+        const int at = (int)piece_at((uint32_t)rq_at, m, group_bytes);
+        load_global_to_lds_16(q_rsrc, dst, g_voff, at);
+        load_global_to_lds_16(do_rsrc, dst + C::TILE, g_voff, at);
     };
     // every wave requests the same kilobyte of statistics (identical bytes, one instruction)
     auto request_stats = [&](int stage) {
