@@ -8,7 +8,9 @@ with the body of every loop entered twice:
   * no accumulator operand of a product in flight is written.
 An instruction is one wait state, s_nop n is n + 1.
 
-Scalar offsets of the requests of query tiles: at most the size of the buffer, which is what their range check is known for."""
+Scalar offsets of the requests of query tiles: at most the size of the buffer, which is what their range check is known for.
+
+Registers of the dQ kernels: as many waves a SIMD as each form is launched for, and no more in scratch memory than is stated beside them."""
 import os
 import re
 import subprocess
@@ -132,6 +134,29 @@ def test_no_request_of_a_query_tile_starts_beyond_its_buffer(listing):
         buffers, unbounded = unbounded_requests(lines)
         assert len(buffers) == 3 and len(unbounded) <= 1, (name, unbounded)
         assert sorted(map(len, buffers.values()))[1:] == [16 if "Li128E" in name else 8] * 2, name      # four tiles in the code, PT pieces each
+
+
+def resources(path):
+    """Registers, and registers kept in scratch, of every kernel by its mangled name."""
+    with open(path) as f:
+        for block in f.read().split("\n  - .agpr_count:")[1:]:
+            field = lambda key: re.search(rf"\.{key}:\s+(\S+)", block).group(1)
+            yield field("name"), (int(field("vgpr_count")), int(field("vgpr_spill_count")))
+
+
+def test_dq_kernels_keep_their_waves(listing):
+    """A SIMD's 512 registers hold three waves of up to 168; the launch bounds only ask for two."""
+    seen = 0
+    for name, (registers, spilled) in resources(listing):
+        m = re.search(r"flash_attn_bwd_dq_kernelILi(64|128)ELb([01])ELNS_8AttnMaskE([012])ELb([01])E", name)
+        if not m:
+            continue
+        D, causal, mask, split = map(int, m.groups())
+        seen += 1
+        if D == 64 and causal and (mask != 2 or split):
+            assert registers <= 168, (name, registers)
+        assert spilled <= (0 if causal or D == 64 else 52), (name, spilled)
+    assert seen == 24
 
 
 def test_what_comes_too_early_is_found():

@@ -93,16 +93,15 @@ __device__ __forceinline__ float dot8_bf16(u32x4 a, u32x4 b) {
     return s;
 }
 
-// What the dK / dV workgroups need of a query row: (lse * log2 e, delta), or for the wide kernel, by groups of four rows, four
-// lse * log2 e and four -delta (16 bytes each: what a lane's scores need; its dP starts from -delta).
+// What the dK / dV workgroups need of a query row: (lse * log2 e, delta), or with fours = 3, for the wide kernel, by groups of four rows
+// four lse * log2 e and four -delta (16 bytes each: what a lane's scores need; its dP starts from -delta).  One pair of stores for
+// both, and nothing for the compiler to keep across the passes of a workgroup (row & 3 is the same in each): as a branch the dQ
+// kernels held two registers more, and at 170 for 168 two waves of <64, causal, Keys, SPLIT> share a SIMD for three.
 __device__ __forceinline__ void store_stats(float2* head, int row, float lse2, float delta, int fours) {
-    if (fours) {
-        float* to = reinterpret_cast<float*>(head + (row & ~3)) + (row & 3);
-        to[0] = lse2;
-        to[4] = -delta;
-    } else {
-        head[row] = make_float2(lse2, delta);
-    }
+    asm volatile("" : "+v"(row));
+    float* at = reinterpret_cast<float*>(head) + (2 * row - (row & fours));
+    at[0] = lse2;
+    at[1 + fours] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, delta) ^ ((uint32_t)fours << 31));
 }
 
 // One wave's 32 columns x D rows accumulator (lane = column l%32, register e of tile dt <-> row
@@ -138,8 +137,8 @@ __device__ __forceinline__ void store_transposed_bf16(const f32x16 (&acc)[D / 32
 // dQ (and the (lse2, delta) pairs)
 // MASK as in the forward kernel;
 // G = query heads per kv head.  SPLIT: 64 query rows per workgroup, the two 32-key sub-tiles of a tile on two waves whose
-// dQ are added through LDS at the end (same use as in the forward kernel: launches with few tiles).  Not causal at D = 128, 39 to
-// 54 registers are too many for two waves a SIMD (160 to 220 bytes a lane in scratch memory; causal none).
+// dQ are added through LDS at the end (same use as in the forward kernel: launches with few tiles).  Not causal at D = 128, 41 to
+// 52 registers are too many for two waves a SIMD (168 to 212 bytes a lane in scratch memory; causal none).
 template <int D, bool CAUSAL, AttnMask MASK, bool SPLIT>
 __device__ __forceinline__ void bwd_dq(int block,
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kp, const uint16_t* __restrict__ Vp,
@@ -2180,7 +2179,7 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
         if (a1 != hipSuccess) return -1;                                                              \
         launch_kernel((flash_attn_bwd_dq_kernel<DD, CC, EE, SS>), grid_q, block, CfgQ<DD>::LDS, stream, \
                            Qp, Kp, Vp, Op, dOp, lse, static_cast<uint16_t*>(dq), st, BH, N, ntq, npad, \
-                           scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single, plan.keys == 256); \
+                           scale, scale_log2, Hq, G, window, kv_lens, key_mask, pair, single, plan.keys == 256 ? 3 : 0); \
     } while (0)
 #define TYR_FAB_DKV(DD, CC, EE, UU, PP)                                                               \
     do {                                                                                              \
