@@ -132,9 +132,12 @@ def test_tiles_of_twice_the_waves_where_they_are_faster(ask, M, N, K, trans_b, s
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,N,D,opt,form", [
-    (1, 32, 32, 315, 64, "0 0", "one"),         # two launches 17.2, one 14.4, 64-key tiles 15.4 us
-    (10, 32, 8, 222, 64, "0 0", "two"),         # 42.7, 53.1, 55.6
-    (9, 8, 8, 66, 64, "0 0", "one"),            # 11.6, 8.1, 10.4
+    (1, 32, 32, 315, 64, "0 0", "half"),        # two launches 16.9, one 14.0, 64-key tiles 11.3 us, two workgroups of which share a CU
+    (10, 32, 8, 222, 64, "0 0", "half"),        # 41.7, -, 35.3
+    (9, 8, 8, 66, 64, "0 0", "half"),           # 11.5, 8.3, 8.0
+    (1, 16, 4, 1042, 64, "0 0", "two"),         # 45.8, 55.8, 67.7
+    (2, 4, 4, 2129, 64, "0 0", "two"),          # 68.6, 81.1, 74.2: too many rows for two workgroups on a CU
+    (7, 8, 8, 143, 64, "0 0", "half"),          # 13.8, 11.4, 9.1: shared CUs in a launch of few more workgroups than CUs
     (1, 2, 2, 2001, 64, "1 0", "one"),          # 39.8, 31.3, 37.3
     (4, 8, 8, 310, 64, "1 0", "half"),          # 20.2, 16.1, 11.3
     (1, 1, 1, 128, 64, "0 0", "half"),          # the train step of one head

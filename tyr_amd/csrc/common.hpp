@@ -419,7 +419,7 @@ __device__ __forceinline__ TileSpan visible_tiles(const uint8_t* mask, int end, 
 // With grouped queries the unit dealt to an XCD is a (batch, kv head) group, whose G heads share one K / V.
 struct AttnOrder {
     int BH, Hq, G, ntr, single;                      // ntr = ranks per head
-    __device__ __forceinline__ void decode(int id, int& bh, int& rank, int& kvbh) const {
+    __host__ __device__ __forceinline__ void decode(int id, int& bh, int& rank, int& kvbh) const {
         const int ngroups = BH / G, hkv = Hq / G;
         if ((ngroups & 7) == 0) {
             const int xcd = id & 7, heads = BH >> 3;

@@ -1850,33 +1850,41 @@ size_t flash_attn_bwd_workspace_bytes(int B, int H, int N) {
 }
 
 namespace {
-// When the last of an XCD's 32 CUs is done, with workgroups of wg + step * steps.  The XCD gets every eighth workgroup of the launch
-// and deals them to its four engines of eight CUs in turn; the next one waits until the engine whose turn it is has a
-// free CU (fab::Parts::order).
-double last_cu(const fab::Parts& p, int ntk, int BHkv, double wg, double step) {
+// One of the eight XCDs, which are alike: it gets every eighth workgroup of a launch and deals them to its four engines of eight CUs
+// in turn; the next one waits until the engine whose turn it is has a free place (fab::Parts::order).
+struct Xcd {
+    int places;                                      // of an engine: 8, or 16 where two workgroups share a CU
+    double free_at[4][16] = {}, started = 0, last = 0;
+    int n = 0;
+    void run(double us) {
+        double* at = std::min_element(free_at[n & 3], free_at[n & 3] + places);
+        ++n;
+        started = std::max(started, *at);
+        *at = started + us;
+        last = std::max(last, *at);
+    }
+};
+// The steps of the dK / dV workgroups that go to the first XCD, in the launch's order (bwd_dkv).
+template <class F> void first_xcd_dkv(const fab::Parts& p, int ntk, int BHkv, F&& run) {
     const bool xcds = BHkv % 8 == 0;
     const int heads = xcds ? BHkv / 8 : BHkv, stride = xcds ? 1 : 8;
-    double busy[4][8] = {}, started = 0, last = 0;
-    int n = 0;
-    auto job = [&](int steps) {
-        double* cu = std::min_element(busy[n & 3], busy[n & 3] + 8);
-        ++n;
-        started = std::max(started, *cu);
-        *cu = started + wg + step * steps;
-        last = std::max(last, *cu);
-    };
     if (p.chunk) {
         for (int kt = 0, at = 0; kt < ntk; ++kt)
             for (const int end = at + p.parts(kt) * heads; at < end; ++at)
-                if (at % stride == 0) job(p.part_steps(kt));
+                if (at % stride == 0) run(p.part_steps(kt));
     } else {
         for (int at = 0; at < heads * ntk; at += stride) {
             int kt;
             p.order(at, heads, xcds, ntk, kt);
-            job(p.steps(kt));
+            run(p.steps(kt));
         }
     }
-    return last;
+}
+// When the last CU is done, with workgroups of wg + step * steps
+double last_cu(const fab::Parts& p, int ntk, int BHkv, double wg, double step) {
+    Xcd x{8};
+    first_xcd_dkv(p, ntk, BHkv, [&](int steps) { x.run(wg + step * steps); });
+    return x.last;
 }
 // traffic of the f32 partials, written and read at 6 TB/s
 double partial_us(const fab::Parts& p, int BHkv, int N, int D) {
@@ -1982,59 +1990,46 @@ size_t ds_bytes(int BH, int N, bool causal, int window) {
 // The four forms of a backward: dQ and dK/dV one after the other (seven products); in one launch; dK/dV leaving dS for dQ (five
 // products, three launches); in one launch with 64-key tiles.
 enum Form { TWO, ONE, DS, HALF, FORMS };
-// One of the eight XCDs, which are alike: 32 CUs that take every eighth workgroup of a launch, in its order, as they get free.
-struct Xcd {
-    double free_at[32], last = 0;
-    int64_t at = 0;
-    int busy = 0;
-    void run(double us, int64_t workgroups) {
-        auto later = [](double x, double y) { return x > y; };
-        int64_t mine = (at + workgroups + 7) / 8 - (at + 7) / 8;
-        for (at += workgroups; mine > 0; --mine) {
-            if (busy == 32) std::pop_heap(free_at, free_at + busy, later); else free_at[busy++] = 0;
-            last = std::max(last, free_at[busy - 1] += us);
-            std::push_heap(free_at, free_at + busy, later);
-        }
-    }
-};
 constexpr size_t kMostDs = (size_t)288 << 20;        // about the 256 MB last-level cache; with 331 MB B5 Hq8 Hkv2 N2724 300 -> 307 us
 int half_steps(int G, int N, bool causal, int window) {                 // of the longest 64-key tile
     const int nq = (N + 63) / 64;
     return G * (causal && window > 0 ? (int)std::min<int64_t>(nq, ((int64_t)window + 62) / 64 + 1) : nq);
 }
 // What each form takes, in microseconds on an MI355X: the workgroups' times (start and end, and a step: 64 queries x 64 or 128 keys)
-// dealt to the CUs in the launch's order, or the estimates that dQ's and dK/dV's own plans are chosen by, weighted as they
+// dealt to the CUs in the launch's order as an XCD deals them (Xcd), or the estimates that dQ's and dK/dV's own plans are chosen by, weighted as they
 // follow one another.  Steps take longer with all CUs busy (`crowd`) and with the mask instructions of a window (`edges`).
-// The constants are near what single workgroups measure and are fitted to make the choice, over 5100 shapes (heads 1 to 32, 64 to 8192
-// rows, every mask; graphs of 12 calls); a form's estimate is within 8 to 14 %.  On 3000 other shapes the form chosen is 0.5 %
-// slower than the best of the four.
+// The constants are near what single workgroups measure and are fitted to make the choice, over 3900 shapes (heads 1 to 32, 64 to 8192
+// rows, every mask; graphs of 12 calls); a form's estimate is within 8 to 11 %.  On 1000 other small launches the form chosen is 0.3 %
+// slower than the best of the four at D = 128 and 0.6 % at 64, at worst 21 % (B13 H16 N159 causal: 46 us with dS, 38 by 256-key tiles) and 17 %.
 // Examples, two / one / dS / half:  D = 128 B1 Hq32 Hkv8 N2000 149 / - / 137 / -, B2 H16 N483 full 36 / 28 / 33 / 34, B5 H8 N217 full 25
-// / 18 / 22 / 20, B2 H8 N685 40 / 38 / 32 / 27; D = 64 B1 H1 N128 10.5 / 7.7 / - / 6.3, B9 H8 N66 full 11.6 / 8.1 / - / 10.4, B10
-// Hq32 Hkv8 N222 full 43 / 53 / - / 56, B1 H2 N2001 40 / 31 / - / 37.
+// / 18 / 22 / 20, B2 H8 N685 40 / 38 / 32 / 27; D = 64 B1 H1 N128 11.4 / 8.3 / - / 6.6, B9 H8 N66 full 11.5 / 8.3 / - / 8.0, B10
+// Hq32 Hkv8 N222 full 42 / - / - / 35, B1 H32 N315 full 16.9 / 14.0 / - / 11.3, B1 Hq16 Hkv4 N1042 full 46 / 56 / - / 68, B1 H2 N2001 41 / 31 / - / 37.
 struct FormModel {
     double half, half_wg, half_step;                 // launch; dK/dV workgroup and step
     double dq_wg, dq_tile;                           // dQ's 64-row workgroups beside either
     double one, part_wg, part_step, sum, traffic;    // launch; dK/dV; the addition of parts and its partials
     double two, two_dq, two_dkv;
     double crowd, edges;
+    double beside;                                   // what a workgroup of HALF takes longer beside a second one on its CU
     double ds, ds_bytes, ds_dkv, ds_tile, ds_mean, ds_sum;      // launches; pairs, per MB of O and dO; dK/dV; product: longest, mean; parts
 };
-constexpr FormModel kModel128{3.1, 3.6, 1.86, 4.1, 0.87, 0.9, 8.4, 2.1, 2.6, 1.6, 6.5, 0.8, 1.31, 0.15, 1.28, 11.2, 0.36, 0.85, 0.23, 1.05, 1.8};
-constexpr FormModel kModel64{2.2, 2.6, 1.08, 2.9, 0.79, 1.5, 5.1, 1.87, 2.6, 0.9, 4.0, 1.06, 1.11, 0.12, 1.09, 0, 0, 0, 0, 0, 0};
-void launch_us(int BH, int BHkv, int N, int D, bool causal, int window, const DkvPlan& plan, double (&us)[FORMS]) {
-    const FormModel& m = D == 128 ? kModel128 : kModel64;
+constexpr FormModel kModel128{3.64, 3.15, 1.77, 3.96, 0.86, 0.544, 7.62, 2.26, 3.06, 1.48, 7, 0.687, 1.34, 0.152, 1.2, 0, 11.4, 0.291, 0.913, 0.215, 1.09, 0.074};
+constexpr FormModel kModel64{1.46, 3.28, 1.04, 2.79, 0.7, 2, 4.63, 1.83, 2.29, 1.14, 2.46, 1.07, 1.14, 0.0436, 1.13, 0.3, 0, 0, 0, 0, 0, 0};
+void launch_us(const FormModel& m, int BH, int BHkv, int N, int D, bool causal, int window, const DkvPlan& plan, double (&us)[FORMS]) {
     const int G = BH / BHkv, nq = (N + 63) / 64, ntk = (N + 127) / 128;
-    const bool edges = window > 0 && window < N, ordered = causal && window <= 0;
+    const bool edges = window > 0 && window < N;
     const int seen = window > 0 ? (int)std::min<int64_t>(nq, ((int64_t)window + 62) / 64 + 1) : nq;      // 64-key tiles of 64 queries
     const fab::Parts& p = plan.parts;
     auto step_scale = [&](int64_t workgroups) {
         return (1.0 + m.crowd * std::min(1.0, std::max(0.0, (workgroups - 200) / 400.0))) * (edges ? m.edges : 1.0);
     };
-    auto dq = [&](Xcd& x, double scale) {
-        // longest first over all heads, or head after head
-        for (int h = 0; h < (ordered || !causal ? 1 : BH); ++h)
-            for (int qt = nq; qt > 0; --qt)
-                x.run(m.dq_wg + m.dq_tile * scale * (causal ? std::min(qt, seen) : nq), ordered || !causal ? BH : 1);
+    auto dq = [&](Xcd& x, int64_t behind, double scale) {                 // dQ's workgroups behind so many others
+        const AttnOrder order{BH, G, G, nq, causal && window <= 0};
+        for (int id = (int)(-behind & 7); id < BH * nq; id += 8) {
+            int bh, rank, kvbh;
+            order.decode(id, bh, rank, kvbh);
+            x.run(m.dq_wg + m.dq_tile * scale * (causal ? std::min(nq - rank, seen) : nq));
+        }
     };
     us[TWO] = m.two + m.two_dq * attn_us(BH, N, D, causal, window, true) + m.two_dkv * plan.us;
     const double sum = p.chunk ? partial_us(p, BHkv, N, D) : 0.0;
@@ -2042,29 +2037,28 @@ void launch_us(int BH, int BHkv, int N, int D, bool causal, int window, const Dk
     int64_t items = 0;
     for (int kt = 0; kt < ntk; ++kt) items += p.parts(kt);
     const int64_t one = items * BHkv + (int64_t)BH * nq, half = (int64_t)(BHkv + BH) * nq;
-    if (one <= 1024) {                               // hardly ever the fastest beyond (2 of 1650 shapes)
-        Xcd x;
+    // Hardly ever the fastest beyond (2 of 1650 shapes); never with whole key tiles and no causal rule at D = 64, where 64-key ones share CUs
+    // or two launches do better (0 of 460; B2 H4 N2129 81 us, 69 in two launches)
+    if (one <= 1024 && (D == 128 || causal || p.chunk)) {
+        Xcd x{8};
         const double scale = step_scale(one), step = m.part_step * scale;
-        if (p.chunk) {
-            for (int kt = 0; kt < ntk; ++kt) x.run(m.part_wg + step * p.part_steps(kt), (int64_t)p.parts(kt) * BHkv);
-        } else {
-            const int heads = BHkv % 8 == 0 ? BHkv / 8 : BHkv;
-            for (int h = 0; h < heads; ++h)
-                for (int kt = 0; kt < ntk; ++kt) x.run(m.part_wg + step * p.steps(kt), BHkv / heads);
-        }
-        dq(x, scale);
+        first_xcd_dkv(p, ntk, BHkv, [&](int steps) { x.run(m.part_wg + step * steps); });
+        dq(x, items * BHkv, scale);
         us[ONE] = m.one + x.last + (p.chunk ? m.sum + m.traffic * sum : 0.0);
     }
-    if (half <= 1600 && half_lds(D, half_steps(G, N, causal, window), false) <= 160 * 1024) {
-        Xcd x;
-        const double scale = step_scale(half), step = m.half_step * (edges ? scale / m.edges : scale);       // its mask is always on
-        for (int kt = 0; kt < nq; ++kt)
-            x.run(m.half_wg + step * G * (std::min(nq, (window > 0 ? kt : 0) + seen) - (causal ? kt : 0)), BHkv);
-        dq(x, scale);
+    const size_t lds = half_lds(D, half_steps(G, N, causal, window), false);
+    if (half <= 1600 && lds <= 160 * 1024) {
+        const bool shared = D == 64 && lds <= 80 * 1024 && !kept_apart(G, N, causal, window, half);      // CUs, by two workgroups
+        Xcd x{shared ? 16 : 8};
+        const double beside = shared ? 1.0 + m.beside * std::min(1.0, std::max(0.0, (half - 256) / 256.0)) : 1.0;
+        const double scale = step_scale(half) * beside, step = m.half_step * (edges ? scale / m.edges : scale);       // its mask is always on
+        const int stride = BHkv % 8 ? 8 : 1, heads = BHkv / (8 / stride);
+        for (int at = 0; at < heads * nq; at += stride) {
+            const int kt = at / heads;
+            x.run(m.half_wg * beside + step * G * (std::min(nq, (window > 0 ? kt : 0) + seen) - (causal ? kt : 0)));
+        }
+        dq(x, (int64_t)BHkv * nq, scale);
         us[HALF] = m.half + x.last;
-        // two workgroups of it on a CU (half_lds).  Smaller launches would take it more often with this too (B1 H32 N315 not causal 14.0 us in
-        // one launch of 128-key tiles, 11.3), but their choice is kept.
-        if (D == 64 && half >= 384 && !kept_apart(G, N, causal, window, half) && half_lds(D, half_steps(G, N, causal, window), false) <= 80 * 1024) us[HALF] *= 0.72;
     }
     if (D == 128 && ntk > 1 && ds_bytes(BH, N, causal, window) <= kMostDs) {
         // product: stages of 32 keys, two workgroups a CU
@@ -2093,7 +2087,7 @@ Launches launches(int BH, int BHkv, int N, int D, bool causal, int window, bool 
         const DkvPlan plan = make_dkv_plan(BHkv, BH / BHkv, N, D, causal, window, cut_tiles);
         const double saved = wide_saves(BHkv, BH / BHkv, N, D, causal, window, plan);
         e = {BH, BHkv, N, D, causal, window, cut_tiles, {plan.parts, saved > 0, {}}};
-        launch_us(BH, BHkv, N, D, causal, window, plan, e.how.us);
+        launch_us(D == 128 ? kModel128 : kModel64, BH, BHkv, N, D, causal, window, plan, e.how.us);
         e.how.us[TWO] -= std::max(0.0, saved);
     }
     return e.how;
@@ -2242,7 +2236,10 @@ int launch_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     do {                                                                                              \
         if (how.both) {                                                                               \
             if (how.half) { TYR_FAB_BOTH(DD, CC, EE, false, true); break; }                           \
-            if (!plan.chunk) { TYR_FAB_BOTH(DD, CC, EE, false, false); break; }                       \
+            if (!plan.chunk) {                                                                        \
+                if constexpr (DD == 128 || CC) TYR_FAB_BOTH(DD, CC, EE, false, false);                \
+                break;                                                                                \
+            }                                                                                         \
             TYR_FAB_BOTH(DD, CC, EE, true, false);                                                    \
             TYR_FAB_SUM(DD);                                                                          \
             break;                                                                                    \
