@@ -1,11 +1,12 @@
 """What the gfx950 assembly of the attention backward has to show (compiled here, no GPU needed).
 
 Wait states around the matrix products that flash_attn_bwd_dkv_wide_kernel issues in asm, where the compiler, which puts
-them in for its own products, does not see any.  Every product of those kernels is checked against the instructions around it,
-with the body of every loop entered twice:
+them in for its own products, does not see any.  Every product of those kernels is checked against the instructions around it
+on every path, over forward and backward branches:
   * no operand is written by an ordinary vector instruction less than 2 wait states before the product,
   * no result is read or written by another kind of instruction less than 8 (16x16x32) or 12 (32x32x16) wait states behind it,
-  * no accumulator operand of a product in flight is written.
+  * no accumulator operand of a product in flight is written,
+  * no product starts from a part of another's result, or from one of another kind, in that time.
 An instruction is one wait state, s_nop n is n + 1.
 
 Scalar offsets of the requests of query tiles: at most the size of the buffer, which is what their range check is known for.
@@ -42,50 +43,99 @@ def operands(line):
     return name, [o for o in ops + [cur.strip()] if o]
 
 
-def straight(lines):
-    """Instructions with every backward branch taken once more."""
-    at = {m.group(1): i for i, l in enumerate(lines) if (m := re.match(r"(\.L\w+):", l))}
-    out = []
-    for i, l in enumerate(lines):
-        if not l.endswith(":"):
-            out.append(l)
-        m = re.match(r"s_c?branch\S*\s+(\.L\w+)", l)
-        if m and at.get(m.group(1), i + 1) <= i:
-            out += [x for x in lines[at[m.group(1)]:i + 1] if not x.endswith(":")]
-    return out
+class Flight:
+    """What may still be under way at a point: register -> wait states that are left, for ordinary writes, results of products (with the
+    product's whole result and kind) and accumulators that products read."""
 
+    def __init__(self):
+        self.written, self.results, self.sources = {}, {}, {}
 
-def violations(code):
-    bad, now = [], 0
-    vector_write, result, source = {}, {}, {}     # register -> wait state of its last write; (wait state, needed) of a product's result, operand
-    for line in code:
+    def merge(self, other):
+        """Takes over what is longer under way in `other`; whether anything was."""
+        grown = False
+        for mine, theirs in ((self.written, other.written), (self.results, other.results), (self.sources, other.sources)):
+            for r, x in theirs.items():
+                have = mine.get(r, (0, *x[1:]))
+                joined = (max(have[0], x[0]), *(p if p == q else None for p, q in zip(have[1:], x[1:])))
+                if mine.get(r) != joined:
+                    mine[r] = joined
+                    grown = True
+        return grown
+
+    def copy(self):
+        out = Flight()
+        out.written, out.results, out.sources = dict(self.written), dict(self.results), dict(self.sources)
+        return out
+
+    def passes(self, states):
+        for d in (self.written, self.results, self.sources):
+            for r in [r for r, x in d.items() if x[0] <= states]:
+                del d[r]
+            for r, x in d.items():
+                d[r] = (x[0] - states, *x[1:])
+
+    def step(self, line):
+        """One instruction; whether it came too early."""
         name, ops = operands(line)
         if name == "s_nop":
-            now += int(ops[0], 0) + 1
-            continue
-        now += 1
+            self.passes(int(ops[0], 0) + 1)
+            return False
         if name.startswith("v_mfma"):
             need = 12 if "32x32" in name else 8
             dst, a, b, c = (registers(o) for o in ops[:4])
-            bad += [line for r in a | b | c if now - vector_write.get(r, -99) <= 2]
-            bad += [line for r in (a | b) & result.keys() if now - result[r][0] <= result[r][1]]
+            bad = any(r in self.written for r in a | b | c) or any(r in self.results for r in a | b)
+            # a product in flight hands its result on to the accumulator of one like it, as a whole
+            bad |= any(self.results[r][1:] != (frozenset(x), name[:12]) for x in (dst, c) for r in x if r in self.results)
+            self.passes(1)
             for r in dst:
-                result[r] = (now, need)
+                self.results[r] = (need, frozenset(dst), name[:12])
             for r in c:
-                source[r] = (now, need)
-            continue
+                self.sources[r] = (need,)
+            return bad
         used = registers(" ".join(ops))
-        bad += [line for r in used & result.keys() if now - result[r][0] <= result[r][1]]
         stores = name.startswith(("global_store", "buffer_", "ds_write", "scratch_store", "s_"))
-        written = set() if stores or not ops else registers(ops[0]) | (registers(ops[1]) if "swap" in name else set())
-        bad += [line for r in written & source.keys() if now - source[r][0] <= source[r][1]]
-        for r in written:
-            result.pop(r, None)
+        writes = set() if stores or not ops else registers(ops[0]) | (registers(ops[1]) if "swap" in name else set())
+        bad = any(r in self.results for r in used) or any(r in self.sources for r in writes)
+        self.passes(1)
+        for r in writes:
+            self.results.pop(r, None)
+            self.written.pop(r, None)
             if name.startswith("v_"):
-                vector_write[r] = now
-            else:
-                vector_write.pop(r, None)
-    return bad
+                self.written[r] = (2,)
+        return bad
+
+
+def violations(lines):
+    """Instructions that come too early on some path: every branch is followed, taken and not, until nothing new is under way."""
+    at = {m.group(1): i for i, l in enumerate(lines) if (m := re.match(r"(\.?\w+):", l))}
+    before = {0: Flight()}
+    todo, bad = [0], set()
+    while todo:
+        i = todo.pop()
+        state = before[i].copy()
+        while i < len(lines):
+            line = lines[i]
+            if not line.endswith(":"):
+                if state.step(line):
+                    bad.add(i)
+                m = re.match(r"s_(c?)branch\S*\s+(\S+)", line)
+                if m:
+                    goal = at[m.group(2)]
+                    if goal not in before:
+                        before[goal] = state.copy()
+                        todo.append(goal)
+                    elif before[goal].merge(state):
+                        todo.append(goal)
+                    if not m.group(1):
+                        break
+                if line.startswith("s_endpgm"):
+                    break
+            elif i in before:                        # a label that is reached from above too
+                if before[i].merge(state):
+                    todo.append(i)
+                state = before[i].copy()
+            i += 1
+    return [lines[i] for i in sorted(bad)]
 
 
 def wide_kernels(path):
@@ -111,7 +161,7 @@ def test_products_in_asm_keep_their_distance(listing):
     assert kernels
     for name, lines in kernels.items():
         assert sum(l.startswith("v_mfma") for l in lines) >= 96, name
-        assert violations(straight(lines)) == [], name
+        assert violations(lines) == [], name
 
 
 def unbounded_requests(code):
@@ -165,5 +215,22 @@ def test_what_comes_too_early_is_found():
     assert violations([mfma, "s_nop 6", "v_mul_f32 v20, v1, v1"]) and not violations([mfma, "s_nop 7", "v_mul_f32 v20, v1, v1"])
     assert violations([mfma, "ds_read_b128 v[0:3], v30"]) and not violations([mfma, mfma])
     acc = "v_mfma_f32_32x32x16_bf16 a[0:15], v[4:7], v[8:11], a[0:15]"
-    assert violations([acc, "s_nop 7", "v_accvgpr_read_b32 v20, a3"])
-    assert violations(straight([".LBB0_1:", "v_mul_f32 v20, v1, v1", mfma, "s_cbranch_scc1 .LBB0_1"]))
+    assert violations([acc, "s_nop 10", "v_accvgpr_read_b32 v20, a3"]) and not violations([acc, "s_nop 11", "v_accvgpr_read_b32 v20, a3"])
+    assert violations([mfma, "v_mfma_f32_16x16x32_bf16 v[2:5], v[12:15], v[8:11], v[2:5]"])          # overlaps a result in flight
+    assert violations([mfma, "v_mfma_f32_32x32x16_bf16 v[16:31], v[4:7], v[8:11], v[0:15]"])         # another kind of product
+
+
+def test_every_branch_is_followed():
+    mfma, use, nop = "v_mfma_f32_16x16x32_bf16 v[0:3], v[4:7], v[8:11], v[0:3]", "v_mul_f32 v20, v1, v1", "s_nop 7"
+    # a loop: the product at its end, the use at its start
+    assert violations([".LBB0_1:", use, mfma, "s_cbranch_scc1 .LBB0_1", "s_endpgm"])
+    assert not violations([".LBB0_1:", use, mfma, nop, "s_cbranch_scc1 .LBB0_1", "s_endpgm"])
+    # a block out of line, behind the kernel's end: from the branch into it, and back
+    away = [mfma, "s_cbranch_scc1 .LBB0_2", nop, ".LBB0_1:", "s_endpgm", ".LBB0_2:"]
+    assert violations(away + [use, "s_branch .LBB0_1"])
+    assert not violations(away + [nop, use, "s_branch .LBB0_1"])
+    back = ["s_cbranch_scc1 .LBB0_2", ".LBB0_1:", mfma, "s_endpgm", ".LBB0_2:"]
+    assert violations(back + ["v_mov_b32 v4, 0", "s_branch .LBB0_1"])
+    assert not violations(back + ["v_mov_b32 v4, 0", "s_nop 0", "s_branch .LBB0_1"])
+    # a block skipped: the use behind it
+    assert violations([mfma, "s_cbranch_execz .LBB0_1", nop, ".LBB0_1:", use, "s_endpgm"])

@@ -46,8 +46,8 @@ __device__ __forceinline__ f32x16 mfma_32x32x16_bf16(bf16x8 a, bf16x8 b, f32x16 
 }
 // Products in asm, for a kernel that fills the register file and says which half of it a result lives in: acc = accumulation
 // registers, vgpr = ordinary ones (begin: the accumulator starts from 0 or c).  The compiler does not see a product in the asm, so
-// the caller keeps two wait states between an ordinary write of a, b or c and the product, and between the product and an ordinary read of
-// its result 19 (32x32x16) or 9 (16x16x32); products in between count.
+// the caller keeps two wait states between an ordinary write of a, b or c and the product, and between the product and any other instruction
+// on its result 12 (32x32x16) or 8 (16x16x32), as the compiler does behind its own; products in between count.
 __device__ __forceinline__ void mfma_32x32x16_bf16_acc(f32x16& c, bf16x8 a, bf16x8 b) {
     asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
