@@ -5,6 +5,7 @@
 //                                             0 = null, any = TYR_HIP_ANY_ORDER; its scratch follows the status
 //   kernels                                   every kernel of the files linked
 //   bwd   B Hq Hkv N D causal window mask ws  status, then "kernel<arguments>:workgroups" each; mask = none | lens | keys
+//   bwd_lds, the same                         "kernel<arguments>:workgroups:bytes of LDS"
 #include <cxxabi.h>
 #include <hip/hip_runtime_api.h>
 
@@ -22,6 +23,7 @@ static std::map<const void*, std::string>& kernels() {
     return m;
 }
 static std::string launched;
+static bool with_lds;
 
 extern "C" {
 void** __hipRegisterFatBinary(const void*) { return nullptr; }
@@ -41,7 +43,7 @@ hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipS
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t lds, hipStream_t) {
     if (lds > 160 * 1024 || grid.x == 0 || grid.x > 0x7fffffffu || block.x > 1024) abort();
-    launched += " " + kernels()[f] + ":" + std::to_string(grid.x);
+    launched += " " + kernels()[f] + ":" + std::to_string(grid.x) + (with_lds ? ":" + std::to_string(lds) : "");
     return hipSuccess;
 }
 }
@@ -78,6 +80,7 @@ int main() {
         }
         in >> B >> Hq >> Hkv >> N >> D >> causal >> window >> mask >> ws;
         launched.clear();
+        with_lds = what == "bwd_lds";
         if (what == "bytes") {
             printf("%zu %zu %zu\n", tyr_hip_flash_attn_bwd_workspace_bytes(B, Hq, N, D),
                    tyr_hip_flash_attn_bwd_parts_workspace_bytes(B, Hq, Hkv, N, D, causal, window),

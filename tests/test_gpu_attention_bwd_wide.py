@@ -20,20 +20,30 @@ def reference(q, k, v, g, visible):
     return ds @ k, sum(d.T @ x for d, x in zip(ds, q)), sum(d.T @ x for d, x in zip(p, g))
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal,mask,window", [
+FIELDS = "B,Hq,Hkv,N,D,causal,mask,window"
+# test_host_launches checks that these take the kernels they are here for
+WIDE = [
     (16, 32, 8, 1025, 128, True, None, 0), (16, 32, 8, 1279, 128, True, None, 0), (16, 32, 32, 960, 128, True, None, 0),
     (16, 32, 8, 513, 64, True, None, 0), (16, 32, 32, 768, 64, True, None, 0),
     (16, 32, 8, 449, 128, False, None, 0), (16, 32, 8, 512, 128, False, None, 0), (17, 12, 4, 513, 64, False, None, 0),
     (16, 32, 8, 1100, 128, True, "lens", 0), (17, 12, 4, 600, 64, False, "lens", 0), (16, 32, 8, 500, 128, False, "lens", 0),
     (16, 32, 8, 1100, 128, True, "keys", 0), (17, 12, 4, 600, 64, False, "keys", 0), (16, 32, 8, 700, 64, True, "keys", 0),
-    (16, 32, 8, 1216, 128, True, None, 600), (16, 32, 8, 1153, 128, True, "lens", 600)])
+    (16, 32, 8, 1216, 128, True, None, 600), (16, 32, 8, 1153, 128, True, "lens", 600),
+    # causal, kv heads that are no multiple of the XCDs (60, 90, 44), or no multiple of eight on each (14, 15): the order's last group of
+    # heads is a part of one
+    (15, 12, 4, 1160, 128, True, None, 0), (15, 18, 6, 929, 128, True, "keys", 0), (11, 12, 4, 1400, 64, True, None, 0),
+    (14, 32, 8, 681, 128, True, "lens", 0), (15, 16, 8, 1100, 64, True, None, 0)]
+TWO_A_CU = [
+    (16, 8, 8, 130, 64, False, None, 0), (6, 8, 8, 320, 64, False, "lens", 0), (8, 16, 4, 385, 64, False, "keys", 0),
+    (3, 16, 16, 283, 64, True, None, 70), (5, 16, 4, 511, 64, True, "lens", 100), (2, 4, 4, 1400, 64, True, None, 129)]
+
+
+@pytest.mark.parametrize(FIELDS, WIDE)
 def test_wide_key_tiles_match_float64(B, Hq, Hkv, N, D, causal, mask, window):
     compare(B, Hq, Hkv, N, D, causal, mask, window)
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal,mask,window", [
-    (16, 8, 8, 130, 64, False, None, 0), (6, 8, 8, 320, 64, False, "lens", 0), (8, 16, 4, 385, 64, False, "keys", 0),
-    (3, 16, 16, 283, 64, True, None, 70), (5, 16, 4, 511, 64, True, "lens", 100), (2, 4, 4, 1400, 64, True, None, 129)])
+@pytest.mark.parametrize(FIELDS, TWO_A_CU)
 def test_two_workgroups_of_64_key_tiles_on_a_cu(B, Hq, Hkv, N, D, causal, mask, window):
     compare(B, Hq, Hkv, N, D, causal, mask, window)
 

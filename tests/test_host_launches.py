@@ -7,6 +7,8 @@ from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 
+from tests.test_gpu_attention_bwd_wide import TWO_A_CU, WIDE
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CHECKED = ["-Xarch_host", "-fsanitize=signed-integer-overflow", "-Xarch_host", "-fsanitize-minimal-runtime", "-Xarch_host",
            "-fno-sanitize-recover=signed-integer-overflow"]
@@ -154,3 +156,18 @@ def test_the_form_of_a_backward_is_the_fastest(ask, B, Hq, Hkv, N, D, opt, form)
     first = got.split()[1]
     kind = {"flash_attn_bwd_dq_kernel": "two", "flash_attn_bwd_stats_kernel": "ds", "flash_attn_bwd_both_kernel": "half" if first.split(":")[0].endswith("true>") else "one"}
     assert kind[first.split("<")[0]] == form, got
+
+
+def test_the_shapes_of_the_wide_tests_take_their_kernels(ask):
+    """dK / dV by key tiles of 256, or one launch of 64-key tiles that leaves a CU (160 KB of LDS, 256 CUs) room for two of more workgroups
+    than CUs: what tests/test_gpu_attention_bwd_wide.py compares has to run them."""
+    def launches(B, Hq, Hkv, N, D, causal, mask, window):
+        got, = ask([f"bwd_lds {B} {Hq} {Hkv} {N} {D} {int(causal)} {window} {mask or 'none'} {1 << 40}"])
+        return [k.rsplit(":", 2) for k in got.split()[1:]]
+    for row in WIDE:
+        (first, _, _), (second, grid, _) = launches(*row)
+        assert first.startswith("flash_attn_bwd_dq_kernel<") and second.startswith("flash_attn_bwd_dkv_wide_kernel<"), row
+        assert int(grid) == row[0] * row[2] * -(-row[3] // 256), row
+    for row in TWO_A_CU:
+        (only, grid, lds), = launches(*row)
+        assert re.fullmatch(r"flash_attn_bwd_both_kernel<64,.*,true>", only) and int(grid) > 256 and 2 * int(lds) <= 160 * 1024, (row, only, lds)
